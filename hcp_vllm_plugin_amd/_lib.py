@@ -53,6 +53,10 @@ EXPORTED_SYMBOLS = (
     "hcp_plan_varlen_tiles",
     "hcp_attn_fwd_varlen",
     "hcp_attn_fwd_varlen_merge",
+    "hcp_plan_fwd_split",
+    "hcp_attn_fwd_lse_split",
+    "hcp_plan_varlen_split",
+    "hcp_attn_fwd_varlen_split",
     "hcp_plan_decode_splits",
     "hcp_decode_workspace_bytes",
     "hcp_decode_splitkv",
@@ -63,7 +67,7 @@ EXPORTED_SYMBOLS = (
     "hcp_gather_paged_kv",
 )
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 
 class KvSegment(ctypes.Structure):
@@ -160,6 +164,25 @@ def _declare(lib: ctypes.CDLL) -> None:
         _P, _I64, _I64, _P, _I64, _I64, _P, _I64,
         _P, _I32, _P, _I32, _I32, _I32, _I32, _F, _I32, _I32, _I32,
         _P, _I64, _I64, _P, _I64, _I32, _I32, _P,
+    ]
+    lib.hcp_plan_fwd_split.restype = ctypes.c_int
+    lib.hcp_plan_fwd_split.argtypes = [_I64, _I64, _I32, _I32, _I32, _I32, _I64, _I32, _P, _P]
+    lib.hcp_attn_fwd_lse_split.restype = ctypes.c_int
+    lib.hcp_attn_fwd_lse_split.argtypes = [
+        _P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32,
+        _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+        _F, _I32, _I64, _I32, _P, _I64, _I64, _P, _I64, _I32,
+        _I32, _I32, _P, ctypes.c_size_t, _I32, _P,
+    ]
+    lib.hcp_plan_varlen_split.restype = ctypes.c_int
+    lib.hcp_plan_varlen_split.argtypes = [
+        _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P, _P, _P, _P, _P,
+    ]
+    lib.hcp_attn_fwd_varlen_split.restype = ctypes.c_int
+    lib.hcp_attn_fwd_varlen_split.argtypes = [
+        _P, _I64, _I64, _P, _I64, _I64, _P, _I64,
+        _P, _I32, _P, _I32, _I32, _P, _I32, _I32, _I32, _I32, _I32, _F, _I32, _I32, _I32,
+        _P, _I64, _I64, _P, _I64, _I32, _P, ctypes.c_size_t, _I32, _P,
     ]
     lib.hcp_plan_decode_splits.restype = ctypes.c_int
     lib.hcp_plan_decode_splits.argtypes = [_P, _I32, _P, _I32, _I32, _I32, _P, _I32, _P]

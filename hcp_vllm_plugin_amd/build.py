@@ -11,19 +11,30 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 OUT = os.path.join(HERE, "libhcp_mi355x.so")
 
-SOURCES = ["abi.hip", "attn_fwd.hip", "decode.hip", "merge.hip", "cache.hip"]
+# (source, extra flags) of each object: the prefill kernels once per column
+# width, so that their instantiations compile side by side
+OBJECTS = [
+    ("attn_fwd.hip", ["-DHCP_FWD_D=128"]),
+    ("attn_fwd.hip", ["-DHCP_FWD_D=256"]),
+    ("attn_fwd.hip", ["-DHCP_FWD_D=64"]),
+    ("decode.hip", []),
+    ("abi.hip", []),
+    ("merge.hip", []),
+    ("cache.hip", []),
+]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
     "-std=c++17",
-    "-shared",
     "-fPIC",
     # packed-FP32 VALU forms are kept out of the generated code on purpose
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -43,23 +54,31 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
-def build(verbose: bool = False) -> str:
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    tmp = OUT + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, "-I", os.path.join(ROOT, "include"), *srcs,
-           "-Wl,-rpath,/opt/rocm/lib", "-o", tmp]
+def _run(cmd: list[str], verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     # hipcc's host pass does not know the GPU-only feature flag; drop that noise
-    err = "\n".join(
-        ln for ln in res.stderr.splitlines() if "packed-fp32-ops" not in ln
-    )
+    err = "\n".join(ln for ln in res.stderr.splitlines() if "packed-fp32-ops" not in ln)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
-    os.replace(tmp, OUT)
+
+
+def build(verbose: bool = False) -> str:
+    cc = hipcc()
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(os.cpu_count() or 1) as pool:
+        objs = [os.path.join(tmp, f"{i}.o") for i in range(len(OBJECTS))]
+        jobs = [pool.submit(_run, [cc, *HIPCC_FLAGS, *flags, "-I", os.path.join(ROOT, "include"),
+                                   "-c", os.path.join(CSRC, src), "-o", obj], verbose)
+                for (src, flags), obj in zip(OBJECTS, objs)]
+        for j in jobs:
+            j.result()
+        lib = OUT + ".tmp"
+        _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs,
+              "-Wl,-rpath,/opt/rocm/lib", "-o", lib], verbose)
+    os.replace(lib, OUT)
     return OUT
 
 

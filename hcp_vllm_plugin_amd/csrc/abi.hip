@@ -5,7 +5,9 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <functional>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <vector>
 
@@ -91,6 +93,160 @@ void set_acc(hcp::FwdParams& p, const AccArgs* a) {
   p.acc_prefix = a->prefix != 0;
 }
 
+// ---- KV split of a prefill launch ------------------------------------------
+constexpr int kNumCus = 256;
+constexpr int kMaxPieces = 4096;    // (query block, head, piece) workgroups of a split launch
+constexpr int kMaxUnits = 4 * kNumCus;  // (query block, head) pairs of a launch worth cutting
+constexpr int kMinPieceTiles = 4;   // a shorter piece is mostly prologue and epilogue
+
+// A query block of a launch: its tiles and how many of the workgroup's four
+// waves have query rows.
+struct Unit {
+  int tiles, waves;
+};
+// How a launch is cut: blocks of more than `tiles` tiles into pieces, except
+// the `whole` longest.
+struct Cut {
+  int tiles = 0, whole = 0;
+};
+
+// Estimated time (us) of a launch over `units` (per head, longest first) cut
+// as `c`: the workgroups, longest first, go to the least loaded CU of one XCD
+// (all XCDs get the same mix).  A CU runs one tile (128 rows x 64 keys) per
+// tile_us whether one or two workgroups share it, so the machine counts as
+// 256 slots; one alone takes about 15% longer per tile, and two with one wave
+// of rows each run side by side.  Constants from measured launches (us):
+// 512 x 32768 at 28 / 4 x 128 whole 490, cut in 2 / 4 / 9 / 16: 311 / 256 /
+// 241 / 254 (estimated 307 / 265 / 247 / 257); 512 x 4096 whole 66, cut in 2 /
+// 8 / 16: 47 / 55 / 70 (47 / 56 / 68); 3001 x 5003 at 14 / 2 x 64 whole 90,
+// cut in 2 / 3: 86 / 81 (82 / 79).
+double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh, int dw,
+                  double limit) {
+  const double tile_us = dw == 64 ? 0.54 : dw == 128 ? 0.97 : 1.75;
+  const double start_us = dw == 256 ? 5.0 : 1.5;  // per workgroup
+  const double part_us = dw == 64 ? 0.006 : dw == 128 ? 0.012 : 0.04;  // per partial
+  const double reduce_us = dw == 256 ? 8.0 : 6.0;  // the second launch
+  // by waves with rows: two workgroups on a CU / one alone
+  static constexpr double kShared[5] = {0.5, 0.5, 0.65, 0.85, 1.0};
+  static constexpr double kAlone[5] = {0.9, 0.9, 1.0, 1.08, 1.15};
+  // one XCD's share of the workgroups (xcd_remap), or the whole machine
+  const bool by_xcd = num_kvh <= hcp::kNumXcd && hcp::kNumXcd % num_kvh == 0;
+  const int share = by_xcd ? hcp::kNumXcd / num_kvh : 1;
+  const int cus = by_xcd ? kNumCus / hcp::kNumXcd : kNumCus;
+  const int64_t per = static_cast<int64_t>(group) * (by_xcd ? 1 : num_kvh);
+  auto pieces = [&](size_t u) {
+    return c.tiles > 0 && static_cast<int>(u) >= c.whole ? hcp::unit_pieces(units[u].tiles, c.tiles)
+                                                         : 1;
+  };
+  int64_t n = 0, parts = 0;
+  for (size_t u = 0; u < units.size(); ++u) {
+    n += pieces(u);
+    if (pieces(u) > 1) parts += pieces(u);
+  }
+  if (c.tiles > 0 && n * group * num_kvh > kMaxPieces) return 1e30;
+  const bool alone = dw < 256 && n * per <= static_cast<int64_t>(cus) * share;
+  const double merge_us =
+      parts > 0 ? reduce_us + static_cast<double>(parts) * group * num_kvh * part_us : 0.0;
+  std::vector<double> sz;  // workgroup times of one head
+  double sum = 0;
+  for (size_t u = 0; u < units.size(); ++u) {
+    const int nt = units[u].tiles, np = pieces(u);
+    const double t = tile_us * (alone ? kAlone : kShared)[units[u].waves];
+    sum += nt * t + np * start_us;
+    for (int i = 0; i < np; ++i)
+      sz.push_back((hcp::piece_begin(nt, np, i + 1) - hcp::piece_begin(nt, np, i)) * t);
+  }
+  // evenly spread at best: not worth simulating when that already loses
+  const double even = 4.0 - start_us + sum * per / (static_cast<double>(cus) * share) + merge_us;
+  if (even >= limit) return even;
+  std::sort(sz.begin(), sz.end(), std::greater<double>());
+  std::vector<double> load(cus, 4.0 - start_us);  // min-heap
+  auto gt = std::greater<double>();
+  for (int64_t j = 0; j < n * per; j += share) {
+    std::pop_heap(load.begin(), load.end(), gt);
+    load.back() += sz[j / per] + start_us;
+    std::push_heap(load.begin(), load.end(), gt);
+  }
+  return *std::max_element(load.begin(), load.end()) + merge_us;
+}
+
+// The cut of a launch over `units`, longest first; tiles 0 when cutting does
+// not pay (6% or more by the estimate).
+Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw) {
+  Cut best;
+  const int heads = group * num_kvh;
+  // past 4 workgroups per CU the dispatch order alone evens the load out to
+  // what the partials of a cut would cost
+  if (units.empty() || static_cast<int64_t>(units.size()) * heads > kMaxUnits) return best;
+  const int mx = units[0].tiles;
+  if (mx < 2 * kMinPieceTiles) return best;
+  double t_best = split_cost(units, best, group, num_kvh, dw, 1e30) * 0.94;
+  // whole blocks spread evenly as they are: no cut can win
+  if (split_cost(units, best, group, num_kvh, dw, 0.0) >= t_best) return best;
+  for (int rounds = 0; rounds < 4; ++rounds) {
+    // rounds > 0: only what is left after `rounds` whole blocks per CU
+    Cut c;
+    c.whole = kNumCus * rounds / heads;
+    if (rounds > 0 && (c.whole == 0 || c.whole >= static_cast<int>(units.size()))) break;
+    const int top = units[c.whole].tiles;
+    for (int k : {2, 3, 4, 5, 6, 8, 9, 12, 16, 20, 24, 32, 40, 48, 64}) {
+      const int tiles = (top + k - 1) / k;
+      if (tiles < kMinPieceTiles) break;
+      if (tiles == c.tiles) continue;
+      c.tiles = tiles;
+      const double t = split_cost(units, c, group, num_kvh, dw, t_best);
+      if (t > 1e29) break;
+      if (t < t_best) {
+        t_best = t;
+        best = c;
+      }
+    }
+  }
+  return best;
+}
+
+int unit_waves(const hcp_varlen_entry& e, int64_t qb) {
+  const int64_t rows = e.q_len - qb * hcp::kFwdBM;
+  return rows >= hcp::kFwdBM ? hcp::kFwdBM / 32 : static_cast<int>((rows + 31) / 32);
+}
+
+int unit_tiles(const hcp_varlen_entry& e, int64_t qb, bool causal, int32_t window) {
+  const int64_t n = hcp::unit_keys(e.kv.len, e.causal_offset, qb, causal, window).n;
+  return static_cast<int>((n + hcp::kFwdBN - 1) / hcp::kFwdBN);
+}
+
+// (O, LSE) partials of `slots` query blocks x num_heads, fp32
+size_t split_ws_o_bytes(int64_t slots, int32_t num_heads, int32_t head_dim) {
+  return static_cast<size_t>(slots) * num_heads * hcp::kFwdBM * hcp::padded_head_dim(head_dim) *
+         sizeof(float);
+}
+size_t split_ws_bytes(int64_t slots, int32_t num_heads, int32_t head_dim) {
+  return split_ws_o_bytes(slots, num_heads, head_dim) +
+         static_cast<size_t>(slots) * num_heads * hcp::kFwdBM * sizeof(float);
+}
+
+// Workspace of a split launch into p; `slots` partials per head.
+int set_split(hcp::FwdParams& p, int32_t piece_tiles, int64_t slots, void* ws, size_t bytes,
+              const char* who) {
+  const size_t need = split_ws_bytes(slots, p.num_heads, p.head_dim);
+  if (!ws || bytes < need)
+    return fail(HCP_EWORKSPACE, "%s: workspace %zu bytes < %zu needed", who, bytes, need);
+  if (!aligned16(ws)) return fail(HCP_EINVAL, "%s: workspace not 16-byte aligned", who);
+  p.piece_tiles = piece_tiles;
+  p.ws_o = static_cast<float*>(ws);
+  p.ws_lse = reinterpret_cast<float*>(static_cast<char*>(ws) +
+                                      split_ws_o_bytes(slots, p.num_heads, p.head_dim));
+  return HCP_OK;
+}
+
+struct SplitArgs {
+  int32_t piece_tiles, whole_blocks;
+  void* ws;
+  size_t bytes;
+  const int32_t* units;  // varlen only
+  int32_t num_units, num_slots;
+};
+
 }  // namespace
 
 extern "C" {
@@ -106,7 +262,7 @@ static int fwd_lse_impl(const char* who, const void* q, const void* k, const voi
                         int64_t v_stride_tok, int64_t v_stride_head, int64_t o_stride_tok,
                         int64_t o_stride_head, int64_t lse_stride_head, float scale,
                         int32_t causal, int64_t causal_offset, int32_t window, int32_t dtype,
-                        void* stream, const AccArgs* acc) {
+                        void* stream, const AccArgs* acc, const SplitArgs* split = nullptr) {
   int rc = check_heads(num_heads, num_kv_heads, head_dim, dtype, who);
   if (rc) return rc;
   if (tq < 0 || tk < 0) return fail(HCP_EINVAL, "%s: negative tq/tk", who);
@@ -157,9 +313,85 @@ static int fwd_lse_impl(const char* who, const void* q, const void* k, const voi
   if (tk > 1 && (k_stride_tok <= 0 || k_stride_tok >= (int64_t{1} << 24)))
     return fail(HCP_EUNSUPPORTED, "%s: k/v token stride must be in (0, 2^24) elements", who);
   set_acc(p, acc);
+  if (split) {
+    if (split->whole_blocks < 0 || split->whole_blocks >= p.num_tiles)
+      return fail(HCP_EINVAL, "%s: whole_blocks %d of %d", who, split->whole_blocks, p.num_tiles);
+    // blocks in dispatch order: the last one first under a causal mask
+    int mp = 1;
+    for (int64_t t = split->whole_blocks; t < p.num_tiles; ++t)
+      mp = std::max(mp, hcp::unit_pieces(unit_tiles(p.single, causal ? p.num_tiles - 1 - t : t,
+                                                    causal != 0, p.window),
+                                         split->piece_tiles));
+    const int64_t slots = static_cast<int64_t>(p.num_tiles - split->whole_blocks) * mp;
+    if (slots * num_heads * 4 > INT32_MAX)
+      return fail(HCP_EINVAL, "%s: too many pieces", who);
+    p.whole_tiles = split->whole_blocks;
+    p.max_pieces = mp;
+    if ((rc = set_split(p, split->piece_tiles, slots, split->ws, split->bytes, who))) return rc;
+  }
   hipError_t e = hcp::launch_fwd(p, head_dim, dtype, causal != 0, false, false,
                                  static_cast<hipStream_t>(stream));
   return launch_status(e, who);
+}
+
+int hcp_plan_fwd_split(int64_t tq, int64_t tk, int32_t num_heads, int32_t num_kv_heads,
+                       int32_t head_dim, int32_t causal, int64_t causal_offset, int32_t window,
+                       int32_t* whole_blocks, size_t* workspace_bytes) try {
+  const char* who = "hcp_plan_fwd_split";
+  int rc = check_heads(num_heads, num_kv_heads, head_dim, HCP_DTYPE_BF16, who);
+  if (rc) return rc;
+  if (tq < 0 || tk < 0 || window < 0 || !whole_blocks || !workspace_bytes)
+    return fail(HCP_EINVAL, "%s: bad arguments", who);
+  *whole_blocks = 0;
+  *workspace_bytes = 0;
+  const int64_t blocks = tq / hcp::kFwdBM + (tq % hcp::kFwdBM != 0);
+  if (tk > (int64_t)INT32_MAX - 256 || blocks > kMaxUnits || blocks * num_heads > kMaxUnits)
+    return 0;
+  hcp_varlen_entry e{};
+  e.q_len = tq;
+  e.causal_offset = causal ? causal_offset : 0;
+  e.kv.len = tk;
+  std::vector<Unit> units;  // in dispatch order (longest first)
+  for (int64_t t = 0; t < blocks; ++t) {
+    const int64_t qb = causal ? blocks - 1 - t : t;
+    units.push_back({unit_tiles(e, qb, causal != 0, causal ? window : 0), unit_waves(e, qb)});
+  }
+  const Cut c = choose_cut(units, num_heads / num_kv_heads, num_kv_heads,
+                           hcp::padded_head_dim(head_dim));
+  if (c.tiles > 0) {
+    int mp = 1;
+    for (size_t t = c.whole; t < units.size(); ++t)
+      mp = std::max(mp, hcp::unit_pieces(units[t].tiles, c.tiles));
+    *whole_blocks = c.whole;
+    *workspace_bytes = split_ws_bytes((blocks - c.whole) * mp, num_heads, head_dim);
+  }
+  return c.tiles;
+} catch (const std::bad_alloc&) {
+  return fail(HCP_EINVAL, "hcp_plan_fwd_split: out of host memory");
+}
+
+int hcp_attn_fwd_lse_split(const void* q, const void* k, const void* v, void* out, float* lse,
+                           int64_t tq, int64_t tk, int32_t num_heads, int32_t num_kv_heads,
+                           int32_t head_dim, int64_t q_stride_tok, int64_t q_stride_head,
+                           int64_t k_stride_tok, int64_t k_stride_head, int64_t v_stride_tok,
+                           int64_t v_stride_head, int64_t o_stride_tok, int64_t o_stride_head,
+                           int64_t lse_stride_head, float scale, int32_t causal,
+                           int64_t causal_offset, int32_t window, const void* acc_out,
+                           int64_t acc_stride_tok, int64_t acc_stride_head,
+                           const float* acc_lse, int64_t acc_lse_stride_head,
+                           int32_t acc_is_prefix, int32_t piece_tiles, int32_t whole_blocks,
+                           void* workspace, size_t workspace_bytes, int32_t dtype,
+                           void* stream) {
+  const char* who = "hcp_attn_fwd_lse_split";
+  if (piece_tiles <= 0) return fail(HCP_EINVAL, "%s: piece_tiles must be > 0", who);
+  const AccArgs acc{acc_out, acc_stride_tok, acc_stride_head, acc_lse, acc_lse_stride_head,
+                    acc_is_prefix};
+  const SplitArgs split{piece_tiles, whole_blocks, workspace, workspace_bytes, nullptr, 0, 0};
+  return fwd_lse_impl(who, q, k, v, out, lse, tq, tk, num_heads, num_kv_heads, head_dim,
+                      q_stride_tok, q_stride_head, k_stride_tok, k_stride_head, v_stride_tok,
+                      v_stride_head, o_stride_tok, o_stride_head, lse_stride_head, scale, causal,
+                      causal_offset, window, dtype, stream, acc_out || acc_lse ? &acc : nullptr,
+                      &split);
 }
 
 int hcp_attn_fwd_lse(const void* q, const void* k, const void* v, void* out, float* lse,
@@ -199,6 +431,30 @@ int hcp_varlen_block_m(int32_t head_dim, int32_t dtype) {
   return hcp::kFwdBM;
 }
 
+static int check_prefill_entry(const hcp_varlen_entry& en, const char* who, int32_t i) {
+  // the kernel counts a segment's keys (and its tiles' key offsets) in int32
+  if (en.kv.len > (int64_t)INT32_MAX - 256)
+    return fail(HCP_EUNSUPPORTED, "%s: entry %d: kv len too large", who, i);
+  // the prefill kernel reads a wave's 16 rows of a paged tile from one block
+  if (en.kv.block_table && (en.kv.stride_tok <= 0 || en.kv.stride_tok >= (int64_t{1} << 24)))
+    return fail(HCP_EUNSUPPORTED, "%s: entry %d: paged token stride must be in (0, 2^24)", who, i);
+  if (!en.kv.block_table && en.kv.len > 1 &&
+      (en.kv.stride_tok <= 0 || en.kv.stride_tok >= (int64_t{1} << 24)))
+    return fail(HCP_EUNSUPPORTED, "%s: entry %d: token stride must be in (0, 2^24)", who, i);
+  if (en.kv.block_table && (en.kv.stride_block <= 0 || en.kv.stride_block >= (int64_t{1} << 31)))
+    return fail(HCP_EUNSUPPORTED, "%s: entry %d: block stride must be in (0, 2^31) elements",
+                who, i);
+  // the kernel's in-block byte offsets are 32-bit
+  if (en.kv.block_table &&
+      static_cast<int64_t>(en.kv.block_size) * en.kv.stride_tok * 2 > (int64_t{1} << 32))
+    return fail(HCP_EUNSUPPORTED, "%s: entry %d: block_size * token stride spans over 4 GiB",
+                who, i);
+  if (en.kv.block_table && en.kv.block_size < hcp::kFwdPagedMinBlock)
+    return fail(HCP_EUNSUPPORTED, "%s: entry %d: paged prefill needs block_size >= %d, got %d",
+                who, i, hcp::kFwdPagedMinBlock, en.kv.block_size);
+  return HCP_OK;
+}
+
 int hcp_plan_varlen_tiles(const hcp_varlen_entry* entries, int32_t num_entries, int32_t causal,
                           int32_t block_m, int32_t* tiles_out, int32_t cap) {
   const char* who = "hcp_plan_varlen_tiles";
@@ -212,26 +468,7 @@ int hcp_plan_varlen_tiles(const hcp_varlen_entry* entries, int32_t num_entries, 
   for (int32_t i = 0; i < num_entries; ++i) {
     const hcp_varlen_entry& en = entries[i];
     if (en.q_len < 0 || en.kv.len < 0) return fail(HCP_EINVAL, "%s: entry %d negative", who, i);
-    // the kernel counts a segment's keys (and its tiles' key offsets) in int32
-    if (en.kv.len > (int64_t)INT32_MAX - 256)
-      return fail(HCP_EUNSUPPORTED, "%s: entry %d: kv len too large", who, i);
-    // the prefill kernel reads a wave's 16 rows of a paged tile from one block
-    if (en.kv.block_table && (en.kv.stride_tok <= 0 || en.kv.stride_tok >= (int64_t{1} << 24)))
-      return fail(HCP_EUNSUPPORTED, "%s: entry %d: paged token stride must be in (0, 2^24)", who, i);
-    if (!en.kv.block_table && en.kv.len > 1 &&
-        (en.kv.stride_tok <= 0 || en.kv.stride_tok >= (int64_t{1} << 24)))
-      return fail(HCP_EUNSUPPORTED, "%s: entry %d: token stride must be in (0, 2^24)", who, i);
-    if (en.kv.block_table && (en.kv.stride_block <= 0 || en.kv.stride_block >= (int64_t{1} << 31)))
-      return fail(HCP_EUNSUPPORTED, "%s: entry %d: block stride must be in (0, 2^31) elements",
-                  who, i);
-    // the kernel's in-block byte offsets are 32-bit
-    if (en.kv.block_table &&
-        static_cast<int64_t>(en.kv.block_size) * en.kv.stride_tok * 2 > (int64_t{1} << 32))
-      return fail(HCP_EUNSUPPORTED, "%s: entry %d: block_size * token stride spans over 4 GiB",
-                  who, i);
-    if (en.kv.block_table && en.kv.block_size < hcp::kFwdPagedMinBlock)
-      return fail(HCP_EUNSUPPORTED, "%s: entry %d: paged prefill needs block_size >= %d, got %d",
-                  who, i, hcp::kFwdPagedMinBlock, en.kv.block_size);
+    if (int rc = check_prefill_entry(en, who, i)) return rc;
     const int64_t nqb = (en.q_len + block_m - 1) / block_m;
     for (int64_t b = 0; b < nqb; ++b) {
       int64_t keys = en.kv.len;
@@ -255,6 +492,87 @@ int hcp_plan_varlen_tiles(const hcp_varlen_entry* entries, int32_t num_entries, 
   return n;
 }
 
+int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries, int32_t causal,
+                          int32_t window, int32_t num_heads, int32_t num_kv_heads,
+                          int32_t head_dim, int32_t* pieces_out, int32_t cap,
+                          int32_t* units_out, int32_t* num_units, int32_t* num_slots,
+                          int32_t* piece_tiles, size_t* workspace_bytes) try {
+  const char* who = "hcp_plan_varlen_split";
+  int rc = check_heads(num_heads, num_kv_heads, head_dim, HCP_DTYPE_BF16, who);
+  if (rc) return rc;
+  if (num_entries < 0 || window < 0 || cap < 0) return fail(HCP_EINVAL, "%s: bad sizes", who);
+  if ((num_entries > 0 && !entries) || !num_units || !num_slots || !piece_tiles ||
+      !workspace_bytes)
+    return fail(HCP_EINVAL, "%s: null pointer", who);
+  *num_units = *num_slots = *piece_tiles = 0;
+  *workspace_bytes = 0;
+  struct U {
+    Unit u;
+    int32_t e, qb;
+  };
+  std::vector<U> blocks;
+  for (int32_t i = 0; i < num_entries; ++i) {
+    const hcp_varlen_entry& en = entries[i];
+    if (en.q_len < 0 || en.kv.len < 0) return fail(HCP_EINVAL, "%s: entry %d negative", who, i);
+    if ((rc = check_prefill_entry(en, who, i))) return rc;
+    const int64_t nqb = en.q_len / hcp::kFwdBM + (en.q_len % hcp::kFwdBM != 0);
+    if (nqb > kMaxUnits || (static_cast<int64_t>(blocks.size()) + nqb) * num_heads > kMaxUnits)
+      return 0;
+    for (int64_t b = 0; b < nqb; ++b)
+      blocks.push_back({{unit_tiles(en, b, causal != 0, causal ? window : 0), unit_waves(en, b)},
+                        i, static_cast<int32_t>(b)});
+  }
+  std::stable_sort(blocks.begin(), blocks.end(),
+                   [](const U& a, const U& b) { return a.u.tiles > b.u.tiles; });
+  std::vector<Unit> units;
+  for (const U& b : blocks) units.push_back(b.u);
+  const Cut c = choose_cut(units, num_heads / num_kv_heads, num_kv_heads,
+                           hcp::padded_head_dim(head_dim));
+  if (c.tiles == 0) return 0;
+  struct P {
+    int32_t cost, e, qb, piece, slot;
+  };
+  std::vector<P> v;
+  int32_t slot = 0, nu = 0;
+  for (size_t j = 0; j < blocks.size(); ++j) {
+    const U& u = blocks[j];
+    const int nt = u.u.tiles;
+    const int np = static_cast<int>(j) < c.whole ? 1 : hcp::unit_pieces(nt, c.tiles);
+    if (static_cast<int64_t>(v.size()) + np > cap || !pieces_out || !units_out)
+      return fail(HCP_EWORKSPACE, "%s: piece cap %d exceeded", who, cap);
+    if (np == 1) {
+      v.push_back({nt, u.e, u.qb, 0, -1});
+      continue;
+    }
+    units_out[4 * nu] = u.e;
+    units_out[4 * nu + 1] = u.qb;
+    units_out[4 * nu + 2] = slot;
+    units_out[4 * nu + 3] = np;
+    ++nu;
+    for (int i = 0; i < np; ++i)
+      v.push_back({hcp::piece_begin(nt, np, i + 1) - hcp::piece_begin(nt, np, i), u.e, u.qb,
+                   i, slot++});
+  }
+  // longest first; among equals the same piece of every block together, so
+  // workgroups in flight at once read the same keys
+  std::stable_sort(v.begin(), v.end(), [](const P& a, const P& b) {
+    return a.cost != b.cost ? a.cost > b.cost : a.piece < b.piece;
+  });
+  for (size_t i = 0; i < v.size(); ++i) {
+    pieces_out[4 * i] = v[i].e;
+    pieces_out[4 * i + 1] = v[i].qb;
+    pieces_out[4 * i + 2] = v[i].piece;
+    pieces_out[4 * i + 3] = v[i].slot;
+  }
+  *num_units = nu;
+  *num_slots = slot;
+  *piece_tiles = c.tiles;
+  *workspace_bytes = split_ws_bytes(slot, num_heads, head_dim);
+  return static_cast<int>(v.size());
+} catch (const std::bad_alloc&) {
+  return fail(HCP_EINVAL, "hcp_plan_varlen_split: out of host memory");
+}
+
 static int fwd_varlen_impl(const char* who, const void* q, int64_t q_stride_tok,
                            int64_t q_stride_head, void* out, int64_t o_stride_tok,
                            int64_t o_stride_head, float* lse, int64_t lse_stride_head,
@@ -262,7 +580,7 @@ static int fwd_varlen_impl(const char* who, const void* q, int64_t q_stride_tok,
                            const int32_t* tiles, int32_t num_tiles, int32_t num_heads,
                            int32_t num_kv_heads, int32_t head_dim, float scale, int32_t causal,
                            int32_t window, int32_t paged, int32_t dtype, void* stream,
-                           const AccArgs* acc) {
+                           const AccArgs* acc, const SplitArgs* split = nullptr) {
   int rc = check_heads(num_heads, num_kv_heads, head_dim, dtype, who);
   if (rc) return rc;
   if (num_entries < 0 || num_tiles < 0) return fail(HCP_EINVAL, "%s: negative counts", who);
@@ -295,6 +613,16 @@ static int fwd_varlen_impl(const char* who, const void* q, int64_t q_stride_tok,
   p.head_dim = head_dim;
   p.scale_log2 = scale * hcp::kLog2e;
   set_acc(p, acc);
+  if (split) {
+    if (split->num_units < 0 || split->num_slots < 0 || (split->num_units > 0 && !split->units))
+      return fail(HCP_EINVAL, "%s: bad split units", who);
+    if (static_cast<int64_t>(split->num_units) * num_heads * 4 > INT32_MAX)
+      return fail(HCP_EINVAL, "%s: too many split units", who);
+    p.units = split->units;
+    p.num_units = split->num_units;
+    if ((rc = set_split(p, split->piece_tiles, split->num_slots, split->ws, split->bytes, who)))
+      return rc;
+  }
   hipError_t e = hcp::launch_fwd(p, head_dim, dtype, causal != 0, paged != 0, true,
                                  static_cast<hipStream_t>(stream));
   return launch_status(e, who);
@@ -329,6 +657,29 @@ int hcp_attn_fwd_varlen_merge(const void* q, int64_t q_stride_tok, int64_t q_str
                          o_stride_tok, o_stride_head, lse, lse_stride_head, entries, num_entries,
                          tiles, num_tiles, num_heads, num_kv_heads, head_dim, scale, causal,
                          window, paged, dtype, stream, &acc);
+}
+
+int hcp_attn_fwd_varlen_split(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                              void* out, int64_t o_stride_tok, int64_t o_stride_head, float* lse,
+                              int64_t lse_stride_head, const hcp_varlen_entry* entries,
+                              int32_t num_entries, const int32_t* pieces, int32_t num_pieces,
+                              int32_t piece_tiles, const int32_t* units, int32_t num_units,
+                              int32_t num_slots, int32_t num_heads, int32_t num_kv_heads,
+                              int32_t head_dim, float scale, int32_t causal, int32_t window,
+                              int32_t paged, const void* acc_out, int64_t acc_stride_tok,
+                              int64_t acc_stride_head, const float* acc_lse,
+                              int64_t acc_lse_stride_head, int32_t acc_is_prefix,
+                              void* workspace, size_t workspace_bytes, int32_t dtype,
+                              void* stream) {
+  const char* who = "hcp_attn_fwd_varlen_split";
+  if (piece_tiles <= 0) return fail(HCP_EINVAL, "%s: piece_tiles must be > 0", who);
+  const AccArgs acc{acc_out, acc_stride_tok, acc_stride_head, acc_lse, acc_lse_stride_head,
+                    acc_is_prefix};
+  const SplitArgs split{piece_tiles, 0, workspace, workspace_bytes, units, num_units, num_slots};
+  return fwd_varlen_impl(who, q, q_stride_tok, q_stride_head, out, o_stride_tok, o_stride_head,
+                         lse, lse_stride_head, entries, num_entries, pieces, num_pieces,
+                         num_heads, num_kv_heads, head_dim, scale, causal, window, paged, dtype,
+                         stream, acc_out || acc_lse ? &acc : nullptr, &split);
 }
 
 int hcp_plan_decode_splits(const hcp_varlen_entry* entries, int32_t num_entries,

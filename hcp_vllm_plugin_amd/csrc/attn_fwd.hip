@@ -57,6 +57,15 @@
 //    diagonal and ragged tiles.  A ragged last tile is bounded by its buffer
 //    descriptor (rows past the segment read as zeros and are masked), so no
 //    load leaves the segment and none is predicated.
+//  * A launch with too few query blocks for 256 CUs (a 512-token chunk of a
+//    32k prompt: 112 workgroups) is cut along the keys (SPLIT instantiations):
+//    a workgroup takes one piece of a block's tiles -- a shorter segment with a
+//    shifted causal offset, the tile loop is the same -- and stores an f32
+//    partial, which fwd_reduce_kernel merges.  28 / 4 x 128 heads, 512 x 32768:
+//    490 -> 248 us; 14 / 2 x 64, 3001 x 5003: 89 -> 76 us (the first 256
+//    workgroups whole, the rest cut to fill what is left of the second round).
+//    The uncut launches keep kernels without the split's registers (the shared
+//    form cost the D = 256 window pass 0.7%).
 //  * The local (paged) segment is read in place through the block table
 //    (hcp_kv_segment), replacing the per-request gather copy of
 //    ring_backend.py:617-624; block ids are fetched ahead of the tile loads.
@@ -117,7 +126,15 @@ __device__ __forceinline__ i16x4 lds_read_tr(const HCP_LDS(char)* p) {
       reinterpret_cast<HCP_LDS(i16x4)*>(const_cast<HCP_LDS(char)*>(p)));
 }
 
-template <int D, typename T, bool CAUSAL, bool PAGED, bool VARLEN, bool PADDED>
+// Workgroup records per KV head and head of its group: whole blocks, then
+// (block, piece) pairs
+__host__ __device__ __forceinline__ int64_t fwd_items(const FwdParams& p, bool varlen,
+                                                              bool split) {
+  if (varlen || !split) return p.num_tiles;
+  return p.whole_tiles + static_cast<int64_t>(p.num_tiles - p.whole_tiles) * p.max_pieces;
+}
+
+template <int D, typename T, bool CAUSAL, bool PAGED, bool VARLEN, bool PADDED, bool SPLIT>
 __global__ __attribute__((amdgpu_flat_work_group_size(kFwdThreads, kFwdThreads),
                           amdgpu_waves_per_eu(D == 256 ? 1 : HCP_FWD_WAVES_PER_EU,
                                               D == 256 ? 1 : HCP_FWD_WAVES_PER_EU))) void
@@ -151,20 +168,33 @@ fa_fwd_kernel(FwdParams p) {
   // ---- work item: (tile, head) ----
   int kvh;
   int64_t item;
-  if (!xcd_remap(blockIdx.x, static_cast<int64_t>(p.num_tiles) * p.group,
-                 p.num_kv_heads, &kvh, &item))
+  if (!xcd_remap(blockIdx.x, fwd_items(p, VARLEN, SPLIT) * p.group, p.num_kv_heads, &kvh, &item))
     return;
-  const int tile = static_cast<int>(item / p.group);
+  const int rec = static_cast<int>(item / p.group);
   const int head = kvh * p.group + static_cast<int>(item % p.group);
 
   hcp_varlen_entry e;
   int qb;
+  int piece = 0, slot = -1;  // slot: workspace partial of this workgroup, -1: none
   if constexpr (VARLEN) {
-    const int ent = p.tiles[2 * tile];
-    qb = p.tiles[2 * tile + 1];
-    e = p.entries[ent];
+    const int32_t* r = p.tiles + static_cast<int64_t>(rec) * (SPLIT ? 4 : 2);
+    e = p.entries[r[0]];
+    qb = r[1];
+    if constexpr (SPLIT) {
+      piece = r[2];
+      slot = r[3];
+    }
   } else {
     e = p.single;
+    int tile = rec;
+    if (SPLIT && rec >= p.whole_tiles) {
+      // pieces outermost: workgroups in flight together read the same keys
+      const int cut = p.num_tiles - p.whole_tiles, r = rec - p.whole_tiles;
+      piece = r / cut;
+      tile = r - piece * cut;
+      slot = tile * p.max_pieces + piece;
+      tile += p.whole_tiles;
+    }
     qb = CAUSAL ? (p.num_tiles - 1 - tile) : tile;  // heaviest first
   }
   // Sliding window (causal only): row i sees keys (off + i - window, off + i].
@@ -179,6 +209,23 @@ fa_fwd_kernel(FwdParams p) {
       e.kv.start += lo;
       e.kv.len -= lo;
       e.causal_offset -= lo;
+    }
+  }
+  // KV split: keep the tiles of this workgroup's piece.  The rest of the
+  // kernel sees a shorter segment and a shifted causal offset.
+  if (SPLIT && slot >= 0) {
+    const int64_t n = unit_keys(e.kv.len, e.causal_offset, qb, CAUSAL, 0).n;
+    const int nt = static_cast<int>((n + BN - 1) / BN);
+    const int np = unit_pieces(nt, p.piece_tiles);
+    if (piece >= np) return;
+    if (np == 1) {
+      slot = -1;
+    } else {
+      const int64_t k0 = static_cast<int64_t>(piece_begin(nt, np, piece)) * BN;
+      const int64_t k1 = static_cast<int64_t>(piece_begin(nt, np, piece + 1)) * BN;
+      e.kv.len = (piece + 1 < np ? k1 : e.kv.len) - k0;
+      e.kv.start += k0;
+      e.causal_offset -= k0;
     }
   }
   // Paged segments are tiled from a 16-key boundary of the request's block
@@ -821,6 +868,27 @@ fa_fwd_kernel(FwdParams p) {
   const int share = wave * 32 * ROWB;
   HCP_LDS(char)* const tbuf[4] = {K0, K1, V0, V1};
   HCP_LDS(char)* const abuf = tbuf[share / TILEB] + share % TILEB;
+  if (SPLIT && slot >= 0) {
+    // KV split: the piece's partial, O normalised in f32, in the lane order
+    // of the accumulator (whole 1 KB runs per store; fwd_reduce_kernel reads
+    // them back in the same order)
+    if (qi_e < q_len) {
+      const float inv = lr_tot > 0.f ? 1.f / lr_tot : 0.f;
+      const int64_t unit = static_cast<int64_t>(slot) * p.num_heads + head;
+      float* const wo = p.ws_o + unit * (BM * D) + wave * (32 * D);
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+          *reinterpret_cast<f32x4*>(wo + ((db * 4 + a) * 64 + lane_e) * 4) =
+              f32x4{oacc[db][4 * a] * inv, oacc[db][4 * a + 1] * inv, oacc[db][4 * a + 2] * inv,
+                    oacc[db][4 * a + 3] * inv};
+      if (ge == 0)
+        p.ws_lse[unit * BM + wave * 32 + r32e] =
+            l_tot > 0.f ? m_ref * kLn2 + __logf(l_tot) : -INFINITY;
+    }
+    return;
+  }
   if (p.acc_o != nullptr && wave_q0 < q_len) {
     const int64_t sb = p.acc_stride_tok * 2;
     const int rows = q_len - wave_q0 < 32 ? static_cast<int>(q_len - wave_q0) : 32;
@@ -911,13 +979,138 @@ fa_fwd_kernel(FwdParams p) {
   }
 }
 
+// Merge of a KV-split pass's partials: one workgroup per (query block, head,
+// 32 rows), each wave a quarter of the columns.  A lane reads its row's
+// partials in the order the forward kernel stored them (1 KB runs), weights
+// them by exp(lse_i - max) and writes the row pieces the forward's own epilogue
+// would have written; with an acc it then does the same merge with it, on the
+// result rounded to the output type.
+template <int D, typename T, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(256) void fwd_reduce_kernel(FwdParams p) {
+  using E = Elem<T>;
+  constexpr int NC = D / 8;  // 64-lane x 16-byte chunks of a wave's 32 rows
+  constexpr int CW = NC / 4; // chunks per wave of this kernel
+  const int lane = threadIdx.x & 63, cw = threadIdx.x >> 6;
+  const int r32 = lane & 31, g = lane >> 5;
+  const int wb = blockIdx.x & 3;  // the forward kernel's wave: rows 32 * wb ..
+  const int64_t uh = blockIdx.x >> 2;
+  const int head = static_cast<int>(uh % p.num_heads);
+  const int unit = static_cast<int>(uh / p.num_heads);
+  int qb, np, slot0;
+  int64_t q_start, q_len;
+  if constexpr (VARLEN) {
+    const int32_t* u = p.units + 4 * static_cast<int64_t>(unit);
+    q_start = p.entries[u[0]].q_start;
+    q_len = p.entries[u[0]].q_len;
+    qb = u[1];
+    slot0 = u[2];
+    np = u[3];
+  } else {
+    const int tile = p.whole_tiles + unit;
+    qb = CAUSAL ? (p.num_tiles - 1 - tile) : tile;
+    q_start = 0;
+    q_len = p.single.q_len;
+    slot0 = unit * p.max_pieces;
+    const int64_t n = unit_keys(p.single.kv.len, p.single.causal_offset, qb, CAUSAL, p.window).n;
+    np = unit_pieces(static_cast<int>((n + kFwdBN - 1) / kFwdBN), p.piece_tiles);
+    if (np == 1) return;  // written by the forward kernel itself
+  }
+  const int64_t qi = static_cast<int64_t>(qb) * kFwdBM + wb * 32 + r32;
+  const bool valid = qi < q_len;
+  const int64_t row = q_start + (valid ? qi : 0);
+  // the running accumulator's LSE is read before the barrier below, lse is
+  // written after it: the two may be one array
+  float la = -INFINITY;
+  if (p.acc_o != nullptr && valid) {
+    la = p.acc_lse[static_cast<int64_t>(head) * p.acc_lse_stride_head + row];
+    if (la == INFINITY) la = -INFINITY;
+  }
+  __syncthreads();
+  if (!valid) return;
+  const int64_t ustride = static_cast<int64_t>(p.num_heads);
+  const int64_t unit0 = static_cast<int64_t>(slot0) * ustride + head;
+  const float* lp = p.ws_lse + unit0 * kFwdBM + wb * 32 + r32;
+  const float* op = p.ws_o + unit0 * (kFwdBM * D) + wb * (32 * D) + (cw * CW * 64 + lane) * 4;
+  float M = -INFINITY;
+  for (int i = 0; i < np; ++i) M = __builtin_fmaxf(M, lp[i * ustride * kFwdBM]);
+  float S = 0.f;
+  f32x4 o[CW];
+#pragma unroll
+  for (int c = 0; c < CW; ++c) o[c] = f32x4{};
+  if (M != -INFINITY) {
+#pragma unroll 2
+    for (int i = 0; i < np; ++i) {
+      const float w = __expf(lp[i * ustride * kFwdBM] - M);
+      S += w;
+#pragma unroll
+      for (int c = 0; c < CW; ++c)
+        o[c] += *reinterpret_cast<const f32x4*>(op + i * ustride * (kFwdBM * D) + c * 256) * w;
+    }
+  }
+  const float inv = S > 0.f ? 1.f / S : 0.f;
+  float lse_row = S > 0.f ? M + __logf(S) : -INFINITY;
+  float w_acc = 0.f, w_own = 1.f;
+  const bool acc = p.acc_o != nullptr, acc_pre = p.acc_prefix != 0;
+  if (acc) {
+    const float l_pre = acc_pre ? la : lse_row, l_suf = acc_pre ? lse_row : la;
+    const float m = __builtin_fmaxf(l_pre, l_suf);
+    float ps = 0.f, ss = 0.f;
+    if (m == -INFINITY) {
+      lse_row = -INFINITY;
+    } else {
+      const float wp = __expf(l_pre - m), ws = __expf(l_suf - m);
+      const float se = wp + ws;
+      ps = wp / se;
+      ss = ws / se;
+      lse_row = m + __logf(se);
+    }
+    w_acc = acc_pre ? ps : ss;
+    w_own = acc_pre ? ss : ps;
+  }
+  char* const orow = reinterpret_cast<char*>(p.out) +
+                     (row * p.o_stride_tok + static_cast<int64_t>(head) * p.o_stride_head) * 2;
+  const char* const arow = reinterpret_cast<const char*>(p.acc_o) +
+                           (row * p.acc_stride_tok + static_cast<int64_t>(head) * p.acc_stride_head) * 2;
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    const int ch = cw * CW + c;  // 4 * db + a of the forward's accumulator
+    const int d0 = 8 * ch + 4 * g;
+    if (d0 >= p.head_dim) continue;
+    u32x2 w;
+    w[0] = pack2<T>(o[c][0] * inv, o[c][1] * inv);
+    w[1] = pack2<T>(o[c][2] * inv, o[c][3] * inv);
+    if (acc) {
+      if (!(w_own > 0.f)) w = u32x2{0, 0};
+      const u32x2 oth = w_acc > 0.f ? ldg8(arow + d0 * 2) : u32x2{0, 0};
+      const u32x2 pre = acc_pre ? oth : w, suf = acc_pre ? w : oth;
+      const float ps = acc_pre ? w_acc : w_own, ss = acc_pre ? w_own : w_acc;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float a0 = E::to_float(static_cast<uint16_t>(pre[h] & 0xffffu));
+        const float a1 = E::to_float(static_cast<uint16_t>(pre[h] >> 16));
+        const float b0 = E::to_float(static_cast<uint16_t>(suf[h] & 0xffffu));
+        const float b1 = E::to_float(static_cast<uint16_t>(suf[h] >> 16));
+        w[h] = pack2<T>(__builtin_fmaf(a0, ps, b0 * ss), __builtin_fmaf(a1, ps, b1 * ss));
+      }
+    }
+    *reinterpret_cast<u32x2*>(orow + d0 * 2) = w;
+  }
+  if (cw == 0 && g == 0 && p.lse != nullptr)
+    p.lse[static_cast<int64_t>(head) * p.lse_stride_head + row] = lse_row;
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launch helpers (called from abi.hip)
 // ---------------------------------------------------------------------------
 template <int D, typename T, bool CAUSAL, bool PAGED, bool VARLEN, bool PADDED>
 static hipError_t launch_fwd_t(const FwdParams& p, int64_t grid, hipStream_t st) {
-  hipLaunchKernelGGL((fa_fwd_kernel<D, T, CAUSAL, PAGED, VARLEN, PADDED>),
-                     dim3(static_cast<unsigned>(grid)), dim3(kFwdThreads), 0, st, p);
+  const dim3 g(static_cast<unsigned>(grid));
+  if (p.piece_tiles > 0)
+    hipLaunchKernelGGL((fa_fwd_kernel<D, T, CAUSAL, PAGED, VARLEN, PADDED, true>), g,
+                       dim3(kFwdThreads), 0, st, p);
+  else
+    hipLaunchKernelGGL((fa_fwd_kernel<D, T, CAUSAL, PAGED, VARLEN, PADDED, false>), g,
+                       dim3(kFwdThreads), 0, st, p);
   return hipGetLastError();
 }
 
@@ -943,24 +1136,34 @@ static hipError_t launch_fwd_d(const FwdParams& p, int64_t grid, bool causal,
                          : launch_fwd_p<D, T, true>(p, grid, causal, paged, varlen, st);
 }
 
-hipError_t launch_fwd(const FwdParams& p, int head_dim, int dtype, bool causal,
-                      bool paged, bool varlen, hipStream_t st) {
+template <int D, typename T>
+static hipError_t launch_reduce_t(const FwdParams& p, bool causal, bool varlen, hipStream_t st) {
+  const int64_t units = varlen ? p.num_units : p.num_tiles - p.whole_tiles;
+  if (units <= 0) return hipSuccess;
+  const dim3 grid(static_cast<unsigned>(units * p.num_heads * 4));
+  if (varlen)
+    hipLaunchKernelGGL((fwd_reduce_kernel<D, T, false, true>), grid, dim3(256), 0, st, p);
+  else if (causal)
+    hipLaunchKernelGGL((fwd_reduce_kernel<D, T, true, false>), grid, dim3(256), 0, st, p);
+  else
+    hipLaunchKernelGGL((fwd_reduce_kernel<D, T, false, false>), grid, dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+// The kernels of one column width: this file is compiled once per width
+// (HCP_FWD_D), side by side.
+template <>
+hipError_t launch_fwd_width<HCP_FWD_D>(const FwdParams& p, int dtype, bool causal, bool paged,
+                                       bool varlen, hipStream_t st) {
+  const bool bf = dtype == HCP_DTYPE_BF16;
   const int64_t grid =
-      xcd_grid_size(static_cast<int64_t>(p.num_tiles) * p.group, p.num_kv_heads);
+      xcd_grid_size(fwd_items(p, varlen, p.piece_tiles > 0) * p.group, p.num_kv_heads);
   if (grid <= 0) return hipSuccess;
-  if (head_dim > 128) {  // 136 .. 256: computed in 256 columns, the tail zero
-    return dtype == HCP_DTYPE_BF16
-               ? launch_fwd_d<256, __bf16>(p, grid, causal, paged, varlen, st)
-               : launch_fwd_d<256, _Float16>(p, grid, causal, paged, varlen, st);
-  }
-  if (head_dim > 64) {  // 72 .. 128: computed in 128 columns, the tail zero
-    return dtype == HCP_DTYPE_BF16
-               ? launch_fwd_d<128, __bf16>(p, grid, causal, paged, varlen, st)
-               : launch_fwd_d<128, _Float16>(p, grid, causal, paged, varlen, st);
-  }
-  return dtype == HCP_DTYPE_BF16
-             ? launch_fwd_d<64, __bf16>(p, grid, causal, paged, varlen, st)
-             : launch_fwd_d<64, _Float16>(p, grid, causal, paged, varlen, st);
+  const hipError_t e = bf ? launch_fwd_d<HCP_FWD_D, __bf16>(p, grid, causal, paged, varlen, st)
+                          : launch_fwd_d<HCP_FWD_D, _Float16>(p, grid, causal, paged, varlen, st);
+  if (e != hipSuccess || p.piece_tiles == 0) return e;
+  return bf ? launch_reduce_t<HCP_FWD_D, __bf16>(p, causal, varlen, st)
+            : launch_reduce_t<HCP_FWD_D, _Float16>(p, causal, varlen, st);
 }
 
 }  // namespace hcp

@@ -44,7 +44,44 @@ struct FwdParams {
   const float* acc_lse;
   int64_t acc_lse_stride_head;
   int32_t acc_prefix;
+  // KV split (piece_tiles 0: none): a (query block, head) whose keys span more
+  // than piece_tiles tiles runs as unit_pieces() workgroups, each writing an
+  // fp32 partial (O normalised, LSE) to the workspace, merged by
+  // fwd_reduce_kernel.  Single entry: the first whole_tiles blocks in dispatch
+  // order stay whole; block t past them, piece i -> slot (t - whole_tiles) *
+  // max_pieces + i.  Varlen: `tiles` holds (entry, q_block, piece, slot)
+  // records, slot -1 for a whole block, and `units` the blocks that were cut.
+  int32_t piece_tiles, max_pieces, whole_tiles;
+  float* ws_o;           // [slot][head][kFwdBM * D], in the kernel's lane order
+  float* ws_lse;         // [slot][head][kFwdBM]
+  const int32_t* units;  // varlen: device (entry, q_block, first slot, pieces) records
+  int32_t num_units;
 };
+
+// Keys [lo, lo + n) of an entry that the rows of query block qb see: the
+// workgroup's key range before it is cut into tiles.
+struct UnitKeys {
+  int64_t lo, n;
+};
+__host__ __device__ inline UnitKeys unit_keys(int64_t kv_len, int64_t causal_offset, int64_t qb,
+                                              bool causal, int32_t window) {
+  UnitKeys u{0, kv_len};
+  if (causal) {
+    const int64_t first = causal_offset + qb * kFwdBM;  // last key of the block's first row
+    if (window > 0 && first - window + 1 > 0)
+      u.lo = first - window + 1 < kv_len ? first - window + 1 : kv_len;
+    const int64_t end = first + kFwdBM < kv_len ? first + kFwdBM : kv_len;
+    u.n = end > u.lo ? end - u.lo : 0;
+  }
+  return u;
+}
+__host__ __device__ inline int unit_pieces(int tiles, int piece_tiles) {
+  return tiles > piece_tiles ? (tiles + piece_tiles - 1) / piece_tiles : 1;
+}
+// first tile of piece i of np (never an empty piece while np <= tiles)
+__host__ __device__ inline int piece_begin(int tiles, int np, int i) {
+  return static_cast<int>(static_cast<int64_t>(tiles) * i / np);
+}
 
 struct DecParams {
   const void* q;
@@ -129,8 +166,25 @@ struct GatherParams {
   void* v_out;
 };
 
-hipError_t launch_fwd(const FwdParams& p, int head_dim, int dtype, bool causal,
-                      bool paged, bool varlen, hipStream_t st);
+// Prefill in D columns (padded_head_dim): the attention kernel and, when p
+// carries a KV split, the merge of its partials into out / lse (and acc).
+template <int D>
+hipError_t launch_fwd_width(const FwdParams& p, int dtype, bool causal, bool paged, bool varlen,
+                            hipStream_t st);
+template <>
+hipError_t launch_fwd_width<64>(const FwdParams&, int, bool, bool, bool, hipStream_t);
+template <>
+hipError_t launch_fwd_width<128>(const FwdParams&, int, bool, bool, bool, hipStream_t);
+template <>
+hipError_t launch_fwd_width<256>(const FwdParams&, int, bool, bool, bool, hipStream_t);
+inline hipError_t launch_fwd(const FwdParams& p, int head_dim, int dtype, bool causal, bool paged,
+                             bool varlen, hipStream_t st) {
+  switch (padded_head_dim(head_dim)) {
+    case 256: return launch_fwd_width<256>(p, dtype, causal, paged, varlen, st);
+    case 128: return launch_fwd_width<128>(p, dtype, causal, paged, varlen, st);
+    default: return launch_fwd_width<64>(p, dtype, causal, paged, varlen, st);
+  }
+}
 hipError_t launch_decode(const DecParams& dp, const RedParams& rp, int head_dim,
                          int dtype, hipStream_t st);
 hipError_t launch_merge(const MergeParams& p, hipStream_t st);

@@ -13,6 +13,8 @@ KV frame.  The work runs in ``hcp_attn_fwd_lse`` (libhcp_mi355x.so).
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -82,6 +84,54 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if ok else _copied(t)
 
 
+# hcp_plan_fwd_split never cuts a launch of more (query block, head) pairs than
+# this, or of fewer keys: those calls are not worth asking about
+_MAX_SPLIT_UNITS = 1024
+_MIN_SPLIT_KEYS = 449
+
+
+def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_prefix):
+    """One pass over (q, k, v): ``hcp_attn_fwd_lse`` (acc None) or
+    ``hcp_attn_fwd_lse_merge``, or -- few query rows over many keys, where
+    those would leave CUs idle -- ``hcp_attn_fwd_lse_split`` on the KV split
+    the library plans, its fp32 partials in stream-ordered scratch from torch's
+    caching allocator."""
+    L = _lib.lib()
+    tq, num_heads, head_dim = q.shape
+    tk, num_kv_heads = k.shape[0], k.shape[1]
+    causal = 0 if causal_offset is None else 1
+    off = 0 if causal_offset is None else int(causal_offset)
+    win = 0 if (window is None or causal_offset is None) else int(window)
+    dtype, device = _lib.dtype_code(q.dtype), q.device
+    with torch.cuda.device(device):
+        head = (
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+            0 if lse is None else lse.data_ptr(),
+            tq, tk, num_heads, num_kv_heads, head_dim,
+            q.stride(0), q.stride(1), k.stride(0), k.stride(1),
+            v.stride(0), v.stride(1), out.stride(0), out.stride(1),
+            0 if lse is None else lse.stride(0),
+            float(scale), causal, off, win,
+        )
+        a = () if acc is None else (acc[0].data_ptr(), acc[0].stride(0), acc[0].stride(1),
+                                    acc[1].data_ptr(), acc[1].stride(0), int(bool(acc_is_prefix)))
+        if tk >= _MIN_SPLIT_KEYS and -(-tq // 128) * num_heads <= _MAX_SPLIT_UNITS:
+            whole, nbytes = ctypes.c_int32(0), ctypes.c_size_t(0)
+            pt = L.hcp_plan_fwd_split(tq, tk, num_heads, num_kv_heads, head_dim, causal, off, win,
+                                      ctypes.addressof(whole), ctypes.addressof(nbytes))
+            _lib.check(pt, name)
+            if pt > 0:
+                ws = torch.empty(nbytes.value, dtype=torch.uint8, device=device)
+                rc = L.hcp_attn_fwd_lse_split(*head, *(a or (0, 0, 0, 0, 0, 0)), pt,
+                                              whole.value, ws.data_ptr(), nbytes.value, dtype,
+                                              _lib.stream_ptr(device))
+                _lib.check(rc, name)
+                return
+        fn = L.hcp_attn_fwd_lse if acc is None else L.hcp_attn_fwd_lse_merge
+        rc = fn(*head, *a, dtype, _lib.stream_ptr(device))
+    _lib.check(rc, name)
+
+
 def ring_attn_with_lse(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -109,8 +159,7 @@ def ring_attn_with_lse(
                                       scale, causal_offset, window)
         return out[..., : q.shape[2]].contiguous(), lse
     q, k, v = _aligned(q), _aligned(k), _aligned(v)
-    tq, num_heads, head_dim = q.shape
-    tk, num_kv_heads = k.shape[0], k.shape[1]
+    tq, num_heads = q.shape[0], q.shape[1]
     out = torch.empty_like(q, memory_format=torch.contiguous_format)
     lse = torch.empty((num_heads, tq), dtype=torch.float32, device=q.device)
     if tq == 0:
@@ -118,19 +167,7 @@ def ring_attn_with_lse(
     if k.stride() != v.stride():
         v = v if v.is_contiguous() else _copied(v)
         k = k if k.is_contiguous() else _copied(k)
-    L = _lib.lib()
-    with torch.cuda.device(q.device):
-        rc = L.hcp_attn_fwd_lse(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-            tq, tk, num_heads, num_kv_heads, head_dim,
-            q.stride(0), q.stride(1), k.stride(0), k.stride(1),
-            v.stride(0), v.stride(1), out.stride(0), out.stride(1), lse.stride(0),
-            float(scale), 0 if causal_offset is None else 1,
-            0 if causal_offset is None else int(causal_offset),
-            0 if (window is None or causal_offset is None) else int(window),
-            _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device),
-        )
-    _lib.check(rc, "hcp_attn_fwd_lse")
+    _launch("hcp_attn_fwd_lse", q, k, v, out, lse, scale, causal_offset, window, None, True)
     return out, lse
 
 
@@ -185,8 +222,7 @@ def ring_attn_merged(
         return output
     q, k, v = _aligned(q), _aligned(k), _aligned(v)
     _check_partial(acc_output, acc_lse, q, "acc")
-    tq, num_heads, head_dim = q.shape
-    tk, num_kv_heads = k.shape[0], k.shape[1]
+    tq, num_heads = q.shape[0], q.shape[1]
     if output is None:
         output = torch.empty_like(q, memory_format=torch.contiguous_format)
     elif output.shape != q.shape or output.dtype != q.dtype or output.stride(-1) != 1:
@@ -200,21 +236,6 @@ def ring_attn_merged(
     if k.stride() != v.stride():
         v = v if v.is_contiguous() else _copied(v)
         k = k if k.is_contiguous() else _copied(k)
-    L = _lib.lib()
-    with torch.cuda.device(q.device):
-        rc = L.hcp_attn_fwd_lse_merge(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(),
-            0 if output_lse is None else output_lse.data_ptr(),
-            tq, tk, num_heads, num_kv_heads, head_dim,
-            q.stride(0), q.stride(1), k.stride(0), k.stride(1),
-            v.stride(0), v.stride(1), output.stride(0), output.stride(1),
-            0 if output_lse is None else output_lse.stride(0),
-            float(scale), 0 if causal_offset is None else 1,
-            0 if causal_offset is None else int(causal_offset),
-            0 if (window is None or causal_offset is None) else int(window),
-            acc_output.data_ptr(), acc_output.stride(0), acc_output.stride(1),
-            acc_lse.data_ptr(), acc_lse.stride(0), int(bool(acc_is_prefix)),
-            _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device),
-        )
-    _lib.check(rc, "hcp_attn_fwd_lse_merge")
+    _launch("hcp_attn_fwd_lse_merge", q, k, v, output, output_lse, scale, causal_offset, window,
+            (acc_output, acc_lse), acc_is_prefix)
     return output

@@ -591,6 +591,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # non-causal peer pass -- ring_backend.py:490-492,786,815,826-830
         self.sliding_window = int(sliding_window) if sliding_window is not None else None
         self.num_queries_per_kv = self.num_heads // self.num_kv_heads
+        self._heads = (self.num_heads, self.num_kv_heads, self.head_size)
 
     # -- paged KV write (the step before the path) ----------------------------
     def do_kv_cache_update(
@@ -1004,8 +1005,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         else:
             lse = torch.empty((self.num_heads, query.shape[0]), dtype=torch.float32,
                               device=query.device)
-            VarlenLaunch(ent, True, True, query.device, keep=keep).run(
-                query, out, lse, self.num_kv_heads, self.scale, w)
+            VarlenLaunch(ent, True, True, query.device, keep=keep, heads=self._heads,
+                         window=w).run(query, out, lse, self.num_kv_heads, self.scale, w)
             _count("attn")
 
     def _forward_prefill(self, query, out, plan: _Plan) -> None:
@@ -1013,7 +1014,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         h = self.num_heads
         if not plan.any_peer:
             lse = torch.empty((h, query.shape[0]), dtype=torch.float32, device=dev)
-            VarlenLaunch(plan.local, True, True, dev).run(query, out, lse, self.num_kv_heads,
+            VarlenLaunch(plan.local, True, True, dev, heads=self._heads,
+                         window=self.sliding_window).run(query, out, lse, self.num_kv_heads,
                                                          self.scale, self.sliding_window)
             _count("attn")
             return
@@ -1024,7 +1026,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                                device=dev)
             for kind in ("contig", "paged"):
                 if rnd[kind]:
-                    VarlenLaunch(rnd[kind], False, kind == "paged", dev).run(
+                    VarlenLaunch(rnd[kind], False, kind == "paged", dev, heads=self._heads).run(
                         query, o_r, lse_r, self.num_kv_heads, self.scale)
                     _count("attn")
             if o_peer is None:
@@ -1040,7 +1042,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # = peer, suffix = local (ring_backend.py:354,820-831), bit for bit.
         # The local entries cover every query row of the plan; rows without a
         # peer have lse_peer = -inf and get the local result.
-        VarlenLaunch(plan.local, True, True, dev).run(
+        VarlenLaunch(plan.local, True, True, dev, heads=self._heads,
+                     window=self.sliding_window).run(
             query, out, None, self.num_kv_heads, self.scale, self.sliding_window,
             acc=(o_peer, lse_peer), acc_is_prefix=True)
         _count("attn")

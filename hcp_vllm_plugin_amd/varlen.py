@@ -288,6 +288,10 @@ def plan_varlen_tiles(entries: list[VarlenEntry], causal: bool) -> list[tuple[in
 # smallest block_size the paged prefill kernel reads in place (a wave's 16
 # rows of a tile must lie in one block); smaller ones are gathered first
 _MIN_PAGED_BLOCK = 16
+# hcp_plan_varlen_split: (query block, head) pairs past which it never cuts a
+# launch, and the most records it writes
+_MAX_SPLIT_UNITS = 1024
+_MAX_PIECES = 4096
 
 
 class VarlenLaunch:
@@ -299,9 +303,15 @@ class VarlenLaunch:
     stream (or synchronise first).
     """
 
-    def __init__(self, entries, causal: bool, paged: bool, device: torch.device, keep=None):
+    def __init__(self, entries, causal: bool, paged: bool, device: torch.device, keep=None,
+                 heads: tuple[int, int, int] | None = None, window: int | None = None):
         """``entries``: a list of VarlenEntry, or an ENTRY_DTYPE array (then
-        ``keep`` holds the tensors its addresses point into)."""
+        ``keep`` holds the tensors its addresses point into).
+
+        ``heads = (num_heads, num_kv_heads, head_dim)`` and ``window`` of the
+        runs to come let the plan cut long key ranges over few query rows into
+        pieces (``hcp_plan_varlen_split``); a run with other values, or a plan
+        built without them, takes the uncut launch."""
         L = _lib.lib()
         self.causal = bool(causal)
         self.paged = bool(paged)
@@ -350,14 +360,40 @@ class VarlenLaunch:
                                      int(self.causal), bm, ctypes.addressof(tiles), cap)
         _lib.check(rc, "hcp_plan_varlen_tiles")
         self.num_tiles = rc
+        split = self._plan_split(L, arr, heads, window)
         if self._gather is None:
-            self._plan_dev, (self.entries_ptr, self.tiles_ptr) = _upload([arr, tiles], device)
+            self._plan_dev, (self.entries_ptr, self.tiles_ptr, *sp) = _upload(
+                [arr, tiles, *split], device)
         else:
             g = self._gather
-            self._plan_dev, (g["paged_ptr"], g["start_ptr"], self.tiles_ptr) = _upload(
-                [g["paged"], g["out_start"], tiles], device)
+            self._plan_dev, (g["paged_ptr"], g["start_ptr"], self.tiles_ptr, *sp) = _upload(
+                [g["paged"], g["out_start"], tiles, *split], device)
             self.entries_ptr = None
+        if split:
+            self._split["ptrs"] = sp
         self.device = device
+
+    def _plan_split(self, L, arr, heads, window):
+        """The KV split of runs with these heads and window: records to upload
+        ([pieces, units]), or [] for the uncut launch."""
+        self._split = None
+        if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS:
+            return []
+        win = int(window or 0) if self.causal else 0
+        pieces = np.empty((_MAX_PIECES, 4), dtype=np.int32)
+        units = np.empty((_MAX_PIECES, 4), dtype=np.int32)
+        nu, ns, pt = (ctypes.c_int32(0) for _ in range(3))
+        nbytes = ctypes.c_size_t(0)
+        rc = L.hcp_plan_varlen_split(
+            _nbytes_addr(arr)[1], self.num_entries, int(self.causal), win, *heads,
+            pieces.ctypes.data, _MAX_PIECES, units.ctypes.data, ctypes.addressof(nu),
+            ctypes.addressof(ns), ctypes.addressof(pt), ctypes.addressof(nbytes))
+        _lib.check(rc, "hcp_plan_varlen_split")
+        if rc == 0:
+            return []
+        self._split = {"key": (*heads, win), "pieces": rc, "units": nu.value, "slots": ns.value,
+                       "piece_tiles": pt.value, "bytes": nbytes.value}
+        return [pieces[:rc], units[:nu.value]]
 
     def _gathered(self, q: torch.Tensor, num_kv_heads: int) -> int:
         """Gather mode: copy every entry's paged keys into a contiguous K/V
@@ -417,6 +453,30 @@ class VarlenLaunch:
             entries_ptr = self.entries_ptr
             if self._gather is not None:
                 entries_ptr = self._gathered(q, num_kv_heads)
+            if acc is not None:
+                a_o, a_lse = acc
+                if a_o.dtype != q.dtype or a_o.stride(-1) != 1 or a_lse.dtype != torch.float32:
+                    raise ValueError("acc must be (out in q.dtype, float32 lse)")
+            sp = self._split
+            if sp is not None and sp["key"] == (num_heads, num_kv_heads, head_dim, win):
+                # fp32 partials: stream-ordered scratch from torch's caching allocator
+                ws = torch.empty(sp["bytes"], dtype=torch.uint8, device=q.device)
+                rc = L.hcp_attn_fwd_varlen_split(
+                    q.data_ptr(), q.stride(0), q.stride(1),
+                    out.data_ptr(), out.stride(0), out.stride(1),
+                    0 if lse is None else lse.data_ptr(), 0 if lse is None else lse.stride(0),
+                    entries_ptr, self.num_entries,
+                    sp["ptrs"][0], sp["pieces"], sp["piece_tiles"],
+                    sp["ptrs"][1], sp["units"], sp["slots"],
+                    num_heads, num_kv_heads, head_dim, float(scale),
+                    int(self.causal), win, int(self.paged),
+                    *((0, 0, 0, 0, 0, 0) if acc is None else
+                      (a_o.data_ptr(), a_o.stride(0), a_o.stride(1),
+                       a_lse.data_ptr(), a_lse.stride(0), int(bool(acc_is_prefix)))),
+                    ws.data_ptr(), sp["bytes"], _lib.dtype_code(q.dtype),
+                    _lib.stream_ptr(q.device))
+                _lib.check(rc, "hcp_attn_fwd_varlen_split")
+                return
             if acc is None:
                 rc = L.hcp_attn_fwd_varlen(
                     q.data_ptr(), q.stride(0), q.stride(1),
@@ -430,9 +490,6 @@ class VarlenLaunch:
                 )
                 _lib.check(rc, "hcp_attn_fwd_varlen")
                 return
-            a_o, a_lse = acc
-            if a_o.dtype != q.dtype or a_o.stride(-1) != 1 or a_lse.dtype != torch.float32:
-                raise ValueError("acc must be (out in q.dtype, float32 lse)")
             rc = L.hcp_attn_fwd_varlen_merge(
                 q.data_ptr(), q.stride(0), q.stride(1),
                 out.data_ptr(), out.stride(0), out.stride(1),
@@ -469,7 +526,8 @@ def varlen_attn_with_lse(
     if lse is None:
         lse = torch.full((q.shape[1], q.shape[0]), float("-inf"), dtype=torch.float32,
                          device=q.device)
-    VarlenLaunch(entries, causal, paged, q.device).run(q, out, lse, num_kv_heads, scale, window)
+    VarlenLaunch(entries, causal, paged, q.device, heads=(q.shape[1], num_kv_heads, q.shape[2]),
+                 window=window).run(q, out, lse, num_kv_heads, scale, window)
     return out, lse
 
 

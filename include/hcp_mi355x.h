@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define HCP_ABI_VERSION 9
+#define HCP_ABI_VERSION 10
 
 typedef enum hcp_status {
   HCP_OK = 0,
@@ -236,6 +236,80 @@ int hcp_attn_fwd_varlen_merge(const void* q, int64_t q_stride_tok,
                               int64_t acc_stride_tok, int64_t acc_stride_head,
                               const float* acc_lse, int64_t acc_lse_stride_head,
                               int32_t acc_is_prefix, int32_t dtype,
+                              void* stream);
+
+/*
+ * KV split of a prefill launch that would leave CUs idle (few query rows over
+ * many keys: a chunk of a long prompt): past the first `whole_blocks` 128-row
+ * query blocks in dispatch order (the last block first when causal), each
+ * block's keys are cut into pieces of at most `piece_tiles` 64-key tiles,
+ * every piece runs as a workgroup of its own into an fp32 partial (O, LSE) in
+ * `workspace`, and a second kernel merges a block's partials into out / lse
+ * (and the acc state, as hcp_attn_fwd_lse_merge does).  hcp_plan_fwd_split
+ * returns the piece_tiles, whole_blocks and workspace bytes to use, or 0 when
+ * the launch is best left whole (then call hcp_attn_fwd_lse / _merge).  Runs
+ * on the CPU only.
+ */
+int hcp_plan_fwd_split(int64_t tq, int64_t tk, int32_t num_heads,
+                       int32_t num_kv_heads, int32_t head_dim, int32_t causal,
+                       int64_t causal_offset, int32_t window,
+                       int32_t* whole_blocks, size_t* workspace_bytes);
+
+/* hcp_attn_fwd_lse (acc_out and acc_lse NULL) or hcp_attn_fwd_lse_merge on a
+ * KV split of piece_tiles > 0 tiles.  Any piece_tiles is correct; the
+ * workspace must hold (ceil(tq / 128) - whole_blocks) * (pieces of the longest
+ * block cut) * num_heads * 128 * (padded head_dim + 1) floats (HCP_EWORKSPACE if not). */
+int hcp_attn_fwd_lse_split(const void* q, const void* k, const void* v, void* out,
+                           float* lse, int64_t tq, int64_t tk, int32_t num_heads,
+                           int32_t num_kv_heads, int32_t head_dim,
+                           int64_t q_stride_tok, int64_t q_stride_head,
+                           int64_t k_stride_tok, int64_t k_stride_head,
+                           int64_t v_stride_tok, int64_t v_stride_head,
+                           int64_t o_stride_tok, int64_t o_stride_head,
+                           int64_t lse_stride_head, float scale, int32_t causal,
+                           int64_t causal_offset, int32_t window,
+                           const void* acc_out, int64_t acc_stride_tok,
+                           int64_t acc_stride_head, const float* acc_lse,
+                           int64_t acc_lse_stride_head, int32_t acc_is_prefix,
+                           int32_t piece_tiles, int32_t whole_blocks,
+                           void* workspace, size_t workspace_bytes,
+                           int32_t dtype, void* stream);
+
+/*
+ * The same for a varlen batch.  Writes up to `cap` (entry, q_block, piece,
+ * slot) int32 records to host memory `pieces_out`, longest first (slot -1: a
+ * block of one piece, written directly), and up to cap (entry, q_block, first
+ * slot, pieces) records of the split blocks to `units_out`; returns the number
+ * of pieces, or 0 when the batch is best left whole (then use
+ * hcp_plan_varlen_tiles).  A cap of 4096 always suffices.  Checks entries as
+ * hcp_plan_varlen_tiles does.  Runs on the CPU only.
+ */
+int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries,
+                          int32_t causal, int32_t window, int32_t num_heads,
+                          int32_t num_kv_heads, int32_t head_dim,
+                          int32_t* pieces_out, int32_t cap, int32_t* units_out,
+                          int32_t* num_units, int32_t* num_slots,
+                          int32_t* piece_tiles, size_t* workspace_bytes);
+
+/* hcp_attn_fwd_varlen (acc NULL) or hcp_attn_fwd_varlen_merge over the pieces
+ * of hcp_plan_varlen_split (same entries, causal, window and heads; `pieces`
+ * and `units` are DEVICE copies of its records). */
+int hcp_attn_fwd_varlen_split(const void* q, int64_t q_stride_tok,
+                              int64_t q_stride_head, void* out,
+                              int64_t o_stride_tok, int64_t o_stride_head,
+                              float* lse, int64_t lse_stride_head,
+                              const hcp_varlen_entry* entries,
+                              int32_t num_entries, const int32_t* pieces,
+                              int32_t num_pieces, int32_t piece_tiles,
+                              const int32_t* units, int32_t num_units,
+                              int32_t num_slots, int32_t num_heads,
+                              int32_t num_kv_heads, int32_t head_dim,
+                              float scale, int32_t causal, int32_t window,
+                              int32_t paged, const void* acc_out,
+                              int64_t acc_stride_tok, int64_t acc_stride_head,
+                              const float* acc_lse, int64_t acc_lse_stride_head,
+                              int32_t acc_is_prefix, void* workspace,
+                              size_t workspace_bytes, int32_t dtype,
                               void* stream);
 
 /*
