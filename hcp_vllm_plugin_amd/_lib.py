@@ -60,6 +60,7 @@ EXPORTED_SYMBOLS = (
     "hcp_plan_decode_splits",
     "hcp_decode_workspace_bytes",
     "hcp_decode_splitkv",
+    "hcp_decode_splitkv_rows",
     "hcp_decode_splitkv_acc",
     "hcp_decode_splitkv_noalloc",
     "hcp_merge_attn_states",
@@ -191,6 +192,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.hcp_decode_splitkv.restype = ctypes.c_int
     lib.hcp_decode_splitkv.argtypes = [
         _P, _I64, _I64, _P, _I32, _P, _I32, _P, _I32, _P, ctypes.c_size_t,
+        _P, _I64, _I64, _P, _I64, _I32, _I32, _I32, _F, _I32, _P,
+    ]
+    lib.hcp_decode_splitkv_rows.restype = ctypes.c_int
+    lib.hcp_decode_splitkv_rows.argtypes = [
+        _P, _I64, _I64, _P, _I32, _P, _I32, _P, _P, _I32, _P, ctypes.c_size_t,
         _P, _I64, _I64, _P, _I64, _I32, _I32, _I32, _F, _I32, _P,
     ]
     lib.hcp_decode_splitkv_acc.restype = ctypes.c_int

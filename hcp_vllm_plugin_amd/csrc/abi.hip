@@ -745,7 +745,7 @@ static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
                        const void* acc_o, int64_t acc_stride_tok, int64_t acc_stride_head,
                        const float* acc_lse, int64_t acc_lse_stride_head, int32_t num_heads,
                        int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype,
-                       void* stream) {
+                       void* stream, const int32_t* rows = nullptr) {
   int rc = check_heads(num_heads, num_kv_heads, head_dim, dtype, who);
   if (rc) return rc;
   if (num_entries < 0 || num_splits < 0 || num_seqs < 0)
@@ -785,6 +785,7 @@ static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
   rp.ws_o = dp.ws_o;
   rp.ws_lse = dp.ws_lse;
   rp.seq_partial_start = seq_partial_start;
+  rp.rows = rows;
   rp.num_seqs = num_seqs;
   rp.out = out;
   rp.o_stride_tok = o_stride_tok;
@@ -815,6 +816,22 @@ int hcp_decode_splitkv(const void* q, int64_t q_stride_tok, int64_t q_stride_hea
                      workspace_bytes, out, o_stride_tok, o_stride_head, lse, lse_stride_head,
                      nullptr, 0, 0, nullptr, 0, num_heads, num_kv_heads, head_dim, scale,
                      dtype, stream);
+}
+
+int hcp_decode_splitkv_rows(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                            const hcp_varlen_entry* entries, int32_t num_entries,
+                            const hcp_decode_split* splits, int32_t num_splits,
+                            const int32_t* seq_partial_start, const int32_t* seq_rows,
+                            int32_t num_seqs, void* workspace, size_t workspace_bytes, void* out,
+                            int64_t o_stride_tok, int64_t o_stride_head, float* lse,
+                            int64_t lse_stride_head, int32_t num_heads, int32_t num_kv_heads,
+                            int32_t head_dim, float scale, int32_t dtype, void* stream) {
+  const char* who = "hcp_decode_splitkv_rows";
+  if (num_seqs > 0 && !seq_rows) return fail(HCP_EINVAL, "%s: null seq_rows", who);
+  return decode_impl(who, q, q_stride_tok, q_stride_head, entries, num_entries, splits,
+                     num_splits, seq_partial_start, num_seqs, workspace, workspace_bytes, out,
+                     o_stride_tok, o_stride_head, lse, lse_stride_head, nullptr, 0, 0, nullptr,
+                     0, num_heads, num_kv_heads, head_dim, scale, dtype, stream, seq_rows);
 }
 
 int hcp_decode_splitkv_acc(const void* q, int64_t q_stride_tok, int64_t q_stride_head,

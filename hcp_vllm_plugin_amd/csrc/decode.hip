@@ -462,6 +462,7 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
   const int ng = p.groups;  // column groups; group gi takes partials gi, gi + ng, ...
   const int sh = blockIdx.x;
   const int seq = sh / p.num_heads, head = sh % p.num_heads;
+  const int row = p.rows != nullptr ? p.rows[seq] : seq;  // of out, lse and acc
   const int tid = threadIdx.x;
   const int d = tid % D, gi = tid / D;
   const int p0 = p.seq_partial_start[seq], p1 = p.seq_partial_start[seq + 1];
@@ -475,10 +476,10 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
   // of them happens before the barriers below, every write after them
   float acc_l = -INFINITY, acc_v = 0.f;
   if (p.acc_lse != nullptr) {
-    acc_l = p.acc_lse[static_cast<int64_t>(head) * p.acc_lse_stride_head + seq];
+    acc_l = p.acc_lse[static_cast<int64_t>(head) * p.acc_lse_stride_head + row];
     if (acc_l == INFINITY) acc_l = -INFINITY;  // merge_attn_states reads +inf as empty
     const uint16_t* arow = reinterpret_cast<const uint16_t*>(p.acc_o) +
-                           seq * p.acc_stride_tok + static_cast<int64_t>(head) * p.acc_stride_head;
+                           row * p.acc_stride_tok + static_cast<int64_t>(head) * p.acc_stride_head;
     acc_v = d < p.head_dim ? Elem<T>::to_float(arow[d]) : 0.f;
   }
 
@@ -537,11 +538,11 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
     o = O / S;
     lse = M + __logf(S);
   }
-  uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + seq * p.o_stride_tok +
+  uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + row * p.o_stride_tok +
                    static_cast<int64_t>(head) * p.o_stride_head;
   if (d < p.head_dim) orow[d] = Elem<T>::from_float(o);
   if (p.lse != nullptr && d == 0)
-    p.lse[static_cast<int64_t>(head) * p.lse_stride_head + seq] = lse;
+    p.lse[static_cast<int64_t>(head) * p.lse_stride_head + row] = lse;
 }
 
 template <int D, typename T>

@@ -101,6 +101,7 @@ struct RedParams {
   const float* ws_o;
   const float* ws_lse;
   const int32_t* seq_partial_start;
+  const int32_t* rows;  // output row of each sequence (NULL: its index)
   int32_t num_seqs;
   void* out;
   int64_t o_stride_tok, o_stride_head;

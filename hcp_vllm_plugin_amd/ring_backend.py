@@ -541,6 +541,7 @@ class _Plan:
         self.local: list = []           # causal entries over the paged cache
         self.peer_rounds: list = []     # per round: {"contig": [...], "paged": [...]}
         self.any_peer = False
+        self.decode: list = []  # single-token rows for the decode kernel: (q row, segments)
         self.ring: list = []  # decode-ring rows: (r, q row, tk, ring state, bt row, block 0)
 
 
@@ -685,8 +686,21 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             if peer_end > 0:
                 _probe_chunk_a_writes(block_table[r], peer_end, pc.block_size)
 
+    def _decode_rows_apart(self, qsl, seq_lens) -> bool:
+        """Whether a mixed batch's single-token rows leave the prefill launch
+        for a decode launch of their own.  In the prefill launch such a row is
+        a 128-row block per query head, each reading its KV head's keys again:
+        about half a microsecond of a CU per 64 keys and head.  The decode
+        launch reads the keys once, but is two more kernels (about 20 us with
+        their planning).  28 / 4 x 128 heads, 512 new tokens next to 32 rows of
+        512 - 8192 keys, two layers: 543 us in one launch each, 398 us apart."""
+        tiles = sum(-(-int(tk) // 64) for r, tk in enumerate(seq_lens) if qsl[r + 1] - qsl[r] == 1)
+        return tiles * self.num_heads * 0.5 / 256 > 20
+
     def _plan(self, layer_name, qsl, seq_lens, block_table, first_blocks, pc, split):
         plan = _Plan()
+        n = len(seq_lens)
+        apart = qsl != list(range(n + 1)) and self._decode_rows_apart(qsl, seq_lens)
         ring_on = _decode_ring_enabled() and bool(DECODE_RING_MAP)
         for r in range(len(seq_lens)):
             qs, qe = qsl[r], qsl[r + 1]
@@ -715,6 +729,15 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 peer_segs.append(segment_paged(pc, row, 0, peer_end))
             else:
                 peer_end = 0
+            if apart and tq == 1:
+                # one query at position tk - 1: inside the prefix it sees the
+                # whole local range, past it the local keys (the last `w` of
+                # them) and every staged chunk
+                lo = peer_end if peer_end < tk else 0
+                segs = [segment_paged(pc, row, lo, tk - lo)]
+                segs = window_tail(segs, self.sliding_window)
+                plan.decode.append((qs, segs + (peer_segs if 0 < peer_end < tk else [])))
+                continue
             if peer_end == 0:
                 plan.local.append(make_entry(qs, tq, segment_paged(pc, row, 0, tk), qpos0))
                 continue
@@ -789,6 +812,11 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         else:
             if plan.local or plan.any_peer:
                 self._forward_prefill(query, out, plan)
+            if plan.decode:
+                DecodeBatch([segs for _, segs in plan.decode], self.num_heads, self.num_kv_heads,
+                            self.head_size, query.device,
+                            rows=[qs for qs, _ in plan.decode]).run(query, out, None, self.scale)
+                _count("decode")
             parts = {}
             for (r, qs, *_r) in plan.ring:
                 parts[r] = self._local_partial(query[qs:qs + 1], ring_local[r])
@@ -984,30 +1012,34 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             tq = np.diff(np.asarray(qsl, dtype=np.int64))
             tk = np.asarray(seq_lens, dtype=np.int64)
             rows = np.arange(n, dtype=np.int64)
-            if is_decode:
-                # one query at the end of its keys: all of them visible, or
-                # the last `w` of them (ring_backend.py:397-398)
-                start = np.zeros(n, np.int64) if w is None else np.maximum(tk - w, 0)
-                tmpl = paged_entry_array(pc, block_table, rows, rows, 1, 0, start, tk - start)
-            else:
-                sel = tq > 0
-                tmpl = paged_entry_array(pc, block_table, rows[sel], qs[sel], tq[sel],
-                                         (tk - tq)[sel], 0, tk[sel])
+            dec = tq == 1
+            if not is_decode and not self._decode_rows_apart(qsl, seq_lens):
+                dec[:] = False
+            pre = (tq > 0) & ~dec
+            # one query at the end of its keys: all of them visible, or
+            # the last `w` of them (ring_backend.py:397-398)
+            start = np.zeros(n, np.int64) if w is None else np.maximum(tk - w, 0)
+            tmpl = (paged_entry_array(pc, block_table, rows[pre], qs[pre], tq[pre],
+                                      (tk - tq)[pre], 0, tk[pre]),
+                    paged_entry_array(pc, block_table, rows[dec], qs[dec], 1, 0, start[dec],
+                                      (tk - start)[dec]))
             _STEP["fast"][key] = tmpl
-        ent = tmpl.copy()
-        ent["k_addr"] = pc.k_addr
-        ent["v_addr"] = pc.v_addr
         keep = (kv_cache, block_table)
-        if is_decode:
-            DecodeBatch.from_entries(ent, self.num_heads, self.num_kv_heads, self.head_size,
-                                     query.device, keep=keep).run(query, out, None, self.scale)
-            _count("decode")
-        else:
+        pre, dec = (t.copy() for t in tmpl)
+        for ent in (pre, dec):
+            ent["k_addr"] = pc.k_addr
+            ent["v_addr"] = pc.v_addr
+        if len(pre):
             lse = torch.empty((self.num_heads, query.shape[0]), dtype=torch.float32,
                               device=query.device)
-            VarlenLaunch(ent, True, True, query.device, keep=keep, heads=self._heads,
+            VarlenLaunch(pre, True, True, query.device, keep=keep, heads=self._heads,
                          window=w).run(query, out, lse, self.num_kv_heads, self.scale, w)
             _count("attn")
+        if len(dec):
+            DecodeBatch.from_entries(
+                dec, self.num_heads, self.num_kv_heads, self.head_size, query.device, keep=keep,
+                rows=None if is_decode else dec["q_start"]).run(query, out, None, self.scale)
+            _count("decode")
 
     def _forward_prefill(self, query, out, plan: _Plan) -> None:
         dev = query.device

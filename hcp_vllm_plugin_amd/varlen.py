@@ -594,12 +594,14 @@ class DecodeBatch:
     """
 
     def __init__(self, segments: list[list[KvSegment]], num_heads: int, num_kv_heads: int,
-                 head_dim: int, device: torch.device, split_tokens: int | None = None):
+                 head_dim: int, device: torch.device, split_tokens: int | None = None,
+                 rows: list[int] | None = None):
+        """``rows``: the q / out / lse row of each sequence (default: its index)."""
         L = _lib.lib()
         entries, seq_of = [], []
         for s, segs in enumerate(segments):
             for seg in segs:
-                entries.append(make_entry(s, 1, seg, 0))
+                entries.append(make_entry(s if rows is None else rows[s], 1, seg, 0))
                 seq_of.append(s)
         self.num_seqs = len(segments)
         self.num_entries = len(entries)
@@ -621,10 +623,7 @@ class DecodeBatch:
         self.num_heads = num_heads
         self.num_kv_heads = num_kv_heads
         self.head_dim = head_dim
-        self._plan_dev, (self.entries_ptr, self.splits_ptr, self.starts_ptr) = _upload(
-            [arr, splits, starts], device)
-        self.ws_bytes = int(L.hcp_decode_workspace_bytes(max(rc, 1), num_heads, head_dim))
-        self.device = device
+        self._upload_plan(arr, splits, starts, rows, device)
         # the segments point at K/V / cache / block-table storage by address
         self._keep = [getattr(e, "_keep", None) for e in entries]
 
@@ -632,12 +631,13 @@ class DecodeBatch:
     def from_entries(cls, entries: np.ndarray, num_heads: int, num_kv_heads: int,
                      head_dim: int, device: torch.device, split_tokens: int | None = None,
                      keep=None, entry_seq: np.ndarray | None = None,
-                     num_seqs: int | None = None) -> "DecodeBatch":
+                     num_seqs: int | None = None, rows=None) -> "DecodeBatch":
         """Entries given as an ENTRY_DTYPE array; ``keep`` holds the tensors
         it points into.  By default one entry per sequence (sequence i = entry
         i = query row i); with ``entry_seq`` (int32, non-decreasing) entry j
         belongs to sequence ``entry_seq[j]`` of ``num_seqs`` -- a sequence's
-        peer chunks and its local segment."""
+        peer chunks and its local segment.  ``rows``: the out / lse row of
+        each sequence (default: its index); the entries' q_start name the q rows."""
         if entries.dtype != ENTRY_DTYPE or not entries.flags.c_contiguous:
             raise ValueError("entry array must be contiguous ENTRY_DTYPE")
         L = _lib.lib()
@@ -672,12 +672,20 @@ class DecodeBatch:
         self.num_heads = num_heads
         self.num_kv_heads = num_kv_heads
         self.head_dim = head_dim
-        self._plan_dev, (self.entries_ptr, self.splits_ptr, self.starts_ptr) = _upload(
-            [arr, splits, starts], device)
-        self.ws_bytes = int(L.hcp_decode_workspace_bytes(max(rc, 1), num_heads, head_dim))
-        self.device = device
+        self._upload_plan(arr, splits, starts, rows, device)
         self._keep = keep
         return self
+
+    def _upload_plan(self, arr, splits, starts, rows, device) -> None:
+        extra = [] if rows is None else [np.ascontiguousarray(rows, dtype=np.int32)]
+        if extra and len(extra[0]) != self.num_seqs:
+            raise ValueError("rows needs one row per sequence")
+        self._plan_dev, (self.entries_ptr, self.splits_ptr, self.starts_ptr, *rp) = _upload(
+            [arr, splits, starts, *extra], device)
+        self.rows_ptr = rp[0] if rp else None
+        self.ws_bytes = int(_lib.lib().hcp_decode_workspace_bytes(
+            max(self.num_splits, 1), self.num_heads, self.head_dim))
+        self.device = device
 
     def rebind(self, entries: np.ndarray, keep=None) -> "DecodeBatch":
         """The same plan (splits, partial slots) over new entries of the same
@@ -707,6 +715,8 @@ class DecodeBatch:
         nothing is allocated; calls overlapping on one GPU race).  Plans whose
         partials exceed ``_lib.NOALLOC_SCRATCH_BYTES`` raise."""
         L = _lib.lib()
+        if self.rows_ptr is not None and (noalloc or acc is not None):
+            raise ValueError("a plan with output rows has neither accumulator nor noalloc form")
         if noalloc:
             if acc is not None:
                 raise ValueError("noalloc decode has no accumulator form")
@@ -736,7 +746,10 @@ class DecodeBatch:
                 self.num_heads, self.num_kv_heads, self.head_dim, float(scale),
                 _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device))
         with torch.cuda.device(q.device):
-            if acc is None:
+            if self.rows_ptr is not None:
+                rc = L.hcp_decode_splitkv_rows(*head[:8], self.rows_ptr, *head[8:], *tail)
+                name = "hcp_decode_splitkv_rows"
+            elif acc is None:
                 rc = L.hcp_decode_splitkv(*head, *tail)
                 name = "hcp_decode_splitkv"
             else:

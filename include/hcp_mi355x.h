@@ -363,6 +363,26 @@ int hcp_decode_splitkv(const void* q, int64_t q_stride_tok,
                        int32_t dtype, void* stream);
 
 /*
+ * hcp_decode_splitkv for sequences that are not all of the batch: the output
+ * row (of out and lse) of sequence s is seq_rows[s], a DEVICE array.  For the
+ * single-token rows of a batch that also holds prefill chunks.
+ */
+int hcp_decode_splitkv_rows(const void* q, int64_t q_stride_tok,
+                            int64_t q_stride_head,
+                            const hcp_varlen_entry* entries,
+                            int32_t num_entries,
+                            const hcp_decode_split* splits,
+                            int32_t num_splits,
+                            const int32_t* seq_partial_start,
+                            const int32_t* seq_rows, int32_t num_seqs,
+                            void* workspace, size_t workspace_bytes, void* out,
+                            int64_t o_stride_tok, int64_t o_stride_head,
+                            float* lse, int64_t lse_stride_head,
+                            int32_t num_heads, int32_t num_kv_heads,
+                            int32_t head_dim, float scale, int32_t dtype,
+                            void* stream);
+
+/*
  * Split-KV decode merged into a running accumulator: the decode ring's step
  * on one node.  Replaces RingDecodeNode.handle_packet's partial over
  * cat(chunk snapshot, growth) and _merge_pair (ring_decode.py:224-237,
