@@ -12,6 +12,7 @@ point raises ``RuntimeError``.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -56,11 +57,13 @@ EXPORTED_SYMBOLS = (
     "hcp_plan_fwd_split",
     "hcp_attn_fwd_lse_split",
     "hcp_plan_varlen_split",
-    "hcp_attn_fwd_varlen_split",
+    "hcp_varlen_launch",
+    "hcp_fetch_metadata",
     "hcp_plan_decode_splits",
     "hcp_decode_workspace_bytes",
     "hcp_decode_splitkv",
-    "hcp_decode_splitkv_rows",
+    "hcp_plan_decode_lists",
+    "hcp_decode_launch",
     "hcp_decode_splitkv_acc",
     "hcp_decode_splitkv_noalloc",
     "hcp_merge_attn_states",
@@ -125,6 +128,82 @@ class DecodeSplit(ctypes.Structure):
     ]
 
 
+class DecodeArgs(ctypes.Structure):
+    """``hcp_decode_args`` (include/hcp_mi355x.h)."""
+
+    _fields_ = [
+        ("q", ctypes.c_uint64),
+        ("q_stride_tok", ctypes.c_int64),
+        ("q_stride_head", ctypes.c_int64),
+        ("works", ctypes.c_uint64),
+        ("seq_partial_start", ctypes.c_uint64),
+        ("seq_rows", ctypes.c_uint64),
+        ("workspace", ctypes.c_uint64),
+        ("workspace_bytes", ctypes.c_uint64),
+        ("acc_o", ctypes.c_uint64),
+        ("acc_stride_tok", ctypes.c_int64),
+        ("acc_stride_head", ctypes.c_int64),
+        ("acc_lse", ctypes.c_uint64),
+        ("acc_lse_stride_head", ctypes.c_int64),
+        ("out", ctypes.c_uint64),
+        ("o_stride_tok", ctypes.c_int64),
+        ("o_stride_head", ctypes.c_int64),
+        ("lse", ctypes.c_uint64),
+        ("lse_stride_head", ctypes.c_int64),
+        ("kv_base", ctypes.c_uint64),
+        ("num_works", ctypes.c_int32),
+        ("num_wgs", ctypes.c_int32),
+        ("num_seqs", ctypes.c_int32),
+        ("num_heads", ctypes.c_int32),
+        ("num_kv_heads", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32),
+        ("dtype", ctypes.c_int32),
+        ("use_scratch", ctypes.c_int32),
+        ("scale", ctypes.c_float),
+        ("reserved", ctypes.c_int32),
+    ]
+
+
+class VarlenArgs(ctypes.Structure):
+    """``hcp_varlen_args`` (include/hcp_mi355x.h)."""
+
+    _fields_ = [
+        ("q", ctypes.c_uint64),
+        ("q_stride_tok", ctypes.c_int64),
+        ("q_stride_head", ctypes.c_int64),
+        ("out", ctypes.c_uint64),
+        ("o_stride_tok", ctypes.c_int64),
+        ("o_stride_head", ctypes.c_int64),
+        ("lse", ctypes.c_uint64),
+        ("lse_stride_head", ctypes.c_int64),
+        ("entries", ctypes.c_uint64),
+        ("tiles", ctypes.c_uint64),
+        ("units", ctypes.c_uint64),
+        ("workspace", ctypes.c_uint64),
+        ("workspace_bytes", ctypes.c_uint64),
+        ("acc_o", ctypes.c_uint64),
+        ("acc_stride_tok", ctypes.c_int64),
+        ("acc_stride_head", ctypes.c_int64),
+        ("acc_lse", ctypes.c_uint64),
+        ("acc_lse_stride_head", ctypes.c_int64),
+        ("kv_base", ctypes.c_uint64),
+        ("num_entries", ctypes.c_int32),
+        ("num_tiles", ctypes.c_int32),
+        ("piece_tiles", ctypes.c_int32),
+        ("num_units", ctypes.c_int32),
+        ("num_slots", ctypes.c_int32),
+        ("num_heads", ctypes.c_int32),
+        ("num_kv_heads", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32),
+        ("dtype", ctypes.c_int32),
+        ("causal", ctypes.c_int32),
+        ("window", ctypes.c_int32),
+        ("paged", ctypes.c_int32),
+        ("acc_is_prefix", ctypes.c_int32),
+        ("scale", ctypes.c_float),
+    ]
+
+
 _lock = threading.Lock()
 _lib = None
 
@@ -179,11 +258,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.hcp_plan_varlen_split.argtypes = [
         _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P, _P, _P, _P, _P,
     ]
-    lib.hcp_attn_fwd_varlen_split.restype = ctypes.c_int
-    lib.hcp_attn_fwd_varlen_split.argtypes = [
-        _P, _I64, _I64, _P, _I64, _I64, _P, _I64,
-        _P, _I32, _P, _I32, _I32, _P, _I32, _I32, _I32, _I32, _I32, _F, _I32, _I32, _I32,
-        _P, _I64, _I64, _P, _I64, _I32, _P, ctypes.c_size_t, _I32, _P,
+    lib.hcp_varlen_launch.restype = ctypes.c_int
+    lib.hcp_varlen_launch.argtypes = [_P, _P]
+    lib.hcp_fetch_metadata.restype = ctypes.c_int
+    lib.hcp_fetch_metadata.argtypes = [
+        _P, _I32, _I64, _P, _I32, _I64, _P, _I32, _I64, _I32, _P, _P,
     ]
     lib.hcp_plan_decode_splits.restype = ctypes.c_int
     lib.hcp_plan_decode_splits.argtypes = [_P, _I32, _P, _I32, _I32, _I32, _P, _I32, _P]
@@ -194,11 +273,12 @@ def _declare(lib: ctypes.CDLL) -> None:
         _P, _I64, _I64, _P, _I32, _P, _I32, _P, _I32, _P, ctypes.c_size_t,
         _P, _I64, _I64, _P, _I64, _I32, _I32, _I32, _F, _I32, _P,
     ]
-    lib.hcp_decode_splitkv_rows.restype = ctypes.c_int
-    lib.hcp_decode_splitkv_rows.argtypes = [
-        _P, _I64, _I64, _P, _I32, _P, _I32, _P, _P, _I32, _P, ctypes.c_size_t,
-        _P, _I64, _I64, _P, _I64, _I32, _I32, _I32, _F, _I32, _P,
+    lib.hcp_plan_decode_lists.restype = ctypes.c_int
+    lib.hcp_plan_decode_lists.argtypes = [
+        _P, _I32, _P, _I32, _I32, _I32, _P, _P, _I32, _P, _P,
     ]
+    lib.hcp_decode_launch.restype = ctypes.c_int
+    lib.hcp_decode_launch.argtypes = [_P, _P]
     lib.hcp_decode_splitkv_acc.restype = ctypes.c_int
     lib.hcp_decode_splitkv_acc.argtypes = [
         _P, _I64, _I64, _P, _I32, _P, _I32, _P, _I32, _P, ctypes.c_size_t,
@@ -270,3 +350,14 @@ def dtype_code(dt: torch.dtype) -> int:
 def stream_ptr(device: torch.device) -> int:
     """Raw hipStream_t of torch's current stream on ``device``."""
     return torch.cuda.current_stream(device).cuda_stream
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, without its two calls into the runtime
+    when ``device`` is the current one already."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _SAME_DEVICE
+    return torch.cuda.device(device)

@@ -580,7 +580,8 @@ static int fwd_varlen_impl(const char* who, const void* q, int64_t q_stride_tok,
                            const int32_t* tiles, int32_t num_tiles, int32_t num_heads,
                            int32_t num_kv_heads, int32_t head_dim, float scale, int32_t causal,
                            int32_t window, int32_t paged, int32_t dtype, void* stream,
-                           const AccArgs* acc, const SplitArgs* split = nullptr) {
+                           const AccArgs* acc, const SplitArgs* split = nullptr,
+                           uint64_t kv_base = 0) {
   int rc = check_heads(num_heads, num_kv_heads, head_dim, dtype, who);
   if (rc) return rc;
   if (num_entries < 0 || num_tiles < 0) return fail(HCP_EINVAL, "%s: negative counts", who);
@@ -607,6 +608,7 @@ static int fwd_varlen_impl(const char* who, const void* q, int64_t q_stride_tok,
   p.entries = entries;
   p.tiles = tiles;
   p.num_tiles = num_tiles;
+  p.kv_base = kv_base;
   p.num_heads = num_heads;
   p.num_kv_heads = num_kv_heads;
   p.group = num_heads / num_kv_heads;
@@ -659,27 +661,21 @@ int hcp_attn_fwd_varlen_merge(const void* q, int64_t q_stride_tok, int64_t q_str
                          window, paged, dtype, stream, &acc);
 }
 
-int hcp_attn_fwd_varlen_split(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
-                              void* out, int64_t o_stride_tok, int64_t o_stride_head, float* lse,
-                              int64_t lse_stride_head, const hcp_varlen_entry* entries,
-                              int32_t num_entries, const int32_t* pieces, int32_t num_pieces,
-                              int32_t piece_tiles, const int32_t* units, int32_t num_units,
-                              int32_t num_slots, int32_t num_heads, int32_t num_kv_heads,
-                              int32_t head_dim, float scale, int32_t causal, int32_t window,
-                              int32_t paged, const void* acc_out, int64_t acc_stride_tok,
-                              int64_t acc_stride_head, const float* acc_lse,
-                              int64_t acc_lse_stride_head, int32_t acc_is_prefix,
-                              void* workspace, size_t workspace_bytes, int32_t dtype,
-                              void* stream) {
-  const char* who = "hcp_attn_fwd_varlen_split";
-  if (piece_tiles <= 0) return fail(HCP_EINVAL, "%s: piece_tiles must be > 0", who);
-  const AccArgs acc{acc_out, acc_stride_tok, acc_stride_head, acc_lse, acc_lse_stride_head,
-                    acc_is_prefix};
-  const SplitArgs split{piece_tiles, 0, workspace, workspace_bytes, units, num_units, num_slots};
-  return fwd_varlen_impl(who, q, q_stride_tok, q_stride_head, out, o_stride_tok, o_stride_head,
-                         lse, lse_stride_head, entries, num_entries, pieces, num_pieces,
-                         num_heads, num_kv_heads, head_dim, scale, causal, window, paged, dtype,
-                         stream, acc_out || acc_lse ? &acc : nullptr, &split);
+int hcp_varlen_launch(const hcp_varlen_args* a, void* stream) {
+  const char* who = "hcp_varlen_launch";
+  if (!a) return fail(HCP_EINVAL, "%s: null arguments", who);
+  if (a->piece_tiles < 0) return fail(HCP_EINVAL, "%s: negative piece_tiles", who);
+  if (a->kv_base & 15) return fail(HCP_EINVAL, "%s: kv_base not 16-byte aligned", who);
+  const AccArgs acc{a->acc_o, a->acc_stride_tok, a->acc_stride_head, a->acc_lse,
+                    a->acc_lse_stride_head, a->acc_is_prefix};
+  const SplitArgs split{a->piece_tiles, 0, a->workspace, a->workspace_bytes, a->units,
+                        a->num_units, a->num_slots};
+  return fwd_varlen_impl(who, a->q, a->q_stride_tok, a->q_stride_head, a->out, a->o_stride_tok,
+                         a->o_stride_head, a->lse, a->lse_stride_head, a->entries, a->num_entries,
+                         a->tiles, a->num_tiles, a->num_heads, a->num_kv_heads, a->head_dim,
+                         a->scale, a->causal, a->window, a->paged, a->dtype, stream,
+                         a->acc_o || a->acc_lse ? &acc : nullptr,
+                         a->piece_tiles > 0 ? &split : nullptr, a->kv_base);
 }
 
 int hcp_plan_decode_splits(const hcp_varlen_entry* entries, int32_t num_entries,
@@ -727,6 +723,138 @@ int hcp_plan_decode_splits(const hcp_varlen_entry* entries, int32_t num_entries,
   return n;
 }
 
+int hcp_plan_decode_lists(const hcp_varlen_entry* entries, int32_t num_entries,
+                          const int32_t* entry_seq, int32_t num_seqs,
+                          int32_t workgroups, int32_t split_tokens, hcp_decode_work* works,
+                          int32_t* work_entry, int32_t cap, int32_t* seq_partial_start,
+                          int32_t* num_wgs) try {
+  const char* who = "hcp_plan_decode_lists";
+  if (num_entries < 0 || num_seqs < 0 || workgroups < 0 || split_tokens < 0 ||
+      (workgroups > 0) == (split_tokens > 0))
+    return fail(HCP_EINVAL, "%s: bad sizes", who);
+  if ((num_entries > 0 && (!entries || !entry_seq)) || !seq_partial_start || !num_wgs ||
+      (cap > 0 && !works))
+    return fail(HCP_EINVAL, "%s: null pointer", who);
+  // lengths in chunks of 32 keys, the kernel's step
+  auto chunks = [&](int32_t i) { return (entries[i].kv.len + 31) / 32; };
+  int64_t total = 0;
+  int32_t cur = 0;
+  for (int32_t i = 0; i < num_entries; ++i) {
+    const int32_t s = entry_seq[i];
+    if (s < 0 || s >= num_seqs || s < cur)
+      return fail(HCP_EINVAL, "%s: entry %d: sequence %d out of order/range", who, i, s);
+    cur = s;
+    if (entries[i].q_len != 1)
+      return fail(HCP_EINVAL, "%s: entry %d: q_len must be 1 for decode", who, i);
+    if (entries[i].kv.len < 0 || entries[i].kv.len > INT32_MAX)
+      return fail(HCP_EINVAL, "%s: entry %d: kv len out of range", who, i);
+    total += chunks(i);
+  }
+  // Each split costs its workgroup its start and its end, as long as about 8
+  // chunks take; the smallest budget (chunks + splits * kSplitCost) that
+  // `wgs` workgroups can hold the batch in is the one to fill them to.  At
+  // least two chunks (64 keys) to a workgroup.
+  constexpr int64_t kSplitCost = 8;
+  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups, (total + 1) / 2));
+  // Chunks of an entry with `left` to go that a workgroup with `room` takes:
+  // none if it would only fit a fragment, the rest if no more than a
+  // fragment would stay, else whole steps of 4 (one for each of the 4 waves).
+  auto take = [&](int64_t left, int64_t room) -> int64_t {
+    room -= kSplitCost;
+    if (left <= room) return left;
+    const int64_t step = room >= 16 ? 4 : 1;
+    const int64_t t = room / step * step;
+    return room < 2 ? 0 : t;
+  };
+  auto fits = [&](int64_t budget) {
+    int64_t w = 0, room = budget;
+    for (int32_t i = 0; i < num_entries; ++i)
+      for (int64_t left = chunks(i); left > 0;) {
+        const int64_t t = take(left, room);
+        if (t > 0) {
+          left -= t;
+          room -= t + kSplitCost;
+        }
+        if (left > 0) {
+          room = budget;
+          if (++w >= wgs) return false;
+        }
+      }
+    return true;
+  };
+  int64_t budget = kSplitCost + std::max<int64_t>(2, (total + wgs - 1) / wgs);
+  if (split_tokens == 0) {
+    int64_t lo = budget, hi = budget + kSplitCost * (num_entries / wgs + 2) + 8;
+    while (!fits(hi)) hi += hi / 2;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) / 2;
+      if (fits(mid)) hi = mid;
+      else lo = mid + 1;
+    }
+    budget = lo;
+  }
+  struct Piece {
+    int32_t entry, begin, end;
+    int64_t wg;
+  };
+  std::vector<Piece> v;
+  int64_t w = 0, room = budget;
+  cur = 0;
+  seq_partial_start[0] = 0;
+  for (int32_t i = 0; i < num_entries; ++i) {
+    while (cur < entry_seq[i]) seq_partial_start[++cur] = static_cast<int32_t>(v.size());
+    const int64_t len = entries[i].kv.len, c = chunks(i);
+    if (split_tokens > 0) {
+      // pieces of at most split_tokens keys, a workgroup each
+      const int64_t np = (len + split_tokens - 1) / split_tokens;
+      const int64_t st = np > 0 ? (len + np - 1) / np : 1;
+      for (int64_t b = 0; b < len; b += st)
+        v.push_back({i, static_cast<int32_t>(b), static_cast<int32_t>(std::min(len, b + st)), w++});
+      continue;
+    }
+    for (int64_t at = 0; at < c;) {
+      const int64_t t = take(c - at, room);
+      if (t > 0) {
+        v.push_back({i, static_cast<int32_t>(at * 32),
+                     static_cast<int32_t>(std::min(len, (at + t) * 32)), w});
+        at += t;
+        room -= t + kSplitCost;
+      }
+      if (at < c) {
+        room = budget;
+        ++w;
+      }
+    }
+  }
+  while (cur < num_seqs) seq_partial_start[++cur] = static_cast<int32_t>(v.size());
+  const int32_t n = static_cast<int32_t>(v.size());
+  if (n > cap) return fail(HCP_EWORKSPACE, "%s: %d splits, cap %d", who, n, cap);
+  // records: the first split of each workgroup in workgroup order, then the
+  // others, each linked from the one before it
+  int32_t heads = 0, more = 0;
+  for (int32_t j = 0; j < n; ++j) heads += j == 0 || v[j].wg != v[j - 1].wg;
+  int32_t h = 0, prev = -1;
+  for (int32_t j = 0; j < n; ++j) {
+    const Piece& x = v[j];
+    const bool head = j == 0 || x.wg != v[j - 1].wg;
+    const int32_t at = head ? h++ : heads + more++;
+    hcp_decode_work& r = works[at];
+    r = hcp_decode_work{};
+    if (work_entry) work_entry[at] = x.entry;
+    r.e = entries[x.entry];
+    r.key_begin = x.begin;
+    r.key_end = x.end;
+    r.slot = j;
+    r.next = -1;
+    if (!head) works[prev].next = at;
+    prev = at;
+  }
+  *num_wgs = heads;
+  return n;
+} catch (const std::bad_alloc&) {
+  return fail(HCP_EINVAL, "hcp_plan_decode_lists: out of host memory");
+}
+
 size_t hcp_decode_workspace_bytes(int32_t num_splits, int32_t num_heads, int32_t head_dim) {
   if (num_splits <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
   head_dim = hcp::padded_head_dim(head_dim);  // partials keep the kernel's width
@@ -735,6 +863,14 @@ size_t hcp_decode_workspace_bytes(int32_t num_splits, int32_t num_heads, int32_t
   const size_t o_al = (o + 255) & ~static_cast<size_t>(255);
   return o_al + n * sizeof(float);
 }
+
+// What hcp_decode_launch can say beyond the plain entry points.
+struct DecodeExtra {
+  const hcp_decode_work* works = nullptr;
+  int32_t num_wgs = 0;
+  const int32_t* rows = nullptr;
+  uint64_t kv_base = 0;
+};
 
 static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
                        int64_t q_stride_head, const hcp_varlen_entry* entries,
@@ -745,13 +881,13 @@ static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
                        const void* acc_o, int64_t acc_stride_tok, int64_t acc_stride_head,
                        const float* acc_lse, int64_t acc_lse_stride_head, int32_t num_heads,
                        int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype,
-                       void* stream, const int32_t* rows = nullptr) {
+                       void* stream, const DecodeExtra& x = DecodeExtra()) {
   int rc = check_heads(num_heads, num_kv_heads, head_dim, dtype, who);
   if (rc) return rc;
   if (num_entries < 0 || num_splits < 0 || num_seqs < 0)
     return fail(HCP_EINVAL, "%s: negative counts", who);
   if (num_seqs == 0) return HCP_OK;
-  if (!q || !out || !seq_partial_start || (num_splits > 0 && (!entries || !splits)))
+  if (!q || !out || !seq_partial_start || (num_splits > 0 && !x.works && (!entries || !splits)))
     return fail(HCP_EINVAL, "%s: null pointer", who);
   if (!aligned16(q)) return fail(HCP_EINVAL, "%s: q not 16-byte aligned", who);
   if ((q_stride_tok | q_stride_head) % 8)
@@ -773,6 +909,9 @@ static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
   dp.entries = entries;
   dp.splits = splits;
   dp.num_splits = num_splits;
+  dp.works = x.works;
+  dp.num_wgs = x.works ? x.num_wgs : num_splits;
+  dp.kv_base = x.kv_base;
   dp.ws_o = static_cast<float*>(workspace);
   dp.ws_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + o_al);
   dp.num_heads = num_heads;
@@ -785,7 +924,7 @@ static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
   rp.ws_o = dp.ws_o;
   rp.ws_lse = dp.ws_lse;
   rp.seq_partial_start = seq_partial_start;
-  rp.rows = rows;
+  rp.rows = x.rows;
   rp.num_seqs = num_seqs;
   rp.out = out;
   rp.o_stride_tok = o_stride_tok;
@@ -816,22 +955,6 @@ int hcp_decode_splitkv(const void* q, int64_t q_stride_tok, int64_t q_stride_hea
                      workspace_bytes, out, o_stride_tok, o_stride_head, lse, lse_stride_head,
                      nullptr, 0, 0, nullptr, 0, num_heads, num_kv_heads, head_dim, scale,
                      dtype, stream);
-}
-
-int hcp_decode_splitkv_rows(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
-                            const hcp_varlen_entry* entries, int32_t num_entries,
-                            const hcp_decode_split* splits, int32_t num_splits,
-                            const int32_t* seq_partial_start, const int32_t* seq_rows,
-                            int32_t num_seqs, void* workspace, size_t workspace_bytes, void* out,
-                            int64_t o_stride_tok, int64_t o_stride_head, float* lse,
-                            int64_t lse_stride_head, int32_t num_heads, int32_t num_kv_heads,
-                            int32_t head_dim, float scale, int32_t dtype, void* stream) {
-  const char* who = "hcp_decode_splitkv_rows";
-  if (num_seqs > 0 && !seq_rows) return fail(HCP_EINVAL, "%s: null seq_rows", who);
-  return decode_impl(who, q, q_stride_tok, q_stride_head, entries, num_entries, splits,
-                     num_splits, seq_partial_start, num_seqs, workspace, workspace_bytes, out,
-                     o_stride_tok, o_stride_head, lse, lse_stride_head, nullptr, 0, 0, nullptr,
-                     0, num_heads, num_kv_heads, head_dim, scale, dtype, stream, seq_rows);
 }
 
 int hcp_decode_splitkv_acc(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
@@ -922,6 +1045,43 @@ int hcp_decode_splitkv_noalloc(const void* q, int64_t q_stride_tok, int64_t q_st
                      num_splits, seq_partial_start, num_seqs, ws, HCP_NOALLOC_SCRATCH_BYTES, out,
                      o_stride_tok, o_stride_head, lse, lse_stride_head, nullptr, 0, 0, nullptr,
                      0, num_heads, num_kv_heads, head_dim, scale, dtype, stream);
+}
+
+int hcp_decode_launch(const hcp_decode_args* a, void* stream) {
+  const char* who = "hcp_decode_launch";
+  if (!a) return fail(HCP_EINVAL, "%s: null arguments", who);
+  if (a->num_works < 0 || a->num_wgs < 0 || a->num_wgs > a->num_works ||
+      (a->num_works > 0 && (!a->works || a->num_wgs == 0)))
+    return fail(HCP_EINVAL, "%s: bad work list", who);
+  if (a->kv_base & 15) return fail(HCP_EINVAL, "%s: kv_base not 16-byte aligned", who);
+  if ((a->acc_o == nullptr) != (a->acc_lse == nullptr))
+    return fail(HCP_EINVAL, "%s: half an accumulator", who);
+  if (reinterpret_cast<uintptr_t>(a->acc_o) % 2)
+    return fail(HCP_EINVAL, "%s: acc_o not 2-byte aligned", who);
+  int rc = check_heads(a->num_heads, a->num_kv_heads, a->head_dim, a->dtype, who);
+  if (rc) return rc;
+  void* ws = a->workspace;
+  size_t bytes = a->workspace_bytes;
+  if (a->use_scratch) {
+    bytes = HCP_NOALLOC_SCRATCH_BYTES;
+    const size_t need = hcp_decode_workspace_bytes(a->num_works, a->num_heads, a->head_dim);
+    if (need > bytes)
+      return fail(HCP_EWORKSPACE, "%s: %d splits x %d heads x head_dim %d need %zu bytes of "
+                  "partials; the library's fixed scratch holds %zu",
+                  who, a->num_works, a->num_heads, a->head_dim, need, bytes);
+    if (a->num_works > 0 && a->num_seqs > 0 && (rc = scratch_on_current_device(&ws, who)))
+      return rc;
+  }
+  DecodeExtra x;
+  x.works = a->works;
+  x.num_wgs = a->num_wgs;
+  x.rows = a->seq_rows;
+  x.kv_base = a->kv_base;
+  return decode_impl(who, a->q, a->q_stride_tok, a->q_stride_head, nullptr, 0, nullptr,
+                     a->num_works, a->seq_partial_start, a->num_seqs, ws, bytes, a->out,
+                     a->o_stride_tok, a->o_stride_head, a->lse, a->lse_stride_head, a->acc_o,
+                     a->acc_stride_tok, a->acc_stride_head, a->acc_lse, a->acc_lse_stride_head,
+                     a->num_heads, a->num_kv_heads, a->head_dim, a->scale, a->dtype, stream, x);
 }
 
 int hcp_merge_attn_states(void* out, int64_t o_stride_tok, int64_t o_stride_head,
@@ -1027,6 +1187,32 @@ int hcp_reshape_and_cache(const void* key, int64_t k_stride_tok, int64_t k_strid
   return launch_status(hcp::launch_cache_write(p, slot_dtype == HCP_DTYPE_I64,
                                                static_cast<hipStream_t>(stream)),
                        who);
+}
+
+int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t qsl_stride,
+                       const void* seq_lens, int32_t lens_dtype, int64_t lens_stride,
+                       const void* block_table, int32_t bt_dtype, int64_t bt_stride, int32_t n,
+                       int64_t* host_out, void* stream) {
+  const char* who = "hcp_fetch_metadata";
+  for (int32_t d : {qsl_dtype, lens_dtype, bt_dtype})
+    if (d != HCP_DTYPE_I32 && d != HCP_DTYPE_I64)
+      return fail(HCP_EUNSUPPORTED, "%s: index dtype %d (int32 or int64)", who, d);
+  if (n < 0) return fail(HCP_EINVAL, "%s: negative n", who);
+  if (!query_start_loc || !host_out || (n > 0 && !seq_lens))
+    return fail(HCP_EINVAL, "%s: null pointer", who);
+  hcp::MetaParams p{};
+  p.qsl = query_start_loc;
+  p.lens = seq_lens;
+  p.bt = block_table;
+  p.qsl_stride = qsl_stride;
+  p.lens_stride = lens_stride;
+  p.bt_stride = bt_stride;
+  p.qsl_wide = qsl_dtype == HCP_DTYPE_I64;
+  p.lens_wide = lens_dtype == HCP_DTYPE_I64;
+  p.bt_wide = bt_dtype == HCP_DTYPE_I64;
+  p.n = n;
+  p.out = host_out;
+  return launch_status(hcp::launch_fetch_metadata(p, static_cast<hipStream_t>(stream)), who);
 }
 
 int hcp_gather_paged_kv(const hcp_varlen_entry* entries, int32_t num_entries,

@@ -306,8 +306,9 @@ fa_fwd_kernel(FwdParams p) {
   const int32_t* bt = reinterpret_cast<const int32_t*>(e.kv.block_table);
   int64_t blockb = 0;
   if constexpr (PAGED) {
-    kseg = reinterpret_cast<const char*>(e.kv.k_addr) + static_cast<int64_t>(kvh) * e.kv.stride_head * 2;
-    vseg = reinterpret_cast<const char*>(e.kv.v_addr) + static_cast<int64_t>(kvh) * e.kv.stride_head * 2;
+    const uint64_t base = p.kv_base + static_cast<uint64_t>(kvh) * e.kv.stride_head * 2;
+    kseg = reinterpret_cast<const char*>(e.kv.k_addr + base);
+    vseg = reinterpret_cast<const char*>(e.kv.v_addr + base);
     bs_shift = 31 - __builtin_clz(e.kv.block_size);
     bs_mask = e.kv.block_size - 1;
     blockb = e.kv.stride_block * 2;

@@ -138,6 +138,13 @@ __device__ __forceinline__ u32x2 ldg8(const void* p) {
   return *reinterpret_cast<gu32x2*>(reinterpret_cast<uintptr_t>(p));
 }
 
+// The same pointer, known to be to global memory: a pointer that was itself
+// loaded from memory is generic to the compiler, and a flat access also
+// counts against the LDS waits.
+template <typename T>
+__device__ __forceinline__ T* global_ptr(T* p) {
+  return (T*)(reinterpret_cast<__attribute__((address_space(1))) T*>(reinterpret_cast<uintptr_t>(p)));
+}
 
 __device__ __forceinline__ float fast_exp2(float x) {
   return __builtin_amdgcn_exp2f(x);  // v_exp_f32; exp2(-inf) = 0
@@ -154,7 +161,7 @@ struct KvAddr {
   __device__ __forceinline__ void init(const hcp_kv_segment& s) {
     k = reinterpret_cast<const char*>(s.k_addr);
     v = reinterpret_cast<const char*>(s.v_addr);
-    bt = reinterpret_cast<const int32_t*>(s.block_table);
+    bt = global_ptr(reinterpret_cast<const int32_t*>(s.block_table));
     stride_tok = s.stride_tok;
     stride_head = s.stride_head;
     stride_block = s.stride_block;

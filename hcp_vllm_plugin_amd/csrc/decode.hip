@@ -52,9 +52,8 @@ struct DecShared {
 
 template <int D, typename T, bool PAGED>
 __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in, int chunk_in,
-                                                  int sp,
-                                                  const hcp_varlen_entry& e,
-                                                  const hcp_decode_split& spl,
+                                                  int sp, const hcp_varlen_entry& e,
+                                                  int64_t kb, int64_t ke,
                                                   char (*bufE)[2 * DecShared<D>::CHB],
                                                   char (*bufO)[2 * DecShared<D>::CHB],
                                                   float (*sm_m)[16], float (*sm_l)[16]) {
@@ -75,7 +74,10 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
   // one from the DMA writes into the other).  Row r's 16-byte slot c sits at
   // slot c ^ (r % CPR): both operand reads below are then conflict-free.
 
-  const int tid = threadIdx.x;
+  // (opaque: what is derived from it is rebuilt for every split, not held in
+  // registers across the workgroup's list)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int c16 = lane & 15;
@@ -89,7 +91,6 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
   const int h0 = kvh * p.group + 16 * chunk;
   KvAddr kva;
   kva.init(e.kv);
-  const int64_t kb = spl.key_begin, ke = spl.key_end;
 
   // A row holds dv <= D valid elements (a multiple of 8): the kernel computes
   // in D columns.  Q's tail is zero; a K/V chunk past dv is fetched from the
@@ -232,6 +233,20 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
     pw[2] = pack2<T>(s1[0], s1[1]);
     pw[3] = pack2<T>(s1[2], s1[3]);
     const V8 pf = as_vec8<V8>(pw);
+    // P enters the PV product as two 16-bit terms, its rounded value and what
+    // the rounding left: the kernel waits on memory, the second product hides.
+    // One term would be exact only for the largest key of each wave's share of
+    // a split, so the error would grow with the length of the splits.
+    auto rest = [&](uint32_t w, float a, float b) __attribute__((always_inline)) {
+      return pack2<T>(a - E::to_float(static_cast<uint16_t>(w & 0xffffu)),
+                      b - E::to_float(static_cast<uint16_t>(w >> 16)));
+    };
+    u32x4 rw;
+    rw[0] = rest(pw[0], s0[0], s0[1]);
+    rw[1] = rest(pw[1], s0[2], s0[3]);
+    rw[2] = rest(pw[2], s1[0], s1[1]);
+    rw[3] = rest(pw[3], s1[2], s1[3]);
+    const V8 rf = as_vec8<V8>(rw);
 
     // 8 keys x NU d in registers -> NU operands of 8 keys each
 #pragma unroll
@@ -244,6 +259,7 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
         a[j] = (u & 1) ? ((x >> 16) | (y & 0xffff0000u)) : ((x & 0xffffu) | (y << 16));
       }
       oacc[u] = E::mfma16(as_vec8<V8>(a), pf, oacc[u]);
+      oacc[u] = E::mfma16(as_vec8<V8>(a), rf, oacc[u]);
     }
   };
 
@@ -254,7 +270,9 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
   // The next chunk's DMA is issued unconditionally (past the wave's last
   // chunk it re-reads the split's last chunk into the buffer nobody reads):
   // with no branch around it, the wait before each compute is exactly "the
-  // previous chunk's loads", not a conservative wait for all of them.
+  // previous chunk's loads", not a conservative wait for all of them.  (Rows
+  // past the descriptor's range instead, which read as zeros without traffic,
+  // measured slower: 16.5 -> 18.6 us at 8 x ~5500 keys of 2 x 64 heads.)
   const int64_t last = nchunks - 1;
   auto next_k0 = [&](int64_t cn) __attribute__((always_inline)) {
     return kb + (cn < last ? cn : last) * kDecChunk;
@@ -385,7 +403,9 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
   // be writing bufE/bufO, which sm_o overlays: drain it before the barrier.
   wait_vmcnt<0>();
   __syncthreads();
-  float (*sm_o)[16][D] = reinterpret_cast<float (*)[16][D]>(&bufE[0][0]);
+  // rows of D + 4 floats: the 16 heads' 16-byte stores fall on different banks
+  float (*sm_o)[16][D + 4] = reinterpret_cast<float (*)[16][D + 4]>(&bufE[0][0]);
+  static_assert(sizeof(float) * W * 16 * (D + 4) <= W * 2 * CHB, "combine staging");
   float l_tot = l_run + __shfl_xor(l_run, 16);
   l_tot += __shfl_xor(l_tot, 32);
   if (g4 == 0) {
@@ -393,9 +413,11 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
     sm_l[wave][c16] = l_tot;
   }
 #pragma unroll
-  for (int u = 0; u < NU; ++u)
+  for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sm_o[wave][c16][NU * (4 * g4 + r) + u] = oacc[u][r];
+    for (int u = 0; u < NU; u += 4)
+      *reinterpret_cast<f32x4*>(&sm_o[wave][c16][NU * (4 * g4 + r) + u]) =
+          f32x4{oacc[u][r], oacc[u + 1][r], oacc[u + 2][r], oacc[u + 3][r]};
   __syncthreads();
 
   for (int idx = tid; idx < G * D; idx += 64 * W) {
@@ -413,13 +435,31 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
     }
     const int head = h0 + h;
     const int64_t slot = static_cast<int64_t>(sp) * p.num_heads + head;
-    p.ws_o[slot * D + d] = L > 0.f ? O / L : 0.f;
-    if (d == 0) p.ws_lse[slot] = L > 0.f ? M * kLn2 + __logf(L) : -INFINITY;
+    global_ptr(p.ws_o)[slot * D + d] = L > 0.f ? O / L : 0.f;
+    if (d == 0) global_ptr(p.ws_lse)[slot] = L > 0.f ? M * kLn2 + __logf(L) : -INFINITY;
   }
+}
+
+// The kernel's one argument, by a pointer the compiler cannot see through:
+// its loads stay where they are used.
+__device__ __forceinline__ const DecParams& fresh_params() {
+  auto k = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return *(const DecParams*)k;
 }
 
 // Paged-ness is a property of each entry (a sequence's peer segment is
 // contiguous, its local segment paged), uniform within a workgroup.
+//
+// A planned launch gives each workgroup a list of records with about the same
+// number of keys in all, one round of the machine: sequences of any lengths
+// leave no CU idle at the end.  A record carries its entry, so that a split
+// starts with one scalar load and not a chain of three.  Split + merge, 28 / 4
+// x 128 heads, before (equal splits in up to four rounds) and after: 16 x 1k-8k
+// keys 46.6 -> 32.4 us, 32 x 0.5k-8k 75 -> 60.5 us (5.6 TB/s), 64 x 0.5k-2k 40.7
+// -> 35 us, 32 x 34k 366 -> 331 us (6.7 TB/s), 33k in one sequence 22.7 -> 20.4
+// us; 8 x 2k-9k at 14 / 2 x 64 16.2 -> 13.1 us.  The last three microseconds or
+// so of the short ones are the chain of latencies (record, block ids, keys).
 template <int D, typename T>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * DecShared<D>::W, 64 * DecShared<D>::W),
                           amdgpu_waves_per_eu(1, 1))) void
@@ -432,32 +472,55 @@ decode_split_kernel(DecParams p) {
   __shared__ float sm_l[W][16];
   int kvh;
   int64_t item;
-  if (!xcd_remap(blockIdx.x, static_cast<int64_t>(p.num_splits) * p.head_chunks,
+  if (!xcd_remap(blockIdx.x, static_cast<int64_t>(p.num_wgs) * p.head_chunks,
                  p.num_kv_heads, &kvh, &item))
     return;
   const int chunk = static_cast<int>(item % p.head_chunks);
-  const hcp_decode_split spl = p.splits[item / p.head_chunks];
-  const int sp = spl.slot;  // workspace partial of this split
-  const hcp_varlen_entry e = p.entries[spl.entry];
-  if (e.kv.block_table != 0)
-    decode_split_body<D, T, true>(p, kvh, chunk, sp, e, spl, bufE, bufO, sm_m, sm_l);
-  else
-    decode_split_body<D, T, false>(p, kvh, chunk, sp, e, spl, bufE, bufO, sm_m, sm_l);
+  int s = static_cast<int>(item / p.head_chunks);
+  while (true) {
+    // the parameters are read afresh for every split: held across the list
+    // they would be spilled
+    const DecParams& p = fresh_params();
+    hcp_decode_work w;
+    if (p.works != nullptr) {
+      w = global_ptr(p.works)[s];
+    } else {
+      const hcp_decode_split spl = global_ptr(p.splits)[s];
+      w.e = global_ptr(p.entries)[spl.entry];
+      w.key_begin = spl.key_begin;
+      w.key_end = spl.key_end;
+      w.slot = spl.slot;  // workspace partial of this split
+      w.next = -1;
+    }
+    if (w.e.kv.block_table != 0) {
+      w.e.kv.k_addr += p.kv_base;
+      w.e.kv.v_addr += p.kv_base;
+      decode_split_body<D, T, true>(p, kvh, chunk, w.slot, w.e, w.key_begin, w.key_end, bufE, bufO,
+                                    sm_m, sm_l);
+    } else {
+      decode_split_body<D, T, false>(p, kvh, chunk, w.slot, w.e, w.key_begin, w.key_end, bufE,
+                                     bufO, sm_m, sm_l);
+    }
+    if (w.next < 0) return;
+    s = w.next;
+    __syncthreads();  // this split has been combined out of the buffers
+  }
 }
 
 // Merge every partial of one (sequence, query head) -- and the running
 // accumulator, when given -- into the output row and its LSE.  One workgroup
 // of D threads per (sequence, head) column group, thread d owns column d;
 // with many partials per sequence (1, 2 or 4 groups) the groups take
-// interleaved shares of the partials and are summed through LDS.  The max over
-// partial LSEs is thread-strided plus a block reduction; the weighted sum
-// issues 8 partials' loads before consuming them, so a long sequence (one
-// request split over the whole machine) is not a chain of dependent loads.
+// interleaved shares of the partials and are merged through LDS.  Bound by
+// latency: a thread issues the LSEs and columns of 16 partials at once, before
+// any maximum is known, and keeps a running maximum over batches of 16 (with
+// the maximum taken first, split + merge of 1 x 2000 keys took 10.7 us, now
+// 9.4).  Merged by the split kernel's last workgroup of each sequence instead,
+// 31 to 64 partials took longer than this launch costs.
 template <int D, typename T>
 __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
-  constexpr int kMaxWaves = 4 * D / 64;
-  __shared__ float sm_max[kMaxWaves];
-  __shared__ float sm_s[4];
+  constexpr int U = 16;
+  __shared__ float sm_m[4], sm_s[4];
   __shared__ float sm_o[4][D];
   const int ng = p.groups;  // column groups; group gi takes partials gi, gi + ng, ...
   const int sh = blockIdx.x;
@@ -465,15 +528,14 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
   const int row = p.rows != nullptr ? p.rows[seq] : seq;  // of out, lse and acc
   const int tid = threadIdx.x;
   const int d = tid % D, gi = tid / D;
-  const int p0 = p.seq_partial_start[seq], p1 = p.seq_partial_start[seq + 1];
-  const int n = p1 - p0;
+  const int p0 = p.seq_partial_start[seq], n = p.seq_partial_start[seq + 1] - p0;
   const int64_t lstep = p.num_heads;
   const float* lcol = p.ws_lse + static_cast<int64_t>(p0) * lstep + head;
   const int64_t ostep = lstep * D;
   const float* ocol = p.ws_o + (static_cast<int64_t>(p0) * lstep + head) * D + d;
 
   // accumulator first: out / lse may alias acc_o / acc_lse, and every read
-  // of them happens before the barriers below, every write after them
+  // of them happens before the barrier below, every write after it
   float acc_l = -INFINITY, acc_v = 0.f;
   if (p.acc_lse != nullptr) {
     acc_l = p.acc_lse[static_cast<int64_t>(head) * p.acc_lse_stride_head + row];
@@ -482,73 +544,72 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
                            row * p.acc_stride_tok + static_cast<int64_t>(head) * p.acc_stride_head;
     acc_v = d < p.head_dim ? Elem<T>::to_float(arow[d]) : 0.f;
   }
-
-  // max over the partial LSEs, thread-strided over the whole block
-  float m = -INFINITY;
-  for (int i = tid; i < n; i += ng * D) m = fmaxf(m, lcol[i * lstep]);
+  // a weighted sum relative to the running maximum m
+  float m = -INFINITY, S = 0.f, O = 0.f;
+  auto rebase = [&](float mn) __attribute__((always_inline)) {
+    const float sc = m == -INFINITY ? 0.f : __expf(m - mn);
+    S *= sc;
+    O *= sc;
+    m = mn;
+  };
+  for (int i0 = gi; i0 < n; i0 += U * ng) {
+    float l[U], v[U];
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  if ((tid & 63) == 0) sm_max[tid >> 6] = m;
-  __syncthreads();
-  float M = acc_l;
-  for (int w = 0; w < ng * D / 64; ++w) M = fmaxf(M, sm_max[w]);
-
-  // this group's share of the weighted sum (S is the same in every column
-  // of the group); 8 partials' loads are issued before they are consumed
-  float S = 0.f, O = 0.f;
-  if (M != -INFINITY) {
-    int i = gi;
-    for (; i + 7 * ng < n; i += 8 * ng) {
-      float l[8], v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        l[j] = lcol[(i + j * ng) * lstep];
-        v[j] = ocol[(i + j * ng) * ostep];
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float w = __expf(l[j] - M);
-        S += w;
-        O += w * v[j];
-      }
+    for (int j = 0; j < U; ++j) {
+      const int i = i0 + j * ng < n ? i0 + j * ng : i0;  // past the last: not summed
+      l[j] = lcol[i * lstep];
+      v[j] = ocol[i * ostep];
     }
-    for (; i < n; i += ng) {
-      const float w = __expf(lcol[i * lstep] - M);
+    float mn = m;
+#pragma unroll
+    for (int j = 0; j < U; ++j) mn = fmaxf(mn, l[j]);
+    if (mn == -INFINITY) continue;
+    rebase(mn);
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const bool in = i0 + j * ng < n;
+      const float w = in ? __expf(l[j] - mn) : 0.f;
       S += w;
-      O += w * ocol[i * ostep];
+      O = in ? __builtin_fmaf(w, v[j], O) : O;
     }
   }
   if (ng > 1) {
-    if (d == 0) sm_s[gi] = S;
+    if (d == 0) {
+      sm_m[gi] = m;
+      sm_s[gi] = S;
+    }
     sm_o[gi][d] = O;
-    __syncthreads();
-    if (gi != 0) return;
-    for (int g2 = 1; g2 < ng; ++g2) {
-      S += sm_s[g2];
-      O += sm_o[g2][d];
-    }
   }
-  float o = 0.f, lse = -INFINITY;
-  if (M != -INFINITY) {
-    if (acc_l != -INFINITY) {
-      const float w = __expf(acc_l - M);
-      S += w;
-      O += w * acc_v;
-    }
-    o = O / S;
-    lse = M + __logf(S);
+  __syncthreads();
+  if (gi != 0) return;
+  for (int g2 = 1; g2 < ng; ++g2) {
+    if (sm_m[g2] == -INFINITY) continue;
+    const float mn = fmaxf(m, sm_m[g2]);
+    rebase(mn);
+    const float w = __expf(sm_m[g2] - mn);
+    S = __builtin_fmaf(w, sm_s[g2], S);
+    O = __builtin_fmaf(w, sm_o[g2][d], O);
   }
+  if (acc_l != -INFINITY) {
+    const float mn = fmaxf(m, acc_l);
+    rebase(mn);
+    const float w = __expf(acc_l - mn);
+    S += w;
+    O = __builtin_fmaf(w, acc_v, O);
+  }
+  const bool any = m != -INFINITY;
   uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + row * p.o_stride_tok +
                    static_cast<int64_t>(head) * p.o_stride_head;
-  if (d < p.head_dim) orow[d] = Elem<T>::from_float(o);
+  if (d < p.head_dim) orow[d] = Elem<T>::from_float(any ? O / S : 0.f);
   if (p.lse != nullptr && d == 0)
-    p.lse[static_cast<int64_t>(head) * p.lse_stride_head + row] = lse;
+    p.lse[static_cast<int64_t>(head) * p.lse_stride_head + row] =
+        any ? m + __logf(S) : -INFINITY;
 }
 
 template <int D, typename T>
 static hipError_t launch_dec_t(const DecParams& dp, const RedParams& rp, hipStream_t st) {
   const int64_t grid =
-      xcd_grid_size(static_cast<int64_t>(dp.num_splits) * dp.head_chunks, dp.num_kv_heads);
+      xcd_grid_size(static_cast<int64_t>(dp.num_wgs) * dp.head_chunks, dp.num_kv_heads);
   if (grid > 0) {
     hipLaunchKernelGGL((decode_split_kernel<D, T>), dim3(static_cast<unsigned>(grid)),
                        dim3(64 * DecShared<D>::W), 0, st, dp);

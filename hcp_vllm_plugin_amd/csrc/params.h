@@ -31,6 +31,7 @@ struct FwdParams {
   const hcp_varlen_entry* entries;  // varlen: device array
   const int32_t* tiles;             // varlen: device (entry, q_block) pairs
   int32_t num_tiles;                // varlen: tiles; else query blocks
+  uint64_t kv_base;                 // varlen, paged: added to the entries' k / v addresses
   int32_t num_heads, num_kv_heads, group;
   int32_t head_dim;  // valid elements per row (<= the kernel's width; the tail is padding)
   float scale_log2;
@@ -86,9 +87,14 @@ __host__ __device__ inline int piece_begin(int tiles, int np, int i) {
 struct DecParams {
   const void* q;
   int64_t q_stride_tok, q_stride_head;
+  // the launch's splits: one record per split, each naming the next of its
+  // workgroup (works), or an entry index and a key range each
+  const hcp_decode_work* works;
   const hcp_varlen_entry* entries;
   const hcp_decode_split* splits;
   int32_t num_splits;
+  int32_t num_wgs;   // workgroups per KV head and head chunk
+  uint64_t kv_base;  // added to the k / v addresses of paged records
   float* ws_o;    // [num_splits, H, D]
   float* ws_lse;  // [num_splits, H]
   int32_t num_heads, num_kv_heads, group;
@@ -167,6 +173,17 @@ struct GatherParams {
   void* v_out;
 };
 
+// One step's metadata, to host memory (fetch_metadata_kernel).
+struct MetaParams {
+  const void* qsl;
+  const void* lens;
+  const void* bt;  // NULL: zeros
+  int64_t qsl_stride, lens_stride, bt_stride;
+  bool qsl_wide, lens_wide, bt_wide;  // int64, else int32
+  int32_t n;
+  int64_t* out;  // [3 n + 1]
+};
+
 // Prefill in D columns (padded_head_dim): the attention kernel and, when p
 // carries a KV split, the merge of its partials into out / lse (and acc).
 template <int D>
@@ -190,6 +207,7 @@ hipError_t launch_decode(const DecParams& dp, const RedParams& rp, int head_dim,
                          int dtype, hipStream_t st);
 hipError_t launch_merge(const MergeParams& p, hipStream_t st);
 hipError_t launch_cache_write(const CacheParams& p, bool slots_i64, hipStream_t st);
+hipError_t launch_fetch_metadata(const MetaParams& p, hipStream_t st);
 hipError_t launch_gather(const GatherParams& p, hipStream_t st);
 
 }  // namespace hcp

@@ -67,7 +67,7 @@ def merge_attn_states(
     if output_lse is not None:
         _chk_lse("output_lse", output_lse, h, t)
     L = _lib.lib()
-    with torch.cuda.device(output.device):
+    with _lib.on_device(output.device):
         rc = L.hcp_merge_attn_states(
             output.data_ptr(), output.stride(0), output.stride(1), _lib.dtype_code(output.dtype),
             output_lse.data_ptr() if output_lse is not None else None,

@@ -103,7 +103,7 @@ def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_p
     off = 0 if causal_offset is None else int(causal_offset)
     win = 0 if (window is None or causal_offset is None) else int(window)
     dtype, device = _lib.dtype_code(q.dtype), q.device
-    with torch.cuda.device(device):
+    with _lib.on_device(device):
         head = (
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             0 if lse is None else lse.data_ptr(),

@@ -233,13 +233,20 @@ ENTRY_DTYPE = np.dtype({
 })
 assert ENTRY_DTYPE.itemsize == ctypes.sizeof(VarlenEntry)
 
+# hcp_decode_work: an entry and its split
+WORK_DTYPE = np.dtype([("e", ENTRY_DTYPE)] + [(f, "<i4") for f in (
+    "key_begin", "key_end", "slot", "next", "r0", "r1", "r2", "r3")])
+assert WORK_DTYPE.itemsize == 128
+
 
 def paged_entry_array(pc: "PagedCache", block_table: torch.Tensor, rows, q_start, q_len,
-                      causal_offset, start, length) -> np.ndarray:
+                      causal_offset, start, length, relative: bool = False) -> np.ndarray:
     """Entries over the paged cache for many requests at once: entry i covers
     query rows [q_start[i], +q_len[i]) and tokens [start[i], +length[i]) of
     block-table row rows[i].  ``block_table`` is the batch's contiguous int32
-    table on the device; all checks are done once for the batch."""
+    table on the device; all checks are done once for the batch.  ``relative``:
+    the K and V addresses relative to ``pc.k_addr``, for a launch given it as
+    ``kv_base``."""
     if block_table.dtype != torch.int32 or not block_table.is_contiguous():
         raise ValueError("block table must be contiguous int32")
     _check_kv_layout(pc.k_addr, pc.v_addr, pc.stride_tok, pc.stride_head, pc.stride_block,
@@ -258,8 +265,8 @@ def paged_entry_array(pc: "PagedCache", block_table: torch.Tensor, rows, q_start
     a["q_start"] = q_start
     a["q_len"] = q_len
     a["causal_offset"] = causal_offset
-    a["k_addr"] = pc.k_addr
-    a["v_addr"] = pc.v_addr
+    a["k_addr"] = 0 if relative else pc.k_addr
+    a["v_addr"] = pc.v_addr - pc.k_addr if relative else pc.v_addr
     a["block_table"] = block_table.data_ptr() + rows * block_table.stride(0) * 4
     a["stride_tok"] = pc.stride_tok
     a["stride_head"] = pc.stride_head
@@ -433,7 +440,7 @@ class VarlenLaunch:
 
     def run(self, q: torch.Tensor, out: torch.Tensor, lse: torch.Tensor | None,
             num_kv_heads: int, scale: float, window: int | None = None,
-            acc=None, acc_is_prefix: bool = True) -> None:
+            acc=None, acc_is_prefix: bool = True, kv_base: int = 0) -> None:
         """``window``: sliding window of a causal launch (query at p sees keys
         p - window < j <= p in its entry's frame); ignored when non-causal.
 
@@ -441,68 +448,49 @@ class VarlenLaunch:
         result in the same launch (``hcp_attn_fwd_varlen_merge``): with
         ``acc_is_prefix`` each row gets merge_attn_states(acc, this pass), the
         local pass taking the peer result as the prefix (ring_backend.py:354).
-        ``lse`` may then be None; otherwise it receives the merged LSE."""
+        ``lse`` may then be None; otherwise it receives the merged LSE.
+
+        ``kv_base``: added to the addresses of paged entries (planned with
+        addresses relative to a layer's cache)."""
         if self.num_tiles == 0:
             return
         if window is not None and window <= 0:
             raise ValueError("window must be a positive number of keys")
+        if kv_base and self._gather is not None:
+            raise ValueError("a gathering launch needs absolute cache addresses")
         num_heads, head_dim = q.shape[1], q.shape[2]
-        L = _lib.lib()
         win = int(window or 0) if self.causal else 0
-        with torch.cuda.device(q.device):
-            entries_ptr = self.entries_ptr
-            if self._gather is not None:
-                entries_ptr = self._gathered(q, num_kv_heads)
-            if acc is not None:
-                a_o, a_lse = acc
-                if a_o.dtype != q.dtype or a_o.stride(-1) != 1 or a_lse.dtype != torch.float32:
-                    raise ValueError("acc must be (out in q.dtype, float32 lse)")
-            sp = self._split
+        a = _lib.VarlenArgs()
+        a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(0), q.stride(1)
+        a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
+        if lse is not None:
+            a.lse, a.lse_stride_head = lse.data_ptr(), lse.stride(0)
+        a.num_entries = self.num_entries
+        a.num_heads, a.num_kv_heads, a.head_dim = num_heads, num_kv_heads, head_dim
+        a.causal, a.window, a.paged = self.causal, win, self.paged
+        a.scale, a.dtype, a.kv_base = float(scale), _lib.dtype_code(q.dtype), kv_base
+        if acc is not None:
+            a_o, a_lse = acc
+            if a_o.dtype != q.dtype or a_o.stride(-1) != 1 or a_lse.dtype != torch.float32:
+                raise ValueError("acc must be (out in q.dtype, float32 lse)")
+            a.acc_o, a.acc_stride_tok, a.acc_stride_head = \
+                a_o.data_ptr(), a_o.stride(0), a_o.stride(1)
+            a.acc_lse, a.acc_lse_stride_head = a_lse.data_ptr(), a_lse.stride(0)
+            a.acc_is_prefix = bool(acc_is_prefix)
+        sp = self._split
+        with _lib.on_device(q.device):
+            a.entries = self.entries_ptr if self._gather is None else \
+                self._gathered(q, num_kv_heads)
             if sp is not None and sp["key"] == (num_heads, num_kv_heads, head_dim, win):
                 # fp32 partials: stream-ordered scratch from torch's caching allocator
                 ws = torch.empty(sp["bytes"], dtype=torch.uint8, device=q.device)
-                rc = L.hcp_attn_fwd_varlen_split(
-                    q.data_ptr(), q.stride(0), q.stride(1),
-                    out.data_ptr(), out.stride(0), out.stride(1),
-                    0 if lse is None else lse.data_ptr(), 0 if lse is None else lse.stride(0),
-                    entries_ptr, self.num_entries,
-                    sp["ptrs"][0], sp["pieces"], sp["piece_tiles"],
-                    sp["ptrs"][1], sp["units"], sp["slots"],
-                    num_heads, num_kv_heads, head_dim, float(scale),
-                    int(self.causal), win, int(self.paged),
-                    *((0, 0, 0, 0, 0, 0) if acc is None else
-                      (a_o.data_ptr(), a_o.stride(0), a_o.stride(1),
-                       a_lse.data_ptr(), a_lse.stride(0), int(bool(acc_is_prefix)))),
-                    ws.data_ptr(), sp["bytes"], _lib.dtype_code(q.dtype),
-                    _lib.stream_ptr(q.device))
-                _lib.check(rc, "hcp_attn_fwd_varlen_split")
-                return
-            if acc is None:
-                rc = L.hcp_attn_fwd_varlen(
-                    q.data_ptr(), q.stride(0), q.stride(1),
-                    out.data_ptr(), out.stride(0), out.stride(1),
-                    lse.data_ptr(), lse.stride(0),
-                    entries_ptr, self.num_entries,
-                    self.tiles_ptr, self.num_tiles,
-                    num_heads, num_kv_heads, head_dim, float(scale),
-                    int(self.causal), win, int(self.paged),
-                    _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device),
-                )
-                _lib.check(rc, "hcp_attn_fwd_varlen")
-                return
-            rc = L.hcp_attn_fwd_varlen_merge(
-                q.data_ptr(), q.stride(0), q.stride(1),
-                out.data_ptr(), out.stride(0), out.stride(1),
-                0 if lse is None else lse.data_ptr(), 0 if lse is None else lse.stride(0),
-                entries_ptr, self.num_entries,
-                self.tiles_ptr, self.num_tiles,
-                num_heads, num_kv_heads, head_dim, float(scale),
-                int(self.causal), win, int(self.paged),
-                a_o.data_ptr(), a_o.stride(0), a_o.stride(1),
-                a_lse.data_ptr(), a_lse.stride(0), int(bool(acc_is_prefix)),
-                _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device),
-            )
-        _lib.check(rc, "hcp_attn_fwd_varlen_merge")
+                a.workspace, a.workspace_bytes = ws.data_ptr(), sp["bytes"]
+                a.tiles, a.num_tiles, a.piece_tiles = sp["ptrs"][0], sp["pieces"], sp["piece_tiles"]
+                a.units, a.num_units, a.num_slots = sp["ptrs"][1], sp["units"], sp["slots"]
+            else:
+                a.tiles, a.num_tiles = self.tiles_ptr, self.num_tiles
+            rc = _lib.lib().hcp_varlen_launch(ctypes.addressof(a), _lib.stream_ptr(q.device))
+        _lib.check(rc, "hcp_varlen_launch")
 
 
 def varlen_attn_with_lse(
@@ -583,6 +571,14 @@ def choose_split_tokens(seg_lens: list[int], num_kv_heads: int, num_cus: int = 2
     return max(minimum, min(maximum, s))
 
 
+def decode_workgroups(heads: int, num_cus: int = 256) -> int:
+    """Workgroups of a decode launch per KV head and head chunk (``heads`` of
+    them).  The split kernel runs one
+    workgroup per CU (128 KB of LDS); its workgroups all get the same number
+    of keys, so one round of the machine drains evenly."""
+    return max(1, num_cus // heads)
+
+
 class DecodeBatch:
     """A planned split-KV decode: entries and splits on the device (the fp32
     partials' workspace is taken per run).
@@ -605,25 +601,12 @@ class DecodeBatch:
                 seq_of.append(s)
         self.num_seqs = len(segments)
         self.num_entries = len(entries)
-        if split_tokens is None:
-            split_tokens = choose_split_tokens([e.kv.len for e in entries],
-                                               num_kv_heads * head_chunks(num_heads, num_kv_heads))
-        self.split_tokens = split_tokens
-        arr = (VarlenEntry * max(self.num_entries, 1))(*entries)
-        seq_arr = (ctypes.c_int32 * max(self.num_entries, 1))(*seq_of)
-        cap = sum(-(-e.kv.len // split_tokens) for e in entries)
-        splits = (DecodeSplit * max(cap, 1))()
-        starts = (ctypes.c_int32 * (self.num_seqs + 1))()
-        rc = L.hcp_plan_decode_splits(ctypes.addressof(arr), self.num_entries,
-                                      ctypes.addressof(seq_arr), self.num_seqs, 0,
-                                      split_tokens, ctypes.addressof(splits), cap,
-                                      ctypes.addressof(starts))
-        _lib.check(rc, "hcp_plan_decode_splits")
-        self.num_splits = rc
-        self.num_heads = num_heads
-        self.num_kv_heads = num_kv_heads
-        self.head_dim = head_dim
-        self._upload_plan(arr, splits, starts, rows, device)
+        arr = np.zeros(max(self.num_entries, 1), dtype=ENTRY_DTYPE)
+        if entries:
+            packed = (VarlenEntry * self.num_entries)(*entries)
+            arr[:] = np.frombuffer(packed, dtype=ENTRY_DTYPE)
+        self._plan(arr, np.asarray(seq_of or [0], dtype=np.int32), num_heads, num_kv_heads,
+                   head_dim, split_tokens, rows, device)
         # the segments point at K/V / cache / block-table storage by address
         self._keep = [getattr(e, "_keep", None) for e in entries]
 
@@ -655,37 +638,56 @@ class DecodeBatch:
                 seq_arr = np.zeros(1, dtype=np.int32)
         self.num_seqs = ns
         self.num_entries = n
-        lens = entries["len"]
-        if split_tokens is None:
-            split_tokens = choose_split_tokens([int(lens.sum())],
-                                               num_kv_heads * head_chunks(num_heads, num_kv_heads))
-        self.split_tokens = split_tokens
         arr = entries if n else np.zeros(1, dtype=ENTRY_DTYPE)
-        cap = int(((lens + split_tokens - 1) // split_tokens).sum())
-        splits = (DecodeSplit * max(cap, 1))()
-        starts = (ctypes.c_int32 * (ns + 1))()
-        rc = L.hcp_plan_decode_splits(arr.ctypes.data, n, seq_arr.ctypes.data, ns, 0,
-                                      split_tokens, ctypes.addressof(splits), cap,
-                                      ctypes.addressof(starts))
-        _lib.check(rc, "hcp_plan_decode_splits")
+        self._plan(arr, seq_arr, num_heads, num_kv_heads, head_dim, split_tokens, rows, device)
+        self._keep = keep
+        return self
+
+    def _plan(self, arr, seq_arr, num_heads, num_kv_heads, head_dim, split_tokens, rows,
+              device) -> None:
+        """Plan and upload: splits of at most ``split_tokens`` keys, one to a
+        workgroup, or (None) an equal share of the batch's keys for every
+        workgroup of the launch (``hcp_plan_decode_lists``)."""
+        L = _lib.lib()
+        n, ns = self.num_entries, self.num_seqs
+        heads = num_kv_heads * head_chunks(num_heads, num_kv_heads)
+        if rows is not None:
+            rows = np.ascontiguousarray(rows, dtype=np.int32)
+            if len(rows) != ns:
+                raise ValueError("rows needs one row per sequence")
+        total = int(arr["len"][:n].sum())
+        if split_tokens is None:
+            wgs = decode_workgroups(heads)
+            cap = n + wgs
+        else:
+            wgs = 0
+            cap = int((-(-arr["len"][:n] // split_tokens)).sum())
+        self.split_tokens = split_tokens or max(1, -(-total // wgs))  # keys to a workgroup
+        works = np.empty(max(cap, 1), dtype=WORK_DTYPE)
+        work_entry = np.empty(max(cap, 1), dtype=np.int32)
+        starts = np.empty(ns + 1, dtype=np.int32)
+        m = ctypes.c_int32(0)
+        rc = L.hcp_plan_decode_lists(
+            arr.ctypes.data, n, seq_arr.ctypes.data, ns, wgs, split_tokens or 0,
+            works.ctypes.data, work_entry.ctypes.data, cap, starts.ctypes.data,
+            ctypes.addressof(m))
+        _lib.check(rc, "hcp_plan_decode_lists")
         self.num_splits = rc
         self.num_heads = num_heads
         self.num_kv_heads = num_kv_heads
         self.head_dim = head_dim
-        self._upload_plan(arr, splits, starts, rows, device)
-        self._keep = keep
-        return self
-
-    def _upload_plan(self, arr, splits, starts, rows, device) -> None:
-        extra = [] if rows is None else [np.ascontiguousarray(rows, dtype=np.int32)]
-        if extra and len(extra[0]) != self.num_seqs:
-            raise ValueError("rows needs one row per sequence")
-        self._plan_dev, (self.entries_ptr, self.splits_ptr, self.starts_ptr, *rp) = _upload(
-            [arr, splits, starts, *extra], device)
-        self.rows_ptr = rp[0] if rp else None
-        self.ws_bytes = int(_lib.lib().hcp_decode_workspace_bytes(
-            max(self.num_splits, 1), self.num_heads, self.head_dim))
+        self.ws_bytes = int(L.hcp_decode_workspace_bytes(max(rc, 1), num_heads, head_dim))
         self.device = device
+        self._works, self._work_entry = works[:rc], work_entry[:rc]
+        extra = [] if rows is None else [rows]
+        self._plan_dev, (w_ptr, s_ptr, *r_ptr) = _upload(
+            [works[:max(rc, 1)], starts, *extra], device)
+        a = self._args = _lib.DecodeArgs()
+        a.works, a.num_works, a.num_wgs = w_ptr, rc, m.value
+        a.seq_partial_start, a.num_seqs = s_ptr, ns
+        a.seq_rows = r_ptr[0] if r_ptr else 0
+        a.workspace_bytes = self.ws_bytes
+        a.num_heads, a.num_kv_heads, a.head_dim = num_heads, num_kv_heads, head_dim
 
     def rebind(self, entries: np.ndarray, keep=None) -> "DecodeBatch":
         """The same plan (splits, partial slots) over new entries of the same
@@ -697,75 +699,57 @@ class DecodeBatch:
             raise ValueError("rebind needs the plan's entry count")
         other = object.__new__(type(self))
         other.__dict__.update(self.__dict__)
-        arr = entries if len(entries) else np.zeros(1, dtype=ENTRY_DTYPE)
-        other._entries_dev, (other.entries_ptr,) = _upload([arr], self.device)
+        other._works = self._works.copy()
+        other._works["e"] = entries[self._work_entry]
+        other._works_dev, (w_ptr,) = _upload([other._works], self.device)
+        other._args = _lib.DecodeArgs.from_buffer_copy(self._args)
+        other._args.works = w_ptr
         other._keep = keep
         return other
 
     def run(self, q: torch.Tensor, out: torch.Tensor, lse: torch.Tensor | None,
             scale: float, acc: tuple[torch.Tensor, torch.Tensor] | None = None,
-            noalloc: bool = False) -> None:
+            noalloc: bool = False, kv_base: int = 0) -> None:
         """Decode into ``out`` (and ``lse``).  With ``acc = (o_acc [S, H, D] in
         q's dtype, lse_acc [H, S] float32)`` the accumulator is merged in by the
-        same launch (``hcp_decode_splitkv_acc``); ``out`` / ``lse`` may be the
-        accumulator's own tensors.
+        same launch; ``out`` / ``lse`` may be the accumulator's own tensors.
 
-        ``noalloc``: run ``hcp_decode_splitkv_noalloc`` instead, whose partials
-        live in the library's fixed per-GPU scratch (no workspace is taken, so
-        nothing is allocated; calls overlapping on one GPU race).  Plans whose
-        partials exceed ``_lib.NOALLOC_SCRATCH_BYTES`` raise."""
+        ``kv_base``: added to the addresses of paged segments (planned with
+        addresses relative to a layer's cache).
+
+        ``noalloc``: the partials live in the library's fixed per-GPU scratch
+        (no workspace is taken, so nothing is allocated; calls overlapping on
+        one GPU race).  Plans whose partials exceed
+        ``_lib.NOALLOC_SCRATCH_BYTES`` raise."""
         L = _lib.lib()
-        if self.rows_ptr is not None and (noalloc or acc is not None):
-            raise ValueError("a plan with output rows has neither accumulator nor noalloc form")
-        if noalloc:
-            if acc is not None:
-                raise ValueError("noalloc decode has no accumulator form")
-            with torch.cuda.device(q.device):
-                rc = L.hcp_decode_splitkv_noalloc(
-                    q.data_ptr(), q.stride(0), q.stride(1),
-                    self.entries_ptr, self.num_entries,
-                    self.splits_ptr, self.num_splits,
-                    self.starts_ptr, self.num_seqs,
-                    out.data_ptr(), out.stride(0), out.stride(1),
-                    lse.data_ptr() if lse is not None else None,
-                    lse.stride(0) if lse is not None else 0,
-                    self.num_heads, self.num_kv_heads, self.head_dim, float(scale),
-                    _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device))
-            _lib.check(rc, "hcp_decode_splitkv_noalloc")
-            return
-        # fp32 partials: stream-ordered scratch from torch's caching allocator
-        workspace = torch.empty(self.ws_bytes, dtype=torch.uint8, device=q.device)
-        head = (q.data_ptr(), q.stride(0), q.stride(1),
-                self.entries_ptr, self.num_entries,
-                self.splits_ptr, self.num_splits,
-                self.starts_ptr, self.num_seqs,
-                workspace.data_ptr(), self.ws_bytes)
-        tail = (out.data_ptr(), out.stride(0), out.stride(1),
-                lse.data_ptr() if lse is not None else None,
-                lse.stride(0) if lse is not None else 0,
-                self.num_heads, self.num_kv_heads, self.head_dim, float(scale),
-                _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device))
-        with torch.cuda.device(q.device):
-            if self.rows_ptr is not None:
-                rc = L.hcp_decode_splitkv_rows(*head[:8], self.rows_ptr, *head[8:], *tail)
-                name = "hcp_decode_splitkv_rows"
-            elif acc is None:
-                rc = L.hcp_decode_splitkv(*head, *tail)
-                name = "hcp_decode_splitkv"
+        if noalloc and acc is not None:
+            raise ValueError("noalloc decode has no accumulator form")
+        a = _lib.DecodeArgs.from_buffer_copy(self._args)
+        a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(0), q.stride(1)
+        a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
+        if lse is not None:
+            a.lse, a.lse_stride_head = lse.data_ptr(), lse.stride(0)
+        a.scale, a.dtype, a.kv_base = float(scale), _lib.dtype_code(q.dtype), kv_base
+        if acc is not None:
+            ao, al = acc
+            if ao.dtype != q.dtype or tuple(ao.shape) != tuple(q.shape) or ao.stride(-1) != 1:
+                raise ValueError("acc o must match q's dtype and shape, contiguous head_dim")
+            if al.dtype != torch.float32 or tuple(al.shape) != (q.shape[1], q.shape[0]) \
+                    or al.stride(1) != 1:
+                raise ValueError("acc lse must be float32 [H, S], contiguous along S")
+            if not (ao.is_cuda and al.is_cuda):
+                raise ValueError("accumulator must be on the GPU")
+            a.acc_o, a.acc_stride_tok, a.acc_stride_head = ao.data_ptr(), ao.stride(0), ao.stride(1)
+            a.acc_lse, a.acc_lse_stride_head = al.data_ptr(), al.stride(0)
+        with _lib.on_device(q.device):
+            if noalloc:
+                a.use_scratch = 1
             else:
-                ao, al = acc
-                if ao.dtype != q.dtype or tuple(ao.shape) != tuple(q.shape) or ao.stride(-1) != 1:
-                    raise ValueError("acc o must match q's dtype and shape, contiguous head_dim")
-                if al.dtype != torch.float32 or tuple(al.shape) != (q.shape[1], q.shape[0]) \
-                        or al.stride(1) != 1:
-                    raise ValueError("acc lse must be float32 [H, S], contiguous along S")
-                if not (ao.is_cuda and al.is_cuda):
-                    raise ValueError("accumulator must be on the GPU")
-                rc = L.hcp_decode_splitkv_acc(
-                    *head, ao.data_ptr(), ao.stride(0), ao.stride(1), al.data_ptr(),
-                    al.stride(0), *tail)
-                name = "hcp_decode_splitkv_acc"
-        _lib.check(rc, name)
+                # fp32 partials: stream-ordered scratch from torch's caching allocator
+                ws = torch.empty(self.ws_bytes, dtype=torch.uint8, device=q.device)
+                a.workspace = ws.data_ptr()
+            rc = L.hcp_decode_launch(ctypes.addressof(a), _lib.stream_ptr(q.device))
+        _lib.check(rc, "hcp_decode_launch")
 
 
 def decode_attn(

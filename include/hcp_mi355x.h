@@ -291,26 +291,52 @@ int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries,
                           int32_t* num_units, int32_t* num_slots,
                           int32_t* piece_tiles, size_t* workspace_bytes);
 
-/* hcp_attn_fwd_varlen (acc NULL) or hcp_attn_fwd_varlen_merge over the pieces
- * of hcp_plan_varlen_split (same entries, causal, window and heads; `pieces`
- * and `units` are DEVICE copies of its records). */
-int hcp_attn_fwd_varlen_split(const void* q, int64_t q_stride_tok,
-                              int64_t q_stride_head, void* out,
-                              int64_t o_stride_tok, int64_t o_stride_head,
-                              float* lse, int64_t lse_stride_head,
-                              const hcp_varlen_entry* entries,
-                              int32_t num_entries, const int32_t* pieces,
-                              int32_t num_pieces, int32_t piece_tiles,
-                              const int32_t* units, int32_t num_units,
-                              int32_t num_slots, int32_t num_heads,
-                              int32_t num_kv_heads, int32_t head_dim,
-                              float scale, int32_t causal, int32_t window,
-                              int32_t paged, const void* acc_out,
-                              int64_t acc_stride_tok, int64_t acc_stride_head,
-                              const float* acc_lse, int64_t acc_lse_stride_head,
-                              int32_t acc_is_prefix, void* workspace,
-                              size_t workspace_bytes, int32_t dtype,
-                              void* stream);
+/*
+ * hcp_attn_fwd_varlen (acc_o and acc_lse NULL) or hcp_attn_fwd_varlen_merge.
+ *   tiles, num_tiles   DEVICE records of hcp_plan_varlen_tiles (piece_tiles 0)
+ *                      or the pieces of hcp_plan_varlen_split (same entries,
+ *                      causal, window and heads), with its units, num_units
+ *                      and num_slots and a workspace of the size it gave
+ *   kv_base            added to k_addr and v_addr of paged entries, so that one
+ *                      plan on the device serves every layer's cache
+ */
+typedef struct hcp_varlen_args {
+  const void* q;
+  int64_t q_stride_tok, q_stride_head;
+  void* out;
+  int64_t o_stride_tok, o_stride_head;
+  float* lse;
+  int64_t lse_stride_head;
+  const hcp_varlen_entry* entries;
+  const int32_t* tiles;
+  const int32_t* units;
+  void* workspace;
+  uint64_t workspace_bytes;
+  const void* acc_o;
+  int64_t acc_stride_tok, acc_stride_head;
+  const float* acc_lse;
+  int64_t acc_lse_stride_head;
+  uint64_t kv_base;
+  int32_t num_entries, num_tiles, piece_tiles, num_units, num_slots;
+  int32_t num_heads, num_kv_heads, head_dim, dtype;
+  int32_t causal, window, paged, acc_is_prefix;
+  float scale;
+} hcp_varlen_args;
+
+int hcp_varlen_launch(const hcp_varlen_args* args, void* stream);
+
+/*
+ * Copies one step's small metadata to host memory: the n + 1 query starts,
+ * the n sequence lengths and the n first block ids (element 0 of each
+ * block-table row; block_table may be NULL: zeros), all widened to int64, into
+ * `host_out` [3 n + 1], which must be page-locked memory the GPU can write.
+ * Index dtypes are HCP_DTYPE_I32 / I64, strides in elements.  One kernel on
+ * `stream`; the caller waits for the stream before reading host_out.
+ */
+int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t qsl_stride,
+                       const void* seq_lens, int32_t lens_dtype, int64_t lens_stride,
+                       const void* block_table, int32_t bt_dtype, int64_t bt_stride,
+                       int32_t n, int64_t* host_out, void* stream);
 
 /*
  * Host-side split planner for hcp_decode_splitkv.  Each entry is one query
@@ -363,24 +389,74 @@ int hcp_decode_splitkv(const void* q, int64_t q_stride_tok,
                        int32_t dtype, void* stream);
 
 /*
- * hcp_decode_splitkv for sequences that are not all of the batch: the output
- * row (of out and lse) of sequence s is seq_rows[s], a DEVICE array.  For the
- * single-token rows of a batch that also holds prefill chunks.
+ * One split of a decode launch with everything its workgroup needs: the
+ * entry (a copy), the key range, the workspace slot and the next record of
+ * the same workgroup (-1: none).
  */
-int hcp_decode_splitkv_rows(const void* q, int64_t q_stride_tok,
-                            int64_t q_stride_head,
-                            const hcp_varlen_entry* entries,
-                            int32_t num_entries,
-                            const hcp_decode_split* splits,
-                            int32_t num_splits,
-                            const int32_t* seq_partial_start,
-                            const int32_t* seq_rows, int32_t num_seqs,
-                            void* workspace, size_t workspace_bytes, void* out,
-                            int64_t o_stride_tok, int64_t o_stride_head,
-                            float* lse, int64_t lse_stride_head,
-                            int32_t num_heads, int32_t num_kv_heads,
-                            int32_t head_dim, float scale, int32_t dtype,
-                            void* stream);
+typedef struct hcp_decode_work {
+  hcp_varlen_entry e;
+  int32_t key_begin, key_end;
+  int32_t slot;
+  int32_t next;
+  int32_t reserved[4];
+} hcp_decode_work;
+
+/*
+ * Host-side planner of hcp_decode_launch.  workgroups > 0 (split_tokens 0)
+ * gives every workgroup an equal share of the batch's keys: the keys of all
+ * entries are laid end to end and cut into at most `workgroups` runs (per KV
+ * head and chunk of 16 query heads), a run that crosses entries becoming
+ * several records of one workgroup.  split_tokens > 0 (workgroups 0) cuts every
+ * entry into pieces of at most that many keys, a workgroup each.  Every key
+ * of an entry is taken (no causal bound).  entry_seq as
+ * hcp_plan_decode_splits.  Writes the records -- record w < num_wgs is the
+ * first of workgroup w --, the entry each came from (work_entry, may be NULL)
+ * and seq_partial_start [num_seqs + 1]; returns the number of records (at most
+ * num_entries + workgroups, or the pieces).  Runs on the CPU only.
+ */
+int hcp_plan_decode_lists(const hcp_varlen_entry* entries, int32_t num_entries,
+                          const int32_t* entry_seq, int32_t num_seqs,
+                          int32_t workgroups, int32_t split_tokens,
+                          hcp_decode_work* works, int32_t* work_entry,
+                          int32_t cap, int32_t* seq_partial_start,
+                          int32_t* num_wgs);
+
+/*
+ * Split-KV decode over planned records (a DEVICE array): as
+ * hcp_decode_splitkv and, with acc_o, hcp_decode_splitkv_acc.
+ *   seq_rows     DEVICE array: the out / lse / acc row of each sequence, for the
+ *                single-token rows of a batch that also holds prefill chunks
+ *                (NULL: row s for sequence s)
+ *   kv_base      added to k_addr and v_addr of paged records, so that one plan on
+ *                the device serves every layer's cache
+ *   use_scratch  partials in the library's scratch, not in workspace (as
+ *                hcp_decode_splitkv_noalloc)
+ */
+typedef struct hcp_decode_args {
+  const void* q;
+  int64_t q_stride_tok, q_stride_head;
+  const hcp_decode_work* works;
+  const int32_t* seq_partial_start;
+  const int32_t* seq_rows;
+  void* workspace;
+  uint64_t workspace_bytes;
+  const void* acc_o;
+  int64_t acc_stride_tok, acc_stride_head;
+  const float* acc_lse;
+  int64_t acc_lse_stride_head;
+  void* out;
+  int64_t o_stride_tok, o_stride_head;
+  float* lse;
+  int64_t lse_stride_head;
+  uint64_t kv_base;
+  int32_t num_works, num_wgs, num_seqs;
+  int32_t num_heads, num_kv_heads, head_dim, dtype;
+  int32_t use_scratch;
+  float scale;
+  int32_t reserved;
+} hcp_decode_args;
+
+int hcp_decode_launch(const hcp_decode_args* args, void* stream);
 
 /*
  * Split-KV decode merged into a running accumulator: the decode ring's step

@@ -1,6 +1,7 @@
-"""The KV-split planners on the CPU: every (query block, tile) of a batch is in
+"""The split planners on the CPU: every (query block, tile) of a prefill batch is in
 exactly one piece, slots are used once, and a launch that fills the machine is
-left whole (``hcp_plan_varlen_split``, ``hcp_plan_fwd_split``)."""
+left whole (``hcp_plan_varlen_split``, ``hcp_plan_fwd_split``); every key of a
+decode batch is in exactly one record (``hcp_plan_decode_lists``)."""
 
 import ctypes
 
@@ -8,7 +9,7 @@ import numpy as np
 import pytest
 
 from hcp_vllm_plugin_amd import _lib
-from hcp_vllm_plugin_amd.varlen import ENTRY_DTYPE
+from hcp_vllm_plugin_amd.varlen import ENTRY_DTYPE, WORK_DTYPE
 
 CAP = 4096
 
@@ -90,3 +91,77 @@ def test_full_launches_stay_whole():
     assert pt > 0 and w.value == 0 and nb.value == 4 * np_ * 28 * 128 * 129 * 4
     assert L.hcp_plan_fwd_split(4, 4, 28, 3, 128, 0, 0, 0, ctypes.addressof(w),
                                 ctypes.addressof(nb)) == _lib.HCP_EINVAL
+
+
+def _lists(lens, seqs, num_seqs, workgroups, split_tokens=0):
+    n = len(lens)
+    a = np.zeros(max(n, 1), dtype=ENTRY_DTYPE)
+    a["q_len"], a["q_start"][:n], a["len"][:n] = 1, seqs, lens
+    cap = n + workgroups + (sum(-(-x // split_tokens) for x in lens) if split_tokens else 0)
+    works = np.zeros(max(cap, 1), dtype=WORK_DTYPE)
+    entry, starts = np.zeros(max(cap, 1), np.int32), np.zeros(num_seqs + 1, np.int32)
+    seq, m = np.asarray(list(seqs) or [0], np.int32), ctypes.c_int32(0)
+    L = _lib.lib()
+    rc = L.hcp_plan_decode_lists(a.ctypes.data, n, seq.ctypes.data, num_seqs, workgroups,
+                                 split_tokens, works.ctypes.data, entry.ctypes.data, cap,
+                                 starts.ctypes.data, ctypes.addressof(m))
+    _lib.check(rc, "hcp_plan_decode_lists")
+    return works[:rc], entry[:rc], starts, m.value
+
+
+@pytest.mark.parametrize("workgroups,split", [(64, 0), (1, 0), (7, 0), (256, 0), (0, 64), (0, 1000)])
+@pytest.mark.parametrize("lens,seqs,num_seqs", [
+    ([2000], [0], 1), ([1], [0], 1), ([32768, 512], [0, 0], 1), ([], [], 3),
+    ([5000, 0, 31, 33, 8192, 64], [0, 0, 1, 3, 3, 4], 6), ([100] * 300, range(300), 300),
+    ([513, 2048, 700, 1999] * 16, range(64), 64),
+])
+def test_decode_lists_cover_every_key_once(lens, seqs, num_seqs, workgroups, split):
+    works, entry, starts, wgs = _lists(lens, seqs, num_seqs, workgroups, split)
+    assert wgs <= (workgroups or len(works))
+    # every record is reached from exactly one workgroup's list
+    seen, loads = set(), []
+    for w in range(wgs):
+        load, j = 0, w
+        while j >= 0:
+            assert j not in seen
+            seen.add(j)
+            load += 8 - (int(works[j]["key_begin"]) - int(works[j]["key_end"])) // 32
+            j = int(works[j]["next"])
+        loads.append(load)
+    assert seen == set(range(len(works)))
+    # slots: one each, in sequence order; key ranges: each entry cut end to end
+    by_slot = np.argsort(works["slot"])
+    assert (works["slot"][by_slot] == np.arange(len(works))).all()
+    pos = [0] * len(lens)
+    for j in by_slot:
+        e, w = int(entry[j]), works[j]
+        assert w["e"]["q_start"] == list(seqs)[e] and w["e"]["len"] == lens[e]
+        assert w["key_begin"] == pos[e] < w["key_end"]
+        pos[e] = int(w["key_end"])
+        assert starts[list(seqs)[e]] <= w["slot"] < starts[list(seqs)[e] + 1]
+        if split:
+            assert w["key_end"] - w["key_begin"] <= split
+    assert pos == list(lens) and starts[0] == 0 and starts[-1] == len(works)
+    if not split and len(works):  # no workgroup far above an even share
+        even = (sum(-(-x // 32) for x in lens) + 8 * len(works)) / workgroups
+        assert max(loads) <= even + 8 + 16
+
+
+def test_decode_lists_refuse_bad_input():
+    L = _lib.lib()
+    a = np.zeros(2, dtype=ENTRY_DTYPE)
+    a["q_len"], a["len"] = 1, 1000
+    works, starts = np.zeros(4, dtype=WORK_DTYPE), np.zeros(3, np.int32)
+    m = ctypes.c_int32(0)
+
+    def call(seq, ns=2, wgs=64, st=0, cap=4):
+        s = np.asarray(seq, np.int32)
+        return L.hcp_plan_decode_lists(a.ctypes.data, 2, s.ctypes.data, ns, wgs, st,
+                                       works.ctypes.data, 0, cap, starts.ctypes.data,
+                                       ctypes.addressof(m))
+
+    assert call([1, 0]) == call([0, 2]) == call([0, 1], wgs=0) == _lib.HCP_EINVAL
+    assert call([0, 1], st=64) == _lib.HCP_EINVAL
+    assert call([0, 1], cap=1) == _lib.HCP_EWORKSPACE
+    a["q_len"] = 2
+    assert call([0, 1]) == _lib.HCP_EINVAL
