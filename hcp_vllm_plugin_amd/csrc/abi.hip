@@ -581,12 +581,12 @@ static int fwd_varlen_impl(const char* who, const void* q, int64_t q_stride_tok,
                            int32_t num_kv_heads, int32_t head_dim, float scale, int32_t causal,
                            int32_t window, int32_t paged, int32_t dtype, void* stream,
                            const AccArgs* acc, const SplitArgs* split = nullptr,
-                           uint64_t kv_base = 0) {
+                           uint64_t kv_base = 0, bool lse_optional = false) {
   int rc = check_heads(num_heads, num_kv_heads, head_dim, dtype, who);
   if (rc) return rc;
   if (num_entries < 0 || num_tiles < 0) return fail(HCP_EINVAL, "%s: negative counts", who);
   if (num_tiles == 0) return HCP_OK;
-  if (!q || !out || (!lse && !acc) || !entries || !tiles)
+  if (!q || !out || (!lse && !acc && !lse_optional) || !entries || !tiles)
     return fail(HCP_EINVAL, "%s: null pointer", who);
   if (acc && (rc = check_acc(*acc, who))) return rc;
   if (!aligned16(q) || !aligned16(out)) return fail(HCP_EINVAL, "%s: q/out not 16-byte aligned", who);
@@ -675,7 +675,7 @@ int hcp_varlen_launch(const hcp_varlen_args* a, void* stream) {
                          a->tiles, a->num_tiles, a->num_heads, a->num_kv_heads, a->head_dim,
                          a->scale, a->causal, a->window, a->paged, a->dtype, stream,
                          a->acc_o || a->acc_lse ? &acc : nullptr,
-                         a->piece_tiles > 0 ? &split : nullptr, a->kv_base);
+                         a->piece_tiles > 0 ? &split : nullptr, a->kv_base, true);
 }
 
 int hcp_plan_decode_splits(const hcp_varlen_entry* entries, int32_t num_entries,

@@ -52,6 +52,7 @@ from __future__ import annotations
 import enum
 import logging
 import os
+import threading
 
 import numpy as np
 import torch
@@ -62,6 +63,7 @@ from .merge import merge_attn_states
 from .ring_attn import COPY_STATS, ring_attn_with_lse
 from .ring_decode import GrowthBuffer, growth_assignee, local_partial, ring_decode_step
 from .varlen import (
+    _MIN_PAGED_BLOCK,
     ENTRY_DTYPE,
     head_major,
     DecodeBatch,
@@ -175,7 +177,8 @@ def _note_staging(k: torch.Tensor) -> None:
     STAGING_STATS["last_chunk_len"] = int(k.shape[0])
 
 
-def _wait_staged(key: tuple[str, str], kv: tuple[torch.Tensor, torch.Tensor]) -> None:
+def _wait_staged(key: tuple[str, str], kv: tuple[torch.Tensor, torch.Tensor],
+                 cur: torch.cuda.Stream | None = None) -> None:
     """Order the current stream after the staging copy of ``key`` (once per
     stream).  A chunk staged on another stream is also marked as used on this
     one, so the caching allocator keeps its memory until this stream's reads
@@ -184,7 +187,8 @@ def _wait_staged(key: tuple[str, str], kv: tuple[torch.Tensor, torch.Tensor]) ->
     if ent is None:
         return
     ev, seen = ent
-    cur = torch.cuda.current_stream(kv[0].device)
+    if cur is None:  # (a caller with many chunks looks it up once)
+        cur = torch.cuda.current_stream(kv[0].device)
     if cur in seen:
         return
     cur.wait_event(ev)
@@ -293,15 +297,24 @@ def _release_staged_for_request(first_block_id: int) -> None:
             drop_chunk_kv(ck)
 
 
-def _contiguous_record(j: int, seq: int, k: torch.Tensor, v: torch.Tensor):
-    """hcp_varlen_entry of decode query row ``seq`` over all of a staged chunk
-    (contiguous k/v ``[n, Hkv, D]``), as an ENTRY_DTYPE record value."""
-    if k.stride() != v.stride() or k.data_ptr() % 16 or v.data_ptr() % 16 or \
-            (k.stride(0) * k.element_size()) % 16 or (k.stride(1) * k.element_size()) % 16 or \
-            not 0 < k.stride(0) < (1 << 24):
-        raise ValueError(f"staged chunk of entry {j}: k/v layout not loadable")
-    return (seq, 1, 0, k.data_ptr(), v.data_ptr(), 0, k.stride(0), k.stride(1), 0, 0,
-            int(k.shape[0]), 0, 0)
+def _set_staged_addresses(ent: np.ndarray, idx: np.ndarray, kvs: list) -> None:
+    """Point entries ``idx`` at all of the staged chunks ``kvs`` (contiguous
+    k/v ``[n, Hkv, D]``), checked as ``segment_contiguous`` checks one."""
+    ks = [k.data_ptr() for k, _ in kvs]
+    vs = [v.data_ptr() for _, v in kvs]
+    st = [k.stride() for k, _ in kvs]
+    if st != [v.stride() for _, v in kvs]:
+        raise ValueError("staged chunk: k/v layout not loadable")
+    ka, va = np.array(ks, dtype=np.uint64), np.array(vs, dtype=np.uint64)
+    sa = np.array(st, dtype=np.int64)
+    es = kvs[0][0].element_size()
+    if ((ka | va) % np.uint64(16)).any() or ((sa[:, :2] * es) % 16).any() or \
+            (sa[:, 0] <= 0).any() or (sa[:, 0] >= 1 << 24).any():
+        raise ValueError("staged chunk: k/v layout not loadable")
+    ent["k_addr"][idx] = ka
+    ent["v_addr"][idx] = va
+    ent["stride_tok"][idx] = sa[:, 0]
+    ent["stride_head"][idx] = sa[:, 1]
 
 
 # Host copy of the step's attention metadata.  vLLM hands every layer the same
@@ -354,12 +367,43 @@ def _host_metadata(attn_metadata):
     qsl_t = attn_metadata.query_start_loc
     sl_t = attn_metadata.seq_lens
     n = sl_t.shape[0]
-    fb = block_table[:, 0] if block_table.shape[1] > 0 else sl_t.new_zeros(n)
-    packed = torch.cat([qsl_t.reshape(-1).to(torch.int64), sl_t.reshape(-1).to(torch.int64),
-                        fb.reshape(-1).to(torch.int64)]).tolist()
-    host = (packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:])
+    if _fetchable(qsl_t, n + 1) and _fetchable(sl_t, n) and block_table.is_cuda:
+        host = _fetch_metadata(qsl_t, sl_t, block_table, n)
+    else:
+        fb = block_table[:, 0] if block_table.shape[1] > 0 else sl_t.new_zeros(n)
+        packed = torch.cat([qsl_t.reshape(-1).to(torch.int64), sl_t.reshape(-1).to(torch.int64),
+                            fb.reshape(-1).to(torch.int64)]).tolist()
+        host = (packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:])
     _STEP.update(meta=attn_metadata, stamp=stamp, host=host, bt=block_table, fast={})
     return host, block_table
+
+
+_INDEX_CODES = {torch.int32: _lib.DTYPE_I32, torch.int64: _lib.DTYPE_I64}
+_fetch_buf = threading.local()  # page-locked, per thread: read before the call returns
+
+
+def _fetchable(t: torch.Tensor, n: int) -> bool:
+    return t.is_cuda and t.dim() == 1 and t.shape[0] == n and t.dtype in _INDEX_CODES
+
+
+def _fetch_metadata(qsl_t, sl_t, block_table, n: int):
+    """The step's metadata as host lists, by one kernel that writes it to
+    page-locked memory and one wait for the stream."""
+    buf = getattr(_fetch_buf, "buf", None)
+    if buf is None or buf.shape[0] < 3 * n + 1:
+        buf = _fetch_buf.buf = torch.empty(max(1024, 4 * n), dtype=torch.int64, pin_memory=True)
+        _fetch_buf.np = buf.numpy()
+    dev = qsl_t.device
+    with _lib.on_device(dev):
+        rc = _lib.lib().hcp_fetch_metadata(
+            qsl_t.data_ptr(), _INDEX_CODES[qsl_t.dtype], qsl_t.stride(0),
+            sl_t.data_ptr(), _INDEX_CODES[sl_t.dtype], sl_t.stride(0),
+            block_table.data_ptr() if block_table.shape[1] > 0 else 0, _lib.DTYPE_I32,
+            block_table.stride(0), n, buf.data_ptr(), _lib.stream_ptr(dev))
+        _lib.check(rc, "hcp_fetch_metadata")
+        torch.cuda.current_stream(dev).synchronize()
+    packed = _fetch_buf.np[:3 * n + 1].tolist()
+    return packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:]
 
 
 def _forward_attn_metadata(layer):
@@ -532,6 +576,13 @@ class HcpRingAttentionBackend(_BackendBase):  # type: ignore[misc,valid-type]
     @staticmethod
     def get_builder_cls():
         return _BuilderCls
+
+
+def _check_base(pc: PagedCache) -> None:
+    """A layer's cache address, the one thing of its layout that a step's plan
+    is not keyed on."""
+    if pc.k_addr % 16 or pc.v_addr % 16:
+        raise ValueError("k/v base addresses must be 16-byte aligned")
 
 
 class _Plan:
@@ -904,150 +955,183 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
     # -- pure decode batches with staged peers ------------------------------------
     def _decode_staged_template(self, seq_lens, block_table, first_blocks, pc, layer_name):
         """The step's decode entries with every field that does not change
-        from layer to layer (lengths, block-table rows, strides of the cache),
-        the split plan over them, and where each layer's addresses go; False
-        if some request's staging is incomplete (the general path then
-        decides, per layer, as the reference does)."""
+        from layer to layer (lengths, block-table rows, strides of the cache;
+        paged addresses relative to the layer's cache), and which staged chunk
+        each contiguous one reads; False if some request's staging is
+        incomplete (the general path then decides, per layer, as the reference
+        does)."""
         n = len(seq_lens)
         w = self.sliding_window
-        seq, kinds, rows, starts, lens, peers = [], [], [], [], [], []
-        for r in range(n):
-            tk = int(seq_lens[r])
-            staged = None
-            if _ring_enabled():
-                staged = self._peer_for_request(first_blocks[r], layer_name, n)
-                if staged is None and PEER_REQ_MAP.get(first_blocks[r]):
-                    return False  # staging still arriving: decided per layer
-            peer_end = min(sum(int(kv[0].shape[0]) for kv in staged), tk) if staged else 0
+        ring_on = _ring_enabled()
+        lone = None  # the single-request fallback of _peer_for_request
+        if n == 1 and ring_on:
+            chunks = {key[0] for key in PEER_KV_STAGING}
+            lone = list(chunks) if len(chunks) == 1 else None
+        seq, kinds, starts, lens, peers = [], [], [], [], []
+        for r, (tk, fb) in enumerate(zip(seq_lens, first_blocks)):
+            peer_end, ck_list, chunk_lens = 0, None, ()
+            if ring_on:
+                ck_list = PEER_REQ_MAP.get(fb)
+                if ck_list is None:
+                    ck_list = lone
+                if ck_list:
+                    kvs = [PEER_KV_STAGING.get((ck, layer_name)) for ck in ck_list]
+                    if any(kv is None for kv in kvs):
+                        return False  # staging still arriving: decided per layer
+                    chunk_lens = [kv[0].shape[0] for kv in kvs]
+                    peer_end = min(sum(chunk_lens), tk)
             # one query at position tk - 1 (ring_backend.py:626-627): inside the
             # prefix it sees the whole local range (:811-817), else the local
             # keys past the prefix plus every staged chunk (:820-830)
             lo = 0 if peer_end == 0 or peer_end >= tk else peer_end
             if w is not None:  # the causal pass sees the last `w` local keys
                 lo = max(lo, tk - w)
-            seq.append(r); kinds.append(0); rows.append(r); starts.append(lo); lens.append(tk - lo)
+            seq.append(r)
+            kinds.append(0)
+            starts.append(lo)
+            lens.append(tk - lo)
             if 0 < peer_end < tk:
-                ck_list = PEER_REQ_MAP.get(first_blocks[r])
-                if ck_list is None:  # the single-request fallback of _peer_for_request
-                    ck_list = [next(iter({key[0] for key in PEER_KV_STAGING}))]
-                for ck, (kk, _vv) in zip(ck_list, staged):
-                    if kk.shape[0] > 0:
-                        seq.append(r); kinds.append(1); rows.append(r); starts.append(0)
-                        lens.append(int(kk.shape[0]))
-                        peers.append((len(seq) - 1, ck, int(kk.shape[0])))
-        m = len(seq)
+                for ck, cl in zip(ck_list, chunk_lens):
+                    if cl > 0:
+                        peers.append((ck, cl))
+                        seq.append(r)
+                        kinds.append(1)
+                        starts.append(0)
+                        lens.append(cl)
         kinds = np.asarray(kinds)
+        seq = np.asarray(seq, dtype=np.int32)
         loc = np.nonzero(kinds == 0)[0]
-        tmpl = np.zeros(m, dtype=ENTRY_DTYPE)
+        tmpl = np.zeros(len(seq), dtype=ENTRY_DTYPE)
         tmpl["q_start"] = seq
         tmpl["q_len"] = 1
-        tmpl["start"] = starts
         tmpl["len"] = lens
-        if len(loc):
-            tmpl[loc] = paged_entry_array(pc, block_table, np.asarray(rows)[loc], tmpl["q_start"][loc],
-                                          1, 0, tmpl["start"][loc], tmpl["len"][loc])
-        first = tmpl.copy()
-        for j, ck, _nt in peers:
-            k, v = PEER_KV_STAGING[(ck, layer_name)]
-            first[j] = _contiguous_record(j, seq[j], k, v)
-        batch = DecodeBatch.from_entries(first, self.num_heads, self.num_kv_heads, self.head_size,
-                                         block_table.device, entry_seq=np.asarray(seq, np.int32),
-                                         num_seqs=n)
-        return {"tmpl": tmpl, "loc": loc, "peers": peers, "batch": batch}
+        tmpl[loc] = paged_entry_array(pc, block_table, seq[loc], seq[loc], 1, 0,
+                                      np.asarray(starts)[loc], tmpl["len"][loc], relative=True)
+        return {"tmpl": tmpl, "seq": seq, "at": np.nonzero(kinds == 1)[0], "peers": peers,
+                "batch": None}
 
     def _forward_decode_staged(self, query, out, seq_lens, block_table, first_blocks, pc,
                                kv_cache, layer_name, ring_on, split) -> bool:
         """A pure decode batch without decode-ring rows: one split-KV launch
         over every request's local paged segment and staged peer chunks, its
         split plan built once per step and reused by every layer, each layer
-        writing only its addresses (the cache, the layer's staged chunks) into
-        the entries and uploading them in one small copy.  False when the
-        general path must run (split env, decode-ring rows, staging that
-        differs from the step's template)."""
+        writing only its staged chunks' addresses into the records and
+        uploading them in one small copy (the cache's address is a launch
+        argument).  False when the general path must run (split env,
+        decode-ring rows, staging that differs from the step's template)."""
         if split > 0 or (_decode_ring_enabled() and DECODE_RING_MAP
                          and any(fb in DECODE_RING_MAP for fb in first_blocks)):
             return False
         # (the staging generation: a chunk staged, dropped or mapped after the
         # template was built -- even for a request the template saw without
-        # peers -- makes the next layer build a new one)
+        # peers -- makes the next layer build a new one; the stream: the plan's
+        # upload is ordered on the one it was made on)
         key = ("dec_staged", self.sliding_window, pc.layout, pc.stride_tok, pc.stride_head,
                pc.stride_block, pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, ring_on,
-               _STAGE_GEN[0])
+               _STAGE_GEN[0], self._heads, _lib.stream_ptr(query.device))
         st = _STEP["fast"].get(key)
         if st is None:
             st = self._decode_staged_template(seq_lens, block_table, first_blocks, pc, layer_name)
             _STEP["fast"][key] = st
         if st is False:
             return False
-        ent = st["tmpl"].copy()
-        ent["k_addr"][st["loc"]] = pc.k_addr
-        ent["v_addr"][st["loc"]] = pc.v_addr
-        keep = [kv_cache, block_table]
-        for j, ck, nt in st["peers"]:
+        _check_base(pc)
+        kvs = []
+        cur = torch.cuda.current_stream(query.device)
+        for ck, nt in st["peers"]:
             kv = PEER_KV_STAGING.get((ck, layer_name))
-            if kv is None or int(kv[0].shape[0]) != nt:
+            if kv is None or kv[0].shape[0] != nt:
                 return False
-            _wait_staged((ck, layer_name), kv)
-            ent[j] = _contiguous_record(j, int(ent["q_start"][j]), kv[0], kv[1])
-            keep.append(kv)
-        st["batch"].rebind(ent, keep).run(query, out, None, self.scale)
+            _wait_staged((ck, layer_name), kv, cur)
+            kvs.append(kv)
+        ent = st["tmpl"]
+        if kvs:
+            ent = ent.copy()
+            _set_staged_addresses(ent, st["at"], kvs)
+        batch = st["batch"]
+        if batch is None:
+            batch = st["batch"] = DecodeBatch.from_entries(
+                ent, self.num_heads, self.num_kv_heads, self.head_size, query.device,
+                keep=block_table, entry_seq=st["seq"], num_seqs=len(seq_lens))
+        elif kvs:
+            batch = batch.rebind(ent, (block_table, kvs))
+        batch.run(query, out, None, self.scale, kv_base=pc.k_addr)
         _count("decode")
         return True
 
     def _forward_local_only(self, query, out, qsl, seq_lens, block_table, pc, kv_cache):
-        """Causal attention of every request over its paged KV, the batch's
-        entries built with array operations (once per step and cache layout,
-        then only the layer's cache address changes): a split-KV decode for a
-        pure decode batch, else one varlen launch."""
+        """Causal attention of every request over its paged KV: a split-KV
+        decode for a pure decode batch, else one varlen launch (and a decode
+        launch for the single-token rows).  Planned and uploaded once per
+        step, cache layout and stream; a layer's launch adds its cache's
+        address."""
         n = len(seq_lens)
         if n == 0:
             return
-        is_decode = qsl == list(range(n + 1))
         w = self.sliding_window
-        key = (is_decode, w, pc.layout, pc.stride_tok, pc.stride_head, pc.stride_block,
-               pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr)
-        tmpl = _STEP["fast"].get(key)
-        if tmpl is None:
-            qs = np.asarray(qsl[:-1], dtype=np.int64)
-            tq = np.diff(np.asarray(qsl, dtype=np.int64))
-            tk = np.asarray(seq_lens, dtype=np.int64)
-            rows = np.arange(n, dtype=np.int64)
-            dec = tq == 1
-            if not is_decode and not self._decode_rows_apart(qsl, seq_lens):
-                dec[:] = False
-            pre = (tq > 0) & ~dec
+        key = ("local", w, pc.layout, pc.stride_tok, pc.stride_head, pc.stride_block,
+               pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, self._heads,
+               _lib.stream_ptr(query.device))
+        st = _STEP["fast"].get(key)
+        if st is None:
+            st = _STEP["fast"][key] = self._plan_local_only(query, qsl, seq_lens, block_table, pc)
+        pre, dec = st
+        _check_base(pc)
+        if pre is not None:
+            if isinstance(pre, np.ndarray):
+                # blocks under 16 tokens are gathered from absolute addresses
+                ent = pre.copy()
+                ent["k_addr"] = pc.k_addr
+                ent["v_addr"] = pc.v_addr
+                VarlenLaunch(ent, True, True, query.device, keep=(kv_cache, block_table),
+                             heads=self._heads, window=w).run(
+                    query, out, None, self.num_kv_heads, self.scale, w)
+            else:
+                pre.run(query, out, None, self.num_kv_heads, self.scale, w, kv_base=pc.k_addr)
+            _count("attn")
+        if dec is not None:
+            dec.run(query, out, None, self.scale, kv_base=pc.k_addr)
+            _count("decode")
+
+    def _plan_local_only(self, query, qsl, seq_lens, block_table, pc):
+        """(prefill launch or None, decode launch or None) of a batch without
+        peers, with addresses relative to the layer's cache; over blocks under
+        16 tokens the prefill's entries instead."""
+        n = len(seq_lens)
+        w = self.sliding_window
+        qs = np.asarray(qsl[:-1], dtype=np.int64)
+        tq = np.diff(np.asarray(qsl, dtype=np.int64))
+        tk = np.asarray(seq_lens, dtype=np.int64)
+        rows = np.arange(n, dtype=np.int64)
+        dec = tq == 1
+        all_dec = qsl == list(range(n + 1))
+        if not all_dec and not self._decode_rows_apart(qsl, seq_lens):
+            dec[:] = False
+        pre = (tq > 0) & ~dec
+        launch = batch = None
+        if pre.any():
+            launch = paged_entry_array(pc, block_table, rows[pre], qs[pre], tq[pre],
+                                       (tk - tq)[pre], 0, tk[pre], relative=True)
+            if pc.block_size >= _MIN_PAGED_BLOCK:
+                launch = VarlenLaunch(launch, True, True, query.device, keep=block_table,
+                                      heads=self._heads, window=w)
+        if dec.any():
             # one query at the end of its keys: all of them visible, or
             # the last `w` of them (ring_backend.py:397-398)
             start = np.zeros(n, np.int64) if w is None else np.maximum(tk - w, 0)
-            tmpl = (paged_entry_array(pc, block_table, rows[pre], qs[pre], tq[pre],
-                                      (tk - tq)[pre], 0, tk[pre]),
-                    paged_entry_array(pc, block_table, rows[dec], qs[dec], 1, 0, start[dec],
-                                      (tk - start)[dec]))
-            _STEP["fast"][key] = tmpl
-        keep = (kv_cache, block_table)
-        pre, dec = (t.copy() for t in tmpl)
-        for ent in (pre, dec):
-            ent["k_addr"] = pc.k_addr
-            ent["v_addr"] = pc.v_addr
-        if len(pre):
-            lse = torch.empty((self.num_heads, query.shape[0]), dtype=torch.float32,
-                              device=query.device)
-            VarlenLaunch(pre, True, True, query.device, keep=keep, heads=self._heads,
-                         window=w).run(query, out, lse, self.num_kv_heads, self.scale, w)
-            _count("attn")
-        if len(dec):
-            DecodeBatch.from_entries(
-                dec, self.num_heads, self.num_kv_heads, self.head_size, query.device, keep=keep,
-                rows=None if is_decode else dec["q_start"]).run(query, out, None, self.scale)
-            _count("decode")
+            batch = DecodeBatch.from_entries(
+                paged_entry_array(pc, block_table, rows[dec], qs[dec], 1, 0, start[dec],
+                                  (tk - start)[dec], relative=True),
+                self.num_heads, self.num_kv_heads, self.head_size, query.device,
+                keep=block_table, rows=None if all_dec else qs[dec])
+        return launch, batch
 
     def _forward_prefill(self, query, out, plan: _Plan) -> None:
         dev = query.device
         h = self.num_heads
         if not plan.any_peer:
-            lse = torch.empty((h, query.shape[0]), dtype=torch.float32, device=dev)
             VarlenLaunch(plan.local, True, True, dev, heads=self._heads,
-                         window=self.sliding_window).run(query, out, lse, self.num_kv_heads,
+                         window=self.sliding_window).run(query, out, None, self.num_kv_heads,
                                                          self.scale, self.sliding_window)
             _count("attn")
             return

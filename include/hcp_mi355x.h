@@ -292,7 +292,8 @@ int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries,
                           int32_t* piece_tiles, size_t* workspace_bytes);
 
 /*
- * hcp_attn_fwd_varlen (acc_o and acc_lse NULL) or hcp_attn_fwd_varlen_merge.
+ * hcp_attn_fwd_varlen (acc_o and acc_lse NULL) or hcp_attn_fwd_varlen_merge;
+ * lse may be NULL in both.
  *   tiles, num_tiles   DEVICE records of hcp_plan_varlen_tiles (piece_tiles 0)
  *                      or the pieces of hcp_plan_varlen_split (same entries,
  *                      causal, window and heads), with its units, num_units
