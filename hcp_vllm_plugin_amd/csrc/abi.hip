@@ -111,24 +111,30 @@ struct Cut {
 };
 
 // Estimated time (us) of a launch over `units` (per head, longest first) cut
-// as `c`: the workgroups, longest first, go to the least loaded CU of one XCD
-// (all XCDs get the same mix).  A CU runs one tile (128 rows x 64 keys) per
-// tile_us whether one or two workgroups share it, so the machine counts as
-// 256 slots; one alone takes about 15% longer per tile, and two with one wave
-// of rows each run side by side.  Constants from measured launches (us):
-// 512 x 32768 at 28 / 4 x 128 whole 490, cut in 2 / 4 / 9 / 16: 311 / 256 /
-// 241 / 254 (estimated 307 / 265 / 247 / 257); 512 x 4096 whole 66, cut in 2 /
-// 8 / 16: 47 / 55 / 70 (47 / 56 / 68); 3001 x 5003 at 14 / 2 x 64 whole 90,
-// cut in 2 / 3: 86 / 81 (82 / 79).
+// as `c`, or a lower bound of it that is already past `limit`.  The workgroups
+// of one XCD (all XCDs get the same mix), longest first, are run through its
+// CUs as the hardware runs them: two to a CU (one at head_dim 256), the next
+// into the first slot that frees.  Two workgroups on a CU take tile_us per
+// tile (128 rows x 64 keys) between them; one alone takes up to 15% longer
+// per tile than two (less when few CUs are busy and the clock is higher), and
+// two with one wave of rows each run side by side.  Measured / estimated, us:
+// 512 x 32768 at 28 / 4 x 128 whole 488 / 495, cut in 2, 4, 9, 16: 320, 257,
+// 248, 262 / 298, 265, 247, 286; 512 x 4096 whole 67 / 64, cut in 2, 4, 8: 48,
+// 47, 55 / 48, 48, 56; 3001 x 5003 at 14 / 2 x 64 whole 93 / 91, cut in 3: 82 /
+// 77, cut in 3 past 18 whole blocks 74 / 75; 600 x 6000 at 16 / 8 x 256 whole
+// 168 / 170, cut in 3: 82 / 79.
 double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh, int dw,
-                  double limit) {
+                  double limit, bool* hopeless = nullptr) {
   const double tile_us = dw == 64 ? 0.54 : dw == 128 ? 0.97 : 1.75;
-  const double start_us = dw == 256 ? 5.0 : 1.5;  // per workgroup
+  const double first_us = dw == 256 ? 5.0 : 3.0;   // start and end of a first workgroup
+  const double start_us = dw == 256 ? 5.0 : 1.0;   // of one that follows
   const double part_us = dw == 64 ? 0.006 : dw == 128 ? 0.012 : 0.04;  // per partial
   const double reduce_us = dw == 256 ? 8.0 : 6.0;  // the second launch
-  // by waves with rows: two workgroups on a CU / one alone
-  static constexpr double kShared[5] = {0.5, 0.5, 0.65, 0.85, 1.0};
-  static constexpr double kAlone[5] = {0.9, 0.9, 1.0, 1.08, 1.15};
+  const int slots = dw == 256 ? 1 : 2;
+  // by waves with rows: work of a tile relative to a full one, and the time of
+  // a workgroup alone on its CU relative to its work
+  static constexpr double kWork[5] = {0.5, 0.5, 0.65, 0.85, 1.0};
+  static constexpr double kAlone[5] = {1.8, 1.8, 1.55, 1.3, 1.15};
   // one XCD's share of the workgroups (xcd_remap), or the whole machine
   const bool by_xcd = num_kvh <= hcp::kNumXcd && hcp::kNumXcd % num_kvh == 0;
   const int share = by_xcd ? hcp::kNumXcd / num_kvh : 1;
@@ -138,40 +144,91 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
     return c.tiles > 0 && static_cast<int>(u) >= c.whole ? hcp::unit_pieces(units[u].tiles, c.tiles)
                                                          : 1;
   };
+  struct Job {
+    double work, alone;
+  };
+  std::vector<Job> jobs;  // workgroups of one head
   int64_t n = 0, parts = 0;
   for (size_t u = 0; u < units.size(); ++u) {
     n += pieces(u);
     if (pieces(u) > 1) parts += pieces(u);
   }
   if (c.tiles > 0 && n * group * num_kvh > kMaxPieces) return 1e30;
-  const bool alone = dw < 256 && n * per <= static_cast<int64_t>(cus) * share;
+  const double busy = std::min(1.0, static_cast<double>(n * per) / (cus * share));
+  const double full_alone = 1.0 + 0.3 * std::max(0.0, busy - 0.5);
   const double merge_us =
       parts > 0 ? reduce_us + static_cast<double>(parts) * group * num_kvh * part_us : 0.0;
-  std::vector<double> sz;  // workgroup times of one head
   double sum = 0;
   for (size_t u = 0; u < units.size(); ++u) {
-    const int nt = units[u].tiles, np = pieces(u);
-    const double t = tile_us * (alone ? kAlone : kShared)[units[u].waves];
-    sum += nt * t + np * start_us;
-    for (int i = 0; i < np; ++i)
-      sz.push_back((hcp::piece_begin(nt, np, i + 1) - hcp::piece_begin(nt, np, i)) * t);
+    const int nt = units[u].tiles, np = pieces(u), w = units[u].waves;
+    const double alone = slots == 1 ? 1.0 : w == 4 ? full_alone : kAlone[w];
+    for (int i = 0; i < np; ++i) {
+      const int tiles = hcp::piece_begin(nt, np, i + 1) - hcp::piece_begin(nt, np, i);
+      jobs.push_back({tiles * tile_us * kWork[w], alone});
+      sum += jobs.back().work + start_us;
+    }
   }
-  // evenly spread at best: not worth simulating when that already loses
-  const double even = 4.0 - start_us + sum * per / (static_cast<double>(cus) * share) + merge_us;
-  if (even >= limit) return even;
-  std::sort(sz.begin(), sz.end(), std::greater<double>());
-  std::vector<double> load(cus, 4.0 - start_us);  // min-heap
-  auto gt = std::greater<double>();
-  for (int64_t j = 0; j < n * per; j += share) {
-    std::pop_heap(load.begin(), load.end(), gt);
-    load.back() += sz[j / per] + start_us;
-    std::push_heap(load.begin(), load.end(), gt);
+  // evenly spread at best: not worth running through when that already loses
+  const double even = sum * per / (static_cast<double>(cus) * share) + merge_us;
+  if (even >= limit) {
+    if (hopeless) *hopeless = true;
+    return even;
   }
-  return *std::max_element(load.begin(), load.end()) + merge_us;
+  std::sort(jobs.begin(), jobs.end(), [](const Job& a, const Job& b) { return a.work > b.work; });
+  struct Cu {
+    double at = 0;        // time its jobs' work stands at
+    Job job[2];
+    int n = 0;
+    double next() const {  // when its next job ends
+      return at + (n == 1 ? job[0].work * job[0].alone : 2 * std::min(job[0].work, job[1].work));
+    }
+  };
+  std::vector<Cu> cu(cus);
+  int64_t j = 0;
+  const int64_t items = n * per;
+  auto give = [&](Cu& x, double extra) {
+    x.job[x.n] = jobs[j / per];
+    x.job[x.n++].work += extra;
+    j += share;
+  };
+  for (int s = 0; s < slots; ++s)
+    for (Cu& x : cu)
+      if (j < items) give(x, first_us);
+  typedef std::pair<double, int> Ev;  // (end of a CU's next job, CU), earliest on top
+  std::vector<Ev> heap;
+  for (int i = 0; i < cus; ++i)
+    if (cu[i].n) heap.push_back({cu[i].next(), i});
+  std::make_heap(heap.begin(), heap.end(), std::greater<Ev>());
+  double end = 0;
+  while (!heap.empty()) {
+    std::pop_heap(heap.begin(), heap.end(), std::greater<Ev>());
+    Cu& x = cu[heap.back().second];
+    end = heap.back().first;
+    if (x.n == 1) {
+      x.n = 0;
+    } else {
+      const double d = std::min(x.job[0].work, x.job[1].work);
+      Job left[2];
+      int m = 0;
+      for (const Job& y : x.job)
+        if (y.work - d > 1e-9) left[m++] = {y.work - d, y.alone};
+      for (int i = 0; i < m; ++i) x.job[i] = left[i];
+      x.n = m;
+    }
+    x.at = end;
+    while (x.n < slots && j < items) give(x, start_us);
+    if (x.n == 0) {
+      heap.pop_back();
+    } else {
+      heap.back().first = x.next();
+      std::push_heap(heap.begin(), heap.end(), std::greater<Ev>());
+    }
+  }
+  return end + merge_us;
 }
 
 // The cut of a launch over `units`, longest first; tiles 0 when cutting does
-// not pay (6% or more by the estimate).
+// not pay (8% or more by the estimate, whose error is about that).
 Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw) {
   Cut best;
   const int heads = group * num_kvh;
@@ -180,22 +237,26 @@ Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw) {
   if (units.empty() || static_cast<int64_t>(units.size()) * heads > kMaxUnits) return best;
   const int mx = units[0].tiles;
   if (mx < 2 * kMinPieceTiles) return best;
-  double t_best = split_cost(units, best, group, num_kvh, dw, 1e30) * 0.94;
+  double t_best = split_cost(units, best, group, num_kvh, dw, 1e30) * 0.92;
   // whole blocks spread evenly as they are: no cut can win
-  if (split_cost(units, best, group, num_kvh, dw, 0.0) >= t_best) return best;
+  bool none = false;
+  split_cost(units, best, group, num_kvh, dw, t_best, &none);
+  if (none) return best;
   for (int rounds = 0; rounds < 4; ++rounds) {
     // rounds > 0: only what is left after `rounds` whole blocks per CU
     Cut c;
     c.whole = kNumCus * rounds / heads;
     if (rounds > 0 && (c.whole == 0 || c.whole >= static_cast<int>(units.size()))) break;
     const int top = units[c.whole].tiles;
-    for (int k : {2, 3, 4, 5, 6, 8, 9, 12, 16, 20, 24, 32, 40, 48, 64}) {
+    for (int k : {2, 3, 4, 6, 9, 12, 16, 24, 32, 48, 64}) {
       const int tiles = (top + k - 1) / k;
       if (tiles < kMinPieceTiles) break;
       if (tiles == c.tiles) continue;
       c.tiles = tiles;
-      const double t = split_cost(units, c, group, num_kvh, dw, t_best);
-      if (t > 1e29) break;
+      bool hopeless = false;
+      const double t = split_cost(units, c, group, num_kvh, dw, t_best, &hopeless);
+      // more pieces only add to the even share: none of them can win either
+      if (hopeless || t > 1e29) break;
       if (t < t_best) {
         t_best = t;
         best = c;
