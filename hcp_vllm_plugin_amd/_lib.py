@@ -64,6 +64,8 @@ EXPORTED_SYMBOLS = (
     "hcp_decode_splitkv",
     "hcp_plan_decode_lists",
     "hcp_decode_launch",
+    "hcp_decode_paged_workspace",
+    "hcp_decode_paged",
     "hcp_decode_splitkv_acc",
     "hcp_decode_splitkv_noalloc",
     "hcp_merge_attn_states",
@@ -204,6 +206,38 @@ class VarlenArgs(ctypes.Structure):
     ]
 
 
+class DecodePagedArgs(ctypes.Structure):
+    """``hcp_decode_paged_args`` (include/hcp_mi355x.h)."""
+
+    _fields_ = [
+        ("q", ctypes.c_uint64),
+        ("q_stride_tok", ctypes.c_int64),
+        ("q_stride_head", ctypes.c_int64),
+        ("kv", KvSegment),
+        ("block_table_stride", ctypes.c_int64),
+        ("block_table_width", ctypes.c_int64),
+        ("seq_lens", ctypes.c_uint64),
+        ("workspace", ctypes.c_uint64),
+        ("workspace_bytes", ctypes.c_uint64),
+        ("out", ctypes.c_uint64),
+        ("o_stride_tok", ctypes.c_int64),
+        ("o_stride_head", ctypes.c_int64),
+        ("lse", ctypes.c_uint64),
+        ("lse_stride_head", ctypes.c_int64),
+        ("lens_dtype", ctypes.c_int32),
+        ("num_seqs", ctypes.c_int32),
+        ("window", ctypes.c_int32),
+        ("num_heads", ctypes.c_int32),
+        ("num_kv_heads", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32),
+        ("dtype", ctypes.c_int32),
+        ("scale", ctypes.c_float),
+    ]
+
+
+# include/hcp_mi355x.h HCP_DECODE_PAGED_MAX_SEQS
+DECODE_PAGED_MAX_SEQS = 1024
+
 _lock = threading.Lock()
 _lib = None
 
@@ -279,6 +313,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     ]
     lib.hcp_decode_launch.restype = ctypes.c_int
     lib.hcp_decode_launch.argtypes = [_P, _P]
+    lib.hcp_decode_paged_workspace.restype = ctypes.c_size_t
+    lib.hcp_decode_paged_workspace.argtypes = [_I32, _I32, _I32, _I32]
+    lib.hcp_decode_paged.restype = ctypes.c_int
+    lib.hcp_decode_paged.argtypes = [_P, _P]
     lib.hcp_decode_splitkv_acc.restype = ctypes.c_int
     lib.hcp_decode_splitkv_acc.argtypes = [
         _P, _I64, _I64, _P, _I32, _P, _I32, _P, _I32, _P, ctypes.c_size_t,

@@ -1145,6 +1145,100 @@ int hcp_decode_launch(const hcp_decode_args* a, void* stream) {
                      a->num_heads, a->num_kv_heads, a->head_dim, a->scale, a->dtype, stream, x);
 }
 
+// Workgroups per KV head and head chunk of hcp_decode_paged: one round of the
+// machine (a workgroup's chunk buffers take 128 KB of a CU's LDS).
+static int32_t paged_wgs(int32_t num_heads, int32_t num_kv_heads) {
+  const int32_t chunks = (num_heads / num_kv_heads + 15) / 16;
+  return std::max(1, kNumCus / (num_kv_heads * chunks));
+}
+
+size_t hcp_decode_paged_workspace(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
+                                  int32_t head_dim) {
+  if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads ||
+      head_dim <= 0)
+    return 0;
+  const size_t parts =
+      hcp_decode_workspace_bytes(num_seqs + paged_wgs(num_heads, num_kv_heads), num_heads, head_dim);
+  return ((parts + 15) & ~static_cast<size_t>(15)) + 2 * sizeof(int32_t) * num_seqs;
+}
+
+int hcp_decode_paged(const hcp_decode_paged_args* a, void* stream) {
+  const char* who = "hcp_decode_paged";
+  if (!a) return fail(HCP_EINVAL, "%s: null arguments", who);
+  int rc = check_heads(a->num_heads, a->num_kv_heads, a->head_dim, a->dtype, who);
+  if (rc) return rc;
+  if (a->num_seqs < 0 || a->window < 0 || a->block_table_width <= 0)
+    return fail(HCP_EINVAL, "%s: bad sizes", who);
+  if (a->num_seqs > HCP_DECODE_PAGED_MAX_SEQS)
+    return fail(HCP_EUNSUPPORTED, "%s: more than %d sequences", who, HCP_DECODE_PAGED_MAX_SEQS);
+  if (a->num_seqs == 0) return HCP_OK;
+  if (!a->q || !a->out || !a->seq_lens || !a->kv.block_table)
+    return fail(HCP_EINVAL, "%s: null pointer", who);
+  if (a->lens_dtype != HCP_DTYPE_I32 && a->lens_dtype != HCP_DTYPE_I64)
+    return fail(HCP_EUNSUPPORTED, "%s: seq_lens dtype %d (int32 or int64)", who, a->lens_dtype);
+  if (!aligned16(a->q) || (a->q_stride_tok | a->q_stride_head) % 8)
+    return fail(HCP_EINVAL, "%s: q not in 16-byte rows", who);
+  if (!(a->scale > 0.f) || !std::isfinite(a->scale))
+    return fail(HCP_EINVAL, "%s: scale must be finite and > 0", who);
+  hcp_kv_segment kv = a->kv;
+  kv.start = 0;
+  kv.len = 1;
+  if ((rc = check_segment(kv, a->head_dim, who, 0))) return rc;
+  // the kernel sums chunks of 32 keys in 32 bits
+  if (a->block_table_width > ((int64_t{1} << 34) / kv.block_size) / a->num_seqs ||
+      a->block_table_width * kv.block_size > INT32_MAX)
+    return fail(HCP_EUNSUPPORTED, "%s: block table names too many keys", who);
+  const size_t need =
+      hcp_decode_paged_workspace(a->num_seqs, a->num_heads, a->num_kv_heads, a->head_dim);
+  if (!a->workspace || a->workspace_bytes < need)
+    return fail(HCP_EWORKSPACE, "%s: workspace %zu bytes < %zu needed", who,
+                static_cast<size_t>(a->workspace_bytes), need);
+  if (!aligned16(a->workspace)) return fail(HCP_EINVAL, "%s: workspace not 16-byte aligned", who);
+  hcp::PagedDecParams p{};
+  hcp::DecParams& dp = p.d;
+  dp.q = a->q;
+  dp.q_stride_tok = a->q_stride_tok;
+  dp.q_stride_head = a->q_stride_head;
+  dp.num_wgs = paged_wgs(a->num_heads, a->num_kv_heads);
+  const size_t slots = static_cast<size_t>(a->num_seqs + dp.num_wgs) * a->num_heads;
+  const size_t o_al = (slots * hcp::padded_head_dim(a->head_dim) * sizeof(float) + 255) &
+                      ~static_cast<size_t>(255);
+  char* const ws = static_cast<char*>(a->workspace);
+  dp.ws_o = reinterpret_cast<float*>(ws);
+  dp.ws_lse = reinterpret_cast<float*>(ws + o_al);
+  dp.num_heads = a->num_heads;
+  dp.num_kv_heads = a->num_kv_heads;
+  dp.group = a->num_heads / a->num_kv_heads;
+  dp.head_chunks = (dp.group + 15) / 16;
+  dp.head_dim = a->head_dim;
+  dp.scale_log2 = a->scale * hcp::kLog2e;
+  p.kv = kv;
+  p.lens = a->seq_lens;
+  p.lens_wide = a->lens_dtype == HCP_DTYPE_I64;
+  p.num_seqs = a->num_seqs;
+  p.bt_stride = a->block_table_stride;
+  p.max_len = a->block_table_width * kv.block_size;
+  p.window = a->window;
+  p.seq_slots = reinterpret_cast<int32_t*>(ws + need - 2 * sizeof(int32_t) * a->num_seqs);
+  hcp::RedParams rp{};
+  rp.ws_o = dp.ws_o;
+  rp.ws_lse = dp.ws_lse;
+  rp.seq_slots = p.seq_slots;
+  rp.lens = p.lens;
+  rp.lens_wide = p.lens_wide;
+  rp.num_seqs = a->num_seqs;
+  rp.out = a->out;
+  rp.o_stride_tok = a->o_stride_tok;
+  rp.o_stride_head = a->o_stride_head;
+  rp.lse = a->lse;
+  rp.lse_stride_head = a->lse_stride_head;
+  rp.num_heads = a->num_heads;
+  rp.head_dim = a->head_dim;
+  return launch_status(hcp::launch_decode_paged(p, rp, a->head_dim, a->dtype,
+                                                static_cast<hipStream_t>(stream)),
+                       who);
+}
+
 int hcp_merge_attn_states(void* out, int64_t o_stride_tok, int64_t o_stride_head,
                           int32_t out_dtype, float* out_lse, int64_t out_lse_stride_head,
                           const void* prefix_out, int64_t p_stride_tok, int64_t p_stride_head,

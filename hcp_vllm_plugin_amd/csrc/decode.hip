@@ -442,10 +442,11 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
 
 // The kernel's one argument, by a pointer the compiler cannot see through:
 // its loads stay where they are used.
-__device__ __forceinline__ const DecParams& fresh_params() {
+template <typename P>
+__device__ __forceinline__ const P& fresh_params() {
   auto k = __builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(k));
-  return *(const DecParams*)k;
+  return *(const P*)k;
 }
 
 // Paged-ness is a property of each entry (a sequence's peer segment is
@@ -480,7 +481,7 @@ decode_split_kernel(DecParams p) {
   while (true) {
     // the parameters are read afresh for every split: held across the list
     // they would be spilled
-    const DecParams& p = fresh_params();
+    const DecParams& p = fresh_params<DecParams>();
     hcp_decode_work w;
     if (p.works != nullptr) {
       w = global_ptr(p.works)[s];
@@ -507,6 +508,154 @@ decode_split_kernel(DecParams p) {
   }
 }
 
+// Keys of sequence r (0 .. max_len) that its one query sees.
+__device__ __forceinline__ int64_t paged_len(const PagedDecParams& p, int r) {
+  int64_t n = p.lens_wide ? global_ptr(reinterpret_cast<const int64_t*>(p.lens))[r]
+                          : global_ptr(reinterpret_cast<const int32_t*>(p.lens))[r];
+  n = n < 0 ? 0 : n < p.max_len ? n : p.max_len;
+  return n;
+}
+
+// A pure decode batch without a plan: lengths and block tables come straight
+// from the step's metadata on the device, so the host neither waits for them
+// nor plans nor uploads.  The keys of all sequences are laid end to end in
+// chunks of 32, each sequence with kStart more for what its split costs to
+// start, and cut into equal shares, one for every workgroup; a workgroup finds
+// its share by a prefix sum over the lengths.  The piece of sequence r in
+// workgroup w is slot w + r: along the batch either w or r grows by one from
+// piece to piece, so no two pieces share a slot and a sequence's slots are
+// consecutive.  Split + merge at 28 / 4 x 128, against a planned launch of the
+// same batch: 1 x 2000 keys 12.1 / 9.6 us, 16 x 1k-8k 35.4 / 32.6 us, 32 x 0.5k-8k
+// 60.7 / 60.9 us -- the two to three microseconds of the sums, for the 100 us a
+// step that reading the lengths, planning and the upload kept the GPU waiting.
+template <int D, typename T>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * DecShared<D>::W, 64 * DecShared<D>::W),
+                          amdgpu_waves_per_eu(1, 1))) void
+decode_paged_kernel(PagedDecParams p_) {
+  constexpr int CHB = DecShared<D>::CHB;
+  constexpr int W = DecShared<D>::W;
+  constexpr int NT = 64 * W;
+  constexpr int EPT = kDecMaxSeqs / NT;  // sequences per thread of the prefix sum
+  constexpr int kStart = 8;              // a split's start and end, in chunks
+  __shared__ __attribute__((aligned(1024))) char bufE[W][2 * CHB];
+  __shared__ __attribute__((aligned(1024))) char bufO[W][2 * CHB];
+  __shared__ float sm_m[W][16];
+  __shared__ float sm_l[W][16];
+  __shared__ int sm_len[kDecMaxSeqs], sm_all[kDecMaxSeqs];  // keys seen, and in the cache
+  __shared__ int sm_w[2][W];
+  __shared__ int sm_cut[4];
+  int kvh;
+  int64_t item;
+  if (!xcd_remap(blockIdx.x, static_cast<int64_t>(p_.d.num_wgs) * p_.d.head_chunks,
+                 p_.d.num_kv_heads, &kvh, &item))
+    return;
+  const int chunk = static_cast<int>(item % p_.d.head_chunks);
+  const int wg = static_cast<int>(item / p_.d.head_chunks);
+  const int n = p_.num_seqs;
+  {
+    // ---- prefix sums over the sequences: chunks, sequences with keys ----
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int c[EPT], cs = 0, zs = 0;
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+      const int r = tid * EPT + j;
+      const int all = r < n ? static_cast<int>(paged_len(p_, r)) : 0;  // max_len < 2^31
+      const int len = p_.window > 0 && all > p_.window ? p_.window : all;
+      if (r < n) {
+        sm_all[r] = all;
+        sm_len[r] = len;
+      }
+      c[j] = (len >> 5) + ((len & 31) != 0);
+      cs += c[j];
+      zs += c[j] > 0;
+    }
+    int ci = cs, zi = zs;  // inclusive over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int a = __shfl_up(ci, o), b = __shfl_up(zi, o);
+      if (lane >= o) {
+        ci += a;
+        zi += b;
+      }
+    }
+    if (lane == 63) {
+      sm_w[0][wave] = ci;
+      sm_w[1][wave] = zi;
+    }
+    if (tid == 0) sm_cut[0] = -1;
+    __syncthreads();
+    int cb = ci - cs, zb = zi - zs;
+    unsigned total = 0, some = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      if (w < wave) {
+        cb += sm_w[0][w];
+        zb += sm_w[1][w];
+      }
+      total += sm_w[0][w];
+      some += sm_w[1][w];
+    }
+    // ---- this workgroup's share: at least two chunks (64 keys) ----
+    const unsigned most = static_cast<unsigned>(p_.d.num_wgs), half = (total + 1) / 2;
+    const unsigned wgs = most < half ? most : half;
+    if (static_cast<unsigned>(wg) < wgs) {
+      const unsigned share = total / wgs;
+      const unsigned start = share < kStart ? share : kStart;
+      const unsigned span = total + start * some, q = span / wgs, rem = span - q * wgs;
+      // cuts at span * w / wgs; the thread whose sequence holds one says which
+      // of its chunks come before it (in steps of 4, one for each wave, where
+      // the shares are long)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const unsigned w = wg + i, x = q * w + rem * w / wgs;
+        unsigned base = cb + start * zb;
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) {
+          const unsigned next = base + (c[j] > 0 ? c[j] + start : 0u);
+          if (x >= base && (x < next || (w == wgs && x == next && c[j] > 0))) {
+            unsigned in = x - base > start ? x - base - start : 0u;
+            if (share >= 16) in = (in + 2) & ~3u;
+            if (w == wgs || in > static_cast<unsigned>(c[j])) in = c[j];
+            sm_cut[2 * i] = tid * EPT + j;
+            sm_cut[2 * i + 1] = in;
+          }
+          base = next;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  const int r0 = __builtin_amdgcn_readfirstlane(sm_cut[0]);
+  if (r0 < 0) return;  // no share
+  const int o0 = __builtin_amdgcn_readfirstlane(sm_cut[1]);
+  const int r1 = __builtin_amdgcn_readfirstlane(sm_cut[2]);
+  const int o1 = __builtin_amdgcn_readfirstlane(sm_cut[3]);
+  for (int r = r0; r <= r1; ++r) {
+    const PagedDecParams& p = fresh_params<PagedDecParams>();
+    const int len = __builtin_amdgcn_readfirstlane(sm_len[r]);
+    const int all = __builtin_amdgcn_readfirstlane(sm_all[r]);
+    const int c = (len >> 5) + ((len & 31) != 0);
+    const int b = r == r0 ? o0 : 0, e_ = r == r1 ? o1 : c;
+    if (b >= e_) continue;
+    if (kvh == 0 && chunk == 0 && threadIdx.x == 0) {
+      if (b == 0) global_ptr(p.seq_slots)[2 * r] = wg + r;
+      if (e_ == c) global_ptr(p.seq_slots)[2 * r + 1] = wg + r;
+    }
+    hcp_varlen_entry e;
+    e.q_start = r;
+    e.q_len = 1;
+    e.causal_offset = 0;
+    e.kv = p.kv;
+    e.kv.block_table = p.kv.block_table + static_cast<uint64_t>(r) * p.bt_stride * 4;
+    e.kv.start = all - len;  // the last `window` keys
+    e.kv.len = len;
+    const int64_t ke = static_cast<int64_t>(e_) * 32;
+    decode_split_body<D, T, true>(p.d, kvh, chunk, wg + r, e, static_cast<int64_t>(b) * 32,
+                                  ke < len ? ke : len, bufE, bufO, sm_m, sm_l);
+    __syncthreads();  // this split has been combined out of the buffers
+  }
+}
+
 // Merge every partial of one (sequence, query head) -- and the running
 // accumulator, when given -- into the output row and its LSE.  One workgroup
 // of D threads per (sequence, head) column group, thread d owns column d;
@@ -528,7 +677,18 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
   const int row = p.rows != nullptr ? p.rows[seq] : seq;  // of out, lse and acc
   const int tid = threadIdx.x;
   const int d = tid % D, gi = tid / D;
-  const int p0 = p.seq_partial_start[seq], n = p.seq_partial_start[seq + 1] - p0;
+  int p0, n;
+  if (p.seq_slots != nullptr) {
+    // (a sequence without keys has no slots: what stands there is not used)
+    const int64_t len = p.lens_wide ? reinterpret_cast<const int64_t*>(p.lens)[seq]
+                                    : reinterpret_cast<const int32_t*>(p.lens)[seq];
+    const int first = p.seq_slots[2 * seq], last = p.seq_slots[2 * seq + 1];
+    p0 = len > 0 ? first : 0;
+    n = len > 0 ? last - first + 1 : 0;
+  } else {
+    p0 = p.seq_partial_start[seq];
+    n = p.seq_partial_start[seq + 1] - p0;
+  }
   const int64_t lstep = p.num_heads;
   const float* lcol = p.ws_lse + static_cast<int64_t>(p0) * lstep + head;
   const int64_t ostep = lstep * D;
@@ -640,6 +800,40 @@ hipError_t launch_decode(const DecParams& dp, const RedParams& rp, int head_dim,
                                    : launch_dec_t<128, _Float16>(dp, rp, st);
   return dtype == HCP_DTYPE_BF16 ? launch_dec_t<64, __bf16>(dp, rp, st)
                                  : launch_dec_t<64, _Float16>(dp, rp, st);
+}
+
+template <int D, typename T>
+static hipError_t launch_dec_paged_t(const PagedDecParams& p, const RedParams& rp,
+                                     hipStream_t st) {
+  const int64_t grid = xcd_grid_size(static_cast<int64_t>(p.d.num_wgs) * p.d.head_chunks,
+                                     p.d.num_kv_heads);
+  hipLaunchKernelGGL((decode_paged_kernel<D, T>), dim3(static_cast<unsigned>(grid)),
+                     dim3(64 * DecShared<D>::W), 0, st, p);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  RedParams r = rp;
+  const int per_seq = (p.d.num_wgs + rp.num_seqs) / rp.num_seqs;
+  r.groups = per_seq >= 48 ? 4 : per_seq >= 24 ? 2 : 1;
+  hipLaunchKernelGGL((decode_reduce_kernel<D, T>),
+                     dim3(static_cast<unsigned>(rp.num_seqs * rp.num_heads)), dim3(D * r.groups),
+                     0, st, r);
+  return hipGetLastError();
+}
+
+hipError_t launch_decode_paged(const PagedDecParams& p, const RedParams& rp, int head_dim,
+                               int dtype, hipStream_t st) {
+  const bool bf = dtype == HCP_DTYPE_BF16;
+  switch (padded_head_dim(head_dim)) {
+    case 256:
+      return bf ? launch_dec_paged_t<256, __bf16>(p, rp, st)
+                : launch_dec_paged_t<256, _Float16>(p, rp, st);
+    case 128:
+      return bf ? launch_dec_paged_t<128, __bf16>(p, rp, st)
+                : launch_dec_paged_t<128, _Float16>(p, rp, st);
+    default:
+      return bf ? launch_dec_paged_t<64, __bf16>(p, rp, st)
+                : launch_dec_paged_t<64, _Float16>(p, rp, st);
+  }
 }
 
 }  // namespace hcp

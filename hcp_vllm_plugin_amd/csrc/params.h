@@ -108,6 +108,11 @@ struct RedParams {
   const float* ws_lse;
   const int32_t* seq_partial_start;
   const int32_t* rows;  // output row of each sequence (NULL: its index)
+  // decode_paged_kernel's launches: first and last slot of each sequence (of
+  // one with keys), in place of seq_partial_start
+  const int32_t* seq_slots;
+  const void* lens;  // with seq_slots: [num_seqs] int32 or int64
+  bool lens_wide;
   int32_t num_seqs;
   void* out;
   int64_t o_stride_tok, o_stride_head;
@@ -121,6 +126,22 @@ struct RedParams {
   int64_t acc_stride_tok, acc_stride_head;
   const float* acc_lse;
   int64_t acc_lse_stride_head;
+};
+
+constexpr int kDecMaxSeqs = 1024;  // sequences of a launch that partitions itself
+
+// A pure decode batch over a paged cache, read straight from the step's
+// metadata: every workgroup works out its own share of the keys.
+struct PagedDecParams {
+  DecParams d;           // no splits; d.num_wgs workgroups per KV head and chunk
+  hcp_kv_segment kv;     // the cache; block_table, start and len are per sequence
+  const void* lens;      // [num_seqs] int32 or int64
+  bool lens_wide;
+  int32_t num_seqs;
+  int64_t bt_stride;     // elements between block-table rows
+  int64_t max_len;       // keys a block-table row can name
+  int32_t window;        // 0: none
+  int32_t* seq_slots;    // [2 * num_seqs]: first and last slot of each sequence
 };
 
 struct MergeParams {
@@ -205,6 +226,8 @@ inline hipError_t launch_fwd(const FwdParams& p, int head_dim, int dtype, bool c
 }
 hipError_t launch_decode(const DecParams& dp, const RedParams& rp, int head_dim,
                          int dtype, hipStream_t st);
+hipError_t launch_decode_paged(const PagedDecParams& p, const RedParams& rp, int head_dim,
+                               int dtype, hipStream_t st);
 hipError_t launch_merge(const MergeParams& p, hipStream_t st);
 hipError_t launch_cache_write(const CacheParams& p, bool slots_i64, hipStream_t st);
 hipError_t launch_fetch_metadata(const MetaParams& p, hipStream_t st);

@@ -68,6 +68,7 @@ from .varlen import (
     head_major,
     DecodeBatch,
     PagedCache,
+    PagedDecode,
     VarlenLaunch,
     make_entry,
     paged_entry_array,
@@ -354,9 +355,11 @@ def invalidate_step_cache() -> None:
     _STEP.update(meta=None, stamp=None, host=None, bt=None, fast={})
 
 
-def _host_metadata(attn_metadata):
+def _host_metadata(attn_metadata, queue=None):
     """(query_start_loc, seq_lens, first block ids) as lists, and the block
-    table as contiguous int32, for this step's metadata."""
+    table as contiguous int32, for this step's metadata.  ``queue``: called,
+    when the metadata is not on the host yet, between queueing its copy and
+    waiting for it."""
     stamp = _meta_stamp(attn_metadata)
     if _STEP["meta"] is attn_metadata and _STEP.get("stamp") == stamp:
         return _STEP["host"], _STEP["bt"]
@@ -368,7 +371,7 @@ def _host_metadata(attn_metadata):
     sl_t = attn_metadata.seq_lens
     n = sl_t.shape[0]
     if _fetchable(qsl_t, n + 1) and _fetchable(sl_t, n) and block_table.is_cuda:
-        host = _fetch_metadata(qsl_t, sl_t, block_table, n)
+        host = _fetch_metadata(qsl_t, sl_t, block_table, n, queue)
     else:
         fb = block_table[:, 0] if block_table.shape[1] > 0 else sl_t.new_zeros(n)
         packed = torch.cat([qsl_t.reshape(-1).to(torch.int64), sl_t.reshape(-1).to(torch.int64),
@@ -386,9 +389,10 @@ def _fetchable(t: torch.Tensor, n: int) -> bool:
     return t.is_cuda and t.dim() == 1 and t.shape[0] == n and t.dtype in _INDEX_CODES
 
 
-def _fetch_metadata(qsl_t, sl_t, block_table, n: int):
+def _fetch_metadata(qsl_t, sl_t, block_table, n: int, queue=None):
     """The step's metadata as host lists, by one kernel that writes it to
-    page-locked memory and one wait for the stream."""
+    page-locked memory and one wait for that kernel; what ``queue`` puts on
+    the stream runs while the host waits and goes on."""
     buf = getattr(_fetch_buf, "buf", None)
     if buf is None or buf.shape[0] < 3 * n + 1:
         buf = _fetch_buf.buf = torch.empty(max(1024, 4 * n), dtype=torch.int64, pin_memory=True)
@@ -401,7 +405,13 @@ def _fetch_metadata(qsl_t, sl_t, block_table, n: int):
             block_table.data_ptr() if block_table.shape[1] > 0 else 0, _lib.DTYPE_I32,
             block_table.stride(0), n, buf.data_ptr(), _lib.stream_ptr(dev))
         _lib.check(rc, "hcp_fetch_metadata")
-        torch.cuda.current_stream(dev).synchronize()
+        if queue is None:
+            torch.cuda.current_stream(dev).synchronize()
+        else:
+            done = torch.cuda.Event()
+            done.record()
+            queue()
+            done.synchronize()
     packed = _fetch_buf.np[:3 * n + 1].tolist()
     return packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:]
 
@@ -583,6 +593,23 @@ def _check_base(pc: PagedCache) -> None:
     is not keyed on."""
     if pc.k_addr % 16 or pc.v_addr % 16:
         raise ValueError("k/v base addresses must be 16-byte aligned")
+
+
+class _Ahead:
+    """A decode layer queued before the host has seen the step's metadata:
+    called by ``_host_metadata`` between queueing the metadata's copy and
+    waiting for it (not at all when the host has it already)."""
+
+    def __init__(self, impl, query, out, meta, pc):
+        self.args = (impl, query, out, meta, pc)
+        self.ran = False
+
+    def __call__(self):
+        impl, query, out, meta, pc = self.args
+        if PagedDecode.takes(meta.block_table, meta.seq_lens, pc.block_size):
+            PagedDecode(pc, meta.block_table, meta.seq_lens, impl.num_heads,
+                        impl.sliding_window).run(query, out, pc, impl.scale)
+            self.ran = True
 
 
 class _Plan:
@@ -836,15 +863,25 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         pc = PagedCache.from_tensor(kv_cache)
         if pc.num_kv_heads != self.num_kv_heads or pc.head_dim != self.head_size:
             raise ValueError("kv_cache shape does not match the layer's heads/head_size")
-        # small metadata tensors: one host sync per step (see _host_metadata)
-        (qsl, seq_lens, first_blocks), block_table = _host_metadata(attn_metadata)
-        BATCH_STATS["max_reqs"] = max(BATCH_STATS["max_reqs"], len(seq_lens))
         ring_on = _ring_enabled()
         split = _split_tokens() if ring_on else 0
+        # One token per request and nothing that gives a request peers: a
+        # decode batch whose lengths and blocks the kernels read themselves.
+        # Its first layer is queued before the host has seen the metadata; a
+        # batch that turns out otherwise runs again as what it is.
+        ahead = None
+        if num_actual == attn_metadata.seq_lens.shape[0] and split == 0 and \
+                not (ring_on and PEER_KV_STAGING) and \
+                not (_decode_ring_enabled() and DECODE_RING_MAP):
+            ahead = _Ahead(self, query, out, attn_metadata, pc)
+        # small metadata tensors: one host sync per step (see _host_metadata)
+        (qsl, seq_lens, first_blocks), block_table = _host_metadata(attn_metadata, ahead)
+        BATCH_STATS["max_reqs"] = max(BATCH_STATS["max_reqs"], len(seq_lens))
         layer_name = getattr(layer, "layer_name", "")
         n = len(seq_lens)
         if self._peer_free(ring_on, split, first_blocks, n):
-            self._forward_local_only(query, out, qsl, seq_lens, block_table, pc, kv_cache)
+            self._forward_local_only(query, out, qsl, seq_lens, block_table, pc, kv_cache,
+                                     attn_metadata.seq_lens, ahead)
             return output
         if WRITE_TRACK["enabled"]:
             self._write_probe(layer_name, qsl, seq_lens, block_table, first_blocks, pc,
@@ -1026,9 +1063,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # template was built -- even for a request the template saw without
         # peers -- makes the next layer build a new one; the stream: the plan's
         # upload is ordered on the one it was made on)
-        key = ("dec_staged", self.sliding_window, pc.layout, pc.stride_tok, pc.stride_head,
-               pc.stride_block, pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, ring_on,
-               _STAGE_GEN[0], self._heads, _lib.stream_ptr(query.device))
+        key = (*self._layout_key("dec_staged", pc), ring_on, _STAGE_GEN[0],
+               _lib.stream_ptr(query.device))
         st = _STEP["fast"].get(key)
         if st is None:
             st = self._decode_staged_template(seq_lens, block_table, first_blocks, pc, layer_name)
@@ -1059,19 +1095,40 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         _count("decode")
         return True
 
-    def _forward_local_only(self, query, out, qsl, seq_lens, block_table, pc, kv_cache):
-        """Causal attention of every request over its paged KV: a split-KV
-        decode for a pure decode batch, else one varlen launch (and a decode
-        launch for the single-token rows).  Planned and uploaded once per
-        step, cache layout and stream; a layer's launch adds its cache's
-        address."""
+    def _layout_key(self, kind: str, pc) -> tuple:
+        """What a step's plan of this kind depends on besides the metadata."""
+        return (kind, self.sliding_window, pc.layout, pc.stride_tok, pc.stride_head,
+                pc.stride_block, pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, self._heads)
+
+    def _forward_local_only(self, query, out, qsl, seq_lens, block_table, pc, kv_cache, lens_t,
+                            ahead):
+        """Causal attention of every request over its paged KV: for a pure
+        decode batch ``PagedDecode``, which needs no plan (``ahead``: already
+        queued for this layer), or, past its limits, a planned split-KV decode;
+        else one varlen launch (and a decode launch for the single-token rows).
+        Planned and uploaded once per step, cache layout and stream; a layer's
+        launch adds its cache's address."""
         n = len(seq_lens)
         if n == 0:
             return
         w = self.sliding_window
-        key = ("local", w, pc.layout, pc.stride_tok, pc.stride_head, pc.stride_block,
-               pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, self._heads,
-               _lib.stream_ptr(query.device))
+        if qsl == list(range(n + 1)) and PagedDecode.takes(block_table, lens_t, pc.block_size):
+            keys = block_table.shape[1] * pc.block_size
+            if min(seq_lens) < 0:
+                raise ValueError("negative segment start/length")
+            if max(seq_lens) > keys:
+                raise ValueError("segment extends past the block-table row")
+            if ahead is None or not ahead.ran:
+                key = self._layout_key("paged", pc)
+                dec = _STEP["fast"].get(key)
+                if dec is None:
+                    dec = _STEP["fast"][key] = PagedDecode(pc, block_table, lens_t,
+                                                           self.num_heads, w)
+                _check_base(pc)
+                dec.run(query, out, pc, self.scale)
+            _count("decode")
+            return
+        key = (*self._layout_key("local", pc), _lib.stream_ptr(query.device))
         st = _STEP["fast"].get(key)
         if st is None:
             st = _STEP["fast"][key] = self._plan_local_only(query, qsl, seq_lens, block_table, pc)

@@ -298,6 +298,7 @@ _MIN_PAGED_BLOCK = 16
 # hcp_plan_varlen_split: (query block, head) pairs past which it never cuts a
 # launch, and the most records it writes
 _MAX_SPLIT_UNITS = 1024
+_MIN_SPLIT_KEYS = 449  # nor one of shorter key ranges
 _MAX_PIECES = 4096
 
 
@@ -384,7 +385,8 @@ class VarlenLaunch:
         """The KV split of runs with these heads and window: records to upload
         ([pieces, units]), or [] for the uncut launch."""
         self._split = None
-        if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS:
+        if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS or not self.num_tiles \
+                or np.frombuffer(arr, dtype=ENTRY_DTYPE)["len"].max() < _MIN_SPLIT_KEYS:
             return []
         win = int(window or 0) if self.causal else 0
         pieces = np.empty((_MAX_PIECES, 4), dtype=np.int32)
@@ -750,6 +752,64 @@ class DecodeBatch:
                 a.workspace = ws.data_ptr()
             rc = L.hcp_decode_launch(ctypes.addressof(a), _lib.stream_ptr(q.device))
         _lib.check(rc, "hcp_decode_launch")
+
+
+class PagedDecode:
+    """A pure decode batch over one paged cache, without a plan
+    (``hcp_decode_paged``): query row r attends to the first ``seq_lens[r]``
+    keys of row r of ``block_table`` (the last ``window`` of them).  Lengths
+    and block ids are read on the device when a run executes; a length past its
+    table row counts as the row's keys, so a caller that refuses such a batch
+    checks the lengths itself.  One object serves every layer whose cache has
+    ``pc``'s layout."""
+
+    def __init__(self, pc: PagedCache, block_table: torch.Tensor, seq_lens: torch.Tensor,
+                 num_heads: int, window: int | None):
+        if block_table.dtype != torch.int32 or block_table.stride(-1) != 1:
+            raise ValueError("block table must be int32 with contiguous rows")
+        _check_kv_layout(pc.k_addr, pc.v_addr, pc.stride_tok, pc.stride_head, pc.stride_block,
+                         pc.cache.element_size())
+        if pc.block_size <= 0 or pc.block_size & (pc.block_size - 1):
+            raise ValueError("block_size must be a power of two")
+        n = seq_lens.shape[0]
+        a = self._args = _lib.DecodePagedArgs()
+        a.kv.block_table = block_table.data_ptr()
+        a.kv.stride_tok, a.kv.stride_head = pc.stride_tok, pc.stride_head
+        a.kv.stride_block, a.kv.block_size = pc.stride_block, pc.block_size
+        a.kv.num_blocks = pc.num_blocks if pc.num_blocks < (1 << 31) else 0
+        a.block_table_stride, a.block_table_width = block_table.stride(0), block_table.shape[1]
+        a.seq_lens = seq_lens.data_ptr()
+        a.lens_dtype = _lib.DTYPE_I64 if seq_lens.dtype == torch.int64 else _lib.DTYPE_I32
+        a.num_seqs, a.window = n, int(window or 0)
+        a.num_heads, a.num_kv_heads, a.head_dim = num_heads, pc.num_kv_heads, pc.head_dim
+        a.workspace_bytes = _lib.lib().hcp_decode_paged_workspace(n, num_heads, pc.num_kv_heads,
+                                                                  pc.head_dim)
+        self._keep = (block_table, seq_lens)
+
+    @staticmethod
+    def takes(block_table: torch.Tensor, seq_lens: torch.Tensor, block_size: int) -> bool:
+        """Whether a batch of this shape runs without a plan."""
+        n = seq_lens.shape[0]
+        width = block_table.shape[1]
+        return (0 < n <= _lib.DECODE_PAGED_MAX_SEQS and width > 0 and block_table.is_cuda
+                and block_table.dtype == torch.int32 and block_table.stride(1) == 1
+                and seq_lens.is_cuda and seq_lens.dim() == 1 and seq_lens.stride(0) == 1
+                and seq_lens.dtype in (torch.int32, torch.int64)
+                and width * block_size < 1 << 31 and width <= ((1 << 34) // block_size) // n)
+
+    def run(self, q: torch.Tensor, out: torch.Tensor, pc: PagedCache, scale: float) -> None:
+        """One layer: its q, out and cache."""
+        a = _lib.DecodePagedArgs.from_buffer_copy(self._args)
+        a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(0), q.stride(1)
+        a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
+        a.kv.k_addr, a.kv.v_addr = pc.k_addr, pc.v_addr
+        a.scale, a.dtype = float(scale), _lib.dtype_code(q.dtype)
+        with _lib.on_device(q.device):
+            # fp32 partials: stream-ordered scratch from torch's caching allocator
+            ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=q.device)
+            a.workspace = ws.data_ptr()
+            rc = _lib.lib().hcp_decode_paged(ctypes.addressof(a), _lib.stream_ptr(q.device))
+        _lib.check(rc, "hcp_decode_paged")
 
 
 def decode_attn(

@@ -460,6 +460,43 @@ typedef struct hcp_decode_args {
 int hcp_decode_launch(const hcp_decode_args* args, void* stream);
 
 /*
+ * Split-KV decode of a pure decode batch over one paged cache, with no plan:
+ * sequence r is query row r and attends to the first seq_lens[r] keys of its
+ * block-table row (the last `window` of them if window > 0).  The lengths and
+ * block tables are read on the device, so the call needs no host copy of
+ * them.  A length below 0 counts as 0 and one past the keys a block-table row
+ * can name (block_table_width * block_size) as that many; the caller checks
+ * them where it must refuse such a batch.  At most
+ * HCP_DECODE_PAGED_MAX_SEQS sequences.
+ *   seq_lens           DEVICE [num_seqs], HCP_DTYPE_I32 or I64 (lens_dtype)
+ *   kv                 the cache; its block_table is the DEVICE int32 table of
+ *                      num_seqs rows of block_table_width ids, block_table_stride
+ *                      elements apart; start and len are ignored
+ *   workspace          hcp_decode_paged_workspace bytes, 16-byte aligned
+ */
+#define HCP_DECODE_PAGED_MAX_SEQS 1024
+typedef struct hcp_decode_paged_args {
+  const void* q;
+  int64_t q_stride_tok, q_stride_head;
+  hcp_kv_segment kv;
+  int64_t block_table_stride, block_table_width;
+  const void* seq_lens;
+  void* workspace;
+  uint64_t workspace_bytes;
+  void* out;
+  int64_t o_stride_tok, o_stride_head;
+  float* lse; /* NULL: not wanted */
+  int64_t lse_stride_head;
+  int32_t lens_dtype, num_seqs, window;
+  int32_t num_heads, num_kv_heads, head_dim, dtype;
+  float scale;
+} hcp_decode_paged_args;
+
+size_t hcp_decode_paged_workspace(int32_t num_seqs, int32_t num_heads,
+                                  int32_t num_kv_heads, int32_t head_dim);
+int hcp_decode_paged(const hcp_decode_paged_args* args, void* stream);
+
+/*
  * Split-KV decode merged into a running accumulator: the decode ring's step
  * on one node.  Replaces RingDecodeNode.handle_packet's partial over
  * cat(chunk snapshot, growth) and _merge_pair (ring_decode.py:224-237,
