@@ -771,7 +771,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         about half a microsecond of a CU per 64 keys and head.  The decode
         launch reads the keys once, but is two more kernels (about 20 us with
         their planning).  28 / 4 x 128 heads, 512 new tokens next to 32 rows of
-        512 - 8192 keys, two layers: 543 us in one launch each, 398 us apart."""
+        512 - 8192 keys, two layers: 543 us in one launch each, 319 us apart."""
         tiles = sum(-(-int(tk) // 64) for r, tk in enumerate(seq_lens) if qsl[r + 1] - qsl[r] == 1)
         return tiles * self.num_heads * 0.5 / 256 > 20
 
@@ -1128,12 +1128,25 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 dec.run(query, out, pc, self.scale)
             _count("decode")
             return
-        key = (*self._layout_key("local", pc), _lib.stream_ptr(query.device))
-        st = _STEP["fast"].get(key)
-        if st is None:
-            st = _STEP["fast"][key] = self._plan_local_only(query, qsl, seq_lens, block_table, pc)
-        pre, dec = st
+        stream = _lib.stream_ptr(query.device)
+        # The single-token rows first: they seldom need a plan, and the
+        # prefill's is made while they run.
+        key = (*self._layout_key("rows", pc), stream)
+        if key not in _STEP["fast"]:
+            _STEP["fast"][key] = self._plan_rows(query, qsl, seq_lens, block_table, pc, lens_t)
+        dec = _STEP["fast"][key]
         _check_base(pc)
+        if dec is not None:
+            if isinstance(dec, tuple):  # a run of rows, unplanned
+                a, b, rows = dec
+                rows.run(query[a:b], out[a:b], pc, self.scale)
+            else:
+                dec.run(query, out, None, self.scale, kv_base=pc.k_addr)
+            _count("decode")
+        key = (*self._layout_key("chunks", pc), stream)
+        if key not in _STEP["fast"]:
+            _STEP["fast"][key] = self._plan_chunks(query, qsl, seq_lens, block_table, pc)
+        pre = _STEP["fast"][key]
         if pre is not None:
             if isinstance(pre, np.ndarray):
                 # blocks under 16 tokens are gathered from absolute addresses
@@ -1146,42 +1159,61 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             else:
                 pre.run(query, out, None, self.num_kv_heads, self.scale, w, kv_base=pc.k_addr)
             _count("attn")
-        if dec is not None:
-            dec.run(query, out, None, self.scale, kv_base=pc.k_addr)
-            _count("decode")
 
-    def _plan_local_only(self, query, qsl, seq_lens, block_table, pc):
-        """(prefill launch or None, decode launch or None) of a batch without
-        peers, with addresses relative to the layer's cache; over blocks under
-        16 tokens the prefill's entries instead."""
-        n = len(seq_lens)
-        w = self.sliding_window
-        qs = np.asarray(qsl[:-1], dtype=np.int64)
+    def _rows_apart(self, qsl, seq_lens):
+        """(query starts, new tokens, keys of each request, which of them are
+        single-token rows for the decode launch) of a batch without peers."""
         tq = np.diff(np.asarray(qsl, dtype=np.int64))
-        tk = np.asarray(seq_lens, dtype=np.int64)
-        rows = np.arange(n, dtype=np.int64)
         dec = tq == 1
-        all_dec = qsl == list(range(n + 1))
-        if not all_dec and not self._decode_rows_apart(qsl, seq_lens):
+        if qsl != list(range(len(qsl))) and not self._decode_rows_apart(qsl, seq_lens):
             dec[:] = False
-        pre = (tq > 0) & ~dec
-        launch = batch = None
-        if pre.any():
-            launch = paged_entry_array(pc, block_table, rows[pre], qs[pre], tq[pre],
-                                       (tk - tq)[pre], 0, tk[pre], relative=True)
-            if pc.block_size >= _MIN_PAGED_BLOCK:
-                launch = VarlenLaunch(launch, True, True, query.device, keep=block_table,
-                                      heads=self._heads, window=w)
-        if dec.any():
-            # one query at the end of its keys: all of them visible, or
-            # the last `w` of them (ring_backend.py:397-398)
-            start = np.zeros(n, np.int64) if w is None else np.maximum(tk - w, 0)
-            batch = DecodeBatch.from_entries(
-                paged_entry_array(pc, block_table, rows[dec], qs[dec], 1, 0, start[dec],
-                                  (tk - start)[dec], relative=True),
-                self.num_heads, self.num_kv_heads, self.head_size, query.device,
-                keep=block_table, rows=None if all_dec else qs[dec])
-        return launch, batch
+        return (np.asarray(qsl[:-1], dtype=np.int64), tq,
+                np.asarray(seq_lens, dtype=np.int64), dec)
+
+    def _plan_chunks(self, query, qsl, seq_lens, block_table, pc):
+        """The prefill launch (or None) of a batch without peers, with
+        addresses relative to the layer's cache; over blocks under 16 tokens
+        its entries instead."""
+        qs, tq, tk, dec = self._rows_apart(qsl, seq_lens)
+        pre = np.nonzero((tq > 0) & ~dec)[0]
+        if len(pre) == 0:
+            return None
+        ent = paged_entry_array(pc, block_table, pre, qs[pre], tq[pre], (tk - tq)[pre], 0, tk[pre],
+                                relative=True)
+        if pc.block_size < _MIN_PAGED_BLOCK:
+            return ent
+        return VarlenLaunch(ent, True, True, query.device, keep=block_table, heads=self._heads,
+                            window=self.sliding_window)
+
+    def _plan_rows(self, query, qsl, seq_lens, block_table, pc, lens_t):
+        """The launch of a batch's single-token rows: (first, end, launch) of a
+        run of query rows without a plan where they are neighbouring requests,
+        as a scheduler lists them, else a planned one; None without such rows.
+        A length past the block table is refused, in a prefill chunk too, before
+        anything of the layer is queued."""
+        qs, tq, tk, dec = self._rows_apart(qsl, seq_lens)
+        limit = block_table.shape[1] * pc.block_size
+        used = tk[tq > 0]
+        if len(used) and used.min() < 0:
+            raise ValueError("negative segment start/length")
+        if len(used) and used.max() > limit:
+            raise ValueError("segment extends past the block-table row")
+        rows = np.nonzero(dec)[0]
+        if len(rows) == 0:
+            return None
+        w = self.sliding_window
+        a, b = int(rows[0]), int(rows[-1]) + 1
+        if b - a == len(rows) and PagedDecode.takes(block_table[a:b], lens_t[a:b], pc.block_size):
+            return (int(qs[a]), int(qs[a]) + b - a,
+                    PagedDecode(pc, block_table[a:b], lens_t[a:b], self.num_heads, w))
+        # one query at the end of its keys: all of them visible, or the last `w`
+        # of them (ring_backend.py:397-398)
+        start = np.zeros(len(rows), np.int64) if w is None else np.maximum(tk[rows] - w, 0)
+        return DecodeBatch.from_entries(
+            paged_entry_array(pc, block_table, rows, qs[rows], 1, 0, start, tk[rows] - start,
+                              relative=True),
+            self.num_heads, self.num_kv_heads, self.head_size, query.device, keep=block_table,
+            rows=None if qsl == list(range(len(qsl))) else qs[rows])
 
     def _forward_prefill(self, query, out, plan: _Plan) -> None:
         dev = query.device
