@@ -11,6 +11,8 @@ table) -- and runs one launch per segment kind:
   every entry, tiles ordered longest-first by ``hcp_plan_varlen_tiles``.
 * ``decode_attn``: split-KV decode of single-token queries; every segment of a
   sequence (peer and local) is split, and one reduce merges all partials.
+* ``PagedDecode``: the same for a whole batch over one paged cache, without a
+  plan: the kernel reads lengths and block tables itself.
 
 Paged layouts the reference reads: vLLM 0.31 ``[nb, Hkv, bs, 2*D]`` with
 K in ``[..., :D]`` and V in ``[..., D:]`` (file_connector.py:13-16,175-179),
@@ -36,6 +38,7 @@ __all__ = [
     "varlen_attn_with_lse",
     "plan_varlen_tiles",
     "DecodeBatch",
+    "PagedDecode",
     "decode_attn",
     "choose_split_tokens",
     "head_major",
@@ -539,7 +542,8 @@ def head_chunks(num_heads: int, num_kv_heads: int) -> int:
 def choose_split_tokens(seg_lens: list[int], num_kv_heads: int, num_cus: int = 256,
                         max_rounds: int = 4, round_keys: int = 2048, minimum: int = 64,
                         maximum: int = 16384) -> int:
-    """Split size from the batch's total key count.
+    """A split size for callers that pass ``split_tokens`` (one workgroup per
+    split), from the batch's key counts.
 
     The split kernel runs one workgroup per CU at a time (its chunk buffers
     take 128 KB of LDS), so the launch is planned in whole rounds of
