@@ -397,6 +397,15 @@ def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def scratch(nbytes: int, device: torch.device) -> torch.Tensor | None:
+    """Stream-ordered scratch from torch's caching allocator for a launch that
+    has another form without it; None when the device has no room for it."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 _SAME_DEVICE = contextlib.nullcontext()
 
 

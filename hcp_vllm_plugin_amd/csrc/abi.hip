@@ -95,7 +95,9 @@ void set_acc(hcp::FwdParams& p, const AccArgs* a) {
 
 // ---- KV split of a prefill launch ------------------------------------------
 constexpr int kNumCus = 256;
-constexpr int kMaxPieces = 4096;    // (query block, head, piece) workgroups of a split launch
+// (query block, head, piece) workgroups of a split launch: 135 MB of partials at
+// head_dim 128
+constexpr int kMaxPieces = 2048;
 constexpr int kMaxUnits = 4 * kNumCus;  // (query block, head) pairs of a launch worth cutting
 constexpr int kMinPieceTiles = 4;   // a shorter piece is mostly prologue and epilogue
 

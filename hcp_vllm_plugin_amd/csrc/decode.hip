@@ -508,6 +508,19 @@ decode_split_kernel(DecParams p) {
   }
 }
 
+// Inclusive prefix sum over the wave's lanes, by DPP moves (inside rows of 16
+// lanes, then row 0 -> 1 and 2 -> 3, then the lower half into the upper):
+// an add each, where six shuffles through LDS take about 100 cycles each.
+__device__ __forceinline__ int wave_prefix(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return x;
+}
+
 // Keys of sequence r (0 .. max_len) that its one query sees.
 __device__ __forceinline__ int64_t paged_len(const PagedDecParams& p, int r) {
   int64_t n = p.lens_wide ? global_ptr(reinterpret_cast<const int64_t*>(p.lens))[r]
@@ -569,15 +582,7 @@ decode_paged_kernel(PagedDecParams p_) {
       cs += c[j];
       zs += c[j] > 0;
     }
-    int ci = cs, zi = zs;  // inclusive over the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int a = __shfl_up(ci, o), b = __shfl_up(zi, o);
-      if (lane >= o) {
-        ci += a;
-        zi += b;
-      }
-    }
+    const int ci = wave_prefix(cs), zi = wave_prefix(zs);
     if (lane == 63) {
       sm_w[0][wave] = ci;
       sm_w[1][wave] = zi;

@@ -94,8 +94,7 @@ def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_p
     """One pass over (q, k, v): ``hcp_attn_fwd_lse`` (acc None) or
     ``hcp_attn_fwd_lse_merge``, or -- few query rows over many keys, where
     those would leave CUs idle -- ``hcp_attn_fwd_lse_split`` on the KV split
-    the library plans, its fp32 partials in stream-ordered scratch from torch's
-    caching allocator."""
+    the library plans."""
     L = _lib.lib()
     tq, num_heads, head_dim = q.shape
     tk, num_kv_heads = k.shape[0], k.shape[1]
@@ -120,10 +119,11 @@ def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_p
             pt = L.hcp_plan_fwd_split(tq, tk, num_heads, num_kv_heads, head_dim, causal, off, win,
                                       ctypes.addressof(whole), ctypes.addressof(nbytes))
             _lib.check(pt, name)
-            if pt > 0:
-                ws = torch.empty(nbytes.value, dtype=torch.uint8, device=device)
-                rc = L.hcp_attn_fwd_lse_split(*head, *(a or (0, 0, 0, 0, 0, 0)), pt,
-                                              whole.value, ws.data_ptr(), nbytes.value, dtype,
+            # fp32 partials; without room for them the launch stays whole
+            ws = _lib.scratch(nbytes.value, device) if pt > 0 else None
+            if ws is not None:
+                rc = L.hcp_attn_fwd_lse_split(*head, *(a or (0, 0, 0, 0, 0, 0)), pt, whole.value,
+                                              ws.data_ptr(), nbytes.value, dtype,
                                               _lib.stream_ptr(device))
                 _lib.check(rc, name)
                 return

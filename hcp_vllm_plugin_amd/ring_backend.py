@@ -298,24 +298,21 @@ def _release_staged_for_request(first_block_id: int) -> None:
             drop_chunk_kv(ck)
 
 
-def _set_staged_addresses(ent: np.ndarray, idx: np.ndarray, kvs: list) -> None:
-    """Point entries ``idx`` at all of the staged chunks ``kvs`` (contiguous
-    k/v ``[n, Hkv, D]``), checked as ``segment_contiguous`` checks one."""
-    ks = [k.data_ptr() for k, _ in kvs]
-    vs = [v.data_ptr() for _, v in kvs]
-    st = [k.stride() for k, _ in kvs]
-    if st != [v.stride() for _, v in kvs]:
+def _chunk_words(kvs: list) -> np.ndarray:
+    """K address, V address, token and head stride of each staged chunk
+    (contiguous k/v ``[n, Hkv, D]``), checked as ``segment_contiguous`` checks
+    one."""
+    rows, low = [], 0
+    for k, v in kvs:
+        st, kp, vp = k.stride(), k.data_ptr(), v.data_ptr()
+        es = k.element_size()
+        low |= kp | vp | st[0] * es | st[1] * es
+        if st != v.stride() or not 0 < st[0] < 1 << 24:
+            raise ValueError("staged chunk: k/v layout not loadable")
+        rows.append((kp, vp, st[0], st[1]))
+    if low % 16:
         raise ValueError("staged chunk: k/v layout not loadable")
-    ka, va = np.array(ks, dtype=np.uint64), np.array(vs, dtype=np.uint64)
-    sa = np.array(st, dtype=np.int64)
-    es = kvs[0][0].element_size()
-    if ((ka | va) % np.uint64(16)).any() or ((sa[:, :2] * es) % 16).any() or \
-            (sa[:, 0] <= 0).any() or (sa[:, 0] >= 1 << 24).any():
-        raise ValueError("staged chunk: k/v layout not loadable")
-    ent["k_addr"][idx] = ka
-    ent["v_addr"][idx] = va
-    ent["stride_tok"][idx] = sa[:, 0]
-    ent["stride_head"][idx] = sa[:, 1]
+    return np.array(rows, dtype=np.uint64)
 
 
 # Host copy of the step's attention metadata.  vLLM hands every layer the same
@@ -410,8 +407,10 @@ def _fetch_metadata(qsl_t, sl_t, block_table, n: int, queue=None):
         else:
             done = torch.cuda.Event()
             done.record()
-            queue()
-            done.synchronize()
+            try:
+                queue()
+            finally:
+                done.synchronize()  # the buffer is not left to be written later
     packed = _fetch_buf.np[:3 * n + 1].tolist()
     return packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:]
 
@@ -1080,17 +1079,18 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 return False
             _wait_staged((ck, layer_name), kv, cur)
             kvs.append(kv)
-        ent = st["tmpl"]
-        if kvs:
-            ent = ent.copy()
-            _set_staged_addresses(ent, st["at"], kvs)
+        words = _chunk_words(kvs) if kvs else None
         batch = st["batch"]
         if batch is None:
+            ent, at = st["tmpl"].copy(), st["at"]
+            if kvs:
+                for i, f in enumerate(("k_addr", "v_addr", "stride_tok", "stride_head")):
+                    ent[f][at] = words[:, i]
             batch = st["batch"] = DecodeBatch.from_entries(
                 ent, self.num_heads, self.num_kv_heads, self.head_size, query.device,
                 keep=block_table, entry_seq=st["seq"], num_seqs=len(seq_lens))
         elif kvs:
-            batch = batch.rebind(ent, (block_table, kvs))
+            batch = batch.rebind_chunks(st["at"], words, (block_table, kvs))
         batch.run(query, out, None, self.scale, kv_base=pc.k_addr)
         _count("decode")
         return True

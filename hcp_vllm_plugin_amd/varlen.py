@@ -240,6 +240,8 @@ assert ENTRY_DTYPE.itemsize == ctypes.sizeof(VarlenEntry)
 WORK_DTYPE = np.dtype([("e", ENTRY_DTYPE)] + [(f, "<i4") for f in (
     "key_begin", "key_end", "slot", "next", "r0", "r1", "r2", "r3")])
 assert WORK_DTYPE.itemsize == 128
+_CHUNK_WORDS = np.array([ENTRY_DTYPE.fields[f][1] // 8 for f in (
+    "k_addr", "v_addr", "stride_tok", "stride_head")])
 
 
 def paged_entry_array(pc: "PagedCache", block_table: torch.Tensor, rows, q_start, q_len,
@@ -302,7 +304,7 @@ _MIN_PAGED_BLOCK = 16
 # launch, and the most records it writes
 _MAX_SPLIT_UNITS = 1024
 _MIN_SPLIT_KEYS = 449  # nor one of shorter key ranges
-_MAX_PIECES = 4096
+_MAX_PIECES = 2048
 
 
 class VarlenLaunch:
@@ -486,9 +488,11 @@ class VarlenLaunch:
         with _lib.on_device(q.device):
             a.entries = self.entries_ptr if self._gather is None else \
                 self._gathered(q, num_kv_heads)
+            # fp32 partials of a cut launch; without room for them it stays whole
+            ws = None
             if sp is not None and sp["key"] == (num_heads, num_kv_heads, head_dim, win):
-                # fp32 partials: stream-ordered scratch from torch's caching allocator
-                ws = torch.empty(sp["bytes"], dtype=torch.uint8, device=q.device)
+                ws = _lib.scratch(sp["bytes"], q.device)
+            if ws is not None:
                 a.workspace, a.workspace_bytes = ws.data_ptr(), sp["bytes"]
                 a.tiles, a.num_tiles, a.piece_tiles = sp["ptrs"][0], sp["pieces"], sp["piece_tiles"]
                 a.units, a.num_units, a.num_slots = sp["ptrs"][1], sp["units"], sp["slots"]
@@ -685,6 +689,7 @@ class DecodeBatch:
         self.ws_bytes = int(L.hcp_decode_workspace_bytes(max(rc, 1), num_heads, head_dim))
         self.device = device
         self._works, self._work_entry = works[:rc], work_entry[:rc]
+        self._chunk_rows = None
         extra = [] if rows is None else [rows]
         self._plan_dev, (w_ptr, s_ptr, *r_ptr) = _upload(
             [works[:max(rc, 1)], starts, *extra], device)
@@ -698,16 +703,36 @@ class DecodeBatch:
     def rebind(self, entries: np.ndarray, keep=None) -> "DecodeBatch":
         """The same plan (splits, partial slots) over new entries of the same
         layout and lengths -- another layer's cache and staged chunks: only
-        the entries go to the device (one small asynchronous copy)."""
+        the records go to the device (one small asynchronous copy)."""
         if entries.dtype != ENTRY_DTYPE or not entries.flags.c_contiguous:
             raise ValueError("entry array must be contiguous ENTRY_DTYPE")
         if len(entries) != self.num_entries:
             raise ValueError("rebind needs the plan's entry count")
+        works = self._works.copy()
+        works["e"] = entries[self._work_entry]
+        return self._with_works(works, keep)
+
+    def rebind_chunks(self, at: np.ndarray, rows: np.ndarray, keep=None) -> "DecodeBatch":
+        """``rebind`` of the contiguous entries ``at`` alone: row i of ``rows``
+        (uint64) is the K address, V address, token and head stride of entry
+        at[i]."""
+        if self._chunk_rows is None:  # records of contiguous entries, and which of them
+            which = np.full(self.num_entries, -1, dtype=np.int64)
+            which[at] = np.arange(len(at))
+            rec = np.nonzero(which[self._work_entry] >= 0)[0]
+            self._chunk_rows = (rec, which[self._work_entry[rec]])
+        rec, src = self._chunk_rows
+        works = self._works.copy()
+        # hcp_decode_work as 16 words: k_addr, v_addr, stride_tok, stride_head
+        words = works.view(np.uint64).reshape(-1, 16)
+        words[rec[:, None], _CHUNK_WORDS] = rows[src]
+        return self._with_works(works, keep)
+
+    def _with_works(self, works: np.ndarray, keep) -> "DecodeBatch":
         other = object.__new__(type(self))
         other.__dict__.update(self.__dict__)
-        other._works = self._works.copy()
-        other._works["e"] = entries[self._work_entry]
-        other._works_dev, (w_ptr,) = _upload([other._works], self.device)
+        other._works = works
+        other._works_dev, (w_ptr,) = _upload([works], self.device)
         other._args = _lib.DecodeArgs.from_buffer_copy(self._args)
         other._args.works = w_ptr
         other._keep = keep

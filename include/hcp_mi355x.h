@@ -281,7 +281,7 @@ int hcp_attn_fwd_lse_split(const void* q, const void* k, const void* v, void* ou
  * block of one piece, written directly), and up to cap (entry, q_block, first
  * slot, pieces) records of the split blocks to `units_out`; returns the number
  * of pieces, or 0 when the batch is best left whole (then use
- * hcp_plan_varlen_tiles).  A cap of 4096 always suffices.  Checks entries as
+ * hcp_plan_varlen_tiles).  A cap of 2048 always suffices.  Checks entries as
  * hcp_plan_varlen_tiles does.  Runs on the CPU only.
  */
 int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries,

@@ -7,8 +7,6 @@ The tolerances are the unsplit passes': the partials are f32, so a split adds
 only the f32 rounding of the merge.
 """
 
-import ctypes
-
 import pytest
 import torch
 
@@ -151,3 +149,19 @@ def test_split_under_capture_and_streams(dev):
         torch.cuda.synchronize()
         assert torch.equal(go, eo) and torch.equal(gl, el)
         ring_attn_with_lse(q, k, v, scale_for(d), 0)
+
+
+def test_no_room_for_the_partials(dev, monkeypatch):
+    """Without memory for the workspace a launch that would be cut runs whole."""
+    h, hkv, d, tq, tk = 14, 2, 64, 40, 9000
+    q, k, v = _qkv(17, tq, tk, h, hkv, d, torch.bfloat16)
+    asked = []
+    monkeypatch.setattr(_lib, "scratch", lambda n, device: asked.append(n))
+    o_ref, l_ref = orc.attn_with_lse(q, k, v, scale_for(d), tk - tq)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    for o, l in (ring_attn_with_lse(qd, kd, vd, scale_for(d), tk - tq),
+                 varlen_attn_with_lse(qd, [make_entry(0, tq, segment_contiguous(kd, vd), tk - tq)],
+                                      True, hkv, scale_for(d))):
+        torch.cuda.synchronize()
+        assert max_err(o, o_ref) <= OUT_TOL[torch.bfloat16] and max_err(l, l_ref) <= LSE_TOL
+    assert len(asked) == 2 and all(n > 0 for n in asked)
