@@ -59,6 +59,7 @@ EXPORTED_SYMBOLS = (
     "hcp_plan_varlen_split",
     "hcp_varlen_launch",
     "hcp_fetch_metadata",
+    "hcp_wait_metadata",
     "hcp_plan_decode_splits",
     "hcp_decode_workspace_bytes",
     "hcp_decode_splitkv",
@@ -296,8 +297,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.hcp_varlen_launch.argtypes = [_P, _P]
     lib.hcp_fetch_metadata.restype = ctypes.c_int
     lib.hcp_fetch_metadata.argtypes = [
-        _P, _I32, _I64, _P, _I32, _I64, _P, _I32, _I64, _I32, _P, _P,
+        _P, _I32, _I64, _P, _I32, _I64, _P, _I32, _I64, _I32, _I64, _P, _P,
     ]
+    lib.hcp_wait_metadata.restype = ctypes.c_int
+    lib.hcp_wait_metadata.argtypes = [_P, _I64, _P]
     lib.hcp_plan_decode_splits.restype = ctypes.c_int
     lib.hcp_plan_decode_splits.argtypes = [_P, _I32, _P, _I32, _I32, _I32, _P, _I32, _P]
     lib.hcp_decode_workspace_bytes.restype = ctypes.c_size_t

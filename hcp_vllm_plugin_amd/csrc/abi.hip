@@ -2,6 +2,7 @@
 // planners and kernel launches.  Declarations and their reference citations
 // are in include/hcp_mi355x.h.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1349,7 +1350,7 @@ int hcp_reshape_and_cache(const void* key, int64_t k_stride_tok, int64_t k_strid
 int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t qsl_stride,
                        const void* seq_lens, int32_t lens_dtype, int64_t lens_stride,
                        const void* block_table, int32_t bt_dtype, int64_t bt_stride, int32_t n,
-                       int64_t* host_out, void* stream) {
+                       int64_t token, int64_t* host_out, void* stream) {
   const char* who = "hcp_fetch_metadata";
   for (int32_t d : {qsl_dtype, lens_dtype, bt_dtype})
     if (d != HCP_DTYPE_I32 && d != HCP_DTYPE_I64)
@@ -1368,8 +1369,25 @@ int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t q
   p.lens_wide = lens_dtype == HCP_DTYPE_I64;
   p.bt_wide = bt_dtype == HCP_DTYPE_I64;
   p.n = n;
+  p.token = token;
   p.out = host_out;
   return launch_status(hcp::launch_fetch_metadata(p, static_cast<hipStream_t>(stream)), who);
+}
+
+int hcp_wait_metadata(const int64_t* host_out, int64_t token, void* stream) {
+  const char* who = "hcp_wait_metadata";
+  if (!host_out) return fail(HCP_EINVAL, "%s: null pointer", who);
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(50);
+  for (int i = 0;; ++i) {
+    if (__atomic_load_n(host_out, __ATOMIC_ACQUIRE) == token) return HCP_OK;
+    if ((i & 1023) == 1023 && std::chrono::steady_clock::now() > until) break;
+  }
+  // a long queue ahead of the copy, or an error: wait for the stream itself
+  const hipError_t e = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return launch_status(e, who);
+  if (__atomic_load_n(host_out, __ATOMIC_ACQUIRE) != token)
+    return fail(HCP_ELAUNCH, "%s: the copy did not arrive", who);
+  return HCP_OK;
 }
 
 int hcp_gather_paged_kv(const hcp_varlen_entry* entries, int32_t num_entries,

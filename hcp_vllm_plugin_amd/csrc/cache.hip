@@ -103,23 +103,30 @@ hipError_t launch_gather(const GatherParams& p, hipStream_t st) {
 
 // One step's metadata -- query starts, lengths, first block ids -- widened
 // into page-locked host memory: one kernel in place of three conversions, a
-// concatenation and a copy, each a launch the host waits through.
+// concatenation and a copy, each a launch the host waits through.  One
+// workgroup: when all its values are out at system scope, thread 0 writes the
+// caller's token before them, which the host waits for without the stream.
 __global__ __launch_bounds__(256) void fetch_metadata_kernel(MetaParams p) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
   auto get = [](const void* a, bool wide, int64_t at) {
     return wide ? reinterpret_cast<const int64_t*>(a)[at]
                 : static_cast<int64_t>(reinterpret_cast<const int32_t*>(a)[at]);
   };
-  if (i <= p.n) p.out[i] = get(p.qsl, p.qsl_wide, i * p.qsl_stride);
-  if (i < p.n) {
-    p.out[p.n + 1 + i] = get(p.lens, p.lens_wide, i * p.lens_stride);
-    p.out[2 * p.n + 1 + i] = p.bt != nullptr ? get(p.bt, p.bt_wide, i * p.bt_stride) : 0;
+  int64_t* const out = p.out + 1;
+  for (int i = threadIdx.x; i <= p.n; i += 256) {
+    out[i] = get(p.qsl, p.qsl_wide, i * p.qsl_stride);
+    if (i < p.n) {
+      out[p.n + 1 + i] = get(p.lens, p.lens_wide, i * p.lens_stride);
+      out[2 * p.n + 1 + i] = p.bt != nullptr ? get(p.bt, p.bt_wide, i * p.bt_stride) : 0;
+    }
   }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(p.out, p.token, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 hipError_t launch_fetch_metadata(const MetaParams& p, hipStream_t st) {
-  hipLaunchKernelGGL(fetch_metadata_kernel, dim3(static_cast<unsigned>(p.n / 256 + 1)), dim3(256),
-                     0, st, p);
+  hipLaunchKernelGGL(fetch_metadata_kernel, dim3(1), dim3(256), 0, st, p);
   return hipGetLastError();
 }
 

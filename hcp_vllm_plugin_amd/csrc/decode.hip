@@ -538,8 +538,8 @@ __device__ __forceinline__ int64_t paged_len(const PagedDecParams& p, int r) {
 // workgroup w is slot w + r: along the batch either w or r grows by one from
 // piece to piece, so no two pieces share a slot and a sequence's slots are
 // consecutive.  Split + merge at 28 / 4 x 128, against a planned launch of the
-// same batch: 1 x 2000 keys 12.1 / 9.6 us, 16 x 1k-8k 35.4 / 32.6 us, 32 x 0.5k-8k
-// 60.7 / 60.9 us -- the two to three microseconds of the sums, for the 100 us a
+// same batch: 1 x 2000 keys 11.5 / 9.6 us, 16 x 1k-8k 34.6 / 32.6 us, 32 x 0.5k-8k
+// 60.2 / 60.6 us -- the two microseconds of the sums, for the 100 us a
 // step that reading the lengths, planning and the upload kept the GPU waiting.
 template <int D, typename T>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * DecShared<D>::W, 64 * DecShared<D>::W),

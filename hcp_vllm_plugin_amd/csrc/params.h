@@ -202,7 +202,8 @@ struct MetaParams {
   int64_t qsl_stride, lens_stride, bt_stride;
   bool qsl_wide, lens_wide, bt_wide;  // int64, else int32
   int32_t n;
-  int64_t* out;  // [3 n + 1]
+  int64_t token;
+  int64_t* out;  // [3 n + 2]: the token, then the values
 };
 
 // Prefill in D columns (padded_head_dim): the attention kernel and, when p

@@ -388,30 +388,29 @@ def _fetchable(t: torch.Tensor, n: int) -> bool:
 
 def _fetch_metadata(qsl_t, sl_t, block_table, n: int, queue=None):
     """The step's metadata as host lists, by one kernel that writes it to
-    page-locked memory and one wait for that kernel; what ``queue`` puts on
+    page-locked memory and one wait for that memory; what ``queue`` puts on
     the stream runs while the host waits and goes on."""
     buf = getattr(_fetch_buf, "buf", None)
-    if buf is None or buf.shape[0] < 3 * n + 1:
-        buf = _fetch_buf.buf = torch.empty(max(1024, 4 * n), dtype=torch.int64, pin_memory=True)
+    if buf is None or buf.shape[0] < 3 * n + 2:
+        buf = _fetch_buf.buf = torch.zeros(max(1024, 4 * n), dtype=torch.int64, pin_memory=True)
         _fetch_buf.np = buf.numpy()
-    dev = qsl_t.device
+        _fetch_buf.token = 0
+    token = _fetch_buf.token = _fetch_buf.token + 1
+    dev, L = qsl_t.device, _lib.lib()
     with _lib.on_device(dev):
-        rc = _lib.lib().hcp_fetch_metadata(
+        stream = _lib.stream_ptr(dev)
+        rc = L.hcp_fetch_metadata(
             qsl_t.data_ptr(), _INDEX_CODES[qsl_t.dtype], qsl_t.stride(0),
             sl_t.data_ptr(), _INDEX_CODES[sl_t.dtype], sl_t.stride(0),
             block_table.data_ptr() if block_table.shape[1] > 0 else 0, _lib.DTYPE_I32,
-            block_table.stride(0), n, buf.data_ptr(), _lib.stream_ptr(dev))
+            block_table.stride(0), n, token, buf.data_ptr(), stream)
         _lib.check(rc, "hcp_fetch_metadata")
-        if queue is None:
-            torch.cuda.current_stream(dev).synchronize()
-        else:
-            done = torch.cuda.Event()
-            done.record()
-            try:
+        try:
+            if queue is not None:
                 queue()
-            finally:
-                done.synchronize()  # the buffer is not left to be written later
-    packed = _fetch_buf.np[:3 * n + 1].tolist()
+        finally:  # the buffer is not left to be written later
+            _lib.check(L.hcp_wait_metadata(buf.data_ptr(), token, stream), "hcp_wait_metadata")
+    packed = _fetch_buf.np[1:3 * n + 2].tolist()
     return packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:]
 
 

@@ -11,7 +11,7 @@
  *   - Strides are in ELEMENTS of the tensor's own dtype.  The last dimension
  *     (head_dim) must be contiguous.
  *   - Every launch is asynchronous on `stream` (a hipStream_t, NULL = default
- *     stream).  No entry point synchronizes the device.
+ *     stream).  No entry point but hcp_wait_metadata waits for the device.
  *   - Return value: HCP_OK (0) or a negative hcp_status.  Nothing throws or
  *     aborts across this boundary; hcp_last_error() gives a thread-local text
  *     of the last failure on the calling thread.
@@ -330,14 +330,18 @@ int hcp_varlen_launch(const hcp_varlen_args* args, void* stream);
  * Copies one step's small metadata to host memory: the n + 1 query starts,
  * the n sequence lengths and the n first block ids (element 0 of each
  * block-table row; block_table may be NULL: zeros), all widened to int64, into
- * `host_out` [3 n + 1], which must be page-locked memory the GPU can write.
- * Index dtypes are HCP_DTYPE_I32 / I64, strides in elements.  One kernel on
- * `stream`; the caller waits for the stream before reading host_out.
+ * `host_out` [1 + 3 n + 1], which must be page-locked memory the GPU can
+ * write: first `token`, written last, then the values.  Index dtypes are
+ * HCP_DTYPE_I32 / I64, strides in elements.  One kernel on `stream`.
+ * hcp_wait_metadata returns when host_out[0] is `token` (which must not have
+ * stood there before): it watches the memory, and after 50 ms waits for
+ * `stream`.  It is the one entry point that waits.
  */
 int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t qsl_stride,
                        const void* seq_lens, int32_t lens_dtype, int64_t lens_stride,
                        const void* block_table, int32_t bt_dtype, int64_t bt_stride,
-                       int32_t n, int64_t* host_out, void* stream);
+                       int32_t n, int64_t token, int64_t* host_out, void* stream);
+int hcp_wait_metadata(const int64_t* host_out, int64_t token, void* stream);
 
 /*
  * Host-side split planner for hcp_decode_splitkv.  Each entry is one query
