@@ -207,6 +207,7 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
     std::pop_heap(heap.begin(), heap.end(), std::greater<Ev>());
     Cu& x = cu[heap.back().second];
     end = heap.back().first;
+    if (end + merge_us >= limit) break;  // jobs end in order of time: it loses
     if (x.n == 1) {
       x.n = 0;
     } else {

@@ -14,6 +14,7 @@ KV frame.  The work runs in ``hcp_attn_fwd_lse`` (libhcp_mi355x.so).
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -90,6 +91,18 @@ _MAX_SPLIT_UNITS = 1024
 _MIN_SPLIT_KEYS = 449
 
 
+@functools.lru_cache(maxsize=1024)
+def _split_plan(tq, tk, num_heads, num_kv_heads, head_dim, causal, off, win):
+    """(piece_tiles, whole_blocks, workspace bytes) of a launch's KV split. It
+    follows from the sizes alone and takes 7 to 37 us of the host to find, so
+    the layers of a step share it (1.5 us). <= 0: the launch stays whole (and
+    reports what is wrong with the sizes, where that is the reason)."""
+    whole, nbytes = ctypes.c_int32(0), ctypes.c_size_t(0)
+    pt = _lib.lib().hcp_plan_fwd_split(tq, tk, num_heads, num_kv_heads, head_dim, causal, off, win,
+                                       ctypes.addressof(whole), ctypes.addressof(nbytes))
+    return pt, whole.value, nbytes.value
+
+
 def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_prefix):
     """One pass over (q, k, v): ``hcp_attn_fwd_lse`` (acc None) or
     ``hcp_attn_fwd_lse_merge``, or -- few query rows over many keys, where
@@ -115,15 +128,13 @@ def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_p
         a = () if acc is None else (acc[0].data_ptr(), acc[0].stride(0), acc[0].stride(1),
                                     acc[1].data_ptr(), acc[1].stride(0), int(bool(acc_is_prefix)))
         if tk >= _MIN_SPLIT_KEYS and -(-tq // 128) * num_heads <= _MAX_SPLIT_UNITS:
-            whole, nbytes = ctypes.c_int32(0), ctypes.c_size_t(0)
-            pt = L.hcp_plan_fwd_split(tq, tk, num_heads, num_kv_heads, head_dim, causal, off, win,
-                                      ctypes.addressof(whole), ctypes.addressof(nbytes))
-            _lib.check(pt, name)
+            pt, whole, nbytes = _split_plan(tq, tk, num_heads, num_kv_heads, head_dim, causal,
+                                            off, win)
             # fp32 partials; without room for them the launch stays whole
-            ws = _lib.scratch(nbytes.value, device) if pt > 0 else None
+            ws = _lib.scratch(nbytes, device) if pt > 0 else None
             if ws is not None:
-                rc = L.hcp_attn_fwd_lse_split(*head, *(a or (0, 0, 0, 0, 0, 0)), pt, whole.value,
-                                              ws.data_ptr(), nbytes.value, dtype,
+                rc = L.hcp_attn_fwd_lse_split(*head, *(a or (0, 0, 0, 0, 0, 0)), pt, whole,
+                                              ws.data_ptr(), nbytes, dtype,
                                               _lib.stream_ptr(device))
                 _lib.check(rc, name)
                 return
