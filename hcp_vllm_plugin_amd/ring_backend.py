@@ -367,7 +367,8 @@ def _host_metadata(attn_metadata, queue=None):
     qsl_t = attn_metadata.query_start_loc
     sl_t = attn_metadata.seq_lens
     n = sl_t.shape[0]
-    if _fetchable(qsl_t, n + 1) and _fetchable(sl_t, n) and block_table.is_cuda:
+    if _fetchable(qsl_t, n + 1) and _fetchable(sl_t, n) and block_table.is_cuda \
+            and block_table.shape[0] >= n:  # (the copy reads a first block per request)
         host = _fetch_metadata(qsl_t, sl_t, block_table, n, queue)
     else:
         fb = block_table[:, 0] if block_table.shape[1] > 0 else sl_t.new_zeros(n)
@@ -877,6 +878,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         BATCH_STATS["max_reqs"] = max(BATCH_STATS["max_reqs"], len(seq_lens))
         layer_name = getattr(layer, "layer_name", "")
         n = len(seq_lens)
+        if len(first_blocks) < n and qsl[n] > qsl[len(first_blocks)]:
+            raise ValueError("the block table has no row for a request")
         if self._peer_free(ring_on, split, first_blocks, n):
             self._forward_local_only(query, out, qsl, seq_lens, block_table, pc, kv_cache,
                                      attn_metadata.seq_lens, ahead)

@@ -266,6 +266,8 @@ def paged_entry_array(pc: "PagedCache", block_table: torch.Tensor, rows, q_start
     nblk = (start + length + pc.block_size - 1) // pc.block_size
     if ((length > 0) & (nblk > block_table.shape[1])).any():
         raise ValueError("segment extends past the block-table row")
+    if ((length > 0) & ((rows < 0) | (rows >= block_table.shape[0]))).any():
+        raise ValueError("the block table has no row for a request")
     a = np.zeros(len(rows), dtype=ENTRY_DTYPE)
     a["q_start"] = q_start
     a["q_len"] = q_len
@@ -801,6 +803,8 @@ class PagedDecode:
         if pc.block_size <= 0 or pc.block_size & (pc.block_size - 1):
             raise ValueError("block_size must be a power of two")
         n = seq_lens.shape[0]
+        if block_table.dim() != 2 or block_table.shape[0] < n:
+            raise ValueError("the block table has no row for a request")
         a = self._args = _lib.DecodePagedArgs()
         a.kv.block_table = block_table.data_ptr()
         a.kv.stride_tok, a.kv.stride_head = pc.stride_tok, pc.stride_head
@@ -819,6 +823,8 @@ class PagedDecode:
     def takes(block_table: torch.Tensor, seq_lens: torch.Tensor, block_size: int) -> bool:
         """Whether a batch of this shape runs without a plan."""
         n = seq_lens.shape[0]
+        if block_table.dim() != 2 or block_table.shape[0] < n:
+            return False
         width = block_table.shape[1]
         return (0 < n <= _lib.DECODE_PAGED_MAX_SEQS and width > 0 and block_table.is_cuda
                 and block_table.dtype == torch.int32 and block_table.stride(1) == 1

@@ -1,0 +1,60 @@
+"""The backend's host side of a step, on the CPU: metadata that does not fit
+together is refused before anything is queued."""
+
+import types
+
+import numpy as np
+import pytest
+import torch
+
+from hcp_vllm_plugin_amd import ring_backend as rb
+from hcp_vllm_plugin_amd.varlen import PagedCache, PagedDecode, paged_entry_array
+
+
+@pytest.fixture(autouse=True)
+def _clean():
+    rb.invalidate_step_cache()
+    yield
+    rb.invalidate_step_cache()
+
+
+def _meta(qsl, lens, bt):
+    return types.SimpleNamespace(
+        num_actual_tokens=qsl[-1], query_start_loc=torch.tensor(qsl, dtype=torch.int32),
+        seq_lens=torch.tensor(lens, dtype=torch.int32),
+        block_table=torch.tensor(bt, dtype=torch.int32))
+
+
+def _forward(meta):
+    impl = rb.HcpRingAttentionImpl(4, 64, 0.125, 2)
+    layer = types.SimpleNamespace(layer_name="model.layers.0.self_attn.attn")
+    q = torch.zeros(meta.num_actual_tokens, 4, 64, dtype=torch.bfloat16)
+    cache = torch.zeros(8, 2, 16, 128, dtype=torch.bfloat16)
+    return impl.forward(layer, q, None, None, cache, meta, torch.zeros_like(q))
+
+
+@pytest.mark.parametrize("qsl", [[0, 1, 2, 3], [0, 4, 5, 9]])
+def test_block_table_without_a_row_for_a_request(qsl):
+    with pytest.raises(ValueError, match="no row for a request"):
+        _forward(_meta(qsl, [20, 20, 20], [[0, 1], [2, 3]]))
+
+
+def test_block_table_rows_of_entries_and_unplanned_batches():
+    pc = PagedCache.from_tensor(torch.zeros(8, 2, 16, 128, dtype=torch.bfloat16))
+    bt = torch.zeros(2, 4, dtype=torch.int32)
+    for rows, lens in (([0, 2], [5, 5]), ([-1, 0], [5, 5])):
+        with pytest.raises(ValueError, match="no row for a request"):
+            paged_entry_array(pc, bt, rows, rows, 1, 0, 0, np.asarray(lens))
+    # a row that nothing is read through may lie past the table
+    assert len(paged_entry_array(pc, bt, [0, 2], [0, 1], 1, 0, 0, np.asarray([5, 0]))) == 2
+    with pytest.raises(ValueError, match="no row for a request"):
+        PagedDecode(pc, bt, torch.ones(3, dtype=torch.int32), 4, None)
+
+    def on_gpu(t):  # what `takes` looks at
+        return types.SimpleNamespace(shape=t.shape, dtype=t.dtype, stride=t.stride, dim=t.dim,
+                                     is_cuda=True)
+
+    lens = on_gpu(torch.ones(2, dtype=torch.int32))
+    assert PagedDecode.takes(on_gpu(bt), lens, 16)
+    assert not PagedDecode.takes(on_gpu(bt[:1]), lens, 16)
+    assert not PagedDecode.takes(on_gpu(bt[0]), lens, 16)
