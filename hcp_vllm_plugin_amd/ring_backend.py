@@ -315,11 +315,23 @@ def _chunk_words(kvs: list) -> np.ndarray:
     return np.array(rows, dtype=np.uint64)
 
 
-# Host copy of the step's attention metadata.  vLLM hands every layer the same
-# metadata object, so one device->host copy serves all layers of a step (the
-# reference syncs three times per layer, ring_backend.py:604-605).  Holding the
-# object keeps its identity from being reused by a later step's metadata.
-_STEP: dict = {"meta": None, "stamp": None, "host": None, "bt": None, "fast": {}}
+class _Step:
+    """What a step's layers share: the host copy of its metadata, its block
+    table as contiguous int32, and the plans made from them (``fast``).  A
+    layer keeps the record it got, so another thread's step can neither take
+    the plans away under it nor be given them."""
+
+    __slots__ = ("meta", "stamp", "host", "bt", "fast")
+
+    def __init__(self, meta, stamp, host, bt):
+        self.meta, self.stamp, self.host, self.bt, self.fast = meta, stamp, host, bt, {}
+
+
+# The newest step.  vLLM hands every layer the same metadata object, so one
+# device->host copy serves all layers of a step (the reference syncs three
+# times per layer, ring_backend.py:604-605).  Holding the object keeps its
+# identity from being reused by a later step's metadata.
+_STEP: dict = {"step": None, "fast": {}}
 
 
 def _version_of(t: torch.Tensor) -> int:
@@ -349,17 +361,23 @@ def invalidate_step_cache() -> None:
     """Drop the cached host copy of the step's metadata and the plans built
     from it: for a caller that rewrites the metadata tensors behind torch's
     back (a kernel writing into them directly) before reusing the object."""
-    _STEP.update(meta=None, stamp=None, host=None, bt=None, fast={})
+    _STEP.update(step=None, fast={})
 
 
-def _host_metadata(attn_metadata, queue=None):
+def _host_metadata(attn_metadata):
     """(query_start_loc, seq_lens, first block ids) as lists, and the block
-    table as contiguous int32, for this step's metadata.  ``queue``: called,
-    when the metadata is not on the host yet, between queueing its copy and
-    waiting for it."""
+    table as contiguous int32, for this step's metadata."""
+    st = _step(attn_metadata)
+    return st.host, st.bt
+
+
+def _step(attn_metadata, queue=None) -> _Step:
+    """This step's record.  ``queue``: called, when the metadata is not on the
+    host yet, between queueing its copy and waiting for it."""
     stamp = _meta_stamp(attn_metadata)
-    if _STEP["meta"] is attn_metadata and _STEP.get("stamp") == stamp:
-        return _STEP["host"], _STEP["bt"]
+    st = _STEP["step"]
+    if st is not None and st.meta is attn_metadata and st.stamp == stamp:
+        return st
     block_table = attn_metadata.block_table
     if block_table.dtype != torch.int32:
         block_table = block_table.to(torch.int32)
@@ -375,8 +393,9 @@ def _host_metadata(attn_metadata, queue=None):
         packed = torch.cat([qsl_t.reshape(-1).to(torch.int64), sl_t.reshape(-1).to(torch.int64),
                             fb.reshape(-1).to(torch.int64)]).tolist()
         host = (packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:])
-    _STEP.update(meta=attn_metadata, stamp=stamp, host=host, bt=block_table, fast={})
-    return host, block_table
+    st = _Step(attn_metadata, stamp, host, block_table)
+    _STEP.update(step=st, fast=st.fast)
+    return st
 
 
 _INDEX_CODES = {torch.int32: _lib.DTYPE_I32, torch.int64: _lib.DTYPE_I64}
@@ -596,7 +615,7 @@ def _check_base(pc: PagedCache) -> None:
 
 class _Ahead:
     """A decode layer queued before the host has seen the step's metadata:
-    called by ``_host_metadata`` between queueing the metadata's copy and
+    called by ``_step`` between queueing the metadata's copy and
     waiting for it (not at all when the host has it already)."""
 
     def __init__(self, impl, query, out, meta, pc):
@@ -873,25 +892,25 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 not (ring_on and PEER_KV_STAGING) and \
                 not (_decode_ring_enabled() and DECODE_RING_MAP):
             ahead = _Ahead(self, query, out, attn_metadata, pc)
-        # small metadata tensors: one host sync per step (see _host_metadata)
-        (qsl, seq_lens, first_blocks), block_table = _host_metadata(attn_metadata, ahead)
+        # small metadata tensors: one host sync per step (see _step)
+        step = _step(attn_metadata, ahead)
+        (qsl, seq_lens, first_blocks), block_table = step.host, step.bt
         BATCH_STATS["max_reqs"] = max(BATCH_STATS["max_reqs"], len(seq_lens))
         layer_name = getattr(layer, "layer_name", "")
         n = len(seq_lens)
         if len(first_blocks) < n and qsl[n] > qsl[len(first_blocks)]:
             raise ValueError("the block table has no row for a request")
         if self._peer_free(ring_on, split, first_blocks, n):
-            self._forward_local_only(query, out, qsl, seq_lens, block_table, pc, kv_cache,
-                                     attn_metadata.seq_lens, ahead)
+            self._forward_local_only(query, out, step, pc, kv_cache, attn_metadata.seq_lens,
+                                     ahead)
             return output
         if WRITE_TRACK["enabled"]:
             self._write_probe(layer_name, qsl, seq_lens, block_table, first_blocks, pc,
                               ring_on, split)
 
         is_decode = n > 0 and qsl == list(range(n + 1))
-        if is_decode and self._forward_decode_staged(query, out, seq_lens, block_table,
-                                                     first_blocks, pc, kv_cache, layer_name,
-                                                     ring_on, split):
+        if is_decode and self._forward_decode_staged(query, out, step, pc, layer_name, ring_on,
+                                                     split):
             return output
         plan = self._plan(layer_name, qsl, seq_lens, block_table, first_blocks, pc, split)
         ring_local = self._ring_local_segments(plan, pc, key, value, layer_name)
@@ -1048,8 +1067,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         return {"tmpl": tmpl, "seq": seq, "at": np.nonzero(kinds == 1)[0], "peers": peers,
                 "batch": None}
 
-    def _forward_decode_staged(self, query, out, seq_lens, block_table, first_blocks, pc,
-                               kv_cache, layer_name, ring_on, split) -> bool:
+    def _forward_decode_staged(self, query, out, step, pc, layer_name, ring_on, split) -> bool:
         """A pure decode batch without decode-ring rows: one split-KV launch
         over every request's local paged segment and staged peer chunks, its
         split plan built once per step and reused by every layer, each layer
@@ -1057,6 +1075,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         uploading them in one small copy (the cache's address is a launch
         argument).  False when the general path must run (split env,
         decode-ring rows, staging that differs from the step's template)."""
+        (_qsl, seq_lens, first_blocks), block_table = step.host, step.bt
         if split > 0 or (_decode_ring_enabled() and DECODE_RING_MAP
                          and any(fb in DECODE_RING_MAP for fb in first_blocks)):
             return False
@@ -1066,10 +1085,10 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # upload is ordered on the one it was made on)
         key = (*self._layout_key("dec_staged", pc), ring_on, _STAGE_GEN[0],
                _lib.stream_ptr(query.device))
-        st = _STEP["fast"].get(key)
+        st = step.fast.get(key)
         if st is None:
             st = self._decode_staged_template(seq_lens, block_table, first_blocks, pc, layer_name)
-            _STEP["fast"][key] = st
+            step.fast[key] = st
         if st is False:
             return False
         _check_base(pc)
@@ -1102,14 +1121,14 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         return (kind, self.sliding_window, pc.layout, pc.stride_tok, pc.stride_head,
                 pc.stride_block, pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, self._heads)
 
-    def _forward_local_only(self, query, out, qsl, seq_lens, block_table, pc, kv_cache, lens_t,
-                            ahead):
+    def _forward_local_only(self, query, out, step, pc, kv_cache, lens_t, ahead):
         """Causal attention of every request over its paged KV: for a pure
         decode batch ``PagedDecode``, which needs no plan (``ahead``: already
         queued for this layer), or, past its limits, a planned split-KV decode;
         else one varlen launch (and a decode launch for the single-token rows).
         Planned and uploaded once per step, cache layout and stream; a layer's
         launch adds its cache's address."""
+        (qsl, seq_lens, _first), block_table, fast = step.host, step.bt, step.fast
         n = len(seq_lens)
         if n == 0:
             return
@@ -1122,10 +1141,9 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 raise ValueError("segment extends past the block-table row")
             if ahead is None or not ahead.ran:
                 key = self._layout_key("paged", pc)
-                dec = _STEP["fast"].get(key)
+                dec = fast.get(key)
                 if dec is None:
-                    dec = _STEP["fast"][key] = PagedDecode(pc, block_table, lens_t,
-                                                           self.num_heads, w)
+                    dec = fast[key] = PagedDecode(pc, block_table, lens_t, self.num_heads, w)
                 _check_base(pc)
                 dec.run(query, out, pc, self.scale)
             _count("decode")
@@ -1134,9 +1152,9 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # The single-token rows first: they seldom need a plan, and the
         # prefill's is made while they run.
         key = (*self._layout_key("rows", pc), stream)
-        if key not in _STEP["fast"]:
-            _STEP["fast"][key] = self._plan_rows(query, qsl, seq_lens, block_table, pc, lens_t)
-        dec = _STEP["fast"][key]
+        dec = fast.get(key, fast)  # (fast itself: not planned yet)
+        if dec is fast:
+            dec = fast[key] = self._plan_rows(query, qsl, seq_lens, block_table, pc, lens_t)
         _check_base(pc)
         if dec is not None:
             if isinstance(dec, tuple):  # a run of rows, unplanned
@@ -1146,9 +1164,9 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 dec.run(query, out, None, self.scale, kv_base=pc.k_addr)
             _count("decode")
         key = (*self._layout_key("chunks", pc), stream)
-        if key not in _STEP["fast"]:
-            _STEP["fast"][key] = self._plan_chunks(query, qsl, seq_lens, block_table, pc)
-        pre = _STEP["fast"][key]
+        pre = fast.get(key, fast)
+        if pre is fast:
+            pre = fast[key] = self._plan_chunks(query, qsl, seq_lens, block_table, pc)
         if pre is not None:
             if isinstance(pre, np.ndarray):
                 # blocks under 16 tokens are gathered from absolute addresses

@@ -58,3 +58,23 @@ def test_block_table_rows_of_entries_and_unplanned_batches():
     assert PagedDecode.takes(on_gpu(bt), lens, 16)
     assert not PagedDecode.takes(on_gpu(bt[:1]), lens, 16)
     assert not PagedDecode.takes(on_gpu(bt[0]), lens, 16)
+
+
+def test_another_threads_step_leaves_a_layers_plans_alone(monkeypatch):
+    """While a layer plans, another thread's step replaces the newest one: the
+    layer goes on with its own plans, which the other step does not get."""
+    mine, other = _meta([0, 3, 8], [20, 30], [[0, 1], [2, 3]]), _meta([0, 2], [9], [[4, 5]])
+    calls = []
+
+    def planner(name):
+        def plan(self, *a):
+            calls.append(name)
+            rb._host_metadata(other)
+        return plan
+
+    monkeypatch.setattr(rb._lib, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(rb.HcpRingAttentionImpl, "_plan_rows", planner("rows"))
+    monkeypatch.setattr(rb.HcpRingAttentionImpl, "_plan_chunks", planner("chunks"))
+    _forward(mine)
+    assert calls == ["rows", "chunks"]
+    assert rb._host_metadata(other)[0][1] == [9] and not rb._STEP["fast"]
