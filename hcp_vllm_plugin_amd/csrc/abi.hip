@@ -1228,8 +1228,7 @@ int hcp_decode_paged(const hcp_decode_paged_args* a, void* stream) {
   rp.ws_o = dp.ws_o;
   rp.ws_lse = dp.ws_lse;
   rp.seq_slots = p.seq_slots;
-  rp.lens = p.lens;
-  rp.lens_wide = p.lens_wide;
+  rp.num_slots = a->num_seqs + dp.num_wgs;
   rp.num_seqs = a->num_seqs;
   rp.out = a->out;
   rp.o_stride_tok = a->o_stride_tok;

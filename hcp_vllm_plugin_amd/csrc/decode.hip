@@ -579,6 +579,11 @@ decode_paged_kernel(PagedDecParams p_) {
         sm_len[r] = len;
       }
       c[j] = (len >> 5) + ((len & 31) != 0);
+      // the reduce goes by the slots alone: a sequence without keys says so
+      if (r < n && c[j] == 0 && wg == 0 && kvh == 0 && chunk == 0) {
+        global_ptr(p_.seq_slots)[2 * r] = 0;
+        global_ptr(p_.seq_slots)[2 * r + 1] = -1;
+      }
       cs += c[j];
       zs += c[j] > 0;
     }
@@ -684,12 +689,11 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
   const int d = tid % D, gi = tid / D;
   int p0, n;
   if (p.seq_slots != nullptr) {
-    // (a sequence without keys has no slots: what stands there is not used)
-    const int64_t len = p.lens_wide ? reinterpret_cast<const int64_t*>(p.lens)[seq]
-                                    : reinterpret_cast<const int32_t*>(p.lens)[seq];
+    // kept inside the workspace whatever stands there: a caller that changes
+    // the lengths while the split kernel reads them leaves pairs unwritten
     const int first = p.seq_slots[2 * seq], last = p.seq_slots[2 * seq + 1];
-    p0 = len > 0 ? first : 0;
-    n = len > 0 ? last - first + 1 : 0;
+    p0 = first < 0 ? 0 : first < p.num_slots ? first : p.num_slots;
+    n = (last < -1 ? -1 : last < p.num_slots ? last : p.num_slots - 1) - p0 + 1;
   } else {
     p0 = p.seq_partial_start[seq];
     n = p.seq_partial_start[seq + 1] - p0;

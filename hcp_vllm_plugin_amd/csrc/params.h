@@ -108,11 +108,10 @@ struct RedParams {
   const float* ws_lse;
   const int32_t* seq_partial_start;
   const int32_t* rows;  // output row of each sequence (NULL: its index)
-  // decode_paged_kernel's launches: first and last slot of each sequence (of
-  // one with keys), in place of seq_partial_start
+  // decode_paged_kernel's launches: first and last of the num_slots slots of
+  // each sequence (first > last: none), in place of seq_partial_start
   const int32_t* seq_slots;
-  const void* lens;  // with seq_slots: [num_seqs] int32 or int64
-  bool lens_wide;
+  int32_t num_slots;
   int32_t num_seqs;
   void* out;
   int64_t o_stride_tok, o_stride_head;
@@ -141,7 +140,7 @@ struct PagedDecParams {
   int64_t bt_stride;     // elements between block-table rows
   int64_t max_len;       // keys a block-table row can name
   int32_t window;        // 0: none
-  int32_t* seq_slots;    // [2 * num_seqs]: first and last slot of each sequence
+  int32_t* seq_slots;    // [2 * num_seqs]: first and last slot of each sequence (0, -1: no keys)
 };
 
 struct MergeParams {

@@ -472,7 +472,9 @@ int hcp_decode_launch(const hcp_decode_args* args, void* stream);
  * can name (block_table_width * block_size) as that many; the caller checks
  * them where it must refuse such a batch.  At most
  * HCP_DECODE_PAGED_MAX_SEQS sequences.
- *   seq_lens           DEVICE [num_seqs], HCP_DTYPE_I32 or I64 (lens_dtype)
+ *   seq_lens           DEVICE [num_seqs], HCP_DTYPE_I32 or I64 (lens_dtype); if
+ *                      they change before the launch has run, the results are
+ *                      undefined, but no access leaves the workspace or the cache
  *   kv                 the cache; its block_table is the DEVICE int32 table of
  *                      num_seqs rows of block_table_width ids, block_table_stride
  *                      elements apart; start and len are ignored
