@@ -74,7 +74,7 @@ EXPORTED_SYMBOLS = (
     "hcp_gather_paged_kv",
 )
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 
 class KvSegment(ctypes.Structure):
@@ -297,7 +297,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.hcp_varlen_launch.argtypes = [_P, _P]
     lib.hcp_fetch_metadata.restype = ctypes.c_int
     lib.hcp_fetch_metadata.argtypes = [
-        _P, _I32, _I64, _P, _I32, _I64, _P, _I32, _I64, _I32, _I64, _P, _P,
+        _P, _I32, _I64, _P, _I32, _I64, _P, _I32, _I64, _I32, _I64, _P, _I64, _P, _P,
     ]
     lib.hcp_wait_metadata.restype = ctypes.c_int
     lib.hcp_wait_metadata.argtypes = [_P, _I64, _P]

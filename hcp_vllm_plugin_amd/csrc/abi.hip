@@ -1350,7 +1350,8 @@ int hcp_reshape_and_cache(const void* key, int64_t k_stride_tok, int64_t k_strid
 int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t qsl_stride,
                        const void* seq_lens, int32_t lens_dtype, int64_t lens_stride,
                        const void* block_table, int32_t bt_dtype, int64_t bt_stride, int32_t n,
-                       int64_t token, int64_t* host_out, void* stream) {
+                       int64_t max_len, int64_t* dev_out, int64_t token, int64_t* host_out,
+                       void* stream) {
   const char* who = "hcp_fetch_metadata";
   for (int32_t d : {qsl_dtype, lens_dtype, bt_dtype})
     if (d != HCP_DTYPE_I32 && d != HCP_DTYPE_I64)
@@ -1371,6 +1372,8 @@ int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t q
   p.n = n;
   p.token = token;
   p.out = host_out;
+  p.max_len = max_len;
+  p.dev = dev_out;
   return launch_status(hcp::launch_fetch_metadata(p, static_cast<hipStream_t>(stream)), who);
 }
 

@@ -521,12 +521,10 @@ __device__ __forceinline__ int wave_prefix(int x) {
   return x;
 }
 
-// Keys of sequence r (0 .. max_len) that its one query sees.
+// Length r as the caller gives it.
 __device__ __forceinline__ int64_t paged_len(const PagedDecParams& p, int r) {
-  int64_t n = p.lens_wide ? global_ptr(reinterpret_cast<const int64_t*>(p.lens))[r]
-                          : global_ptr(reinterpret_cast<const int32_t*>(p.lens))[r];
-  n = n < 0 ? 0 : n < p.max_len ? n : p.max_len;
-  return n;
+  return p.lens_wide ? global_ptr(reinterpret_cast<const int64_t*>(p.lens))[r]
+                     : global_ptr(reinterpret_cast<const int32_t*>(p.lens))[r];
 }
 
 // A pure decode batch without a plan: lengths and block tables come straight
@@ -554,7 +552,7 @@ decode_paged_kernel(PagedDecParams p_) {
   __shared__ __attribute__((aligned(1024))) char bufO[W][2 * CHB];
   __shared__ float sm_m[W][16];
   __shared__ float sm_l[W][16];
-  __shared__ int sm_len[kDecMaxSeqs], sm_all[kDecMaxSeqs];  // keys seen, and in the cache
+  __shared__ int sm_len[kDecMaxSeqs], sm_all[kDecMaxSeqs];  // keys seen, in the cache (-1: not run)
   __shared__ int sm_w[2][W];
   __shared__ int sm_cut[4];
   int kvh;
@@ -572,18 +570,15 @@ decode_paged_kernel(PagedDecParams p_) {
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       const int r = tid * EPT + j;
-      const int all = r < n ? static_cast<int>(paged_len(p_, r)) : 0;  // max_len < 2^31
+      const int64_t given = r < n ? paged_len(p_, r) : 0;
+      const int all =  // keys that the sequence's query sees; max_len < 2^31
+          static_cast<int>(given < 0 ? 0 : given < p_.max_len ? given : p_.max_len);
       const int len = p_.window > 0 && all > p_.window ? p_.window : all;
       if (r < n) {
-        sm_all[r] = all;
+        sm_all[r] = given == HCP_LEN_NOT_RUN ? -1 : all;
         sm_len[r] = len;
       }
       c[j] = (len >> 5) + ((len & 31) != 0);
-      // the reduce goes by the slots alone: a sequence without keys says so
-      if (r < n && c[j] == 0 && wg == 0 && kvh == 0 && chunk == 0) {
-        global_ptr(p_.seq_slots)[2 * r] = 0;
-        global_ptr(p_.seq_slots)[2 * r + 1] = -1;
-      }
       cs += c[j];
       zs += c[j] > 0;
     }
@@ -636,9 +631,8 @@ decode_paged_kernel(PagedDecParams p_) {
     __syncthreads();
   }
   const int r0 = __builtin_amdgcn_readfirstlane(sm_cut[0]);
-  if (r0 < 0) return;  // no share
   const int o0 = __builtin_amdgcn_readfirstlane(sm_cut[1]);
-  const int r1 = __builtin_amdgcn_readfirstlane(sm_cut[2]);
+  const int r1 = r0 < 0 ? -2 : __builtin_amdgcn_readfirstlane(sm_cut[2]);  // -1, -2: no share
   const int o1 = __builtin_amdgcn_readfirstlane(sm_cut[3]);
   for (int r = r0; r <= r1; ++r) {
     const PagedDecParams& p = fresh_params<PagedDecParams>();
@@ -663,6 +657,15 @@ decode_paged_kernel(PagedDecParams p_) {
     decode_split_body<D, T, true>(p.d, kvh, chunk, wg + r, e, static_cast<int64_t>(b) * 32,
                                   ke < len ? ke : len, bufE, bufO, sm_m, sm_l);
     __syncthreads();  // this split has been combined out of the buffers
+  }
+  // the reduce goes by the slots alone: a sequence without keys says so
+  if (wg == 0 && kvh == 0 && chunk == 0) {
+    const PagedDecParams& p = fresh_params<PagedDecParams>();
+    for (int r = threadIdx.x; r < p.num_seqs; r += NT) {
+      if (sm_len[r] > 0) continue;
+      global_ptr(p.seq_slots)[2 * r] = 0;
+      global_ptr(p.seq_slots)[2 * r + 1] = sm_all[r] < 0 ? -2 : -1;
+    }
   }
 }
 
@@ -693,7 +696,8 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
     // the lengths while the split kernel reads them leaves pairs unwritten
     const int first = p.seq_slots[2 * seq], last = p.seq_slots[2 * seq + 1];
     p0 = first < 0 ? 0 : first < p.num_slots ? first : p.num_slots;
-    n = (last < -1 ? -1 : last < p.num_slots ? last : p.num_slots - 1) - p0 + 1;
+    n = (last < -2 ? -2 : last < p.num_slots ? last : p.num_slots - 1) - p0 + 1;
+    if (n < 0) return;  // not run
   } else {
     p0 = p.seq_partial_start[seq];
     n = p.seq_partial_start[seq + 1] - p0;

@@ -109,7 +109,8 @@ struct RedParams {
   const int32_t* seq_partial_start;
   const int32_t* rows;  // output row of each sequence (NULL: its index)
   // decode_paged_kernel's launches: first and last of the num_slots slots of
-  // each sequence (first > last: none), in place of seq_partial_start
+  // each sequence (first > last: none, by more than 1: its row is left as it
+  // is), in place of seq_partial_start
   const int32_t* seq_slots;
   int32_t num_slots;
   int32_t num_seqs;
@@ -140,7 +141,8 @@ struct PagedDecParams {
   int64_t bt_stride;     // elements between block-table rows
   int64_t max_len;       // keys a block-table row can name
   int32_t window;        // 0: none
-  int32_t* seq_slots;    // [2 * num_seqs]: first and last slot of each sequence (0, -1: no keys)
+  int32_t* seq_slots;    // [2 * num_seqs]: first and last slot of each sequence (0, -1: no keys;
+                         // 0, -2: HCP_LEN_NOT_RUN)
 };
 
 struct MergeParams {
@@ -203,6 +205,8 @@ struct MetaParams {
   int32_t n;
   int64_t token;
   int64_t* out;  // [3 n + 2]: the token, then the values
+  int64_t max_len;
+  int64_t* dev;  // [2 n] or NULL: the lengths of a plain decode batch, the lengths
 };
 
 // Prefill in D columns (padded_head_dim): the attention kernel and, when p

@@ -70,6 +70,7 @@ from .varlen import (
     PagedCache,
     PagedDecode,
     VarlenLaunch,
+    _upload,
     make_entry,
     paged_entry_array,
     segment_contiguous,
@@ -315,16 +316,41 @@ def _chunk_words(kvs: list) -> np.ndarray:
     return np.array(rows, dtype=np.uint64)
 
 
+# (what torch.cuda.is_current_stream_capturing calls, looked up once)
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing",
+                     torch.cuda.is_current_stream_capturing)
+
+
 class _Step:
     """What a step's layers share: the host copy of its metadata, its block
-    table as contiguous int32, and the plans made from them (``fast``).  A
-    layer keeps the record it got, so another thread's step can neither take
-    the plans away under it nor be given them."""
+    table as contiguous int32, its lengths on the device as the host saw them
+    (``lens``, None where the copy took the general path) and the plans made
+    from them (``fast``).  A layer keeps the record it got, so another thread's
+    step can neither take the plans away under it nor be given them."""
 
-    __slots__ = ("meta", "stamp", "host", "bt", "fast")
+    __slots__ = ("meta", "stamp", "host", "bt", "lens", "owner", "fast")
 
-    def __init__(self, meta, stamp, host, bt):
-        self.meta, self.stamp, self.host, self.bt, self.fast = meta, stamp, host, bt, {}
+    def __init__(self, meta, stamp, host, bt, lens, owner):
+        self.meta, self.stamp, self.host, self.bt = meta, stamp, host, bt
+        self.lens, self.owner, self.fast = lens, owner, {}
+
+    def lens_on(self, stream: int, device: torch.device, given: torch.Tensor):
+        """The lengths for launches on ``stream`` that read them on the device,
+        or None.  Not the caller's tensor: that may be refilled for the next
+        step while they are queued.  ``lens`` itself is written again by the
+        next step of its thread on its stream, in order there; any other
+        thread or stream gets a copy of the host's.  Under capture it is the
+        caller's, whose contents at each replay are what a graph runs on."""
+        if _capturing():
+            return given
+        if self.lens is None or self.owner == (threading.get_ident(), stream):
+            return self.lens
+        own = self.fast.get(("lens", stream))
+        if own is None:
+            words = np.asarray(self.host[1], dtype=np.int64)
+            dev, _ = _upload([words], device)
+            own = self.fast[("lens", stream)] = dev[:words.nbytes].view(torch.int64)
+        return own
 
 
 # The newest step.  vLLM hands every layer the same metadata object, so one
@@ -385,21 +411,24 @@ def _step(attn_metadata, queue=None) -> _Step:
     qsl_t = attn_metadata.query_start_loc
     sl_t = attn_metadata.seq_lens
     n = sl_t.shape[0]
+    lens = owner = None
     if _fetchable(qsl_t, n + 1) and _fetchable(sl_t, n) and block_table.is_cuda \
             and block_table.shape[0] >= n:  # (the copy reads a first block per request)
-        host = _fetch_metadata(qsl_t, sl_t, block_table, n, queue)
+        host, lens, owner = _fetch_metadata(qsl_t, sl_t, block_table, n, queue)
     else:
         fb = block_table[:, 0] if block_table.shape[1] > 0 else sl_t.new_zeros(n)
         packed = torch.cat([qsl_t.reshape(-1).to(torch.int64), sl_t.reshape(-1).to(torch.int64),
                             fb.reshape(-1).to(torch.int64)]).tolist()
         host = (packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:])
-    st = _Step(attn_metadata, stamp, host, block_table)
+    st = _Step(attn_metadata, stamp, host, block_table, lens, owner)
     _STEP.update(step=st, fast=st.fast)
     return st
 
 
 _INDEX_CODES = {torch.int32: _lib.DTYPE_I32, torch.int64: _lib.DTYPE_I64}
-_fetch_buf = threading.local()  # page-locked, per thread: read before the call returns
+# per thread: the page-locked block (read before the call returns) and the
+# words on the device
+_fetch_buf = threading.local()
 
 
 def _fetchable(t: torch.Tensor, n: int) -> bool:
@@ -407,31 +436,39 @@ def _fetchable(t: torch.Tensor, n: int) -> bool:
 
 
 def _fetch_metadata(qsl_t, sl_t, block_table, n: int, queue=None):
-    """The step's metadata as host lists, by one kernel that writes it to
-    page-locked memory and one wait for that memory; what ``queue`` puts on
+    """The step's metadata as host lists, its lengths on the device and whose
+    they are (thread and stream), by one kernel that writes both (the former to
+    page-locked memory) and one wait for that memory; what ``queue`` puts on
     the stream runs while the host waits and goes on."""
-    buf = getattr(_fetch_buf, "buf", None)
-    if buf is None or buf.shape[0] < 3 * n + 2:
-        buf = _fetch_buf.buf = torch.zeros(max(1024, 4 * n), dtype=torch.int64, pin_memory=True)
-        _fetch_buf.np = buf.numpy()
-        _fetch_buf.token = 0
-    token = _fetch_buf.token = _fetch_buf.token + 1
     dev, L = qsl_t.device, _lib.lib()
     with _lib.on_device(dev):
         stream = _lib.stream_ptr(dev)
+        f = _fetch_buf
+        if getattr(f, "key", None) != (dev, stream, n):
+            # the lengths, for a launch queued ahead and for all others:
+            # written by each step of this thread and stream, in order
+            f.words = torch.empty(2 * n, dtype=torch.int64, device=dev)
+            f.ahead, f.lens = f.words[:n], f.words[n:]
+            f.key = (dev, stream, n)
+            if getattr(f, "buf", None) is None or f.buf.shape[0] < 3 * n + 2:
+                f.buf = torch.zeros(max(1024, 4 * n), dtype=torch.int64, pin_memory=True)
+                f.np, f.token = f.buf.numpy(), 0
+        f.token += 1
         rc = L.hcp_fetch_metadata(
             qsl_t.data_ptr(), _INDEX_CODES[qsl_t.dtype], qsl_t.stride(0),
             sl_t.data_ptr(), _INDEX_CODES[sl_t.dtype], sl_t.stride(0),
             block_table.data_ptr() if block_table.shape[1] > 0 else 0, _lib.DTYPE_I32,
-            block_table.stride(0), n, token, buf.data_ptr(), stream)
+            block_table.stride(0), n, 0 if queue is None else queue.max_len, f.words.data_ptr(),
+            f.token, f.buf.data_ptr(), stream)
         _lib.check(rc, "hcp_fetch_metadata")
         try:
             if queue is not None:
-                queue()
+                queue(f.ahead)
         finally:  # the buffer is not left to be written later
-            _lib.check(L.hcp_wait_metadata(buf.data_ptr(), token, stream), "hcp_wait_metadata")
-    packed = _fetch_buf.np[1:3 * n + 2].tolist()
-    return packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:]
+            _lib.check(L.hcp_wait_metadata(f.buf.data_ptr(), f.token, stream), "hcp_wait_metadata")
+    packed = f.np[1:3 * n + 2].tolist()
+    return ((packed[:n + 1], packed[n + 1:2 * n + 1], packed[2 * n + 1:]), f.lens,
+            (threading.get_ident(), stream))
 
 
 def _forward_attn_metadata(layer):
@@ -616,18 +653,21 @@ def _check_base(pc: PagedCache) -> None:
 class _Ahead:
     """A decode layer queued before the host has seen the step's metadata:
     called by ``_step`` between queueing the metadata's copy and
-    waiting for it (not at all when the host has it already)."""
+    waiting for it (not at all when the host has it already).  The copy's
+    kernel looks whether the batch is what the layer was queued for, with
+    lengths within ``max_len``; if not, the layer writes nothing."""
 
     def __init__(self, impl, query, out, meta, pc):
         self.args = (impl, query, out, meta, pc)
-        self.ran = False
+        self.max_len = meta.block_table.shape[1] * pc.block_size
+        self.dec = None
 
-    def __call__(self):
+    def __call__(self, lens):
         impl, query, out, meta, pc = self.args
-        if PagedDecode.takes(meta.block_table, meta.seq_lens, pc.block_size):
-            PagedDecode(pc, meta.block_table, meta.seq_lens, impl.num_heads,
-                        impl.sliding_window).run(query, out, pc, impl.scale)
-            self.ran = True
+        if PagedDecode.takes(meta.block_table, lens, pc.block_size):
+            self.dec = PagedDecode(pc, meta.block_table, lens, impl.num_heads,
+                                   impl.sliding_window)
+            self.dec.run(query, out, pc, impl.scale)
 
 
 class _Plan:
@@ -890,7 +930,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         ahead = None
         if num_actual == attn_metadata.seq_lens.shape[0] and split == 0 and \
                 not (ring_on and PEER_KV_STAGING) and \
-                not (_decode_ring_enabled() and DECODE_RING_MAP):
+                not (DECODE_RING_MAP and _decode_ring_enabled()):
             ahead = _Ahead(self, query, out, attn_metadata, pc)
         # small metadata tensors: one host sync per step (see _step)
         step = _step(attn_metadata, ahead)
@@ -998,7 +1038,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
     def _peer_free(ring_on: bool, split: int, first_blocks, n: int) -> bool:
         """No request of the batch takes a peer segment or the decode ring:
         the plain causal pass over the paged cache (ring_backend.py:783-789)."""
-        if _decode_ring_enabled() and DECODE_RING_MAP and \
+        if DECODE_RING_MAP and _decode_ring_enabled() and \
                 any(fb in DECODE_RING_MAP for fb in first_blocks):
             return False
         if not ring_on:
@@ -1133,28 +1173,26 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         if n == 0:
             return
         w = self.sliding_window
-        if qsl == list(range(n + 1)) and PagedDecode.takes(block_table, lens_t, pc.block_size):
-            keys = block_table.shape[1] * pc.block_size
-            if min(seq_lens) < 0:
-                raise ValueError("negative segment start/length")
-            if max(seq_lens) > keys:
-                raise ValueError("segment extends past the block-table row")
-            if ahead is None or not ahead.ran:
-                key = self._layout_key("paged", pc)
-                dec = fast.get(key)
-                if dec is None:
-                    dec = fast[key] = PagedDecode(pc, block_table, lens_t, self.num_heads, w)
-                _check_base(pc)
-                dec.run(query, out, pc, self.scale)
-            _count("decode")
-            return
         stream = _lib.stream_ptr(query.device)
+        if qsl == list(range(n + 1)):
+            lens = step.lens_on(stream, query.device, lens_t)
+            key = (*self._layout_key("paged", pc), stream, lens is lens_t)
+            dec = fast.get(key)
+            if dec is None:
+                dec = fast[key] = self._plan_paged(seq_lens, block_table, pc, lens, ahead)
+            if dec:
+                if ahead is None or ahead.dec is None:
+                    _check_base(pc)
+                    dec.run(query, out, pc, self.scale)
+                _count("decode")
+                return
         # The single-token rows first: they seldom need a plan, and the
         # prefill's is made while they run.
         key = (*self._layout_key("rows", pc), stream)
         dec = fast.get(key, fast)  # (fast itself: not planned yet)
         if dec is fast:
-            dec = fast[key] = self._plan_rows(query, qsl, seq_lens, block_table, pc, lens_t)
+            lens = step.lens_on(stream, query.device, lens_t)
+            dec = fast[key] = self._plan_rows(query, qsl, seq_lens, block_table, pc, lens)
         _check_base(pc)
         if dec is not None:
             if isinstance(dec, tuple):  # a run of rows, unplanned
@@ -1179,6 +1217,19 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             else:
                 pre.run(query, out, None, self.num_kv_heads, self.scale, w, kv_base=pc.k_addr)
             _count("attn")
+
+    def _plan_paged(self, seq_lens, block_table, pc, lens, ahead):
+        """A pure decode batch without a plan, or False past its limits.
+        Lengths that the block table cannot name are refused."""
+        if lens is None or not PagedDecode.takes(block_table, lens, pc.block_size):
+            return False
+        if min(seq_lens) < 0:
+            raise ValueError("negative segment start/length")
+        if max(seq_lens) > block_table.shape[1] * pc.block_size:
+            raise ValueError("segment extends past the block-table row")
+        if ahead is not None and ahead.dec is not None and ahead.args[3].block_table is block_table:
+            return ahead.dec
+        return PagedDecode(pc, block_table, lens, self.num_heads, self.sliding_window)
 
     def _rows_apart(self, qsl, seq_lens):
         """(query starts, new tokens, keys of each request, which of them are
@@ -1205,7 +1256,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         return VarlenLaunch(ent, True, True, query.device, keep=block_table, heads=self._heads,
                             window=self.sliding_window)
 
-    def _plan_rows(self, query, qsl, seq_lens, block_table, pc, lens_t):
+    def _plan_rows(self, query, qsl, seq_lens, block_table, pc, lens):
         """The launch of a batch's single-token rows: (first, end, launch) of a
         run of query rows without a plan where they are neighbouring requests,
         as a scheduler lists them, else a planned one; None without such rows.
@@ -1223,9 +1274,10 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             return None
         w = self.sliding_window
         a, b = int(rows[0]), int(rows[-1]) + 1
-        if b - a == len(rows) and PagedDecode.takes(block_table[a:b], lens_t[a:b], pc.block_size):
+        if b - a == len(rows) and lens is not None and \
+                PagedDecode.takes(block_table[a:b], lens[a:b], pc.block_size):
             return (int(qs[a]), int(qs[a]) + b - a,
-                    PagedDecode(pc, block_table[a:b], lens_t[a:b], self.num_heads, w))
+                    PagedDecode(pc, block_table[a:b], lens[a:b], self.num_heads, w))
         # one query at the end of its keys: all of them visible, or the last `w`
         # of them (ring_backend.py:397-398)
         start = np.zeros(len(rows), np.int64) if w is None else np.maximum(tk[rows] - w, 0)

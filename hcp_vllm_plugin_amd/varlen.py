@@ -264,10 +264,13 @@ def paged_entry_array(pc: "PagedCache", block_table: torch.Tensor, rows, q_start
     if (start < 0).any() or (length < 0).any():
         raise ValueError("negative segment start/length")
     nblk = (start + length + pc.block_size - 1) // pc.block_size
-    if ((length > 0) & (nblk > block_table.shape[1])).any():
+    num_rows, width = block_table.shape
+    # (as unsigned numbers: a negative row lies past the last one)
+    past = rows.view(np.uint64) >= num_rows
+    if ((length > 0) & ((nblk > width) | past)).any():
+        if ((length > 0) & past).any():
+            raise ValueError("the block table has no row for a request")
         raise ValueError("segment extends past the block-table row")
-    if ((length > 0) & ((rows < 0) | (rows >= block_table.shape[0]))).any():
-        raise ValueError("the block table has no row for a request")
     a = np.zeros(len(rows), dtype=ENTRY_DTYPE)
     a["q_start"] = q_start
     a["q_len"] = q_len

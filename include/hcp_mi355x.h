@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define HCP_ABI_VERSION 10
+#define HCP_ABI_VERSION 11
 
 typedef enum hcp_status {
   HCP_OK = 0,
@@ -331,7 +331,11 @@ int hcp_varlen_launch(const hcp_varlen_args* args, void* stream);
  * the n sequence lengths and the n first block ids (element 0 of each
  * block-table row; block_table may be NULL: zeros), all widened to int64, into
  * `host_out` [1 + 3 n + 1], which must be page-locked memory the GPU can
- * write: first `token`, written last, then the values.  Index dtypes are
+ * write: first `token`, written last, then the values.  dev_out [2 n] (DEVICE,
+ * may be NULL) gets n lengths as int64 for a plain decode batch -- query r
+ * starts at row r, every length is in 0 .. max_len -- or n times
+ * HCP_LEN_NOT_RUN for any other, then the n lengths as they are: a launch on
+ * either runs on what the host sees, whatever becomes of seq_lens.  Index dtypes are
  * HCP_DTYPE_I32 / I64, strides in elements.  One kernel on `stream`.
  * hcp_wait_metadata returns when host_out[0] is `token` (which must not have
  * stood there before): it watches the memory, and after 50 ms waits for
@@ -340,7 +344,8 @@ int hcp_varlen_launch(const hcp_varlen_args* args, void* stream);
 int hcp_fetch_metadata(const void* query_start_loc, int32_t qsl_dtype, int64_t qsl_stride,
                        const void* seq_lens, int32_t lens_dtype, int64_t lens_stride,
                        const void* block_table, int32_t bt_dtype, int64_t bt_stride,
-                       int32_t n, int64_t token, int64_t* host_out, void* stream);
+                       int32_t n, int64_t max_len, int64_t* dev_out, int64_t token,
+                       int64_t* host_out, void* stream);
 int hcp_wait_metadata(const int64_t* host_out, int64_t token, void* stream);
 
 /*
@@ -472,7 +477,8 @@ int hcp_decode_launch(const hcp_decode_args* args, void* stream);
  * can name (block_table_width * block_size) as that many; the caller checks
  * them where it must refuse such a batch.  At most
  * HCP_DECODE_PAGED_MAX_SEQS sequences.
- *   seq_lens           DEVICE [num_seqs], HCP_DTYPE_I32 or I64 (lens_dtype); if
+ *   seq_lens           DEVICE [num_seqs], HCP_DTYPE_I32 or I64 (lens_dtype); the
+ *                      row of an int64 HCP_LEN_NOT_RUN is not written; if
  *                      they change before the launch has run, the results are
  *                      undefined, but no access leaves the workspace or the cache
  *   kv                 the cache; its block_table is the DEVICE int32 table of
@@ -481,6 +487,7 @@ int hcp_decode_launch(const hcp_decode_args* args, void* stream);
  *   workspace          hcp_decode_paged_workspace bytes, 16-byte aligned
  */
 #define HCP_DECODE_PAGED_MAX_SEQS 1024
+#define HCP_LEN_NOT_RUN INT64_MIN
 typedef struct hcp_decode_paged_args {
   const void* q;
   int64_t q_stride_tok, q_stride_head;

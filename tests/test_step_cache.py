@@ -73,6 +73,7 @@ def test_another_threads_step_leaves_a_layers_plans_alone(monkeypatch):
         return plan
 
     monkeypatch.setattr(rb._lib, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(rb, "_capturing", lambda: False)
     monkeypatch.setattr(rb.HcpRingAttentionImpl, "_plan_rows", planner("rows"))
     monkeypatch.setattr(rb.HcpRingAttentionImpl, "_plan_chunks", planner("chunks"))
     _forward(mine)
