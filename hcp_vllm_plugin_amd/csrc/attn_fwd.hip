@@ -884,9 +884,11 @@ fa_fwd_kernel(FwdParams p) {
           *reinterpret_cast<f32x4*>(wo + ((db * 4 + a) * 64 + lane_e) * 4) =
               f32x4{oacc[db][4 * a] * inv, oacc[db][4 * a + 1] * inv, oacc[db][4 * a + 2] * inv,
                     oacc[db][4 * a + 3] * inv};
+      // (a sum that is NaN leaves a NaN here: the merge must not take the piece
+      // for one without keys)
       if (ge == 0)
         p.ws_lse[unit * BM + wave * 32 + r32e] =
-            l_tot > 0.f ? m_ref * kLn2 + __logf(l_tot) : -INFINITY;
+            l_tot == 0.f ? -INFINITY : m_ref * kLn2 + __logf(l_tot);
     }
     return;
   }
@@ -1038,15 +1040,16 @@ __global__ __launch_bounds__(256) void fwd_reduce_kernel(FwdParams p) {
   f32x4 o[CW];
 #pragma unroll
   for (int c = 0; c < CW; ++c) o[c] = f32x4{};
-  if (M != -INFINITY) {
+  // A NaN LSE (scores that hold a NaN) makes the sums NaN and the row with
+  // them, its LSE -inf: what the uncut launch writes.
+  const float ref = M == -INFINITY ? 0.f : M;
 #pragma unroll 2
-    for (int i = 0; i < np; ++i) {
-      const float w = __expf(lp[i * ustride * kFwdBM] - M);
-      S += w;
+  for (int i = 0; i < np; ++i) {
+    const float w = __expf(lp[i * ustride * kFwdBM] - ref);
+    S += w;
 #pragma unroll
-      for (int c = 0; c < CW; ++c)
-        o[c] += *reinterpret_cast<const f32x4*>(op + i * ustride * (kFwdBM * D) + c * 256) * w;
-    }
+    for (int c = 0; c < CW; ++c)
+      o[c] += *reinterpret_cast<const f32x4*>(op + i * ustride * (kFwdBM * D) + c * 256) * w;
   }
   const float inv = S > 0.f ? 1.f / S : 0.f;
   float lse_row = S > 0.f ? M + __logf(S) : -INFINITY;

@@ -1,0 +1,80 @@
+"""NaN and infinite inputs: a row comes out as the launch that is not cut (or
+the batch that is not taken apart) gives it, on whatever kernels it runs."""
+
+import pytest
+import torch
+
+from hcp_vllm_plugin_amd import ring_attn_merged, ring_attn_with_lse
+from tests._util import randn, scale_for
+from tests.test_gpu_split import _qkv, _split
+
+pytestmark = pytest.mark.gpu
+
+NAN, INF = float("nan"), float("inf")
+
+
+def _same(got, want, tol, strict=True):
+    """NaN and infinities in the same places, the rest within ``tol``.  Not
+    ``strict``: infinite or NaN alike -- an infinite V meets a P that is 0 in 16
+    bits (and gives NaN) relative to one maximum and not to another."""
+    got, want = got.float(), want.float()
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    if strict:
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(got == INF, want == INF) and torch.equal(got == -INF, want == -INF)
+    ok = torch.isfinite(want)
+    assert not ok.any() or (got[ok] - want[ok]).abs().max().item() <= tol
+
+
+def _poison(q, k, v, what):
+    """``what`` at one query row, at keys of one or several pieces, or in V."""
+    if what == "q":
+        q[5, 1, 3], q[40, 0, 0] = NAN, INF
+    elif what == "k":
+        k[700, :, 1] = NAN
+    elif what == "k all":
+        k[:, 0, 1] = NAN
+    elif what == "k inf":
+        k[3, :, 2] = INF
+    else:
+        v[700, :, 4], v[100, :, 5] = NAN, INF
+    return q, k, v
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h,hkv,d", [(8, 2, 128), (4, 2, 64), (4, 4, 256)])
+@pytest.mark.parametrize("what", ["q", "k", "k all", "k inf", "v"])
+@pytest.mark.parametrize("off,window", [(None, 0), (872, 0), (872, 400)])
+def test_cut_prefill_rows(dev, dtype, h, hkv, d, what, off, window):
+    tq, tk = 150, 1000
+    q, k, v = (x.to(dev) for x in _poison(*_qkv(d, tq, tk, h, hkv, d, dtype), what))
+    scale = scale_for(d)
+    whole, whole_l = _split(q, k, v, scale, off, window, 100, 0)  # one piece: nothing is cut
+    acc_o = randn(torch.Generator().manual_seed(1), (tq, h, d), dtype).to(dev)
+    acc_l = torch.full((h, tq), 1.0, device=dev)
+    acc_l[:, 3:9] = -INF
+    want, want_l = _split(q, k, v, scale, off, window, 100, 0, (acc_o, acc_l))
+    # P and the output round to the dtype, the partials to f32
+    tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * 4 * max(
+        1.0, whole.float().nan_to_num(0, 0, 0).abs().max().item())
+    for piece in (1, 4):
+        out, lse = _split(q, k, v, scale, off, window, piece, 0)
+        _same(out, whole, tol, what != "v")
+        _same(lse, whole_l, 1e-3)
+        out, lse = _split(q, k, v, scale, off, window, piece, 0, (acc_o, acc_l))
+        _same(out, want, tol, what != "v")
+        _same(lse, want_l, 1e-3)
+
+
+def test_planned_cut_and_whole_agree(dev):
+    """The entry points, where the planner cuts: a NaN query row is NaN."""
+    q, k, v = _qkv(1, 16, 8192, 14, 2, 64, torch.bfloat16)
+    q[7] = NAN
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    out, lse = ring_attn_with_lse(qd, kd, vd, scale_for(64), None)
+    assert torch.isnan(out[7]).all() and (lse[:, 7] == -INF).all()
+    rest = [i for i in range(16) if i != 7]
+    assert torch.isfinite(out[rest]).all() and torch.isfinite(lse[:, rest]).all()
+    merged = ring_attn_merged(qd, kd, vd, scale_for(64), None, torch.ones_like(out),
+                              torch.zeros_like(lse))
+    assert (merged[7] == 1).all()  # a side without weight, as in the merge after a whole pass
