@@ -163,7 +163,7 @@ class DecodeArgs(ctypes.Structure):
         ("dtype", ctypes.c_int32),
         ("use_scratch", ctypes.c_int32),
         ("scale", ctypes.c_float),
-        ("reserved", ctypes.c_int32),
+        ("keep_nan", ctypes.c_int32),
     ]
 
 
@@ -232,6 +232,7 @@ class DecodePagedArgs(ctypes.Structure):
         ("num_kv_heads", ctypes.c_int32),
         ("head_dim", ctypes.c_int32),
         ("dtype", ctypes.c_int32),
+        ("keep_nan", ctypes.c_int32),
         ("scale", ctypes.c_float),
     ]
 

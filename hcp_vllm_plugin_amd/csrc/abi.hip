@@ -935,6 +935,7 @@ struct DecodeExtra {
   int32_t num_wgs = 0;
   const int32_t* rows = nullptr;
   uint64_t kv_base = 0;
+  bool keep_nan = false;
 };
 
 static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
@@ -977,6 +978,7 @@ static int decode_impl(const char* who, const void* q, int64_t q_stride_tok,
   dp.works = x.works;
   dp.num_wgs = x.works ? x.num_wgs : num_splits;
   dp.kv_base = x.kv_base;
+  dp.keep_nan = x.keep_nan;
   dp.ws_o = static_cast<float*>(workspace);
   dp.ws_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + o_al);
   dp.num_heads = num_heads;
@@ -1142,6 +1144,7 @@ int hcp_decode_launch(const hcp_decode_args* a, void* stream) {
   x.num_wgs = a->num_wgs;
   x.rows = a->seq_rows;
   x.kv_base = a->kv_base;
+  x.keep_nan = a->keep_nan != 0;
   return decode_impl(who, a->q, a->q_stride_tok, a->q_stride_head, nullptr, 0, nullptr,
                      a->num_works, a->seq_partial_start, a->num_seqs, ws, bytes, a->out,
                      a->o_stride_tok, a->o_stride_head, a->lse, a->lse_stride_head, a->acc_o,
@@ -1216,6 +1219,7 @@ int hcp_decode_paged(const hcp_decode_paged_args* a, void* stream) {
   dp.head_chunks = (dp.group + 15) / 16;
   dp.head_dim = a->head_dim;
   dp.scale_log2 = a->scale * hcp::kLog2e;
+  dp.keep_nan = a->keep_nan != 0;
   p.kv = kv;
   p.lens = a->seq_lens;
   p.lens_wide = a->lens_dtype == HCP_DTYPE_I64;

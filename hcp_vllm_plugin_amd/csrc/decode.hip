@@ -435,8 +435,12 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
     }
     const int head = h0 + h;
     const int64_t slot = static_cast<int64_t>(sp) * p.num_heads + head;
-    global_ptr(p.ws_o)[slot * D + d] = L > 0.f ? O / L : 0.f;
-    if (d == 0) global_ptr(p.ws_lse)[slot] = L > 0.f ? M * kLn2 + __logf(L) : -INFINITY;
+    // a sum that is NaN counts as a split without keys unless the caller wants
+    // the NaN in the row
+    const float none = p.keep_nan && L != L ? L : 0.f;
+    global_ptr(p.ws_o)[slot * D + d] = L > 0.f ? O / L : none;
+    if (d == 0)
+      global_ptr(p.ws_lse)[slot] = L > 0.f ? M * kLn2 + __logf(L) : none == 0.f ? -INFINITY : none;
   }
 }
 
@@ -736,12 +740,14 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
     float mn = m;
 #pragma unroll
     for (int j = 0; j < U; ++j) mn = fmaxf(mn, l[j]);
-    if (mn == -INFINITY) continue;
+    // (relative to 0 where no partial has keys: their weights are 0, but one
+    // with a NaN LSE makes the sums NaN)
+    const float ref = mn == -INFINITY ? 0.f : mn;
     rebase(mn);
 #pragma unroll
     for (int j = 0; j < U; ++j) {
       const bool in = i0 + j * ng < n;
-      const float w = in ? __expf(l[j] - mn) : 0.f;
+      const float w = in ? __expf(l[j] - ref) : 0.f;
       S += w;
       O = in ? __builtin_fmaf(w, v[j], O) : O;
     }
@@ -756,13 +762,14 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
   __syncthreads();
   if (gi != 0) return;
   for (int g2 = 1; g2 < ng; ++g2) {
-    if (sm_m[g2] == -INFINITY) continue;
+    if (sm_s[g2] == 0.f) continue;
     const float mn = fmaxf(m, sm_m[g2]);
     rebase(mn);
     const float w = __expf(sm_m[g2] - mn);
     S = __builtin_fmaf(w, sm_s[g2], S);
     O = __builtin_fmaf(w, sm_o[g2][d], O);
   }
+  const bool nan = S != S;  // the partials' own
   if (acc_l != -INFINITY) {
     const float mn = fmaxf(m, acc_l);
     rebase(mn);
@@ -770,13 +777,13 @@ __global__ __launch_bounds__(4 * D) void decode_reduce_kernel(RedParams p) {
     S += w;
     O = __builtin_fmaf(w, acc_v, O);
   }
-  const bool any = m != -INFINITY;
+  const bool any = m != -INFINITY || nan;
   uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + row * p.o_stride_tok +
                    static_cast<int64_t>(head) * p.o_stride_head;
   if (d < p.head_dim) orow[d] = Elem<T>::from_float(any ? O / S : 0.f);
   if (p.lse != nullptr && d == 0)
     p.lse[static_cast<int64_t>(head) * p.lse_stride_head + row] =
-        any ? m + __logf(S) : -INFINITY;
+        any && !nan ? m + __logf(S) : -INFINITY;
 }
 
 template <int D, typename T>

@@ -678,6 +678,7 @@ class _Plan:
         self.peer_rounds: list = []     # per round: {"contig": [...], "paged": [...]}
         self.any_peer = False
         self.decode: list = []  # single-token rows for the decode kernel: (q row, segments)
+        self.decode_peer = False  # one of them has a peer segment
         self.ring: list = []  # decode-ring rows: (r, q row, tk, ring state, bt row, block 0)
 
 
@@ -872,7 +873,10 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 lo = peer_end if peer_end < tk else 0
                 segs = [segment_paged(pc, row, lo, tk - lo)]
                 segs = window_tail(segs, self.sliding_window)
-                plan.decode.append((qs, segs + (peer_segs if 0 < peer_end < tk else [])))
+                if 0 < peer_end < tk and peer_segs:
+                    segs += peer_segs
+                    plan.decode_peer = True
+                plan.decode.append((qs, segs))
                 continue
             if peer_end == 0:
                 plan.local.append(make_entry(qs, tq, segment_paged(pc, row, 0, tk), qpos0))
@@ -961,9 +965,13 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             if plan.local or plan.any_peer:
                 self._forward_prefill(query, out, plan)
             if plan.decode:
+                # NaN scores as the prefill launches leave them: in the row, or,
+                # where these merge with peers, a side without weight
+                keep_nan = not (plan.any_peer or plan.decode_peer)
                 DecodeBatch([segs for _, segs in plan.decode], self.num_heads, self.num_kv_heads,
                             self.head_size, query.device,
-                            rows=[qs for qs, _ in plan.decode]).run(query, out, None, self.scale)
+                            rows=[qs for qs, _ in plan.decode]).run(
+                    query, out, None, self.scale, keep_nan=keep_nan)
                 _count("decode")
             parts = {}
             for (r, qs, *_r) in plan.ring:
@@ -1187,7 +1195,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 _count("decode")
                 return
         # The single-token rows first: they seldom need a plan, and the
-        # prefill's is made while they run.
+        # prefill's is made while they run.  In the prefill launch a NaN score
+        # makes its row NaN (a decode batch leaves the split out): here too.
         key = (*self._layout_key("rows", pc), stream)
         dec = fast.get(key, fast)  # (fast itself: not planned yet)
         if dec is fast:
@@ -1197,9 +1206,10 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         if dec is not None:
             if isinstance(dec, tuple):  # a run of rows, unplanned
                 a, b, rows = dec
-                rows.run(query[a:b], out[a:b], pc, self.scale)
+                rows.run(query[a:b], out[a:b], pc, self.scale, keep_nan=True)
             else:
-                dec.run(query, out, None, self.scale, kv_base=pc.k_addr)
+                dec.run(query, out, None, self.scale, kv_base=pc.k_addr,
+                        keep_nan=qsl != list(range(n + 1)))
             _count("decode")
         key = (*self._layout_key("chunks", pc), stream)
         pre = fast.get(key, fast)

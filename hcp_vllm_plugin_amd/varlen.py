@@ -745,13 +745,16 @@ class DecodeBatch:
 
     def run(self, q: torch.Tensor, out: torch.Tensor, lse: torch.Tensor | None,
             scale: float, acc: tuple[torch.Tensor, torch.Tensor] | None = None,
-            noalloc: bool = False, kv_base: int = 0) -> None:
+            noalloc: bool = False, kv_base: int = 0, keep_nan: bool = False) -> None:
         """Decode into ``out`` (and ``lse``).  With ``acc = (o_acc [S, H, D] in
         q's dtype, lse_acc [H, S] float32)`` the accumulator is merged in by the
         same launch; ``out`` / ``lse`` may be the accumulator's own tensors.
 
         ``kv_base``: added to the addresses of paged segments (planned with
         addresses relative to a layer's cache).
+
+        ``keep_nan``: a row whose scores hold a NaN comes out NaN, as from a
+        prefill launch; otherwise the splits that hold one are left out.
 
         ``noalloc``: the partials live in the library's fixed per-GPU scratch
         (no workspace is taken, so nothing is allocated; calls overlapping on
@@ -766,6 +769,7 @@ class DecodeBatch:
         if lse is not None:
             a.lse, a.lse_stride_head = lse.data_ptr(), lse.stride(0)
         a.scale, a.dtype, a.kv_base = float(scale), _lib.dtype_code(q.dtype), kv_base
+        a.keep_nan = keep_nan
         if acc is not None:
             ao, al = acc
             if ao.dtype != q.dtype or tuple(ao.shape) != tuple(q.shape) or ao.stride(-1) != 1:
@@ -835,13 +839,14 @@ class PagedDecode:
                 and seq_lens.dtype in (torch.int32, torch.int64)
                 and width * block_size < 1 << 31 and width <= ((1 << 34) // block_size) // n)
 
-    def run(self, q: torch.Tensor, out: torch.Tensor, pc: PagedCache, scale: float) -> None:
-        """One layer: its q, out and cache."""
+    def run(self, q: torch.Tensor, out: torch.Tensor, pc: PagedCache, scale: float,
+            keep_nan: bool = False) -> None:
+        """One layer: its q, out and cache.  ``keep_nan``: as ``DecodeBatch.run``."""
         a = _lib.DecodePagedArgs.from_buffer_copy(self._args)
         a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(0), q.stride(1)
         a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
         a.kv.k_addr, a.kv.v_addr = pc.k_addr, pc.v_addr
-        a.scale, a.dtype = float(scale), _lib.dtype_code(q.dtype)
+        a.scale, a.dtype, a.keep_nan = float(scale), _lib.dtype_code(q.dtype), keep_nan
         with _lib.on_device(q.device):
             # fp32 partials: stream-ordered scratch from torch's caching allocator
             ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=q.device)

@@ -441,6 +441,9 @@ int hcp_plan_decode_lists(const hcp_varlen_entry* entries, int32_t num_entries,
  *                the device serves every layer's cache
  *   use_scratch  partials in the library's scratch, not in workspace (as
  *                hcp_decode_splitkv_noalloc)
+ *   keep_nan     a row whose scores hold a NaN comes out NaN (its LSE -inf), as
+ *                the prefill launches write it; 0: such a split is left out, as
+ *                in hcp_decode_splitkv
  */
 typedef struct hcp_decode_args {
   const void* q;
@@ -463,7 +466,7 @@ typedef struct hcp_decode_args {
   int32_t num_heads, num_kv_heads, head_dim, dtype;
   int32_t use_scratch;
   float scale;
-  int32_t reserved;
+  int32_t keep_nan;
 } hcp_decode_args;
 
 int hcp_decode_launch(const hcp_decode_args* args, void* stream);
@@ -502,6 +505,7 @@ typedef struct hcp_decode_paged_args {
   int64_t lse_stride_head;
   int32_t lens_dtype, num_seqs, window;
   int32_t num_heads, num_kv_heads, head_dim, dtype;
+  int32_t keep_nan; /* as in hcp_decode_args */
   float scale;
 } hcp_decode_paged_args;
 

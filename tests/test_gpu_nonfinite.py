@@ -1,11 +1,16 @@
 """NaN and infinite inputs: a row comes out as the launch that is not cut (or
 the batch that is not taken apart) gives it, on whatever kernels it runs."""
 
+import types
+
 import pytest
 import torch
 
+from hcp_vllm_plugin_amd import ring_backend as rb
 from hcp_vllm_plugin_amd import ring_attn_merged, ring_attn_with_lse
 from tests._util import randn, scale_for
+from tests.test_gpu_backend import _clean  # noqa: F401
+from tests.test_gpu_decode_paged import _batch, _meta
 from tests.test_gpu_split import _qkv, _split
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +83,50 @@ def test_planned_cut_and_whole_agree(dev):
     merged = ring_attn_merged(qd, kd, vd, scale_for(64), None, torch.ones_like(out),
                               torch.zeros_like(lse))
     assert (merged[7] == 1).all()  # a side without weight, as in the merge after a whole pass
+
+
+@pytest.mark.parametrize("lens", [[200, 9000, 40, 5000], [9000, 200, 40, 700]])
+@pytest.mark.parametrize("peers", ["none", "staging of others", "staged"])
+def test_single_token_rows_of_a_mixed_batch(dev, monkeypatch, lens, peers):
+    """Rows with NaN in q, or in one key, as the prefill launch gives them,
+    unplanned and planned; next to a staged peer, which the prefill launches
+    merge with, a row of NaN scores has no weight."""
+    h, hkv, d = 8, 2, 128
+    tq = [1, 64, 1, 1] if lens[0] == 200 else [64, 1, 1, 1]
+    qsl = [0]
+    for t in tq:
+        qsl.append(qsl[-1] + t)
+    _, cache, bt = _batch(7, lens, h, hkv, d, torch.bfloat16, "v031", 16)
+    if peers != "staged":  # one key of the third request, in a block of its own
+        cache[bt[2, 1], :, 3, 5] = NAN
+    gen = torch.Generator().manual_seed(2)
+    q = randn(gen, (qsl[-1], h, d), torch.bfloat16)
+    q[qsl[-1] - 1] = NAN
+    impl = rb.HcpRingAttentionImpl(h, d, scale_for(d), hkv)
+    layer = types.SimpleNamespace(layer_name="model.layers.0.self_attn.attn")
+    bt[:, 0] = torch.arange(4, dtype=torch.int32)  # the requests' names, still blocks of the cache
+    if peers == "staging of others":
+        rb.stage_peer_kv("c", "another.layer", torch.zeros(16, hkv, d, dtype=q.dtype, device=dev),
+                         torch.zeros(16, hkv, d, dtype=q.dtype, device=dev))
+        rb.map_request_peer(2, ["c"])
+    elif peers == "staged":
+        for r in (1, 2):
+            rb.stage_peer_kv("c%d" % r, layer.layer_name,
+                             randn(gen, (32, hkv, d), q.dtype).to(dev),
+                             randn(gen, (32, hkv, d), q.dtype).to(dev))
+            rb.map_request_peer(r, ["c%d" % r])
+    got = []
+    for apart in (False, True):
+        monkeypatch.setattr(rb.HcpRingAttentionImpl, "_decode_rows_apart",
+                            lambda self, *a, apart=apart: apart)
+        out = torch.full((qsl[-1], h, d), 7.0, dtype=q.dtype, device=dev)
+        impl.forward(layer, q.to(dev), None, None, cache.to(dev), _meta(dev, qsl, lens, bt), out)
+        torch.cuda.synchronize()
+        got.append(out)
+    assert rb.IMPL_STATS["decode_hip"] == 1
+    bad = got[0].float()
+    if peers == "staged":
+        assert torch.isfinite(bad).all() and (bad[-1] == 0).all()
+    else:
+        assert torch.isnan(bad[-1]).all() and torch.isnan(bad[qsl[2]]).all()
+    _same(got[1], got[0], 2 * 1.5e-2)
