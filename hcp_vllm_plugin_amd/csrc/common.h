@@ -89,6 +89,28 @@ __device__ __forceinline__ uint32_t pack2<_Float16>(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), f16x2));
 }
 
+// Two floats >= 0 (or NaN) as two dwords of two 16-bit elements: hi is below
+// the float, lo what is left of it.  Unlike a rounded term and its remainder
+// neither is 0 or negative where the float is above 2^-23: products with an
+// infinity stay that infinity.
+template <typename T>
+__device__ __forceinline__ void two_terms(float a, float b, uint32_t& hi, uint32_t& lo);
+template <>
+__device__ __forceinline__ void two_terms<__bf16>(float a, float b, uint32_t& hi, uint32_t& lo) {
+  const uint32_t x = __builtin_elementwise_sub_sat(__float_as_uint(a), 1u) & 0xffff0000u;
+  const uint32_t y = __builtin_elementwise_sub_sat(__float_as_uint(b), 1u) & 0xffff0000u;
+  hi = (x >> 16) | y;
+  lo = pack2<__bf16>(a - __uint_as_float(x), b - __uint_as_float(y));
+}
+template <>
+__device__ __forceinline__ void two_terms<_Float16>(float a, float b, uint32_t& hi, uint32_t& lo) {
+  constexpr float kLeast = 0x1p-24f;  // the smallest fp16: what lo rounds to, at least
+  hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(__builtin_fmaxf(a - kLeast, 0.f),
+                                                              __builtin_fmaxf(b - kLeast, 0.f)));
+  lo = pack2<_Float16>(a - Elem<_Float16>::to_float(static_cast<uint16_t>(hi & 0xffffu)),
+                       b - Elem<_Float16>::to_float(static_cast<uint16_t>(hi >> 16)));
+}
+
 // acc + lo + hi of a dword of two 16-bit elements, in f32: one v_dot2_f32_*
 // against (1, 1), so the sum is of the rounded values themselves.
 template <typename T>

@@ -227,26 +227,22 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
 #pragma unroll
     for (int u = 0; u < NU; ++u) oacc[u] *= alpha;
 
-    u32x4 pw;
-    pw[0] = pack2<T>(s0[0], s0[1]);
-    pw[1] = pack2<T>(s0[2], s0[3]);
-    pw[2] = pack2<T>(s1[0], s1[1]);
-    pw[3] = pack2<T>(s1[2], s1[3]);
-    const V8 pf = as_vec8<V8>(pw);
-    // P enters the PV product as two 16-bit terms, its rounded value and what
-    // the rounding left: the kernel waits on memory, the second product hides.
-    // One term would be exact only for the largest key of each wave's share of
-    // a split, so the error would grow with the length of the splits.
-    auto rest = [&](uint32_t w, float a, float b) __attribute__((always_inline)) {
-      return pack2<T>(a - E::to_float(static_cast<uint16_t>(w & 0xffffu)),
-                      b - E::to_float(static_cast<uint16_t>(w >> 16)));
+    // P enters the PV product as two 16-bit terms: the kernel waits on memory,
+    // the second product hides.  One rounded term would be exact only for the
+    // largest key of each wave's share of a split, so the error would grow with
+    // the length of the splits.
+    u32x4 pw, rw;
+    auto put = [&](int i, float a, float b) __attribute__((always_inline)) {
+      uint32_t hi, lo;
+      two_terms<T>(a, b, hi, lo);
+      pw[i] = hi;
+      rw[i] = lo;
     };
-    u32x4 rw;
-    rw[0] = rest(pw[0], s0[0], s0[1]);
-    rw[1] = rest(pw[1], s0[2], s0[3]);
-    rw[2] = rest(pw[2], s1[0], s1[1]);
-    rw[3] = rest(pw[3], s1[2], s1[3]);
-    const V8 rf = as_vec8<V8>(rw);
+    put(0, s0[0], s0[1]);
+    put(1, s0[2], s0[3]);
+    put(2, s1[0], s1[1]);
+    put(3, s1[2], s1[3]);
+    const V8 pf = as_vec8<V8>(pw), rf = as_vec8<V8>(rw);
 
     // 8 keys x NU d in registers -> NU operands of 8 keys each
 #pragma unroll

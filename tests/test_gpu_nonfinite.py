@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from hcp_vllm_plugin_amd import ring_backend as rb
+from hcp_vllm_plugin_amd.varlen import PagedCache, PagedDecode, decode_attn, segment_contiguous
 from hcp_vllm_plugin_amd import ring_attn_merged, ring_attn_with_lse
 from tests._util import randn, scale_for
 from tests.test_gpu_backend import _clean  # noqa: F401
@@ -130,3 +131,41 @@ def test_single_token_rows_of_a_mixed_batch(dev, monkeypatch, lens, peers):
     else:
         assert torch.isnan(bad[-1]).all() and torch.isnan(bad[qsl[2]]).all()
     _same(got[1], got[0], 2 * 1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h,hkv,d", [(8, 2, 128), (4, 2, 64), (4, 4, 256)])
+def test_decode_with_infinite_values(dev, dtype, h, hkv, d):
+    """An infinite V element makes its output column infinite, with its sign,
+    whatever its key's weight rounds to (the largest weight of the row, 1,
+    among them); the other columns stay what they are."""
+    n = 1500
+    gen = torch.Generator().manual_seed(d)
+    q = randn(gen, (2, h, d), dtype) * 0.2
+    k, v = randn(gen, (n, hkv, d), dtype), randn(gen, (n, hkv, d), dtype)
+    kd = k.float().reshape(n, hkv, d).repeat_interleave(h // hkv, 1)
+    sc = torch.einsum("thd,nhd->thn", q.float(), kd) * scale_for(d)
+    top = sc.argmax(-1)[0]  # the first row's heaviest key of each head
+    keys = torch.unique(torch.cat([top, torch.tensor([0, 31, 32, 700, n - 2])]))
+    inf = v.clone()
+    for i, key in enumerate(keys.tolist()):
+        inf[key, :, i] = INF if i % 2 else -INF
+    col = torch.arange(len(keys))
+    pc_cache = torch.zeros(100, hkv, 16, 2 * d, dtype=dtype)
+    pc_cache[torch.arange(n) // 16, :, torch.arange(n) % 16] = torch.cat([k, inf], -1)
+    cache = pc_cache.to(dev)
+    bt = torch.arange(100, dtype=torch.int32, device=dev).repeat(2, 1)
+    lens = torch.tensor([n, n], dtype=torch.int32, device=dev)
+    qd, kdev, vdev, idev = q.to(dev), k.to(dev), v.to(dev), inf.to(dev)
+    want = decode_attn(qd, [[segment_contiguous(kdev, vdev)]] * 2, hkv, scale_for(d))
+    flat = decode_attn(qd, [[segment_contiguous(kdev, idev)]] * 2, hkv, scale_for(d))
+    paged = torch.empty_like(flat)
+    pc = PagedCache.from_tensor(cache)
+    PagedDecode(pc, bt, lens, h, None).run(qd, paged, pc, scale_for(d))
+    torch.cuda.synchronize()
+    ref = torch.where(col % 2 == 1, INF, -INF).to(dev)
+    tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * 4
+    for out in (flat, paged):
+        hit = out[..., :len(keys)].float()
+        assert (hit == ref).all(), [(keys[c].item(), hit[..., c].tolist()) for c in col if not (hit[..., c] == ref[c]).all()]
+        assert (out[..., len(keys):].float() - want[..., len(keys):].float()).abs().max() <= tol
