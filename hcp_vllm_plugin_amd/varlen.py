@@ -608,7 +608,6 @@ class DecodeBatch:
                  head_dim: int, device: torch.device, split_tokens: int | None = None,
                  rows: list[int] | None = None):
         """``rows``: the q / out / lse row of each sequence (default: its index)."""
-        L = _lib.lib()
         entries, seq_of = [], []
         for s, segs in enumerate(segments):
             for seg in segs:
@@ -616,12 +615,12 @@ class DecodeBatch:
                 seq_of.append(s)
         self.num_seqs = len(segments)
         self.num_entries = len(entries)
-        arr = np.zeros(max(self.num_entries, 1), dtype=ENTRY_DTYPE)
-        if entries:
-            packed = (VarlenEntry * self.num_entries)(*entries)
-            arr[:] = np.frombuffer(packed, dtype=ENTRY_DTYPE)
-        self._plan(arr, np.asarray(seq_of or [0], dtype=np.int32), num_heads, num_kv_heads,
-                   head_dim, split_tokens, rows, device)
+        n = max(self.num_entries, 1)
+        arr = (VarlenEntry * n)(*entries)
+        seq_arr = (ctypes.c_int32 * n)(*seq_of)
+        self._plan(ctypes.addressof(arr), ctypes.addressof(seq_arr),
+                   [e.kv.len for e in entries], num_heads, num_kv_heads, head_dim, split_tokens,
+                   rows, device)
         # the segments point at K/V / cache / block-table storage by address
         self._keep = [getattr(e, "_keep", None) for e in entries]
 
@@ -638,7 +637,6 @@ class DecodeBatch:
         each sequence (default: its index); the entries' q_start name the q rows."""
         if entries.dtype != ENTRY_DTYPE or not entries.flags.c_contiguous:
             raise ValueError("entry array must be contiguous ENTRY_DTYPE")
-        L = _lib.lib()
         self = cls.__new__(cls)
         n = len(entries)
         if entry_seq is None:
@@ -654,38 +652,39 @@ class DecodeBatch:
         self.num_seqs = ns
         self.num_entries = n
         arr = entries if n else np.zeros(1, dtype=ENTRY_DTYPE)
-        self._plan(arr, seq_arr, num_heads, num_kv_heads, head_dim, split_tokens, rows, device)
+        self._plan(arr.ctypes.data, seq_arr.ctypes.data, arr["len"][:n].tolist(), num_heads,
+                   num_kv_heads, head_dim, split_tokens, rows, device)
         self._keep = keep
         return self
 
-    def _plan(self, arr, seq_arr, num_heads, num_kv_heads, head_dim, split_tokens, rows,
-              device) -> None:
+    def _plan(self, entries_addr, seq_addr, lens, num_heads, num_kv_heads, head_dim, split_tokens,
+              rows, device) -> None:
         """Plan and upload: splits of at most ``split_tokens`` keys, one to a
         workgroup, or (None) an equal share of the batch's keys for every
         workgroup of the launch (``hcp_plan_decode_lists``)."""
         L = _lib.lib()
         n, ns = self.num_entries, self.num_seqs
-        heads = num_kv_heads * head_chunks(num_heads, num_kv_heads)
-        if rows is not None:
-            rows = np.ascontiguousarray(rows, dtype=np.int32)
-            if len(rows) != ns:
-                raise ValueError("rows needs one row per sequence")
-        total = int(arr["len"][:n].sum())
+        if rows is not None and len(rows) != ns:
+            raise ValueError("rows needs one row per sequence")
         if split_tokens is None:
-            wgs = decode_workgroups(heads)
+            wgs = decode_workgroups(num_kv_heads * head_chunks(num_heads, num_kv_heads))
             cap = n + wgs
         else:
             wgs = 0
-            cap = int((-(-arr["len"][:n] // split_tokens)).sum())
-        self.split_tokens = split_tokens or max(1, -(-total // wgs))  # keys to a workgroup
-        works = np.empty(max(cap, 1), dtype=WORK_DTYPE)
-        work_entry = np.empty(max(cap, 1), dtype=np.int32)
-        starts = np.empty(ns + 1, dtype=np.int32)
+            cap = sum(-(-x // split_tokens) for x in lens)
+        self.split_tokens = split_tokens or max(1, -(-sum(lens) // wgs))  # keys to a workgroup
+        # one block: partial starts, rows and records (uploaded), entry of each record
+        rows_at = (4 * (ns + 1) + 255) & ~255
+        works_at = rows_at + (0 if rows is None else (4 * ns + 255) & ~255)
+        entry_at = works_at + 128 * max(cap, 1)
+        block = np.empty(entry_at + 4 * max(cap, 1), dtype=np.uint8)
+        base = block.ctypes.data
+        if rows is not None:
+            block[rows_at:rows_at + 4 * ns].view(np.int32)[:] = rows
         m = ctypes.c_int32(0)
         rc = L.hcp_plan_decode_lists(
-            arr.ctypes.data, n, seq_arr.ctypes.data, ns, wgs, split_tokens or 0,
-            works.ctypes.data, work_entry.ctypes.data, cap, starts.ctypes.data,
-            ctypes.addressof(m))
+            entries_addr, n, seq_addr, ns, wgs, split_tokens or 0, base + works_at,
+            base + entry_at, cap, base, ctypes.addressof(m))
         _lib.check(rc, "hcp_plan_decode_lists")
         self.num_splits = rc
         self.num_heads = num_heads
@@ -693,51 +692,36 @@ class DecodeBatch:
         self.head_dim = head_dim
         self.ws_bytes = int(L.hcp_decode_workspace_bytes(max(rc, 1), num_heads, head_dim))
         self.device = device
-        self._works, self._work_entry = works[:rc], work_entry[:rc]
+        # the records as words: copying those is one memcpy, copying records
+        # goes field by field
+        self._words = block[works_at:works_at + 128 * rc].view(np.uint64).reshape(rc, 16)
+        self._work_entry = block[entry_at:entry_at + 4 * rc].view(np.int32)
         self._chunk_rows = None
-        extra = [] if rows is None else [rows]
-        self._plan_dev, (w_ptr, s_ptr, *r_ptr) = _upload(
-            [works[:max(rc, 1)], starts, *extra], device)
+        self._plan_dev, (dev,) = _upload([block[:works_at + 128 * max(rc, 1)]], device)
         a = self._args = _lib.DecodeArgs()
-        a.works, a.num_works, a.num_wgs = w_ptr, rc, m.value
-        a.seq_partial_start, a.num_seqs = s_ptr, ns
-        a.seq_rows = r_ptr[0] if r_ptr else 0
+        a.works, a.num_works, a.num_wgs = dev + works_at, rc, m.value
+        a.seq_partial_start, a.num_seqs = dev, ns
+        a.seq_rows = 0 if rows is None else dev + rows_at
         a.workspace_bytes = self.ws_bytes
         a.num_heads, a.num_kv_heads, a.head_dim = num_heads, num_kv_heads, head_dim
 
-    def rebind(self, entries: np.ndarray, keep=None) -> "DecodeBatch":
-        """The same plan (splits, partial slots) over new entries of the same
-        layout and lengths -- another layer's cache and staged chunks: only
-        the records go to the device (one small asynchronous copy)."""
-        if entries.dtype != ENTRY_DTYPE or not entries.flags.c_contiguous:
-            raise ValueError("entry array must be contiguous ENTRY_DTYPE")
-        if len(entries) != self.num_entries:
-            raise ValueError("rebind needs the plan's entry count")
-        works = self._works.copy()
-        works["e"] = entries[self._work_entry]
-        return self._with_works(works, keep)
-
     def rebind_chunks(self, at: np.ndarray, rows: np.ndarray, keep=None) -> "DecodeBatch":
-        """``rebind`` of the contiguous entries ``at`` alone: row i of ``rows``
-        (uint64) is the K address, V address, token and head stride of entry
-        at[i]."""
+        """The same plan (splits, partial slots) over other chunks of the same
+        lengths -- another layer's: row i of ``rows`` (uint64) is the K address,
+        V address, token and head stride of the contiguous entry at[i].  Only the
+        records go to the device (one small asynchronous copy)."""
         if self._chunk_rows is None:  # records of contiguous entries, and which of them
             which = np.full(self.num_entries, -1, dtype=np.int64)
             which[at] = np.arange(len(at))
             rec = np.nonzero(which[self._work_entry] >= 0)[0]
             self._chunk_rows = (rec, which[self._work_entry[rec]])
         rec, src = self._chunk_rows
-        works = self._works.copy()
-        # hcp_decode_work as 16 words: k_addr, v_addr, stride_tok, stride_head
-        words = works.view(np.uint64).reshape(-1, 16)
+        words = self._words.copy()
         words[rec[:, None], _CHUNK_WORDS] = rows[src]
-        return self._with_works(works, keep)
-
-    def _with_works(self, works: np.ndarray, keep) -> "DecodeBatch":
         other = object.__new__(type(self))
         other.__dict__.update(self.__dict__)
-        other._works = works
-        other._works_dev, (w_ptr,) = _upload([works], self.device)
+        other._words = words
+        other._works_dev, (w_ptr,) = _upload([words], self.device)
         other._args = _lib.DecodeArgs.from_buffer_copy(self._args)
         other._args.works = w_ptr
         other._keep = keep

@@ -1,0 +1,76 @@
+"""What planning a launch costs the host, on the CPU: the planners' own calls
+counted, and the plans of equal batches equal."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from hcp_vllm_plugin_amd import varlen as V
+
+CPU = torch.device("cpu")
+
+
+@pytest.fixture
+def uploads(monkeypatch):
+    """Byte counts of what each plan uploads, and the blocks themselves."""
+    got = []
+
+    def upload(arrays, device):
+        offs, raw = [], b""  # (addresses: offsets in the block)
+        for a in arrays:
+            offs.append(len(raw))
+            n, addr = V._nbytes_addr(a)
+            raw += ctypes.string_at(addr, n)
+            raw += b"\0" * (-len(raw) % 256)
+        got.append(raw)
+        return None, offs
+
+    monkeypatch.setattr(V, "_upload", upload)
+    return got
+
+
+def _seg(n):
+    s = V.KvSegment()
+    s.k_addr = s.v_addr = 4096
+    s.stride_tok, s.stride_head, s.len = 128, n * 128, n
+    return s
+
+
+@pytest.mark.parametrize("rows", [None, [7, 3]])
+@pytest.mark.parametrize("split", [None, 64, 1000])
+def test_decode_plans_of_both_forms_agree(uploads, rows, split):
+    """Segments as objects and the same as an entry array: the same records,
+    where the launch arguments say."""
+    segs = [[_seg(5000), _seg(33)], [_seg(700)]]
+    a = V.DecodeBatch(segs, 28, 4, 128, CPU, split, rows=rows)
+    ent = np.zeros(3, dtype=V.ENTRY_DTYPE)
+    for i, (s, seg) in enumerate([(0, segs[0][0]), (0, segs[0][1]), (1, segs[1][0])]):
+        e = V.make_entry(s if rows is None else rows[s], 1, seg, 0)
+        ent[i] = np.frombuffer(e, dtype=V.ENTRY_DTYPE)[0]
+    b = V.DecodeBatch.from_entries(ent, 28, 4, 128, CPU, split, rows=rows, num_seqs=2,
+                                   entry_seq=np.array([0, 0, 1], np.int32))
+    assert a.split_tokens == b.split_tokens and a.num_splits == b.num_splits == a._args.num_works
+    raw, other = uploads
+    works = np.frombuffer(raw, V.WORK_DTYPE, a.num_splits, a._args.works)
+    same = np.frombuffer(other, V.WORK_DTYPE, a.num_splits, b._args.works)
+    starts = np.frombuffer(raw, np.int32, 3, a._args.seq_partial_start)
+    assert (works == same).all() and starts[0] == 0 and starts[2] == a.num_splits
+    assert int((works["key_end"] - works["key_begin"]).sum()) == 5733
+    if rows is None:
+        assert a._args.seq_rows == 0
+    else:
+        assert np.frombuffer(raw, np.int32, 2, a._args.seq_rows).tolist() == rows
+    with pytest.raises(ValueError, match="one row per sequence"):
+        V.DecodeBatch(segs, 28, 4, 128, CPU, split, rows=[1, 2, 3])
+
+
+def test_decode_plan_is_one_host_block(uploads, monkeypatch):
+    """... not an array each for records, starts, rows and their conversions:
+    a hop plans again after every growth append."""
+    made = []
+    empty = np.empty
+    monkeypatch.setattr(np, "empty", lambda *a, **k: made.append(a) or empty(*a, **k))
+    V.DecodeBatch([[_seg(32768), _seg(512)]], 28, 4, 128, CPU)
+    assert len(made) == 1
