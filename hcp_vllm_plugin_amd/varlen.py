@@ -22,6 +22,7 @@ and vLLM 0.23 ``[nb, 2, bs, Hkv, D]`` (ring_backend.py:601,617-624).
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import numpy as np
@@ -312,6 +313,34 @@ _MIN_SPLIT_KEYS = 449  # nor one of shorter key ranges
 _MAX_PIECES = 2048
 
 
+@functools.lru_cache(maxsize=64)
+def _varlen_cut(q_lens: bytes, kv_lens: bytes, offsets: bytes | None, window: int, heads):
+    """(pieces, units, arguments) of the KV split of a launch with these sizes
+    (int64 each; ``offsets`` None: not causal), None where it stays whole.  It
+    follows from the sizes alone and takes 15 to 30 us of the host to find
+    (known, 3 us), so the layers of a step share it."""
+    n = len(q_lens) // 8
+    ent = np.zeros(n, dtype=ENTRY_DTYPE)
+    ent["q_len"], ent["len"] = np.frombuffer(q_lens, np.int64), np.frombuffer(kv_lens, np.int64)
+    if offsets is not None:
+        ent["causal_offset"] = np.frombuffer(offsets, np.int64)
+    ent["stride_tok"] = 1  # the real strides were checked with the tiles
+    pieces, units = np.empty((2, _MAX_PIECES, 4), dtype=np.int32)
+    nu, ns, pt = (ctypes.c_int32(0) for _ in range(3))
+    nbytes = ctypes.c_size_t(0)
+    rc = _lib.lib().hcp_plan_varlen_split(
+        ent.ctypes.data, n, int(offsets is not None), window, *heads, pieces.ctypes.data,
+        _MAX_PIECES, units.ctypes.data, ctypes.addressof(nu), ctypes.addressof(ns),
+        ctypes.addressof(pt), ctypes.addressof(nbytes))
+    _lib.check(rc, "hcp_plan_varlen_split")
+    if rc == 0:
+        return None
+    pieces, units = pieces[:rc].copy(), units[:nu.value].copy()
+    pieces.flags.writeable = units.flags.writeable = False  # shared by every launch of these sizes
+    return pieces, units, {"key": (*heads, window), "pieces": rc, "units": nu.value,
+                           "slots": ns.value, "piece_tiles": pt.value, "bytes": nbytes.value}
+
+
 class VarlenLaunch:
     """A planned varlen launch: entries and tile list uploaded to the device.
 
@@ -378,7 +407,7 @@ class VarlenLaunch:
                                      int(self.causal), bm, ctypes.addressof(tiles), cap)
         _lib.check(rc, "hcp_plan_varlen_tiles")
         self.num_tiles = rc
-        split = self._plan_split(L, arr, heads, window)
+        split = self._plan_split(arr, heads, window)
         if self._gather is None:
             self._plan_dev, (self.entries_ptr, self.tiles_ptr, *sp) = _upload(
                 [arr, tiles, *split], device)
@@ -391,28 +420,23 @@ class VarlenLaunch:
             self._split["ptrs"] = sp
         self.device = device
 
-    def _plan_split(self, L, arr, heads, window):
+    def _plan_split(self, arr, heads, window):
         """The KV split of runs with these heads and window: records to upload
         ([pieces, units]), or [] for the uncut launch."""
         self._split = None
-        if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS or not self.num_tiles \
-                or np.frombuffer(arr, dtype=ENTRY_DTYPE)["len"].max() < _MIN_SPLIT_KEYS:
+        if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS or not self.num_tiles:
+            return []
+        ent = np.frombuffer(arr, dtype=ENTRY_DTYPE, count=self.num_entries)
+        if ent["len"].max() < _MIN_SPLIT_KEYS:
             return []
         win = int(window or 0) if self.causal else 0
-        pieces = np.empty((_MAX_PIECES, 4), dtype=np.int32)
-        units = np.empty((_MAX_PIECES, 4), dtype=np.int32)
-        nu, ns, pt = (ctypes.c_int32(0) for _ in range(3))
-        nbytes = ctypes.c_size_t(0)
-        rc = L.hcp_plan_varlen_split(
-            _nbytes_addr(arr)[1], self.num_entries, int(self.causal), win, *heads,
-            pieces.ctypes.data, _MAX_PIECES, units.ctypes.data, ctypes.addressof(nu),
-            ctypes.addressof(ns), ctypes.addressof(pt), ctypes.addressof(nbytes))
-        _lib.check(rc, "hcp_plan_varlen_split")
-        if rc == 0:
+        cut = _varlen_cut(ent["q_len"].tobytes(), ent["len"].tobytes(),
+                          ent["causal_offset"].tobytes() if self.causal else None, win,
+                          tuple(heads))
+        if cut is None:
             return []
-        self._split = {"key": (*heads, win), "pieces": rc, "units": nu.value, "slots": ns.value,
-                       "piece_tiles": pt.value, "bytes": nbytes.value}
-        return [pieces[:rc], units[:nu.value]]
+        pieces, units, self._split = cut[0], cut[1], dict(cut[2])
+        return [pieces, units]
 
     def _gathered(self, q: torch.Tensor, num_kv_heads: int) -> int:
         """Gather mode: copy every entry's paged keys into a contiguous K/V

@@ -74,3 +74,49 @@ def test_decode_plan_is_one_host_block(uploads, monkeypatch):
     monkeypatch.setattr(np, "empty", lambda *a, **k: made.append(a) or empty(*a, **k))
     V.DecodeBatch([[_seg(32768), _seg(512)]], 28, 4, 128, CPU)
     assert len(made) == 1
+
+
+@pytest.mark.parametrize("causal,window", [(True, None), (True, 300), (False, None)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_launches_of_equal_sizes_share_a_cut(uploads, monkeypatch, causal, window, paged):
+    """The search for the KV split runs once for the layers of a step, at other
+    addresses too; other sizes, offsets, windows or heads get their own."""
+    V._varlen_cut.cache_clear()
+    L = V._lib.lib()
+    calls, plan = [], L.hcp_plan_varlen_split
+    monkeypatch.setattr(L, "hcp_plan_varlen_split", lambda *a: calls.append(a) or plan(*a))
+
+    def launch(addr, keys=32768, heads=(28, 4, 128), new=512, win=window):
+        e = np.zeros(2, dtype=V.ENTRY_DTYPE)
+        e["q_len"], e["q_start"], e["len"] = [new, 3], [0, new], [keys, 700]
+        e["causal_offset"] = e["len"] - e["q_len"] if causal else 0
+        e["k_addr"] = e["v_addr"] = addr
+        e["stride_tok"], e["stride_head"] = 512, 128
+        if paged:
+            e["block_table"], e["stride_block"], e["block_size"] = addr, 8192, 16
+        return V.VarlenLaunch(e, causal, paged, CPU, heads=heads, window=win)
+
+    first = launch(4096)
+    assert len(calls) == 1
+    for i in range(3):
+        same = launch(8192 * (i + 1))
+        assert same._split == first._split
+    assert len(calls) == 1
+    if window is None:  # 512 x 32768 at 28 heads is cut, whatever the form
+        assert first._split is not None and first._split["pieces"] > 2 * 4
+        up = uploads[-1]
+        assert first._split["pieces"] * 16 + first._split["units"] * 16 < len(up)
+    launch(4096, keys=30000), launch(4096, heads=(14, 2, 64)), launch(4096, new=500)
+    launch(4096, win=900)
+    assert len(calls) == (5 if causal else 4)  # a window is nothing to a launch without a mask
+    assert V._varlen_cut.cache_info().maxsize == 64
+
+
+def test_a_launchs_arguments_are_its_own(uploads):
+    """(The addresses of the uploaded records go into them.)"""
+    e = np.zeros(1, dtype=V.ENTRY_DTYPE)
+    e["q_len"], e["len"], e["stride_tok"], e["stride_head"] = 64, 8192, 512, 128
+    a = V.VarlenLaunch(e, False, False, CPU, heads=(28, 4, 128))
+    b = V.VarlenLaunch(e, False, False, CPU, heads=(28, 4, 128))
+    a._split["ptrs"] = "a"
+    assert b._split["ptrs"] != "a" and a._split is not b._split
