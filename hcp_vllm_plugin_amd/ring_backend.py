@@ -823,21 +823,33 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             if peer_end > 0:
                 _probe_chunk_a_writes(block_table[r], peer_end, pc.block_size)
 
-    def _decode_rows_apart(self, qsl, seq_lens) -> bool:
+    def _decode_rows_apart(self, qsl, seq_lens, each_layer: bool = False) -> bool:
         """Whether a mixed batch's single-token rows leave the prefill launch
         for a decode launch of their own.  In the prefill launch such a row is
-        a 128-row block per query head, each reading its KV head's keys again:
-        about half a microsecond of a CU per 64 keys and head.  The decode
-        launch reads the keys once, but is two more kernels (about 20 us with
-        their planning).  28 / 4 x 128 heads, 512 new tokens next to 32 rows of
-        512 - 8192 keys, two layers: 543 us in one launch each, 319 us apart."""
-        tiles = sum(-(-int(tk) // 64) for r, tk in enumerate(seq_lens) if qsl[r + 1] - qsl[r] == 1)
-        return tiles * self.num_heads * 0.5 / 256 > 20
+        a 128-row block per query head, one of whose four waves has a row, each
+        reading its KV head's keys (the window's) again: 0.27, 0.49 or 0.88 us of
+        a CU per 64 keys and head at 64, 128 or 256 columns.  The decode launch
+        reads the keys once, but is two more kernels; where a plan is made once
+        per step it pays past 20 us of the machine, where each layer makes its
+        own (``each_layer``: staged or split peers) only past 150 us.
+
+        256 new tokens next to the rows, us per layer in one launch / apart:
+        28 / 4 x 128, 16 x 1536 keys (20 us by this count) 73 / 80, 8 x 4096 (27)
+        88 / 80, 32 x 4096 (109) 224 / 97; 14 / 2 x 64, 32 x 4096 (30) 100 / 80;
+        16 / 8 x 256, 2 x 8192 (14) 100 / 91; with 1024 staged keys each, 28 / 4 x
+        128, 8 x 4096 (34) 213 / 244, 32 x 4096 (136) 493 / 503."""
+        w = self.sliding_window
+        keys = [tk if w is None else min(tk, w)
+                for r, tk in enumerate(seq_lens) if qsl[r + 1] - qsl[r] == 1]
+        tile_us = {64: 0.27, 128: 0.49, 256: 0.88}[
+            next(c for c in (64, 128, 256) if self.head_size <= c)]
+        est = sum(-(-tk // 64) for tk in keys) * self.num_heads * tile_us / 256
+        return est > (150 if each_layer else 20)
 
     def _plan(self, layer_name, qsl, seq_lens, block_table, first_blocks, pc, split):
         plan = _Plan()
         n = len(seq_lens)
-        apart = qsl != list(range(n + 1)) and self._decode_rows_apart(qsl, seq_lens)
+        apart = qsl != list(range(n + 1)) and self._decode_rows_apart(qsl, seq_lens, True)
         ring_on = _decode_ring_enabled() and bool(DECODE_RING_MAP)
         for r in range(len(seq_lens)):
             qs, qe = qsl[r], qsl[r + 1]

@@ -79,3 +79,28 @@ def test_another_threads_step_leaves_a_layers_plans_alone(monkeypatch):
     _forward(mine)
     assert calls == ["rows", "chunks"]
     assert rb._host_metadata(other)[0][1] == [9] and not rb._STEP["fast"]
+
+
+@pytest.mark.parametrize("heads,d,rows,window,each_layer,apart", [
+    (28, 128, [16384] * 2, None, False, True),
+    (28, 128, [16384] * 2, 128, False, False),   # the prefill launch reads the window alone
+    (28, 128, [16384] * 64, 128, False, False),
+    (28, 128, [16384] * 64, 4096, False, True),
+    (28, 128, [4096] * 8, None, False, True),
+    (14, 64, [4096] * 8, None, False, False),    # half the columns, half the heads
+    (14, 64, [4096] * 32, None, False, True),
+    (16, 256, [4096] * 8, None, False, True),
+    (28, 128, [5120] * 32, None, True, False),   # a plan in every layer costs more
+    (28, 128, [34000] * 32, None, True, True),
+    (28, 128, [], None, False, False),
+])
+def test_rows_that_leave_the_prefill_launch(heads, d, rows, window, each_layer, apart):
+    """Next to two prefill chunks of many keys, which do not count."""
+    impl = rb.HcpRingAttentionImpl(heads, d, 0.125, 2, sliding_window=window)
+    qsl, lens = [0, 300], [60000]
+    for n in rows:
+        qsl.append(qsl[-1] + 1)
+        lens.append(n)
+    qsl.append(qsl[-1] + 300)
+    lens.append(60000)
+    assert impl._decode_rows_apart(qsl, lens, *([True] if each_layer else [])) == apart
