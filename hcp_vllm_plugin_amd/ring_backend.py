@@ -674,7 +674,9 @@ class _Plan:
     """Launch descriptors for one forward call."""
 
     def __init__(self):
-        self.local: list = []           # causal entries over the paged cache
+        # causal entries over the paged cache: (q row, rows, request, first key,
+        # keys, causal offset)
+        self.local: list = []
         self.peer_rounds: list = []     # per round: {"contig": [...], "paged": [...]}
         self.any_peer = False
         self.decode: list = []  # single-token rows for the decode kernel: (q row, segments)
@@ -856,11 +858,10 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             tq, tk = qe - qs, seq_lens[r]
             if tq == 0:
                 continue
-            row = block_table[r]
             if ring_on and tq == 1:
                 dr = DECODE_RING_MAP.get(first_blocks[r])
                 if dr is not None:
-                    plan.ring.append((r, qs, tk, dr, row, first_blocks[r]))
+                    plan.ring.append((r, qs, tk, dr, block_table[r], first_blocks[r]))
                     continue
             qpos0 = tk - tq
             staged = None
@@ -875,7 +876,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                         peer_segs.append(segment_contiguous(kk, vv))
             elif split > 0:
                 peer_end = min(split, tk)
-                peer_segs.append(segment_paged(pc, row, 0, peer_end))
+                peer_segs.append(segment_paged(pc, block_table[r], 0, peer_end))
             else:
                 peer_end = 0
             if apart and tq == 1:
@@ -883,7 +884,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 # whole local range, past it the local keys (the last `w` of
                 # them) and every staged chunk
                 lo = peer_end if peer_end < tk else 0
-                segs = [segment_paged(pc, row, lo, tk - lo)]
+                segs = [segment_paged(pc, block_table[r], lo, tk - lo)]
                 segs = window_tail(segs, self.sliding_window)
                 if 0 < peer_end < tk and peer_segs:
                     segs += peer_segs
@@ -891,16 +892,14 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 plan.decode.append((qs, segs))
                 continue
             if peer_end == 0:
-                plan.local.append(make_entry(qs, tq, segment_paged(pc, row, 0, tk), qpos0))
+                plan.local.append((qs, tq, r, 0, tk, qpos0))
                 continue
             n_a = max(0, min(tq, peer_end - qpos0))
             if n_a > 0:
-                plan.local.append(make_entry(qs, n_a, segment_paged(pc, row, 0, tk), qpos0))
+                plan.local.append((qs, n_a, r, 0, tk, qpos0))
             if n_a < tq:
                 qb0, nb = qs + n_a, tq - n_a
-                plan.local.append(make_entry(
-                    qb0, nb, segment_paged(pc, row, peer_end, tk - peer_end),
-                    qpos0 + n_a - peer_end))
+                plan.local.append((qb0, nb, r, peer_end, tk - peer_end, qpos0 + n_a - peer_end))
                 for i, seg in enumerate(peer_segs):
                     while len(plan.peer_rounds) <= i:
                         plan.peer_rounds.append({"contig": [], "paged": []})
@@ -957,8 +956,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         if len(first_blocks) < n and qsl[n] > qsl[len(first_blocks)]:
             raise ValueError("the block table has no row for a request")
         if self._peer_free(ring_on, split, first_blocks, n):
-            self._forward_local_only(query, out, step, pc, kv_cache, attn_metadata.seq_lens,
-                                     ahead)
+            self._forward_local_only(query, out, step, pc, attn_metadata.seq_lens, ahead)
             return output
         if WRITE_TRACK["enabled"]:
             self._write_probe(layer_name, qsl, seq_lens, block_table, first_blocks, pc,
@@ -971,11 +969,11 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         plan = self._plan(layer_name, qsl, seq_lens, block_table, first_blocks, pc, split)
         ring_local = self._ring_local_segments(plan, pc, key, value, layer_name)
         if is_decode:
-            lse = self._forward_decode(query, out, plan, n, ring_local)
+            lse = self._forward_decode(query, out, plan, block_table, pc, n, ring_local)
             parts = {r: (out[qs:qs + 1], lse[:, qs:qs + 1]) for (r, qs, *_r) in plan.ring}
         else:
             if plan.local or plan.any_peer:
-                self._forward_prefill(query, out, plan)
+                self._forward_prefill(query, out, plan, step, pc)
             if plan.decode:
                 # NaN scores as the prefill launches leave them: in the row, or,
                 # where these merge with peers, a side without weight
@@ -1181,7 +1179,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         return (kind, self.sliding_window, pc.layout, pc.stride_tok, pc.stride_head,
                 pc.stride_block, pc.block_size, pc.num_blocks, pc.v_addr - pc.k_addr, self._heads)
 
-    def _forward_local_only(self, query, out, step, pc, kv_cache, lens_t, ahead):
+    def _forward_local_only(self, query, out, step, pc, lens_t, ahead):
         """Causal attention of every request over its paged KV: for a pure
         decode batch ``PagedDecode``, which needs no plan (``ahead``: already
         queued for this layer), or, past its limits, a planned split-KV decode;
@@ -1228,16 +1226,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         if pre is fast:
             pre = fast[key] = self._plan_chunks(query, qsl, seq_lens, block_table, pc)
         if pre is not None:
-            if isinstance(pre, np.ndarray):
-                # blocks under 16 tokens are gathered from absolute addresses
-                ent = pre.copy()
-                ent["k_addr"] = pc.k_addr
-                ent["v_addr"] = pc.v_addr
-                VarlenLaunch(ent, True, True, query.device, keep=(kv_cache, block_table),
-                             heads=self._heads, window=w).run(
-                    query, out, None, self.num_kv_heads, self.scale, w)
-            else:
-                pre.run(query, out, None, self.num_kv_heads, self.scale, w, kv_base=pc.k_addr)
+            self._run_chunks(pre, query, out, block_table, pc)
             _count("attn")
 
     def _plan_paged(self, seq_lens, block_table, pc, lens, ahead):
@@ -1271,12 +1260,32 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         pre = np.nonzero((tq > 0) & ~dec)[0]
         if len(pre) == 0:
             return None
-        ent = paged_entry_array(pc, block_table, pre, qs[pre], tq[pre], (tk - tq)[pre], 0, tk[pre],
-                                relative=True)
+        return self._chunk_launch(
+            paged_entry_array(pc, block_table, pre, qs[pre], tq[pre], (tk - tq)[pre], 0, tk[pre],
+                              relative=True), query, block_table, pc)
+
+    def _chunk_launch(self, ent, query, block_table, pc):
+        """The causal launch of entries with addresses relative to a layer's
+        cache; over blocks under 16 tokens, which are gathered from absolute
+        addresses, the entries."""
         if pc.block_size < _MIN_PAGED_BLOCK:
             return ent
         return VarlenLaunch(ent, True, True, query.device, keep=block_table, heads=self._heads,
                             window=self.sliding_window)
+
+    def _run_chunks(self, pre, query, out, block_table, pc, acc=None):
+        """A layer's run of what ``_chunk_launch`` made, merged with ``acc`` as
+        its prefix."""
+        if isinstance(pre, np.ndarray):
+            ent = pre.copy()
+            ent["k_addr"] = pc.k_addr
+            ent["v_addr"] = pc.v_addr
+            pre, base = VarlenLaunch(ent, True, True, query.device, keep=(pc.cache, block_table),
+                                     heads=self._heads, window=self.sliding_window), 0
+        else:
+            base = pc.k_addr
+        pre.run(query, out, None, self.num_kv_heads, self.scale, self.sliding_window, acc=acc,
+                kv_base=base)
 
     def _plan_rows(self, query, qsl, seq_lens, block_table, pc, lens):
         """The launch of a batch's single-token rows: (first, end, launch) of a
@@ -1309,13 +1318,25 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
             self.num_heads, self.num_kv_heads, self.head_size, query.device, keep=block_table,
             rows=None if qsl == list(range(len(qsl))) else qs[rows])
 
-    def _forward_prefill(self, query, out, plan: _Plan) -> None:
+    def _local_launch(self, query, plan: _Plan, step, pc):
+        """The launch of a plan's local entries, shared by the layers that plan
+        the same ones (a layer whose staging differs makes its own)."""
+        _check_base(pc)
+        key = (*self._layout_key("local", pc), _lib.stream_ptr(query.device), tuple(plan.local))
+        pre = step.fast.get(key)
+        if pre is None:
+            a = np.array(plan.local, dtype=np.int64).reshape(-1, 6)
+            pre = step.fast[key] = self._chunk_launch(
+                paged_entry_array(pc, step.bt, a[:, 2], a[:, 0], a[:, 1], a[:, 5], a[:, 3],
+                                  a[:, 4], relative=True), query, step.bt, pc)
+        return pre
+
+    def _forward_prefill(self, query, out, plan: _Plan, step, pc) -> None:
         dev = query.device
         h = self.num_heads
+        local = self._local_launch(query, plan, step, pc)
         if not plan.any_peer:
-            VarlenLaunch(plan.local, True, True, dev, heads=self._heads,
-                         window=self.sliding_window).run(query, out, None, self.num_kv_heads,
-                                                         self.scale, self.sliding_window)
+            self._run_chunks(local, query, out, step.bt, pc)
             _count("attn")
             return
         o_peer = lse_peer = None
@@ -1341,23 +1362,20 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # = peer, suffix = local (ring_backend.py:354,820-831), bit for bit.
         # The local entries cover every query row of the plan; rows without a
         # peer have lse_peer = -inf and get the local result.
-        VarlenLaunch(plan.local, True, True, dev, heads=self._heads,
-                     window=self.sliding_window).run(
-            query, out, None, self.num_kv_heads, self.scale, self.sliding_window,
-            acc=(o_peer, lse_peer), acc_is_prefix=True)
+        self._run_chunks(local, query, out, step.bt, pc, acc=(o_peer, lse_peer))
         _count("attn")
         _count("merge")
 
-    def _forward_decode(self, query, out, plan: _Plan, n: int, ring_local=None):
+    def _forward_decode(self, query, out, plan: _Plan, block_table, pc, n: int, ring_local=None):
         """One split-KV launch for the whole decode batch; decode-ring rows
         get their owner-local partial (with LSE) from the same launch."""
         segs: list[list] = [[] for _ in range(n)]
         w = self.sliding_window
-        for e in plan.local:
-            kv = e.kv
+        for (qs, _tq, r, start, length, off) in plan.local:
+            kv = segment_paged(pc, block_table[r], start, length)
             if w is not None:  # the causal local pass sees keys (off - w, off]
-                kv = trim_segment(kv, min(kv.len, max(0, e.causal_offset - w + 1)))
-            segs[e.q_start].append(kv)
+                kv = trim_segment(kv, min(kv.len, max(0, off - w + 1)))
+            segs[qs].append(kv)
         for rnd in plan.peer_rounds:
             for kind in ("contig", "paged"):
                 for e in rnd[kind]:

@@ -324,6 +324,8 @@ def _varlen_cut(q_lens: bytes, kv_lens: bytes, offsets: bytes | None, window: in
     ent["q_len"], ent["len"] = np.frombuffer(q_lens, np.int64), np.frombuffer(kv_lens, np.int64)
     if offsets is not None:
         ent["causal_offset"] = np.frombuffer(offsets, np.int64)
+    if ent["len"].max() < _MIN_SPLIT_KEYS:
+        return None
     ent["stride_tok"] = 1  # the real strides were checked with the tiles
     pieces, units = np.empty((2, _MAX_PIECES, 4), dtype=np.int32)
     nu, ns, pt = (ctypes.c_int32(0) for _ in range(3))
@@ -427,8 +429,6 @@ class VarlenLaunch:
         if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS or not self.num_tiles:
             return []
         ent = np.frombuffer(arr, dtype=ENTRY_DTYPE, count=self.num_entries)
-        if ent["len"].max() < _MIN_SPLIT_KEYS:
-            return []
         win = int(window or 0) if self.causal else 0
         cut = _varlen_cut(ent["q_len"].tobytes(), ent["len"].tobytes(),
                           ent["causal_offset"].tobytes() if self.causal else None, win,
