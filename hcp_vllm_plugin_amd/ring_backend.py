@@ -1169,7 +1169,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
                 ent, self.num_heads, self.num_kv_heads, self.head_size, query.device,
                 keep=block_table, entry_seq=st["seq"], num_seqs=len(seq_lens))
         elif kvs:
-            batch = batch.rebind_chunks(st["at"], words, (block_table, kvs))
+            batch = batch.rebind_chunks(words, (block_table, kvs))
         batch.run(query, out, None, self.scale, kv_base=pc.k_addr)
         _count("decode")
         return True

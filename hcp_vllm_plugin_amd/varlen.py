@@ -639,6 +639,7 @@ class DecodeBatch:
                 seq_of.append(s)
         self.num_seqs = len(segments)
         self.num_entries = len(entries)
+        self._contiguous = None
         n = max(self.num_entries, 1)
         arr = (VarlenEntry * n)(*entries)
         seq_arr = (ctypes.c_int32 * n)(*seq_of)
@@ -678,6 +679,7 @@ class DecodeBatch:
         arr = entries if n else np.zeros(1, dtype=ENTRY_DTYPE)
         self._plan(arr.ctypes.data, seq_arr.ctypes.data, arr["len"][:n].tolist(), num_heads,
                    num_kv_heads, head_dim, split_tokens, rows, device)
+        self._contiguous = entries["block_table"] == 0
         self._keep = keep
         return self
 
@@ -729,16 +731,19 @@ class DecodeBatch:
         a.workspace_bytes = self.ws_bytes
         a.num_heads, a.num_kv_heads, a.head_dim = num_heads, num_kv_heads, head_dim
 
-    def rebind_chunks(self, at: np.ndarray, rows: np.ndarray, keep=None) -> "DecodeBatch":
+    def rebind_chunks(self, rows: np.ndarray, keep=None) -> "DecodeBatch":
         """The same plan (splits, partial slots) over other chunks of the same
         lengths -- another layer's: row i of ``rows`` (uint64) is the K address,
-        V address, token and head stride of the contiguous entry at[i].  Only the
-        records go to the device (one small asynchronous copy)."""
+        V address, token and head stride of the plan's i-th contiguous entry.
+        Only the records go to the device (one small asynchronous copy)."""
+        if self._contiguous is None:
+            raise ValueError("rebind_chunks needs a plan made from an entry array")
         if self._chunk_rows is None:  # records of contiguous entries, and which of them
-            which = np.full(self.num_entries, -1, dtype=np.int64)
-            which[at] = np.arange(len(at))
-            rec = np.nonzero(which[self._work_entry] >= 0)[0]
+            which = np.cumsum(self._contiguous) - 1
+            rec = np.nonzero(self._contiguous[self._work_entry])[0]
             self._chunk_rows = (rec, which[self._work_entry[rec]])
+        if len(rows) != np.count_nonzero(self._contiguous):
+            raise ValueError("rebind_chunks needs one row per contiguous entry")
         rec, src = self._chunk_rows
         words = self._words.copy()
         words[rec[:, None], _CHUNK_WORDS] = rows[src]

@@ -120,3 +120,30 @@ def test_a_launchs_arguments_are_its_own(uploads):
     b = V.VarlenLaunch(e, False, False, CPU, heads=(28, 4, 128))
     a._split["ptrs"] = "a"
     assert b._split["ptrs"] != "a" and a._split is not b._split
+
+
+def test_rebound_chunks_follow_the_entries(uploads):
+    """Row i of a rebind goes to the records of the i-th contiguous entry and
+    to no other, whatever a rebind before it was given; one with another
+    number of rows is refused."""
+    ent = np.zeros(5, dtype=V.ENTRY_DTYPE)
+    ent["q_len"], ent["len"] = 1, [3000, 900, 5000, 64, 7000]
+    ent["block_table"], ent["k_addr"] = [4096, 0, 0, 8192, 0], [1, 2, 3, 4, 5]
+    seq = np.array([0, 0, 1, 2, 2], np.int32)
+    plan = V.DecodeBatch.from_entries(ent, 28, 4, 128, CPU, entry_seq=seq, num_seqs=3)
+    at0 = plan._args.works
+    for base in (100, 200):
+        rows = (np.arange(12, dtype=np.uint64) + base).reshape(3, 4)
+        got = plan.rebind_chunks(rows)
+        works = np.frombuffer(uploads[-1], V.WORK_DTYPE, plan.num_splits, got._args.works)
+        before = np.frombuffer(uploads[0], V.WORK_DTYPE, plan.num_splits, at0)
+        for w, old in zip(works, before):
+            at = {2: 0, 3: 1, 5: 2}.get(int(old["e"]["k_addr"]))
+            fields = [int(w["e"][f]) for f in ("k_addr", "v_addr", "stride_tok", "stride_head")]
+            assert fields == ([int(old["e"]["k_addr"]), 0, 0, 0] if at is None
+                              else rows[at].tolist())
+            assert w["key_begin"] == old["key_begin"] and w["next"] == old["next"]
+        plan = got  # a copy inherits what it memoised
+    for wrong in (rows[:2], np.zeros((4, 4), np.uint64)):
+        with pytest.raises(ValueError, match="one row per contiguous entry"):
+            plan.rebind_chunks(wrong)
