@@ -14,8 +14,11 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 import threading
+import time
+from typing import NamedTuple
 
 import torch  # noqa: F401  (must be loaded first: shares its HIP runtime)
 
@@ -54,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "hcp_plan_varlen_tiles",
     "hcp_attn_fwd_varlen",
     "hcp_attn_fwd_varlen_merge",
+    "hcp_split_limits",
     "hcp_plan_fwd_split",
     "hcp_attn_fwd_lse_split",
     "hcp_plan_varlen_split",
@@ -281,6 +285,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         _P, _I32, _P, _I32, _I32, _I32, _I32, _F, _I32, _I32, _I32,
         _P, _I64, _I64, _P, _I64, _I32, _I32, _P,
     ]
+    lib.hcp_split_limits.restype = ctypes.c_int
+    lib.hcp_split_limits.argtypes = [_I32, _P, _P, _P, _P]
     lib.hcp_plan_fwd_split.restype = ctypes.c_int
     lib.hcp_plan_fwd_split.argtypes = [_I64, _I64, _I32, _I32, _I32, _I32, _I64, _I32, _P, _P]
     lib.hcp_attn_fwd_lse_split.restype = ctypes.c_int
@@ -401,12 +407,46 @@ def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+class SplitLimits(NamedTuple):
+    """``hcp_split_limits`` (include/hcp_mi355x.h)."""
+
+    max_units: int
+    min_keys: int
+    max_pieces: int
+    max_workspace: int
+
+
+@functools.lru_cache(maxsize=None)  # one entry per head_dim
+def split_limits(head_dim: int) -> SplitLimits:
+    if not 0 < head_dim <= 256:  # refused by the launch: nothing to cut
+        return SplitLimits(0, 1 << 62, 0, 0)
+    n = [ctypes.c_int32(0) for _ in range(3)]
+    ws = ctypes.c_size_t(0)
+    check(lib().hcp_split_limits(head_dim, *(ctypes.addressof(x) for x in n),
+                                 ctypes.addressof(ws)), "hcp_split_limits")
+    return SplitLimits(*(x.value for x in n), ws.value)
+
+
+# per device: the last size there was no room for, and until when not to ask
+# for as much again (a failed allocation empties torch's cache and waits for
+# the device: not in every layer of every step)
+_no_room: dict = {}
+_NO_ROOM_S = 1.0
+
+
 def scratch(nbytes: int, device: torch.device) -> torch.Tensor | None:
     """Stream-ordered scratch from torch's caching allocator for a launch that
     has another form without it; None when the device has no room for it."""
+    held = _no_room.get(device.index)
+    if held is not None:
+        if time.monotonic() >= held[1]:
+            _no_room.pop(device.index, None)
+        elif nbytes >= held[0]:
+            return None
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
     except torch.OutOfMemoryError:
+        _no_room[device.index] = (nbytes, time.monotonic() + _NO_ROOM_S)
         return None
 
 

@@ -96,8 +96,8 @@ void set_acc(hcp::FwdParams& p, const AccArgs* a) {
 
 // ---- KV split of a prefill launch ------------------------------------------
 constexpr int kNumCus = 256;
-// (query block, head, piece) workgroups of a split launch: 135 MB of partials at
-// head_dim 128
+// (query block, head, piece) workgroups of a split launch, and the slots of its
+// workspace: 135 MB of partials at head_dim 128 (hcp_split_limits)
 constexpr int kMaxPieces = 2048;
 constexpr int kMaxUnits = 4 * kNumCus;  // (query block, head) pairs of a launch worth cutting
 constexpr int kMinPieceTiles = 4;   // a shorter piece is mostly prologue and epilogue
@@ -126,14 +126,15 @@ struct Cut {
 // 47, 55 / 48, 48, 56; 3001 x 5003 at 14 / 2 x 64 whole 93 / 91, cut in 3: 82 /
 // 77, cut in 3 past 18 whole blocks 74 / 75; 600 x 6000 at 16 / 8 x 256 whole
 // 168 / 170, cut in 3: 82 / 79.
+// `padded`: every cut block has as many slots in the workspace as the longest.
 double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh, int dw,
-                  double limit, bool* hopeless = nullptr) {
+                  bool padded, double limit, bool* hopeless = nullptr) {
   const double tile_us = dw == 64 ? 0.54 : dw == 128 ? 0.97 : 1.75;
   const double first_us = dw == 256 ? 5.0 : 3.0;   // start and end of a first workgroup
   const double start_us = dw == 256 ? 5.0 : 1.0;   // of one that follows
   const double part_us = dw == 64 ? 0.006 : dw == 128 ? 0.012 : 0.04;  // per partial
   const double reduce_us = dw == 256 ? 8.0 : 6.0;  // the second launch
-  const int slots = dw == 256 ? 1 : 2;
+  const int per_cu = dw == 256 ? 1 : 2;
   // by waves with rows: work of a tile relative to a full one, and the time of
   // a workgroup alone on its CU relative to its work
   static constexpr double kWork[5] = {0.5, 0.5, 0.65, 0.85, 1.0};
@@ -151,12 +152,14 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
     double work, alone;
   };
   std::vector<Job> jobs;  // workgroups of one head
-  int64_t n = 0, parts = 0;
+  int64_t n = 0, parts = 0, most = 1;
   for (size_t u = 0; u < units.size(); ++u) {
     n += pieces(u);
     if (pieces(u) > 1) parts += pieces(u);
+    most = std::max<int64_t>(most, pieces(u));
   }
-  if (c.tiles > 0 && n * group * num_kvh > kMaxPieces) return 1e30;
+  const int64_t slots = padded ? (static_cast<int64_t>(units.size()) - c.whole) * most : parts;
+  if (c.tiles > 0 && std::max(n, slots) * group * num_kvh > kMaxPieces) return 1e30;
   const double busy = std::min(1.0, static_cast<double>(n * per) / (cus * share));
   const double full_alone = 1.0 + 0.3 * std::max(0.0, busy - 0.5);
   const double merge_us =
@@ -164,7 +167,7 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
   double sum = 0;
   for (size_t u = 0; u < units.size(); ++u) {
     const int nt = units[u].tiles, np = pieces(u), w = units[u].waves;
-    const double alone = slots == 1 ? 1.0 : w == 4 ? full_alone : kAlone[w];
+    const double alone = per_cu == 1 ? 1.0 : w == 4 ? full_alone : kAlone[w];
     for (int i = 0; i < np; ++i) {
       const int tiles = hcp::piece_begin(nt, np, i + 1) - hcp::piece_begin(nt, np, i);
       jobs.push_back({tiles * tile_us * kWork[w], alone});
@@ -194,7 +197,7 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
     x.job[x.n++].work += extra;
     j += share;
   };
-  for (int s = 0; s < slots; ++s)
+  for (int s = 0; s < per_cu; ++s)
     for (Cu& x : cu)
       if (j < items) give(x, first_us);
   typedef std::pair<double, int> Ev;  // (end of a CU's next job, CU), earliest on top
@@ -220,7 +223,7 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
       x.n = m;
     }
     x.at = end;
-    while (x.n < slots && j < items) give(x, start_us);
+    while (x.n < per_cu && j < items) give(x, start_us);
     if (x.n == 0) {
       heap.pop_back();
     } else {
@@ -233,7 +236,7 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
 
 // The cut of a launch over `units`, longest first; tiles 0 when cutting does
 // not pay (8% or more by the estimate, whose error is about that).
-Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw) {
+Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw, bool padded) {
   Cut best;
   const int heads = group * num_kvh;
   // past 4 workgroups per CU the dispatch order alone evens the load out to
@@ -241,10 +244,10 @@ Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw) {
   if (units.empty() || static_cast<int64_t>(units.size()) * heads > kMaxUnits) return best;
   const int mx = units[0].tiles;
   if (mx < 2 * kMinPieceTiles) return best;
-  double t_best = split_cost(units, best, group, num_kvh, dw, 1e30) * 0.92;
+  double t_best = split_cost(units, best, group, num_kvh, dw, padded, 1e30) * 0.92;
   // whole blocks spread evenly as they are: no cut can win
   bool none = false;
-  split_cost(units, best, group, num_kvh, dw, t_best, &none);
+  split_cost(units, best, group, num_kvh, dw, padded, t_best, &none);
   if (none) return best;
   for (int rounds = 0; rounds < 4; ++rounds) {
     // rounds > 0: only what is left after `rounds` whole blocks per CU
@@ -258,7 +261,7 @@ Cut choose_cut(const std::vector<Unit>& units, int group, int num_kvh, int dw) {
       if (tiles == c.tiles) continue;
       c.tiles = tiles;
       bool hopeless = false;
-      const double t = split_cost(units, c, group, num_kvh, dw, t_best, &hopeless);
+      const double t = split_cost(units, c, group, num_kvh, dw, padded, t_best, &hopeless);
       // more pieces only add to the even share: none of them can win either
       if (hopeless || t > 1e29) break;
       if (t < t_best) {
@@ -399,6 +402,17 @@ static int fwd_lse_impl(const char* who, const void* q, const void* k, const voi
   return launch_status(e, who);
 }
 
+int hcp_split_limits(int32_t head_dim, int32_t* max_units, int32_t* min_keys, int32_t* max_pieces,
+                     size_t* max_workspace) {
+  if (head_dim <= 0 || head_dim > 256 || !max_units || !min_keys || !max_pieces || !max_workspace)
+    return fail(HCP_EINVAL, "hcp_split_limits: bad arguments");
+  *max_units = kMaxUnits;
+  *min_keys = (2 * kMinPieceTiles - 1) * hcp::kFwdBN + 1;  // a block of two pieces
+  *max_pieces = kMaxPieces;
+  *max_workspace = split_ws_bytes(kMaxPieces, 1, head_dim);
+  return HCP_OK;
+}
+
 int hcp_plan_fwd_split(int64_t tq, int64_t tk, int32_t num_heads, int32_t num_kv_heads,
                        int32_t head_dim, int32_t causal, int64_t causal_offset, int32_t window,
                        int32_t* whole_blocks, size_t* workspace_bytes) try {
@@ -422,7 +436,7 @@ int hcp_plan_fwd_split(int64_t tq, int64_t tk, int32_t num_heads, int32_t num_kv
     units.push_back({unit_tiles(e, qb, causal != 0, causal ? window : 0), unit_waves(e, qb)});
   }
   const Cut c = choose_cut(units, num_heads / num_kv_heads, num_kv_heads,
-                           hcp::padded_head_dim(head_dim));
+                           hcp::padded_head_dim(head_dim), true);
   if (c.tiles > 0) {
     int mp = 1;
     for (size_t t = c.whole; t < units.size(); ++t)
@@ -592,7 +606,7 @@ int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries, 
   std::vector<Unit> units;
   for (const U& b : blocks) units.push_back(b.u);
   const Cut c = choose_cut(units, num_heads / num_kv_heads, num_kv_heads,
-                           hcp::padded_head_dim(head_dim));
+                           hcp::padded_head_dim(head_dim), false);
   if (c.tiles == 0) return 0;
   struct P {
     int32_t cost, e, qb, piece, slot;

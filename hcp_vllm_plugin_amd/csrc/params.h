@@ -129,7 +129,7 @@ struct RedParams {
   int64_t acc_lse_stride_head;
 };
 
-constexpr int kDecMaxSeqs = 1024;  // sequences of a launch that partitions itself
+constexpr int kDecMaxSeqs = HCP_DECODE_PAGED_MAX_SEQS;  // sequences of a launch that partitions itself
 
 // A pure decode batch over a paged cache, read straight from the step's
 // metadata: every workgroup works out its own share of the keys.

@@ -85,12 +85,6 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if ok else _copied(t)
 
 
-# hcp_plan_fwd_split never cuts a launch of more (query block, head) pairs than
-# this, or of fewer keys: those calls are not worth asking about
-_MAX_SPLIT_UNITS = 1024
-_MIN_SPLIT_KEYS = 449
-
-
 @functools.lru_cache(maxsize=1024)
 def _split_plan(tq, tk, num_heads, num_kv_heads, head_dim, causal, off, win):
     """(piece_tiles, whole_blocks, workspace bytes) of a launch's KV split. It
@@ -127,7 +121,8 @@ def _launch(name, q, k, v, out, lse, scale, causal_offset, window, acc, acc_is_p
         )
         a = () if acc is None else (acc[0].data_ptr(), acc[0].stride(0), acc[0].stride(1),
                                     acc[1].data_ptr(), acc[1].stride(0), int(bool(acc_is_prefix)))
-        if tk >= _MIN_SPLIT_KEYS and -(-tq // 128) * num_heads <= _MAX_SPLIT_UNITS:
+        lim = _lib.split_limits(head_dim)
+        if tk >= lim.min_keys and -(-tq // 128) * num_heads <= lim.max_units:
             pt, whole, nbytes = _split_plan(tq, tk, num_heads, num_kv_heads, head_dim, causal,
                                             off, win)
             # fp32 partials; without room for them the launch stays whole

@@ -306,11 +306,6 @@ def plan_varlen_tiles(entries: list[VarlenEntry], causal: bool) -> list[tuple[in
 # smallest block_size the paged prefill kernel reads in place (a wave's 16
 # rows of a tile must lie in one block); smaller ones are gathered first
 _MIN_PAGED_BLOCK = 16
-# hcp_plan_varlen_split: (query block, head) pairs past which it never cuts a
-# launch, and the most records it writes
-_MAX_SPLIT_UNITS = 1024
-_MIN_SPLIT_KEYS = 449  # nor one of shorter key ranges
-_MAX_PIECES = 2048
 
 
 @functools.lru_cache(maxsize=64)
@@ -324,15 +319,16 @@ def _varlen_cut(q_lens: bytes, kv_lens: bytes, offsets: bytes | None, window: in
     ent["q_len"], ent["len"] = np.frombuffer(q_lens, np.int64), np.frombuffer(kv_lens, np.int64)
     if offsets is not None:
         ent["causal_offset"] = np.frombuffer(offsets, np.int64)
-    if ent["len"].max() < _MIN_SPLIT_KEYS:
+    lim = _lib.split_limits(heads[2])
+    if ent["len"].max() < lim.min_keys:
         return None
     ent["stride_tok"] = 1  # the real strides were checked with the tiles
-    pieces, units = np.empty((2, _MAX_PIECES, 4), dtype=np.int32)
+    pieces, units = np.empty((2, lim.max_pieces, 4), dtype=np.int32)
     nu, ns, pt = (ctypes.c_int32(0) for _ in range(3))
     nbytes = ctypes.c_size_t(0)
     rc = _lib.lib().hcp_plan_varlen_split(
         ent.ctypes.data, n, int(offsets is not None), window, *heads, pieces.ctypes.data,
-        _MAX_PIECES, units.ctypes.data, ctypes.addressof(nu), ctypes.addressof(ns),
+        lim.max_pieces, units.ctypes.data, ctypes.addressof(nu), ctypes.addressof(ns),
         ctypes.addressof(pt), ctypes.addressof(nbytes))
     _lib.check(rc, "hcp_plan_varlen_split")
     if rc == 0:
@@ -426,7 +422,8 @@ class VarlenLaunch:
         """The KV split of runs with these heads and window: records to upload
         ([pieces, units]), or [] for the uncut launch."""
         self._split = None
-        if heads is None or self.num_tiles * heads[0] > _MAX_SPLIT_UNITS or not self.num_tiles:
+        if heads is None or not self.num_tiles or \
+                self.num_tiles * heads[0] > _lib.split_limits(heads[2]).max_units:
             return []
         ent = np.frombuffer(arr, dtype=ENTRY_DTYPE, count=self.num_entries)
         win = int(window or 0) if self.causal else 0

@@ -255,6 +255,15 @@ int hcp_plan_fwd_split(int64_t tq, int64_t tk, int32_t num_heads,
                        int64_t causal_offset, int32_t window,
                        int32_t* whole_blocks, size_t* workspace_bytes);
 
+/*
+ * What the two split planners keep to: no cut of a launch of more than
+ * max_units (128-row query block, head) pairs, nor of one whose entries all
+ * have fewer than min_keys keys (not worth asking about); at most max_pieces
+ * records from hcp_plan_varlen_split, and max_workspace bytes from either.
+ */
+int hcp_split_limits(int32_t head_dim, int32_t* max_units, int32_t* min_keys,
+                     int32_t* max_pieces, size_t* max_workspace);
+
 /* hcp_attn_fwd_lse (acc_out and acc_lse NULL) or hcp_attn_fwd_lse_merge on a
  * KV split of piece_tiles > 0 tiles.  Any piece_tiles is correct; the
  * workspace must hold (ceil(tq / 128) - whole_blocks) * (pieces of the longest
@@ -281,7 +290,7 @@ int hcp_attn_fwd_lse_split(const void* q, const void* k, const void* v, void* ou
  * block of one piece, written directly), and up to cap (entry, q_block, first
  * slot, pieces) records of the split blocks to `units_out`; returns the number
  * of pieces, or 0 when the batch is best left whole (then use
- * hcp_plan_varlen_tiles).  A cap of 2048 always suffices.  Checks entries as
+ * hcp_plan_varlen_tiles).  hcp_split_limits' max_pieces is cap enough.  Checks entries as
  * hcp_plan_varlen_tiles does.  Runs on the CPU only.
  */
 int hcp_plan_varlen_split(const hcp_varlen_entry* entries, int32_t num_entries,
