@@ -139,6 +139,7 @@ double split_cost(const std::vector<Unit>& units, Cut c, int group, int num_kvh,
   // a workgroup alone on its CU relative to its work
   static constexpr double kWork[5] = {0.5, 0.5, 0.65, 0.85, 1.0};
   static constexpr double kAlone[5] = {1.8, 1.8, 1.55, 1.3, 1.15};
+  static_assert(HCP_FWD_WAVES == 4, "measured with four waves to a workgroup");
   // one XCD's share of the workgroups (xcd_remap), or the whole machine
   const bool by_xcd = num_kvh <= hcp::kNumXcd && hcp::kNumXcd % num_kvh == 0;
   const int share = by_xcd ? hcp::kNumXcd / num_kvh : 1;
@@ -836,8 +837,9 @@ int hcp_plan_decode_lists(const hcp_varlen_entry* entries, int32_t num_entries,
   constexpr int64_t kSplitCost = 8;
   const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups, (total + 1) / 2));
   // Chunks of an entry with `left` to go that a workgroup with `room` takes:
-  // none if it would only fit a fragment, the rest if no more than a
-  // fragment would stay, else whole steps of 4 (one for each of the 4 waves).
+  // the rest if there is room for it, else whole steps of 4 (one for each of
+  // the 4 waves; single chunks in a small share), but none if the room, less
+  // the split's own cost, is under 2.
   auto take = [&](int64_t left, int64_t room) -> int64_t {
     room -= kSplitCost;
     if (left <= room) return left;

@@ -991,6 +991,7 @@ fa_fwd_kernel(FwdParams p) {
 template <int D, typename T, bool CAUSAL, bool VARLEN>
 __global__ __launch_bounds__(256) void fwd_reduce_kernel(FwdParams p) {
   using E = Elem<T>;
+  static_assert(HCP_FWD_WAVES == 4, "four workgroups to a query block of four waves' rows");
   constexpr int NC = D / 8;  // 64-lane x 16-byte chunks of a wave's 32 rows
   constexpr int CW = NC / 4; // chunks per wave of this kernel
   const int lane = threadIdx.x & 63, cw = threadIdx.x >> 6;

@@ -93,3 +93,22 @@ def test_profiling_run_has_the_partials(monkeypatch):
     assert asked == [(_lib.split_limits(80).max_workspace, "gpu")]
     cpu = torch.ones(2, 2)
     assert impl.forward(None, None, None, None, None, None, cpu).sum() == 0 and len(asked) == 1
+
+
+# (query rows, keys) of a launch of one request: pieces, at least
+@pytest.mark.parametrize("heads,causal,window,new,keys,least", [
+    ((28, 4, 128), 1, 0, 512, 32768, 4 * 4), ((28, 4, 128), 0, 0, 512, 32768, 4 * 4),
+    ((14, 2, 64), 1, 0, 512, 32768, 4 * 4), ((16, 8, 256), 1, 0, 512, 32768, 4 * 2),
+    ((12, 3, 128), 0, 0, 16, 4099, 2), ((28, 4, 128), 1, 0, 16, 4099, 2),
+    ((28, 4, 128), 1, 700, 16, 4099, 1),  # the window's 12 tiles: whole
+])
+def test_varlen_launches_that_are_cut(heads, causal, window, new, keys, least):
+    from tests.test_split_plan import _entries, _plan as plan_varlen
+
+    pieces, units, slots, _, nbytes = plan_varlen(_entries([(0, new, keys)], causal), causal,
+                                                  window, heads)
+    if least == 1:
+        assert len(pieces) == 0 and nbytes == 0
+        return
+    assert len(pieces) >= least and len(units) >= 1 and slots >= 2
+    assert 0 < nbytes <= _lib.split_limits(heads[2]).max_workspace
