@@ -1,5 +1,5 @@
 """GPU parity: an attention pass and the LSE merge after it in one launch
-(hcp_attn_fwd_lse_merge via ring_attn_merged, hcp_attn_fwd_varlen_merge via
+(hcp_attn_fwd_lse_merge via ring_attn_merged, hcp_varlen_launch with acc_o via
 VarlenLaunch.run(acc=...)).
 
 The fused result must equal the two-step path -- ring_attn_with_lse /

@@ -1,4 +1,4 @@
-"""GPU parity: split-KV decode (hcp_decode_splitkv) against the oracle.
+"""GPU parity: split-KV decode (hcp_decode_launch) against the oracle.
 
 Each sequence has one query token, a contiguous peer segment and a paged
 local segment (all keys visible, ring_backend.py:663-679 / :820-830 with
@@ -147,7 +147,7 @@ def test_decode_empty_sequence(dev):
 
 
 # ---------------------------------------------------------------------------
-# hcp_decode_splitkv_acc: the decode merged into a running accumulator
+# hcp_decode_launch with acc_o: the decode merged into a running accumulator
 # ---------------------------------------------------------------------------
 def _acc_case(dev, dtype, seg_lens, split, seed, in_place=False, acc_lse_fill=None):
     h, hkv, d = 28, 4, 128

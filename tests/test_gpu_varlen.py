@@ -1,4 +1,4 @@
-"""GPU parity: batched varlen prefill (hcp_attn_fwd_varlen) with the local
+"""GPU parity: batched varlen prefill (hcp_varlen_launch) with the local
 segment read in place from the paged cache, the peer segment from packed
 contiguous KV, and one merge -- against the oracle's per-request
 gather + attention + merge (ring_backend.py:611-832).

@@ -1,13 +1,13 @@
-"""GPU parity of the allocation-free decode entry point.
+"""GPU parity of the allocation-free decode.
 
-``hcp_decode_splitkv_noalloc`` runs the split-KV decode with its fp32 split
-partials in the library's fixed per-GPU scratch instead of a caller
-workspace.  Its output and LSE must equal ``hcp_decode_splitkv``'s on the same
-plan bit for bit (same kernels, same arithmetic), on two calls in a row, the
-second with a smaller batch (the scratch keeps the first call's partials);
-and a plan whose partials exceed the scratch is refused on the host before
-anything is launched.  Both entry points are called through the C ABI
-(``DecodeBatch.run`` binds them with ctypes).
+``DecodeBatch.run(noalloc=True)`` (``hcp_decode_launch`` with ``use_scratch``)
+runs the split-KV decode with its fp32 split partials in the library's fixed
+per-GPU scratch instead of a caller workspace.  Its output and LSE must equal
+the workspace form's on the same plan bit for bit (same kernels, same
+arithmetic), on two calls in a row, the second with a smaller batch (the
+scratch keeps the first call's partials); and a plan whose partials exceed the
+scratch is refused on the host before anything is launched.  (The C entry
+``hcp_decode_splitkv_noalloc`` itself is called by test_gpu_c_entries.py.)
 """
 
 import pytest
