@@ -1193,7 +1193,6 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         n = len(seq_lens)
         if n == 0:
             return
-        w = self.sliding_window
         stream = _lib.stream_ptr(query.device)
         if qsl == list(range(n + 1)):
             lens = step.lens_on(stream, query.device, lens_t)

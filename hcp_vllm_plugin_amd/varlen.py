@@ -30,7 +30,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import DecodeSplit, KvSegment, VarlenEntry
+from ._lib import KvSegment, VarlenEntry
 
 __all__ = [
     "PagedCache",
@@ -41,7 +41,6 @@ __all__ = [
     "DecodeBatch",
     "PagedDecode",
     "decode_attn",
-    "choose_split_tokens",
     "head_major",
 ]
 
@@ -569,49 +568,11 @@ def head_chunks(num_heads: int, num_kv_heads: int) -> int:
     return -(-(num_heads // num_kv_heads) // 16)
 
 
-def choose_split_tokens(seg_lens: list[int], num_kv_heads: int, num_cus: int = 256,
-                        max_rounds: int = 4, round_keys: int = 2048, minimum: int = 64,
-                        maximum: int = 16384) -> int:
-    """A split size for callers that pass ``split_tokens`` (one workgroup per
-    split), from the batch's key counts.
-
-    The split kernel runs one workgroup per CU at a time (its chunk buffers
-    take 128 KB of LDS), so the launch is planned in whole rounds of
-    ``num_cus`` (split, KV head) workgroups: one round while the work is
-    small (a single long request -- a decode-ring hop -- spread over the whole
-    machine), up to ``max_rounds`` once each workgroup would stream more than
-    ``round_keys`` keys, so the launch drains evenly while each split stays
-    long enough that its fp32 partial is small next to the K/V it summarises.
-    Several rounds: rounded up to 64 keys.  One round: the smallest split
-    whose pieces fill at most one workgroup per CU.
-    """
-    total = sum(seg_lens) * num_kv_heads
-    if total == 0:
-        return minimum
-    rounds = min(max_rounds, max(1, -(-total // (num_cus * round_keys))))
-    s = -(-total // (rounds * num_cus))
-    if rounds == 1:
-        # one round: the smallest split whose pieces (every segment cut into
-        # ceil(len / s) of them) fit the machine, so a single long request
-        # occupies every CU
-        lens = [n for n in seg_lens if n > 0]
-        lo, hi = max(minimum, s), max(max(lens), minimum)
-        while lo < hi:
-            mid = (lo + hi) // 2
-            if sum(-(-n // mid) for n in lens) * num_kv_heads <= num_cus:
-                hi = mid
-            else:
-                lo = mid + 1
-        return min(maximum, lo)
-    s = ((s + 63) // 64) * 64
-    return max(minimum, min(maximum, s))
-
-
 def decode_workgroups(heads: int, num_cus: int = 256) -> int:
     """Workgroups of a decode launch per KV head and head chunk (``heads`` of
-    them).  The split kernel runs one
-    workgroup per CU (128 KB of LDS); its workgroups all get the same number
-    of keys, so one round of the machine drains evenly."""
+    them).  The split kernel runs one workgroup per CU (128 KB of LDS); its
+    workgroups all get the same number of keys, so one round of the machine
+    drains evenly."""
     return max(1, num_cus // heads)
 
 
