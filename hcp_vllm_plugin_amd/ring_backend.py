@@ -1336,9 +1336,8 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
     def _forward_prefill(self, query, out, plan: _Plan, step, pc) -> None:
         dev = query.device
         h = self.num_heads
-        local = self._local_launch(query, plan, step, pc)
         if not plan.any_peer:
-            self._run_chunks(local, query, out, step.bt, pc)
+            self._run_chunks(self._local_launch(query, plan, step, pc), query, out, step.bt, pc)
             _count("attn")
             return
         o_peer = lse_peer = None
@@ -1364,7 +1363,9 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # = peer, suffix = local (ring_backend.py:354,820-831), bit for bit.
         # The local entries cover every query row of the plan; rows without a
         # peer have lse_peer = -inf and get the local result.
-        self._run_chunks(local, query, out, step.bt, pc, acc=(o_peer, lse_peer))
+        # (planned, in a step's first layer, while the peer launches run)
+        self._run_chunks(self._local_launch(query, plan, step, pc), query, out, step.bt, pc,
+                         acc=(o_peer, lse_peer))
         _count("attn")
         _count("merge")
 
