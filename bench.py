@@ -191,7 +191,7 @@ def bench_decode(dev, steps, warmup):
         "ms": ms,
         "bytes": total,
         "gbs": total / (ms * 1e-3) / 1e9,
-        "split_tokens": batch.split_tokens,
+        "keys_per_workgroup": batch.split_tokens,
         "splits": batch.num_splits,
         "seqs": seqs,
         "peer_len": peer_len,
@@ -1115,7 +1115,7 @@ def main():
             "unit": "GB/s",
             "bytes": dec["bytes"],
             "frac_hbm": round(dec["gbs"] / PEAK_HBM_GBS, 4),
-            "split_tokens": dec["split_tokens"],
+            "keys_per_workgroup": dec["keys_per_workgroup"],
             "splits": dec["splits"],
             "roofline": {
                 "bound": "hbm",
