@@ -833,20 +833,22 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         a CU per 64 keys and head at 64, 128 or 256 columns.  The decode launch
         reads the keys once, but is two more kernels; where a plan is made once
         per step it pays past 20 us of the machine, where each layer makes its
-        own (``each_layer``: staged or split peers) only past 150 us.
+        own (``each_layer``: staged or split peers) past 60 us and 6 us a row.
 
         256 new tokens next to the rows, us per layer in one launch / apart:
-        28 / 4 x 128, 16 x 1536 keys (20 us by this count) 73 / 80, 8 x 4096 (27)
-        88 / 80, 32 x 4096 (109) 224 / 97; 14 / 2 x 64, 32 x 4096 (30) 100 / 80;
-        16 / 8 x 256, 2 x 8192 (14) 100 / 91; with 1024 staged keys each, 28 / 4 x
-        128, 8 x 4096 (34) 213 / 244, 32 x 4096 (136) 493 / 503."""
+        28 / 4 x 128, 16 x 1536 keys (20 us by this count) 73 / 79, 8 x 4096 (27)
+        87 / 79, 32 x 4096 (109) 224 / 96; 14 / 2 x 64, 32 x 4096 (30) 99 / 79;
+        16 / 8 x 256, 2 x 8192 (14) 98 / 90.  With 1024 staged keys each, 28 / 4 x
+        128, 2 x 24576 (42) 145 / 164, 2 x 49152 (83) 201 / 171; 8 x 12000 (86) 221 /
+        240, 8 x 16384 (115) 268 / 249; 32 x 8192 (244) 497 / 503, 32 x 16384 (462)
+        849 / 519."""
         w = self.sliding_window
         keys = [tk if w is None else min(tk, w)
                 for r, tk in enumerate(seq_lens) if qsl[r + 1] - qsl[r] == 1]
         tile_us = {64: 0.27, 128: 0.49, 256: 0.88}[
             next(c for c in (64, 128, 256) if self.head_size <= c)]
         est = sum(-(-tk // 64) for tk in keys) * self.num_heads * tile_us / 256
-        return est > (150 if each_layer else 20)
+        return est > (60 + 6 * len(keys) if each_layer else 20)
 
     def _plan(self, layer_name, qsl, seq_lens, block_table, first_blocks, pc, split):
         plan = _Plan()

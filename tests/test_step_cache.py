@@ -91,7 +91,10 @@ def test_another_threads_step_leaves_a_layers_plans_alone(monkeypatch):
     (14, 64, [4096] * 32, None, False, True),
     (16, 256, [4096] * 8, None, False, True),
     (28, 128, [5120] * 32, None, True, False),   # a plan in every layer costs more
-    (28, 128, [34000] * 32, None, True, True),
+    (28, 128, [9216] * 32, None, True, False),
+    (28, 128, [17408] * 32, None, True, True),
+    (28, 128, [25600] * 2, None, True, False),
+    (28, 128, [50176] * 2, None, True, True),
     (28, 128, [], None, False, False),
 ])
 def test_rows_that_leave_the_prefill_launch(heads, d, rows, window, each_layer, apart):
