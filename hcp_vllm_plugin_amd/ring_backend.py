@@ -414,6 +414,9 @@ def _step(attn_metadata, queue=None) -> _Step:
     lens = owner = None
     if _fetchable(qsl_t, n + 1) and _fetchable(sl_t, n) and block_table.is_cuda \
             and block_table.shape[0] >= n:  # (the copy reads a first block per request)
+        # (the lengths of this thread's step before are written over: its record
+        # goes first, in case this one fails)
+        _STEP.update(step=None, fast={})
         host, lens, owner = _fetch_metadata(qsl_t, sl_t, block_table, n, queue)
     else:
         fb = block_table[:, 0] if block_table.shape[1] > 0 else sl_t.new_zeros(n)
@@ -926,7 +929,7 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         if output_scale is not None or output_block_scale is not None:
             raise NotImplementedError("fused output quant not supported")
         if attn_metadata is None:  # profiling run
-            if output.is_cuda:
+            if output.is_cuda and not _capturing():
                 # the partials of a cut launch, so that the engine's peak has them
                 _lib.scratch(_lib.split_limits(self.head_size).max_workspace, output.device)
             return output.fill_(0)
@@ -1196,9 +1199,10 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         if n == 0:
             return
         stream = _lib.stream_ptr(query.device)
+        lens = step.lens_on(stream, query.device, lens_t)
+        on = (stream, 0 if lens is None else lens.data_ptr())
         if qsl == list(range(n + 1)):
-            lens = step.lens_on(stream, query.device, lens_t)
-            key = (*self._layout_key("paged", pc), stream, lens is lens_t)
+            key = (*self._layout_key("paged", pc), on)
             dec = fast.get(key)
             if dec is None:
                 dec = fast[key] = self._plan_paged(seq_lens, block_table, pc, lens, ahead)
@@ -1211,10 +1215,9 @@ class HcpRingAttentionImpl(_ImplBase):  # type: ignore[misc,valid-type]
         # The single-token rows first: they seldom need a plan, and the
         # prefill's is made while they run.  In the prefill launch a NaN score
         # makes its row NaN (a decode batch leaves the split out): here too.
-        key = (*self._layout_key("rows", pc), stream)
+        key = (*self._layout_key("rows", pc), on)
         dec = fast.get(key, fast)  # (fast itself: not planned yet)
         if dec is fast:
-            lens = step.lens_on(stream, query.device, lens_t)
             dec = fast[key] = self._plan_rows(query, qsl, seq_lens, block_table, pc, lens)
         _check_base(pc)
         if dec is not None:

@@ -98,3 +98,23 @@ def test_queued_ahead_writes_only_a_decode_batch(dev):
             impl.forward(LAYER, qd, None, None, cached, _meta(dev, [0, 1, 2, 3], bad, bt), out)
         torch.cuda.synchronize()
         assert (out == 7).all()
+
+
+def test_a_step_that_failed_leaves_no_lengths_behind(dev):
+    """A step refused while its first layer was being queued has written its
+    lengths; the step before it, still the caller's, runs on its own."""
+    lens, other = [900, 17, 2500], [5, 3, 7]
+    q, cache, bt = _batch(1, lens, H, HKV, D, torch.bfloat16, "v031", 16)
+    qd, cached = q.to(dev), cache.to(dev)
+    impl = rb.HcpRingAttentionImpl(H, D, scale_for(D), HKV)
+    meta = _meta(dev, [0, 1, 2, 3], lens, bt)
+    first, second = torch.empty_like(qd), torch.empty_like(qd)
+    impl.forward(LAYER, qd, None, None, cached, meta, first)
+    odd = torch.zeros(cached.numel() + 1, dtype=qd.dtype, device=dev)[1:].view(cached.shape)
+    with pytest.raises(ValueError, match="16-byte aligned"):
+        impl.forward(LAYER, qd, None, None, odd, _meta(dev, [0, 1, 2, 3], other, bt), second)
+    impl.forward(LAYER, qd, None, None, cached, meta, second)
+    torch.cuda.synchronize()
+    assert torch.equal(first, second)
+    ref = _reference(q, cache, bt, lens, "v031", scale_for(D), 0)
+    assert max_err(second, ref) <= OUT_TOL[torch.bfloat16]

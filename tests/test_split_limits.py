@@ -87,10 +87,14 @@ def test_no_room_is_remembered_for_a_while(monkeypatch):
 def test_profiling_run_has_the_partials(monkeypatch):
     asked = []
     monkeypatch.setattr(_lib, "scratch", lambda n, device: asked.append((n, device)))
+    capturing = [False]
+    monkeypatch.setattr(rb, "_capturing", lambda: capturing[0])
     out = types.SimpleNamespace(is_cuda=True, device="gpu", fill_=lambda v: ("filled", v))
     impl = rb.HcpRingAttentionImpl(28, 80, 0.1, 4)
     assert impl.forward(None, None, None, None, None, None, out) == ("filled", 0)
     assert asked == [(_lib.split_limits(80).max_workspace, "gpu")]
+    capturing[0] = True  # not into a graph's pool
+    assert impl.forward(None, None, None, None, None, None, out) == ("filled", 0)
     cpu = torch.ones(2, 2)
     assert impl.forward(None, None, None, None, None, None, cpu).sum() == 0 and len(asked) == 1
 

@@ -107,3 +107,31 @@ def test_rows_that_leave_the_prefill_launch(heads, d, rows, window, each_layer, 
     qsl.append(qsl[-1] + 300)
     lens.append(60000)
     assert impl._decode_rows_apart(qsl, lens, *([True] if each_layer else [])) == apart
+
+
+def test_whose_lengths_a_launch_reads(monkeypatch):
+    """The step's own on the thread and stream that wrote them; anywhere else a
+    copy of the host's, one for each stream; the caller's under capture."""
+    import threading
+
+    words = torch.zeros(4, dtype=torch.int64)
+    step = rb._Step(None, None, ([0, 1, 2], [70, 80], [0, 1]), None, words[2:],
+                    (threading.get_ident(), 5))
+    given = torch.ones(2, dtype=torch.int32)
+    capturing = [False]
+    monkeypatch.setattr(rb, "_capturing", lambda: capturing[0])
+    monkeypatch.setattr(rb, "_upload", lambda arrays, device: (
+        torch.from_numpy(np.concatenate([a.view(np.uint8) for a in arrays])), [0]))
+    assert step.lens_on(5, None, given) is step.lens
+    other = step.lens_on(6, None, given)
+    assert other.tolist() == [70, 80] and step.lens_on(6, None, given) is other
+    seen = []
+    t = threading.Thread(target=lambda: seen.append(step.lens_on(5, None, given)))
+    t.start()
+    t.join()
+    assert seen[0].tolist() == [70, 80] and seen[0].data_ptr() != step.lens.data_ptr()
+    capturing[0] = True
+    assert step.lens_on(5, None, given) is given
+    capturing[0] = False
+    step.lens = None  # metadata that came another way: nothing runs unplanned
+    assert step.lens_on(5, None, given) is None
