@@ -50,7 +50,10 @@ struct DecShared {
   static constexpr int W = D == 256 ? 2 : 4;     // waves per workgroup
 };
 
-template <int D, typename T, bool PAGED>
+// KEEP_NAN: scores that hold a NaN make their row NaN, as in the prefill
+// kernels; without it their split is left out.  (A parameter read where the
+// partial is stored costs every split 0.1 to 0.3 us.)
+template <int D, typename T, bool PAGED, bool KEEP_NAN>
 __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in, int chunk_in,
                                                   int sp, const hcp_varlen_entry& e,
                                                   int64_t kb, int64_t ke,
@@ -431,12 +434,9 @@ __device__ __forceinline__ void decode_split_body(const DecParams& p, int kvh_in
     }
     const int head = h0 + h;
     const int64_t slot = static_cast<int64_t>(sp) * p.num_heads + head;
-    // a sum that is NaN counts as a split without keys unless the caller wants
-    // the NaN in the row
-    const float none = p.keep_nan && L != L ? L : 0.f;
-    global_ptr(p.ws_o)[slot * D + d] = L > 0.f ? O / L : none;
-    if (d == 0)
-      global_ptr(p.ws_lse)[slot] = L > 0.f ? M * kLn2 + __logf(L) : none == 0.f ? -INFINITY : none;
+    const bool some = KEEP_NAN ? L != 0.f : L > 0.f;
+    global_ptr(p.ws_o)[slot * D + d] = some ? O / L : 0.f;
+    if (d == 0) global_ptr(p.ws_lse)[slot] = some ? M * kLn2 + __logf(L) : -INFINITY;
   }
 }
 
@@ -461,7 +461,7 @@ __device__ __forceinline__ const P& fresh_params() {
 // -> 35 us, 32 x 34k 366 -> 331 us (6.7 TB/s), 33k in one sequence 22.7 -> 20.4
 // us; 8 x 2k-9k at 14 / 2 x 64 16.2 -> 13.1 us.  The last three microseconds or
 // so of the short ones are the chain of latencies (record, block ids, keys).
-template <int D, typename T>
+template <int D, typename T, bool KEEP_NAN>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * DecShared<D>::W, 64 * DecShared<D>::W),
                           amdgpu_waves_per_eu(1, 1))) void
 decode_split_kernel(DecParams p) {
@@ -496,10 +496,10 @@ decode_split_kernel(DecParams p) {
     if (w.e.kv.block_table != 0) {
       w.e.kv.k_addr += p.kv_base;
       w.e.kv.v_addr += p.kv_base;
-      decode_split_body<D, T, true>(p, kvh, chunk, w.slot, w.e, w.key_begin, w.key_end, bufE, bufO,
+      decode_split_body<D, T, true, KEEP_NAN>(p, kvh, chunk, w.slot, w.e, w.key_begin, w.key_end, bufE, bufO,
                                     sm_m, sm_l);
     } else {
-      decode_split_body<D, T, false>(p, kvh, chunk, w.slot, w.e, w.key_begin, w.key_end, bufE,
+      decode_split_body<D, T, false, KEEP_NAN>(p, kvh, chunk, w.slot, w.e, w.key_begin, w.key_end, bufE,
                                      bufO, sm_m, sm_l);
     }
     if (w.next < 0) return;
@@ -539,7 +539,7 @@ __device__ __forceinline__ int64_t paged_len(const PagedDecParams& p, int r) {
 // same batch: 1 x 2000 keys 11.5 / 9.6 us, 16 x 1k-8k 34.6 / 32.6 us, 32 x 0.5k-8k
 // 60.2 / 60.6 us -- the two microseconds of the sums, for the 100 us a
 // step that reading the lengths, planning and the upload kept the GPU waiting.
-template <int D, typename T>
+template <int D, typename T, bool KEEP_NAN>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * DecShared<D>::W, 64 * DecShared<D>::W),
                           amdgpu_waves_per_eu(1, 1))) void
 decode_paged_kernel(PagedDecParams p_) {
@@ -654,7 +654,7 @@ decode_paged_kernel(PagedDecParams p_) {
     e.kv.start = all - len;  // the last `window` keys
     e.kv.len = len;
     const int64_t ke = static_cast<int64_t>(e_) * 32;
-    decode_split_body<D, T, true>(p.d, kvh, chunk, wg + r, e, static_cast<int64_t>(b) * 32,
+    decode_split_body<D, T, true, KEEP_NAN>(p.d, kvh, chunk, wg + r, e, static_cast<int64_t>(b) * 32,
                                   ke < len ? ke : len, bufE, bufO, sm_m, sm_l);
     __syncthreads();  // this split has been combined out of the buffers
   }
@@ -787,8 +787,11 @@ static hipError_t launch_dec_t(const DecParams& dp, const RedParams& rp, hipStre
   const int64_t grid =
       xcd_grid_size(static_cast<int64_t>(dp.num_wgs) * dp.head_chunks, dp.num_kv_heads);
   if (grid > 0) {
-    hipLaunchKernelGGL((decode_split_kernel<D, T>), dim3(static_cast<unsigned>(grid)),
-                       dim3(64 * DecShared<D>::W), 0, st, dp);
+    const dim3 g(static_cast<unsigned>(grid)), b(64 * DecShared<D>::W);
+    if (dp.keep_nan)
+      hipLaunchKernelGGL((decode_split_kernel<D, T, true>), g, b, 0, st, dp);
+    else
+      hipLaunchKernelGGL((decode_split_kernel<D, T, false>), g, b, 0, st, dp);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
@@ -823,8 +826,11 @@ static hipError_t launch_dec_paged_t(const PagedDecParams& p, const RedParams& r
                                      hipStream_t st) {
   const int64_t grid = xcd_grid_size(static_cast<int64_t>(p.d.num_wgs) * p.d.head_chunks,
                                      p.d.num_kv_heads);
-  hipLaunchKernelGGL((decode_paged_kernel<D, T>), dim3(static_cast<unsigned>(grid)),
-                     dim3(64 * DecShared<D>::W), 0, st, p);
+  const dim3 g(static_cast<unsigned>(grid)), b(64 * DecShared<D>::W);
+  if (p.d.keep_nan)
+    hipLaunchKernelGGL((decode_paged_kernel<D, T, true>), g, b, 0, st, p);
+  else
+    hipLaunchKernelGGL((decode_paged_kernel<D, T, false>), g, b, 0, st, p);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   RedParams r = rp;

@@ -100,7 +100,7 @@ struct DecParams {
   int32_t num_heads, num_kv_heads, group;
   int32_t head_chunks;  // ceil(group / 16): workgroups per (split, KV head)
   int32_t head_dim;     // valid elements per row (<= the kernel's width)
-  bool keep_nan;        // NaN scores make their row NaN (else their split is left out)
+  bool keep_nan;  // NaN scores make their row NaN (else their split is left out): picks the kernel
   float scale_log2;
 };
 
