@@ -116,7 +116,9 @@ __global__ __launch_bounds__(256) void fetch_metadata_kernel(MetaParams p) {
                 : static_cast<int64_t>(reinterpret_cast<const int32_t*>(a)[at]);
   };
   int64_t* const out = p.out + 1;
-  const int tid = threadIdx.x;
+  // one wave up to 63 requests (its barriers are free: 3.1 -> 2.8 us at 16
+  // requests), four for more
+  const int tid = threadIdx.x, nt = blockDim.x;
   bool plain = p.n <= kDecMaxSeqs;  // more never run without a plan
   auto request = [&](int i) {
     const int64_t start = get(p.qsl, p.qsl_wide, i * p.qsl_stride);
@@ -130,8 +132,8 @@ __global__ __launch_bounds__(256) void fetch_metadata_kernel(MetaParams p) {
   int64_t len[kDecMaxSeqs / 256];
 #pragma unroll
   for (int j = 0; j < kDecMaxSeqs / 256; ++j)
-    if (tid + 256 * j < p.n) len[j] = request(tid + 256 * j);
-  for (int i = tid + kDecMaxSeqs; i < p.n; i += 256) request(i);
+    if (tid + nt * j < p.n) len[j] = request(tid + nt * j);
+  for (int i = tid + kDecMaxSeqs; i < p.n; i += nt) request(i);
   if (tid == 0) {
     const int64_t end = get(p.qsl, p.qsl_wide, p.n * p.qsl_stride);
     out[p.n] = end;
@@ -149,14 +151,14 @@ __global__ __launch_bounds__(256) void fetch_metadata_kernel(MetaParams p) {
     };
 #pragma unroll
     for (int j = 0; j < kDecMaxSeqs / 256; ++j)
-      if (tid + 256 * j < p.n) keep(tid + 256 * j, len[j]);
-    for (int i = tid + kDecMaxSeqs; i < p.n; i += 256)
+      if (tid + nt * j < p.n) keep(tid + nt * j, len[j]);
+    for (int i = tid + kDecMaxSeqs; i < p.n; i += nt)
       keep(i, get(p.lens, p.lens_wide, i * p.lens_stride));
   }
 }
 
 hipError_t launch_fetch_metadata(const MetaParams& p, hipStream_t st) {
-  hipLaunchKernelGGL(fetch_metadata_kernel, dim3(1), dim3(256), 0, st, p);
+  hipLaunchKernelGGL(fetch_metadata_kernel, dim3(1), dim3(p.n < 64 ? 64 : 256), 0, st, p);
   return hipGetLastError();
 }
 
